@@ -18,6 +18,7 @@
 #include "obme_batch_kernels.h"
 #include "obme_internal.h"
 #include "obme_npd_kernels.h"
+#include "obme_wave_kernels.h"
 
 using namespace obme;
 
@@ -44,19 +45,6 @@ extern "C" const char* obme_last_error(void) { return g_last_error.c_str(); }
 extern "C" const char* obme_version(void) { return "obme 0.1.0 gfx950"; }
 
 // ------------------------------------------------------------------ kernels
-
-// The sweep: lane per water column, workgroups of blockDim.x = 64 NW
-// consecutive columns of one row (obme_npd_kernels.h).  FP32 is held to 128
-// VGPRs (4 waves per SIMD, the occupancy at which the 512x512 grid's 4096
-// waves fill the chip once).
-constexpr int SWEEP_MAX_THREADS = 512;
-template <int MODEL, int CARB, typename FT, int MODE, bool UNIFORM, int FM = -1, int EXTRA = 0, bool MASKX = true,
-          int SCHEME = OBME_UPWIND1>
-__global__ void __launch_bounds__(SWEEP_MAX_THREADS, (sizeof(FT) == 4 && (EXTRA & 2) == 0) ? 4 : 1)
-k_column_lane(StepArgs<FT> a)
-{
-    column_lane<MODEL, CARB, FT, MODE, UNIFORM, FM, EXTRA, MASKX, true, SCHEME>(a, (int)blockDim.x);
-}
 
 // The O2 gas exchange's per-column coefficients (GasExchange.jl:127-146):
 // k / Δz_top and the air-side concentration C_air α at the column's surface
@@ -180,16 +168,6 @@ __global__ void __launch_bounds__(256) k_sediment_state(StepArgs<FT> a, int s0, 
     a.sedG[col] = ge;
 }
 
-// The model's default formulations (fm_code): LOBSTER Mondo light,
-// quadratic mortality and grazing; NPZD analytical light, linear
-// mortality, quadratic grazing, Q10 on.  The FP32 fused step on full
-// columns is compiled for these with the choices folded in.
-template <int MODEL>
-constexpr int default_fm()
-{
-    return MODEL == OBME_LOBSTER ? (0 | (1 << 1) | (1 << 2)) : (1 | (0 << 1) | (1 << 2) | (1 << 3));
-}
-
 // CO2 flux and pH on n points (SoA, FP64).
 __global__ void __launch_bounds__(256) k_co2_flux(const double* __restrict__ DIC, const double* __restrict__ Alk,
                                                   const double* __restrict__ T, const double* __restrict__ S,
@@ -235,6 +213,11 @@ struct obme_handle {
     double* d_surfc = nullptr; // [SURF_PACK][surfc_cols] surface constants of the current stepper call
     int surfc_cols = 0;        // Nx*Ny, or 1 when the call's T and S are the same in every column
     bool surfc_ready = false;  // d_surfc holds the constants of this call's T and S
+    int srec_steps = 1;        // steps of surface records that d_srec holds
+    void* d_fast = nullptr;    // FP64: the transitions' constants (FastParams<double>)
+    void* d_toprec = nullptr;  // the top cells' records of k_top_steps (scaling with the CO2 flux)
+    int toprec_steps = 0;      // steps of them that d_toprec holds
+    bool default_forms = false;   // the model's default formulations (the FP32 kernels' compiled-in choices)
     int sink_idx[MAX_SINK];
     int sweep_waves;           // waves per workgroup of the sweep (1, 2, 4 or 8)
     bool uniform;
@@ -376,6 +359,8 @@ static obme_status upload_geometry(obme_handle* h)
             lev[LEV_DN * Nz + k] = (FT)(h->zf[Nz] - h->zc[Nz - 1]);
         }
         lev[LEV_INVDZ * Nz + k] = (FT)(1.0 / h->dz[k]);
+        lev[LEV_WR * Nz + k] = (FT)(0.5 * std::exp(h->cfg.par.water_red_attenuation * h->zc[k]));
+        lev[LEV_WB * Nz + k] = (FT)(0.5 * std::exp(h->cfg.par.water_blue_attenuation * h->zc[k]));
     }
     HIP_TRY(hipMalloc(&h->d_lev, lev.size() * sizeof(FT)));
     HIP_TRY(hipMemcpy(h->d_lev, lev.data(), lev.size() * sizeof(FT), hipMemcpyHostToDevice));
@@ -417,8 +402,7 @@ static obme_status upload_geometry(obme_handle* h)
 }
 
 // Waves per workgroup of the sweep: a workgroup covers 64 NW consecutive
-// columns of a row.  4 measured fastest on the 512x512x64 LOBSTER step;
-// obme_autotune times every choice.
+// columns.
 static const int SWEEP_WAVES[] = {1, 2, 4, 8};
 static const int N_SWEEP_WAVES = sizeof(SWEEP_WAVES) / sizeof(SWEEP_WAVES[0]);
 static bool valid_sweep_waves(int nw)
@@ -427,6 +411,39 @@ static bool valid_sweep_waves(int nw)
         if (SWEEP_WAVES[q] == nw) return true;
     return false;
 }
+
+// The default: the fewest waves on the fullest of the 256 CUs, and of those the
+// widest workgroup, whose waves walk in step and make longer runs per level.
+// (us per FP32 step of 64 levels with 1 | 2 | 4 | 8 waves: 512 x 512 278 | 266
+// | 257 | 247, 256 x 256 63 | 96 | 64 | 100; the hooks on 384 x 384 264 | 269 |
+// 286 | 320.)
+static int default_sweep_waves(size_t ncol)
+{
+    constexpr size_t CUS = 256;
+    int best = 8;
+    size_t least = (size_t)-1;
+    for (int nw = 8; nw >= 1; nw /= 2) {
+        const size_t groups = (ncol + 64 * nw - 1) / (64 * nw);
+        const size_t on_cu = (groups + CUS - 1) / CUS * nw;
+        if (on_cu < least) {
+            least = on_cu;
+            best = nw;
+        }
+    }
+    return best;
+}
+
+// Steps of per-column records of a launch that a handle keeps room for: as
+// many as fit RECORD_BYTES, 1 to WAVE_MAX_STEPS.
+constexpr size_t RECORD_BYTES = (size_t)128 << 20;
+constexpr int TOP_REC = 9;   // k_top_steps: three values per stage
+static int steps_within(size_t bytes, size_t per_step)
+{
+    return (int)std::max<size_t>(1, std::min<size_t>(WAVE_MAX_STEPS, bytes / std::max<size_t>(1, per_step)));
+}
+
+template <typename FT>
+static StepArgs<FT> make_args(const obme_handle* h, void* const* tracers);
 
 extern "C" obme_status obme_create(const obme_config* cfg, obme_handle** out)
 {
@@ -508,14 +525,25 @@ extern "C" obme_status obme_create(const obme_config* cfg, obme_handle** out)
         obme_destroy(h);
         return st;
     }
-    // a workgroup's waves walk in step, so wider workgroups make longer
-    // contiguous runs per level: the widest that a row fills
-    h->sweep_waves = g.Nx >= 512 ? 8 : g.Nx >= 256 ? 4 : g.Nx >= 128 ? 2 : 1;
+    if (h->prec == OBME_FP64) {
+        const FastParams<double> f = make_args<double>(h, nullptr).f;
+        if (hipMalloc(&h->d_fast, sizeof(f)) != hipSuccess ||
+            hipMemcpy(h->d_fast, &f, sizeof(f), hipMemcpyHostToDevice) != hipSuccess) {
+            obme_destroy(h);
+            return fail(OBME_ERR_NOMEM, "constants");
+        }
+    }
+    h->sweep_waves = default_sweep_waves((size_t)g.Nx * g.Ny);
     if (const char* e = std::getenv("OBME_SWEEP_WAVES")) {
         const int nw = std::atoi(e);
         if (valid_sweep_waves(nw)) h->sweep_waves = nw;
     }
     h->scaling = cfg->scaling.n_groups > 0;
+    {
+        const FastParams<float> f = make_fast_params<float>(cfg->npd);
+        h->default_forms =
+            fm_code(f) == (cfg->model == OBME_NPZD ? default_fm<OBME_NPZD>() : default_fm<OBME_LOBSTER>());
+    }
     h->scheme = cfg->sinking.scheme;
     h->staged = h->scheme != OBME_UPWIND1;
     h->co2_inline = h->scaling && cfg->model == OBME_LOBSTER && cfg->carbonate_system && cfg->co2.enabled;
@@ -528,7 +556,16 @@ extern "C" obme_status obme_create(const obme_config* cfg, obme_handle** out)
     if (cfg->model == OBME_LOBSTER && cfg->carbonate_system && cfg->co2.enabled) {
         size_t ncol = (size_t)g.Nx * g.Ny;
         size_t es = (h->prec == OBME_FP64) ? 8 : 4;
-        hipError_t e1 = hipMalloc(&h->d_srec, SURF_REC * ncol * es);
+        // the records of several steps, for the launches that take several
+        h->srec_steps = h->co2_inline ? 1 : steps_within(RECORD_BYTES, SURF_REC * ncol * es);
+        hipError_t e1 = hipMalloc(&h->d_srec, h->srec_steps * SURF_REC * ncol * es);
+        if (h->co2_inline) {
+            h->toprec_steps = steps_within(RECORD_BYTES, TOP_REC * ncol * es);
+            if (hipMalloc(&h->d_toprec, h->toprec_steps * TOP_REC * ncol * es) != hipSuccess) {
+                obme_destroy(h);
+                return fail(OBME_ERR_NOMEM, "top-cell records");
+            }
+        }
         hipError_t e2 = hipMalloc((void**)&h->d_Hprev, ncol * sizeof(double));
         hipError_t e3 = (h->prec == OBME_FP64) ? hipSuccess : hipMalloc((void**)&h->d_topres, 2 * ncol * sizeof(float));
         if (e1 != hipSuccess || e2 != hipSuccess || e3 != hipSuccess) {
@@ -565,6 +602,8 @@ extern "C" obme_status obme_destroy(obme_handle* h)
     if (h->d_Tprof) (void)hipFree(h->d_Tprof);
     if (h->d_Sprof) (void)hipFree(h->d_Sprof);
     if (h->d_srec) (void)hipFree(h->d_srec);
+    if (h->d_toprec) (void)hipFree(h->d_toprec);
+    if (h->d_fast) (void)hipFree(h->d_fast);
     if (h->d_Hprev) (void)hipFree(h->d_Hprev);
     if (h->d_topres) (void)hipFree(h->d_topres);
     if (h->d_o2c) (void)hipFree(h->d_o2c);
@@ -600,6 +639,7 @@ extern "C" int32_t obme_required_tracers(const obme_handle* h, char* buf, int32_
 
 // the sweep takes its arguments by value: within the 4 KiB kernel-argument limit
 static_assert(sizeof(StepArgs<double>) <= 4096 && sizeof(StepArgs<float>) <= 4096, "StepArgs exceeds 4 KiB");
+static_assert(sizeof(WaveArgs<double>) <= 4088 && sizeof(WaveArgs<float>) <= 4088, "WaveArgs exceeds 4 KiB");
 
 template <typename FT>
 static StepArgs<FT> make_args(const obme_handle* h, void* const* tracers)
@@ -618,10 +658,15 @@ static StepArgs<FT> make_args(const obme_handle* h, void* const* tracers)
     a.sxy = a.sx * (unsigned)(g.Ny + 2 * g.Hy);
     a.base0 = (unsigned)g.Hx + a.sx * (unsigned)g.Hy + a.sxy * (unsigned)g.Hz;
     a.field_bytes = (unsigned)((size_t)a.sxy * (size_t)(g.Nz + 2 * g.Hz) * sizeof(FT));
-    a.q = convert_params<FT>(c.npd);
-    if (c.oxygen.enabled) {
-        a.q.Rp = (FT)c.oxygen.respiration_oxygen_nitrogen_ratio;
-        a.q.Rn = (FT)c.oxygen.nitrification_oxygen_nitrogen_ratio;
+    a.f = c.oxygen.enabled ? make_fast_params<FT>(c.npd, c.oxygen.respiration_oxygen_nitrogen_ratio,
+                                                  c.oxygen.nitrification_oxygen_nitrogen_ratio)
+                           : make_fast_params<FT>(c.npd);
+    if (sizeof(FT) == 4 && h->sediment) {
+        a.fs = make_sediment_params(c.npd);
+        if (c.oxygen.enabled) {
+            a.fs.oRp = (float)c.oxygen.respiration_oxygen_nitrogen_ratio;
+            a.fs.oRpn = (float)(c.oxygen.respiration_oxygen_nitrogen_ratio - c.oxygen.nitrification_oxygen_nitrogen_ratio);
+        }
     }
     a.kr = (FT)c.par.water_red_attenuation;
     a.kb = (FT)c.par.water_blue_attenuation;
@@ -697,11 +742,6 @@ static StepArgs<FT> make_args(const obme_handle* h, void* const* tracers)
         }
     }
     if (sizeof(FT) == 4) {
-        a.f = make_fast_params(c.npd);
-        if (c.oxygen.enabled) {
-            a.f.oRp = (float)c.oxygen.respiration_oxygen_nitrogen_ratio;
-            a.f.oRpn = (float)(c.oxygen.respiration_oxygen_nitrogen_ratio - c.oxygen.nitrification_oxygen_nitrogen_ratio);
-        }
         const double log2e = 1.4426950408889634;
         a.kr2 = (float)(c.par.water_red_attenuation * log2e);
         a.kb2 = (float)(c.par.water_blue_attenuation * log2e);
@@ -751,6 +791,7 @@ static SurfaceArgs<FT> make_surface_args(const obme_handle* h, void* const* trac
     s.sxy = s.sx * (unsigned)(g.Ny + 2 * g.Hy);
     s.base0 = (unsigned)g.Hx + s.sx * (unsigned)g.Hy + s.sxy * (unsigned)g.Hz;
     s.invdz_top = (FT)(1.0 / h->dz[g.Nz - 1]);
+    s.nsteps = 1;
     // both precisions: Newton warm-started from the column's previous [H+]
     // (FP32 to FP32_NEWTON_TOL, FP64 to a 1e-14 relative step), the
     // reference's damped Newton as the fallback
@@ -764,68 +805,13 @@ template <int MODEL, int CARB, typename FT, int MODE>
 static obme_status launch_lane(obme_handle* h, const StepArgs<FT>& a, hipStream_t s)
 {
     const int cw = 64 * h->sweep_waves;
-    // one-dimensional: tile = xcd_tile(blockIdx.x), row-major over (i tile, j)
-    const unsigned n_tiles = (unsigned)(((h->cfg.grid.Nx + cw - 1) / cw) * h->cfg.grid.Ny);
-    using Kernel = void (*)(StepArgs<FT>);
-    Kernel k = nullptr;
-    if constexpr (MODE == TILE_STAGE) {
-        // centred / WENO sinking, one stage per launch (the general-grid form)
-        k = (h->scheme == OBME_WENO5) ? k_column_lane<MODEL, CARB, FT, MODE, false, -1, 0, true, OBME_WENO5>
-                                      : k_column_lane<MODEL, CARB, FT, MODE, false, -1, 0, true, OBME_CENTERED2>;
-    } else {
-        k = h->uniform ? k_column_lane<MODEL, CARB, FT, MODE, true> : k_column_lane<MODEL, CARB, FT, MODE, false>;
-    }
-    // rows of whole workgroups (Nx a multiple of 64 NW): stores without a
-    // mask; the FP32 step and tendencies compiled with the model's default
-    // formulations
-    const bool whole = h->cfg.grid.Nx % cw == 0;
-    if constexpr (MODE == TILE_TENDENCY) {
-        if (h->scheme == OBME_WENO5) {
-            k = k_column_lane<MODEL, CARB, FT, MODE, false, -1, 0, true, OBME_WENO5>;
-        } else if (h->scheme == OBME_CENTERED2) {
-            k = k_column_lane<MODEL, CARB, FT, MODE, false, -1, 0, true, OBME_CENTERED2>;
-        } else if (whole && h->uniform) {
-            if constexpr (sizeof(FT) == 4) {
-                if (fm_code(a.f) == default_fm<MODEL>())
-                    k = k_column_lane<MODEL, CARB, FT, MODE, true, default_fm<MODEL>(), 0, false>;
-            } else {
-                k = k_column_lane<MODEL, CARB, FT, MODE, true, -1, 0, false>;
-            }
-        }
-    }
-    if constexpr (MODE == TILE_PAR) {
-        if (whole && h->uniform) k = k_column_lane<MODEL, CARB, FT, MODE, true, -1, 0, false>;
-    }
-    if constexpr (MODE == TILE_STEP) {
-        if constexpr (sizeof(FT) == 4) {
-            if (fm_code(a.f) == default_fm<MODEL>()) {
-                constexpr int FM = default_fm<MODEL>();
-                k = whole ? (h->uniform ? k_column_lane<MODEL, CARB, FT, MODE, true, FM, 0, false>
-                                        : k_column_lane<MODEL, CARB, FT, MODE, false, FM, 0, false>)
-                          : (h->uniform ? k_column_lane<MODEL, CARB, FT, MODE, true, FM>
-                                        : k_column_lane<MODEL, CARB, FT, MODE, false, FM>);
-            }
-        } else if (whole) {
-            k = h->uniform ? k_column_lane<MODEL, CARB, FT, MODE, true, -1, 0, false>
-                           : k_column_lane<MODEL, CARB, FT, MODE, false, -1, 0, false>;
-        }
-    }
-    if constexpr (MODE == TILE_STEP) {
-        // negative scaling (1), the inline CO2 flux (2, with 1) and the
-        // sediment (4) in the fused step, with the extra work compiled in
-        const int ex = (h->scaling ? 1 : 0) | (h->co2_inline ? 2 : 0) | (h->sediment ? 4 : 0);
-#define OBME_EXTRA_KERNEL(E)                                                               \
-    (h->uniform ? k_column_lane<MODEL, CARB, FT, MODE, true, -1, E>                       \
-                : k_column_lane<MODEL, CARB, FT, MODE, false, -1, E>)
-        if (ex == 1) k = OBME_EXTRA_KERNEL(1);
-        if (ex == 4) k = OBME_EXTRA_KERNEL(4);
-        if (ex == 5) k = OBME_EXTRA_KERNEL(5);
-        if constexpr ((CARB & 1) != 0) {
-            if (ex == 3) k = OBME_EXTRA_KERNEL(3);
-            if (ex == 7) k = OBME_EXTRA_KERNEL(7);
-        }
-#undef OBME_EXTRA_KERNEL
-    }
+    const size_t ncol = (size_t)h->cfg.grid.Nx * h->cfg.grid.Ny;
+    const unsigned n_tiles = (unsigned)((ncol + cw - 1) / cw);
+    // negative scaling (1), the inline CO2 flux (2, with 1) and the sediment
+    // (4) in the fused step, with the extra work compiled in
+    const int extra = (h->scaling ? 1 : 0) | (h->co2_inline ? 2 : 0) | (h->sediment ? 4 : 0);
+    LaneKernel<FT> k = lane_kernel<MODEL, CARB, FT>(MODE, h->uniform, ncol % cw == 0, h->default_forms,
+                                                    h->scheme, extra);
     LaunchTimer tm(h, OBME_KERNEL_SWEEP, s);
     hipLaunchKernelGGL(k, dim3(n_tiles), dim3(cw), 0, s, a);
     tm.done();
@@ -847,6 +833,115 @@ static obme_status dispatch_model(obme_handle* h, const StepArgs<FT>& a, hipStre
     return launch_lane<OBME_LOBSTER, 0, FT, MODE>(h, a, s);
 }
 
+// The levels-along-the-lanes kernels (obme_wave_kernels.h): levels per lane,
+// lanes per column, columns per wave and waves per workgroup of a launch;
+// levels 0 where the column sweep serves.
+struct WaveShape {
+    int levels = 0, lpc = 0, cpw = 0, nw = 0;
+};
+
+template <typename FT>
+static WaveShape wave_shape(const obme_handle* h, int mode, int nsteps, bool general)
+{
+    WaveShape best;
+    const int Nz = h->cfg.grid.Nz;
+    const long ncol = (long)h->cfg.grid.Nx * h->cfg.grid.Ny;
+    if (Nz < 2 || !h->default_forms) return best;
+    // (FP32 takes the logarithm of the chlorophyll attenuation)
+    if (sizeof(FT) == 4 && !(h->cfg.par.chlorophyll_red_attenuation >= 0 && h->cfg.par.chlorophyll_blue_attenuation >= 0))
+        return best;
+    if (mode == TILE_STEP && h->sediment) {
+        if (h->cfg.sediment.model == OBME_SEDIMENT_SIMPLE_MULTI_G) return best;
+        // NPZD's sinking P takes the light's rounding into the FP64 storage
+        // (obme_sediment_order.h): FP32 keeps the sweep's running sums there
+        if (sizeof(FT) == 4 && h->cfg.model == OBME_NPZD) return best;
+    }
+    // One step or a hook: the sweep moves a level's values in longer runs and
+    // is the faster where its columns fill the chip.  On 64 levels, us per
+    // step, sweep | this: FP32 16 384 columns 59 | 26, 65 536 64 | 81; FP64
+    // 180 | 65, 197 | 247; FP32 hooks 57 | 35, 110 | 158.  From two steps on,
+    // with the state in registers between them, this is the faster everywhere
+    // (262 144 columns, two steps: 507 | 486).  The centred and WENO steps and
+    // the scaling and sediment variants are: a launch per stage and the flux
+    // solve in the walk are what they replace.
+    if (ncol > 40960 && (mode != TILE_STEP || (nsteps < 2 && !general && !h->staged))) return best;
+    double cost = 0.0;
+    for (int i = 0; i < 4 && wave_levels<FT>(i); i++) {
+        const int L = wave_levels<FT>(i);
+        if (L > 2 && (mode != TILE_STEP || general || h->staged)) continue;
+        const int lpc = (Nz + L - 1) / L;
+        if (lpc > 64) continue;
+        const int cpw = 64 / lpc;
+        const double waves = (double)((ncol + cpw - 1) / cpw);
+        // a wave's time goes with its levels per lane (FP64: and half a level
+        // for the prefix sums' double moves), down to two waves per SIMD
+        const double c = (L + (sizeof(FT) == 8 ? 0.5 : 0.0)) * std::max(waves, 2048.0);
+        if (!best.levels || c < cost) {
+            cost = c;
+            best.levels = L;
+            best.lpc = lpc;
+            best.cpw = cpw;
+        }
+    }
+    if (!best.levels) return best;
+    // workgroups of eight waves, fewer where that leaves CUs without one
+    best.nw = 8;
+    const int es = (int)sizeof(FT);
+    while (best.nw > 1 && ((ncol + best.nw * best.cpw - 1) / (best.nw * best.cpw) < 512 ||
+                           (h->ntracers + 1) * best.nw * 64 * best.levels * es > 48 * 1024))
+        best.nw /= 2;
+    return best;
+}
+
+template <int MODEL, int CARB, typename FT>
+static WaveKernel<FT> pick_wave(const obme_handle* h, int mode, const WaveShape& ws, bool general)
+{
+    return wave_kernel<MODEL, CARB, FT>(mode, h->uniform, ws.levels, ws.lpc, general, h->staged);
+}
+
+template <typename FT>
+static WaveKernel<FT> pick_wave_model(const obme_handle* h, int mode, const WaveShape& ws, bool general)
+{
+    const int carb = (h->cfg.carbonate_system ? 1 : 0) | (h->cfg.oxygen.enabled ? 2 : 0);
+    if (h->cfg.model == OBME_NPZD)
+        return carb ? pick_wave<OBME_NPZD, 2, FT>(h, mode, ws, general) : pick_wave<OBME_NPZD, 0, FT>(h, mode, ws, general);
+    if (carb == 3) return pick_wave<OBME_LOBSTER, 3, FT>(h, mode, ws, general);
+    if (carb == 2) return pick_wave<OBME_LOBSTER, 2, FT>(h, mode, ws, general);
+    if (carb == 1) return pick_wave<OBME_LOBSTER, 1, FT>(h, mode, ws, general);
+    return pick_wave<OBME_LOBSTER, 0, FT>(h, mode, ws, general);
+}
+
+// FP32: the constants of the light's chlorophyll powers, with the attenuation
+// in powers of 2 and, for the uniform-grid kernel, the half cell.
+template <typename FT>
+static void wave_light(const obme_handle* h, bool uniform, WaveArgs<FT>& w)
+{
+    const obme_two_band_par& p = h->cfg.par;
+    const double scale = 1.4426950408889634 * (uniform ? h->dz_u / 2 : 1.0);
+    const double lRr = std::log2(p.phytoplankton_chlorophyll_ratio / p.pigment_ratio);
+    w.cr = (float)(p.chlorophyll_red_exponent * lRr + std::log2(p.chlorophyll_red_attenuation * scale));
+    w.cb = (float)(p.chlorophyll_blue_exponent * lRr + std::log2(p.chlorophyll_blue_attenuation * scale));
+}
+
+template <typename FT>
+static obme_status launch_wave(obme_handle* h, const WaveShape& ws, WaveArgs<FT>& w, int mode, bool general, hipStream_t s)
+{
+    WaveKernel<FT> k = pick_wave_model<FT>(h, mode, ws, general);
+    if (!k) return fail(OBME_ERR_UNSUPPORTED, "no kernel of this shape");
+    w.lpc = ws.lpc;
+    w.cpw = ws.cpw;
+    w.fpar = (const FastParams<FT>*)h->d_fast;
+    w.ncol = (unsigned)((size_t)h->cfg.grid.Nx * h->cfg.grid.Ny);
+    const unsigned per_wg = (unsigned)(ws.nw * ws.cpw);
+    const size_t bytes = (size_t)(h->ntracers + 1) * ws.nw * 64 * ws.levels * sizeof(FT) +
+                         (sizeof(FT) == 8 ? sizeof(FastParams<FT>) : 0);
+    LaunchTimer tm(h, OBME_KERNEL_SWEEP, s);
+    hipLaunchKernelGGL(k, dim3((w.ncol + per_wg - 1) / per_wg), dim3(64 * ws.nw), bytes, s, w);
+    tm.done();
+    HIP_TRY(hipGetLastError());
+    return OBME_OK;
+}
+
 template <typename FT, int MODE>
 static obme_status launch_surface(obme_handle* h, const SurfaceArgs<FT>& sa, hipStream_t s)
 {
@@ -857,6 +952,42 @@ static obme_status launch_surface(obme_handle* h, const SurfaceArgs<FT>& sa, hip
     tm.done();
     HIP_TRY(hipGetLastError());
     return OBME_OK;
+}
+
+// The O2 exchange coefficients of the call's surface T and S.
+template <typename FT>
+static obme_status prepare_o2(obme_handle* h, const StepArgs<FT>& a, hipStream_t s)
+{
+    const long ncol = (long)h->cfg.grid.Nx * h->cfg.grid.Ny;
+    hipLaunchKernelGGL(k_o2_prep<FT>, dim3((unsigned)((ncol + 255) / 256)), dim3(256), 0, s, a, h->cfg.o2,
+                       1.0 / h->dz[h->cfg.grid.Nz - 1], h->d_o2c);
+    HIP_TRY(hipGetLastError());
+    return OBME_OK;
+}
+
+// default_surface_PAR (Light/Light.jl:219) at time t, and the stage clocks
+static const double STAGE_CLOCK[3] = {0.0, 8.0 / 15.0, 8.0 / 15.0 + 5.0 / 12.0 - 17.0 / 60.0};
+static double surface_daylight(double t)
+{
+    const double cv = std::cos(t * 3.141592653589793 / (12 * 3600.0));
+    const double d = 0.0 - cv;  // Julia max(0, cos): NaN propagates, ±0 ordered
+    return 100 * (std::isnan(cv) ? d : (std::signbit(d) ? cv : 0.0));
+}
+
+// The sediment's stepping of the steps from here on, in the launch's
+// arguments: the sediment steps after the three stages take Δt γ1,
+// Δt (γ2 + ζ2), Δt (γ3 + ζ3) (the stage Δt of Oceananigans' RK3, its clock's
+// last_stage_Δt); an AB2 step only where a step's Δt repeats the previous one,
+// which within a step never happens.
+template <typename FT>
+static void sediment_args(const obme_handle* h, double dt, double* storage, StepArgs<FT>& a)
+{
+    a.storage = storage;
+    a.sed_dt[0] = (8.0 / 15.0) * dt;
+    a.sed_dt[1] = (5.0 / 12.0 + -17.0 / 60.0) * dt;
+    a.sed_dt[2] = (3.0 / 4.0 + -5.0 / 12.0) * dt;
+    a.sed_init = h->sed_iter == 0 ? 1 : 0;
+    a.sed_ab2 = (!a.sed_init && a.sed_dt[0] == h->sed_last_dt) ? 1 : 0;
 }
 
 template <typename FT, int MODE>
@@ -870,14 +1001,7 @@ static obme_status run_typed(obme_handle* h, void* const* tracers, void* const* 
     rk3_products(dt, a.rk_a, a.rk_b);
     if (h->cfg.par.surface_mode == OBME_SURFACE_DIURNAL) {
         // default_surface_PAR (Light/Light.jl:219) at the stage clocks
-        const double cst[3] = {0.0, 8.0 / 15.0, 8.0 / 15.0 + 5.0 / 12.0 - 17.0 / 60.0};
-        for (int q = 0; q < 3; q++) {
-            double tq = t + cst[q] * dt;
-            double cv = std::cos(tq * 3.141592653589793 / (12 * 3600.0));
-            double d = 0.0 - cv;  // Julia max(0, cos): NaN propagates, ±0 ordered
-            double v = std::isnan(cv) ? d : (std::signbit(d) ? cv : 0.0);
-            a.PAR0_stage[q] = (FT)(100 * v);
-        }
+        for (int q = 0; q < 3; q++) a.PAR0_stage[q] = (FT)surface_daylight(t + STAGE_CLOCK[q] * dt);
     }
     if (MODE != TILE_STEP) {
         // the hooks: the flux by the surface kernel in tendency mode
@@ -903,10 +1027,8 @@ static obme_status run_typed(obme_handle* h, void* const* tracers, void* const* 
     if (MODE != TILE_PAR && a.o2_on && !h->o2c_ready) {
         // the O2 exchange coefficients of this call's surface T and S (once
         // per obme_step call, which sets o2c_ready around its steps)
-        const long ncol = (long)h->cfg.grid.Nx * h->cfg.grid.Ny;
-        hipLaunchKernelGGL(k_o2_prep<FT>, dim3((unsigned)((ncol + 255) / 256)), dim3(256), 0, s, a, h->cfg.o2,
-                           1.0 / h->dz[h->cfg.grid.Nz - 1], h->d_o2c);
-        HIP_TRY(hipGetLastError());
+        obme_status r = prepare_o2<FT>(h, a, s);
+        if (r != OBME_OK) return r;
         if (MODE == TILE_STEP) h->o2c_ready = true;
     }
     if (MODE == TILE_PAR && h->scaling) {
@@ -922,20 +1044,7 @@ static obme_status run_typed(obme_handle* h, void* const* tracers, void* const* 
         hipLaunchKernelGGL(ks, dim3((unsigned)((ncell + bs - 1) / bs)), dim3(bs), 0, s, a);
         HIP_TRY(hipGetLastError());
     }
-    double sed_last = 0.0;
-    if (MODE == TILE_STEP && h->sediment) {
-        // the sediment steps after the three stages: Δt γ1, Δt (γ2 + ζ2),
-        // Δt (γ3 + ζ3) (the stage Δt of Oceananigans' RK3, its clock's
-        // last_stage_Δt); an AB2 step only where a step's Δt repeats the
-        // previous one, which within a step never happens
-        a.storage = storage;
-        a.sed_dt[0] = (8.0 / 15.0) * dt;
-        a.sed_dt[1] = (5.0 / 12.0 + -17.0 / 60.0) * dt;
-        a.sed_dt[2] = (3.0 / 4.0 + -5.0 / 12.0) * dt;
-        a.sed_init = h->sed_iter == 0 ? 1 : 0;
-        a.sed_ab2 = (!a.sed_init && a.sed_dt[0] == h->sed_last_dt) ? 1 : 0;
-        sed_last = a.sed_dt[2];
-    }
+    if (MODE == TILE_STEP && h->sediment) sediment_args(h, dt, storage, a);
     if constexpr (MODE == TILE_STAGE) {
         if (a.co2_stage) {
             // the stage's top-cell CO2 flux per column, from the stage's inputs
@@ -953,10 +1062,24 @@ static obme_status run_typed(obme_handle* h, void* const* tracers, void* const* 
             if (rs != OBME_OK) return rs;
         }
     }
-    obme_status r = dispatch_model<FT, MODE>(h, a, s);
+    obme_status r = OBME_OK;
+    WaveShape ws;
+    if constexpr (MODE == TILE_TENDENCY || MODE == TILE_PAR) ws = wave_shape<FT>(h, MODE, 1, false);
+    if (ws.levels) {
+        WaveArgs<FT> w;
+        std::memset(&w, 0, sizeof(w));
+        w.a = a;
+        wave_light<FT>(h, false, w);
+        w.nsteps = 1;
+        w.scheme = h->scheme;
+        w.PAR0s[0][0] = a.surface_mode == OBME_SURFACE_DIURNAL ? a.PAR0_stage[0] : a.surface_value;
+        r = launch_wave<FT>(h, ws, w, MODE, false, s);
+    } else {
+        r = dispatch_model<FT, MODE>(h, a, s);
+    }
     if (r == OBME_OK && MODE == TILE_STEP && h->sediment) {
         h->sed_iter += 3;
-        h->sed_last_dt = sed_last;
+        h->sed_last_dt = a.sed_dt[2];
     }
     if (r == OBME_OK && MODE == TILE_TENDENCY && h->sediment) {
         const unsigned ncol = (unsigned)(h->cfg.grid.Nx * h->cfg.grid.Ny);
@@ -975,6 +1098,78 @@ static obme_status run_typed(obme_handle* h, void* const* tracers, void* const* 
     rk3_products(dt, sa.rk_a, sa.rk_b);
     if (MODE == TILE_TENDENCY) sa.GDIC = (FT*)G[7];
     return launch_surface<FT, MODE>(h, sa, s);
+}
+
+// nsteps steps by the levels-along-the-lanes kernels, several per launch.
+template <typename FT>
+static obme_status run_wave_steps(obme_handle* h, const WaveShape& ws, void* const* tracers, const void* T, const void* S,
+                                  double* storage, int nsteps, double t0, double dt, hipStream_t s)
+{
+    WaveArgs<FT> w;
+    std::memset(&w, 0, sizeof(w));
+    w.a = make_args<FT>(h, tracers);
+    StepArgs<FT>& a = w.a;
+    a.dtf = (FT)dt;
+    rk3_products(dt, a.rk_a, a.rk_b);
+    w.rk_c[0] = (float)(dt * (8.0 / 15.0 - 17.0 / 60.0));
+    w.rk_c[1] = (float)(dt * (5.0 / 12.0 - 5.0 / 12.0));
+    a.T3 = (const FT*)T;
+    a.S3 = (const FT*)S;
+    a.topres = a.co2_on ? h->d_topres : nullptr;
+    w.scale = h->scaling;
+    w.sed = h->sediment;
+    w.scheme = h->scheme;
+    const bool general = h->scaling || h->sediment;
+    const bool uniform = h->uniform && !h->staged;
+    wave_light<FT>(h, uniform, w);
+    w.uniform = uniform;
+    if (a.o2_on) {
+        obme_status r = prepare_o2<FT>(h, a, s);
+        if (r != OBME_OK) return r;
+    }
+    int chunk = WAVE_MAX_STEPS;
+    if (a.co2_on) chunk = std::min(chunk, h->srec_steps);
+    if (h->co2_inline) chunk = std::min(chunk, h->toprec_steps);
+    for (int s0 = 0; s0 < nsteps; s0 += chunk) {
+        w.nsteps = std::min(chunk, nsteps - s0);
+        for (int q = 0; q < w.nsteps; q++)
+            for (int st = 0; st < 3; st++)
+                w.PAR0s[q][st] = a.surface_mode == OBME_SURFACE_DIURNAL
+                                     ? (FT)surface_daylight(t0 + (s0 + q) * dt + STAGE_CLOCK[st] * dt)
+                                     : a.surface_value;
+        if (h->sediment) sediment_args(h, dt, storage, a);
+        if (h->co2_inline) {
+            const unsigned ncol = (unsigned)((size_t)h->cfg.grid.Nx * h->cfg.grid.Ny);
+            w.ncol = ncol;
+            w.toprec = nullptr;
+            w.fpar = (const FastParams<FT>*)h->d_fast;
+            auto k = h->cfg.oxygen.enabled ? top_kernel<3, FT>() : top_kernel<1, FT>();
+            LaunchTimer tm(h, OBME_KERNEL_SURFACE, s);
+            hipLaunchKernelGGL(k, dim3((ncol + 63) / 64), dim3(64), 0, s, w, (FT*)h->d_toprec);
+            tm.done();
+            HIP_TRY(hipGetLastError());
+            w.toprec = (const FT*)h->d_toprec;
+        }
+        obme_status r = launch_wave<FT>(h, ws, w, TILE_STEP, general, s);
+        if (r != OBME_OK) return r;
+        if (h->sediment) {
+            h->sed_iter += 3 * (long long)w.nsteps;
+            h->sed_last_dt = a.sed_dt[2];
+        }
+        if (!a.co2_on) continue;
+        SurfaceArgs<FT> sa = make_surface_args<FT>(h, tracers, T, S);
+        if (h->surfc_ready) {
+            sa.surfc = h->d_surfc;
+            sa.surfc_cols = h->surfc_cols;
+        }
+        sa.topres = a.topres;
+        sa.dtf = (FT)dt;
+        rk3_products(dt, sa.rk_a, sa.rk_b);
+        sa.nsteps = w.nsteps;
+        r = launch_surface<FT, TILE_STEP>(h, sa, s);
+        if (r != OBME_OK) return r;
+    }
+    return OBME_OK;
 }
 
 template <int MODE>
@@ -1071,6 +1266,18 @@ extern "C" obme_status obme_step_with_sediment(obme_handle* h, void* const* trac
     }
     obme_status r = OBME_OK;
     h->o2c_ready = false;
+    {
+        const bool general = h->scaling || h->sediment;
+        const bool f64 = h->prec == OBME_FP64;
+        const WaveShape ws = f64 ? wave_shape<double>(h, TILE_STEP, nsteps, general)
+                                 : wave_shape<float>(h, TILE_STEP, nsteps, general);
+        if (ws.levels && nsteps > 0 && (!h->co2_inline || h->toprec_steps > 0)) {
+            r = f64 ? run_wave_steps<double>(h, ws, tracers, T, S, storage, nsteps, t0, dt, s)
+                    : run_wave_steps<float>(h, ws, tracers, T, S, storage, nsteps, t0, dt, s);
+            h->surfc_ready = false;
+            return r;
+        }
+    }
     if (h->staged && nsteps > 0) {
         // centred / WENO sinking: each stage's face values need the stage
         // inputs of the levels below, so a step is three launches of one stage
@@ -1181,24 +1388,29 @@ extern "C" obme_status obme_step_noalloc(obme_handle* h, void* const* tracers, c
     struct Swap {
         obme_handle* h;
         void* srec;
+        int srec_steps;
         double *hprev, *surfc, *o2c;
         float* topres;
         bool timing;
         ~Swap()
         {
             h->d_srec = srec;
+            h->srec_steps = srec_steps;
             h->d_Hprev = hprev;
             h->d_surfc = surfc;
             h->d_o2c = o2c;
             h->d_topres = topres;
             h->timing = timing;
         }
-    } keep{h, h->d_srec, h->d_Hprev, h->d_surfc, h->d_o2c, h->d_topres, h->timing};
+    } keep{h, h->d_srec, h->srec_steps, h->d_Hprev, h->d_surfc, h->d_o2c, h->d_topres, h->timing};
     h->timing = false;
+    // (the records of one step are part of the limit; more steps of them take
+    // what the static array has left, at its end)
+    if (co2)
+        h->srec_steps = 1 + (int)std::min<size_t>(WAVE_MAX_STEPS - 1,
+                                                  (NOALLOC_SCRATCH_BYTES - need) / (SURF_REC * ncol * es));
     size_t off = 0;
     if (co2) {
-        h->d_srec = base + off;
-        off += b_srec;
         h->d_Hprev = (double*)(base + off);
         off += b_hprev;
         h->d_surfc = (double*)(base + off);
@@ -1214,6 +1426,8 @@ extern "C" obme_status obme_step_noalloc(obme_handle* h, void* const* tracers, c
     }
     // (obme_step_with_sediment clears the residuals)
     h->d_topres = b_topres ? (float*)(base + off) : nullptr;
+    off += b_topres;
+    if (co2) h->d_srec = base + off;
     return obme_step_with_sediment(h, tracers, T, S, nullptr, nsteps, dt, t0, s);
 }
 
@@ -1430,8 +1644,8 @@ struct obme_batch {
     std::vector<int> offsets;
     double dz, T;
     int* d_offsets = nullptr;
-    FastParams* d_fpar = nullptr;
-    NPDParams<double>* d_dpar = nullptr;
+    void* d_fpar = nullptr;               // per-column derived constants, FastParams of the element type
+    SedimentParams* d_fsed = nullptr;     // FP32 with a sediment: its transitions' constants
     BatchColumn* d_bcol = nullptr;
     float* d_comp = nullptr;              // FP32: the residual arrays, 4 x offsets[n_columns]
     int plan = -1;
@@ -1513,8 +1727,8 @@ static BatchArgs<FT> batch_args(const obme_batch* b, void* const* tracers, doubl
     std::memset(&a, 0, sizeof(a));
     for (int n = 0; n < 4; n++) a.U[n] = (FT*)tracers[n];
     a.offsets = b->d_offsets;
-    a.fpar = b->d_fpar;
-    a.dpar = b->d_dpar;
+    a.fpar = (const FastParams<FT>*)b->d_fpar;
+    a.fsed = (const SedimentParams*)b->d_fsed;
     a.bcol = b->d_bcol;
     a.dtf = (FT)dt;
     a.dz = (FT)b->dz;
@@ -1648,7 +1862,7 @@ extern "C" obme_status obme_batch_destroy(obme_batch* b)
     if (b->cap_stream) (void)hipStreamDestroy(b->cap_stream);
     if (b->d_offsets) (void)hipFree(b->d_offsets);
     if (b->d_fpar) (void)hipFree(b->d_fpar);
-    if (b->d_dpar) (void)hipFree(b->d_dpar);
+    if (b->d_fsed) (void)hipFree(b->d_fsed);
     if (b->d_bcol) (void)hipFree(b->d_bcol);
     if (b->d_comp) (void)hipFree(b->d_comp);
     if (b->d_sedGm) (void)hipFree(b->d_sedGm);
@@ -1719,8 +1933,11 @@ extern "C" obme_status obme_batch_create(const obme_config* cfg, int32_t n_colum
             return fail(OBME_ERR_HIP, "reading the per-column parameters");
         }
     }
-    std::vector<FastParams> fpar(n_columns);
-    std::vector<NPDParams<double>> dpar(n_columns);
+    const bool f64 = b->prec == OBME_FP64;
+    std::vector<FastParams<float>> fpar(f64 ? 0 : n_columns);
+    std::vector<FastParams<double>> dpar(f64 ? n_columns : 0);
+    const bool fixed = !f64 && cfg->sediment.model != OBME_SEDIMENT_NONE;
+    std::vector<SedimentParams> spar(fixed ? n_columns : 0);
     std::vector<BatchColumn> bcol(n_columns);
     for (int c = 0; c < n_columns; c++) {
         obme_npd_params q = cfg->npd;
@@ -1743,8 +1960,9 @@ extern "C" obme_status obme_batch_create(const obme_config* cfg, int32_t n_colum
         q.zooplankton_assimilation_fraction = get(OBME_BP_ZOO_ASSIMILATION_FRACTION, q.zooplankton_assimilation_fraction);
         q.remineralisation_rate = get(OBME_BP_REMINERALISATION_RATE, q.remineralisation_rate);
         q.small_particle_fraction = get(OBME_BP_SMALL_PARTICLE_FRACTION, q.small_particle_fraction);
-        fpar[c] = make_fast_params(q);
-        dpar[c] = convert_params<double>(q);
+        if (f64) dpar[c] = make_fast_params<double>(q);
+        else fpar[c] = make_fast_params<float>(q);
+        if (fixed) spar[c] = make_sediment_params(q);
         BatchColumn& bc = bcol[c];
         bc.PAR0 = get(OBME_BP_SURFACE_PAR, cfg->par.surface_value);
         bc.wP = -get(OBME_BP_P_SINKING_SPEED, cfg->sinking.speed[1]);
@@ -1761,8 +1979,9 @@ extern "C" obme_status obme_batch_create(const obme_config* cfg, int32_t n_colum
     };
     bool ok = up((void**)&b->d_offsets, b->offsets.data(), b->offsets.size() * sizeof(int)) &&
               up((void**)&b->d_bcol, bcol.data(), bcol.size() * sizeof(BatchColumn));
-    if (ok && b->prec == OBME_FP64) ok = up((void**)&b->d_dpar, dpar.data(), dpar.size() * sizeof(NPDParams<double>));
-    if (ok && b->prec != OBME_FP64) ok = up((void**)&b->d_fpar, fpar.data(), fpar.size() * sizeof(FastParams));
+    if (ok) ok = f64 ? up(&b->d_fpar, dpar.data(), dpar.size() * sizeof(dpar[0]))
+                     : up(&b->d_fpar, fpar.data(), fpar.size() * sizeof(fpar[0]));
+    if (ok && fixed) ok = up((void**)&b->d_fsed, spar.data(), spar.size() * sizeof(spar[0]));
     if (ok && b->prec != OBME_FP64)
         ok = hipMalloc((void**)&b->d_comp, 4 * (size_t)b->offsets[n_columns] * sizeof(float)) == hipSuccess;
     if (ok && cfg->sediment.model == OBME_SEDIMENT_INSTANT_REMINERALISATION) {

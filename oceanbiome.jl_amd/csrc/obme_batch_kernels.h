@@ -45,8 +45,8 @@ struct BatchArgs {
     const int* offsets;             // [n_columns + 1]
     const int* cols;                // this class's column list
     int ncols;                      // entries of `cols`
-    const FastParams* fpar;         // FP32: per-column derived constants
-    const NPDParams<double>* dpar;  // FP64: per-column parameters
+    const FastParams<FT>* fpar;     // per-column derived constants
+    const SedimentParams* fsed;     // FP32 with a sediment: the same, for its transitions
     const BatchColumn* bcol;        // per-column constants
     int nsteps;
     FT dtf, dz, invdz;
@@ -117,10 +117,11 @@ __device__ __forceinline__ void batch_columns(const BatchArgs<FT>& a)
         const FT PAR0 = (FT)bc.PAR0;
         const FT Lt = (FT)bc.Lt;
         const FT wP = (FT)bc.wP, wD = (FT)bc.wD;
-        FastParams fp;
-        NPDParams<double> dp;
-        if constexpr (F32) fp = a.fpar[cc];
-        else dp = a.dpar[cc];
+        constexpr bool FIXED = F32 && SED;
+        using Params = std::conditional_t<FIXED, SedimentParams, FastParams<FT>>;
+        Params fp;
+        if constexpr (FIXED) fp = a.fsed[cc];
+        else fp = a.fpar[cc];
         const float wiP = (float)(bc.wP / (double)a.dz), wiD = (float)(bc.wD / (double)a.dz);
 
         // the sediment of this column, held by the lane of its bottom cell
@@ -250,8 +251,8 @@ __device__ __forceinline__ void batch_columns(const BatchArgs<FT>& a)
                     const bool top = (m == 0) && (r == 0);
                     const FT N = val(0, m), P = val(1, m), Z = val(2, m), Dd = val(3, m);
                     FT G[4];
-                    if constexpr (F32) npzd_fast(fp, N, P, Z, Dd, PARv[m], Lt, G[0], G[1], G[2], G[3]);
-                    else npzd_tendencies(dp, N, P, Z, FT(0), Dd, PARv[m], Lt, G[0], G[1], G[2], G[3]);
+                    if constexpr (FIXED) npzd_sediment(fp, N, P, Z, Dd, PARv[m], Lt, G[0], G[1], G[2], G[3]);
+                    else npzd_fast(fp, N, P, Z, Dd, PARv[m], Lt, G[0], G[1], G[2], G[3]);
                     const FT cPn = (m == 0) ? cP_up : val(1, m > 0 ? m - 1 : 0);
                     const FT cDn = (m == 0) ? cD_up : val(3, m > 0 ? m - 1 : 0);
                     if constexpr (F32) {

@@ -5,7 +5,7 @@
 // Newton, pCO2, CO2 gas-exchange flux).
 //
 // FT = double is the plain FP64 path (the reference's arithmetic, operand
-// order kept; contraction into FMA is the only change).  FT = float is the
+// order kept in the carbonate chemistry; the transitions agree to rounding).  FT = float is the
 // FP32-mixed path: native v_exp/v_log/v_rcp based transcendentals and
 // divisions on the vector ALUs; the carbonate chemistry is always FP64.
 #pragma once
@@ -37,28 +37,6 @@ __device__ __forceinline__ FT jmax(FT x, FT y)
     return (__builtin_isnan(x) || __builtin_isnan(y)) ? d : a;
 }
 
-// Julia eps(x): spacing of floats at |x|; eps(0) is the smallest subnormal.
-__device__ __forceinline__ double jeps(double x)
-{
-    uint64_t b = __double_as_longlong(x);
-    int e = (int)((b >> 52) & 0x7ff);
-    uint64_t r = (e > 52) ? ((uint64_t)(e - 52) << 52) : ((uint64_t)1 << ((e > 1 ? e : 1) - 1));
-    double out = __longlong_as_double(r);
-    return (e == 0x7ff) ? __longlong_as_double(0x7ff8000000000000ull) : out;
-}
-__device__ __forceinline__ float jeps(float x)
-{
-    uint32_t b = __float_as_uint(x);
-    int e = (int)((b >> 23) & 0xff);
-    uint32_t r = (e > 23) ? ((uint32_t)(e - 23) << 23) : ((uint32_t)1 << ((e > 1 ? e : 1) - 1));
-    float out = __uint_as_float(r);
-    return (e == 0xff) ? __uint_as_float(0x7fc00000u) : out;
-}
-
-template <typename FT> struct Tiny;
-template <> struct Tiny<double> { static constexpr double eps0 = 4.9406564584124654e-324; };
-template <> struct Tiny<float> { static constexpr float eps0 = 1.40129846e-45f; };
-
 // Precision-dispatched math.  FP64: the accurate device library.  FP32:
 // the hardware instructions v_exp_f32 (2^x), v_log_f32 (log2 x),
 // v_rcp_f32 and v_sqrt_f32 (about 1 ulp each).
@@ -73,19 +51,86 @@ __device__ __forceinline__ float m_exp(float x) { return __builtin_amdgcn_exp2f(
 __device__ __forceinline__ double m_sqrt(double x) { return sqrt(x); }
 __device__ __forceinline__ float m_sqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
 __device__ __forceinline__ double m_pow(double x, double y) { return pow(x, y); }
-// x^e1 and x^e2 of one base in FP64 as exp(e log x) with the logarithm
-// shared: within a few ulp of pow (the rounding of e log x, |e log x| of
-// order 10, is what exp amplifies), at a third of two pow calls.  x <= 0,
-// NaN and a zero exponent take pow's own special cases.
+// 1/x: the hardware's estimate; FP64 with two Newton steps (36 cycles of a
+// wave where the IEEE quotient takes 65; within 1 ulp, NaN for x = 0 or
+// infinite).
+__device__ __forceinline__ float m_rcp(float x) { return __builtin_amdgcn_rcpf(x); }
+__device__ __forceinline__ double m_rcp(double x)
+{
+    double r = __builtin_amdgcn_rcp(x);
+    r = fma(r, fma(-x, r, 1.0), r);
+    return fma(r, fma(-x, r, 1.0), r);
+}
+// 1/sqrt(x), x > 0 and finite: the same way.
+__device__ __forceinline__ float m_rsqrt(float x) { return __builtin_amdgcn_rsqf(x); }
+__device__ __forceinline__ double m_rsqrt(double x)
+{
+    double y = __builtin_amdgcn_rsq(x);
+    y = fma(0.5 * y, fma(-(x * y), y, 1.0), y);
+    return fma(0.5 * y, fma(-(x * y), y, 1.0), y);
+}
+// log x for a finite x > 0, within 1 ulp: x = 2^k (1 + f), 1 + f in
+// [sqrt(1/2), sqrt(2)), s = f / (2 + f), log(1 + f) = 2 atanh s =
+// f - (f^2/2 - s (f^2/2 + R(s^2))), R the series 2 (z/3 + z^2/5 + ...) to
+// z^9 (z <= 0.0295: the rest is below 2^-55 of the logarithm).  About 150 cycles of a wave
+// where the library's log takes 365.
+__device__ __forceinline__ double log_positive(double x)
+{
+    double m = __builtin_amdgcn_frexp_mant(x);         // [1/2, 1)
+    int k = __builtin_amdgcn_frexp_exp(x);
+    const bool lo = m < 0.70710678118654752;
+    m = lo ? m + m : m;
+    k = lo ? k - 1 : k;
+    const double f = m - 1.0;
+    const double s = f * m_rcp(2.0 + f);
+    const double z = s * s;
+    double R = fma(z, 2.0 / 19, 2.0 / 17);
+    R = fma(z, R, 2.0 / 15);
+    R = fma(z, R, 2.0 / 13);
+    R = fma(z, R, 2.0 / 11);
+    R = fma(z, R, 2.0 / 9);
+    R = fma(z, R, 2.0 / 7);
+    R = fma(z, R, 2.0 / 5);
+    R = fma(z, R, 2.0 / 3);
+    R = z * R;
+    const double h = 0.5 * f * f;
+    const double dk = (double)k;
+    // ln 2 in two parts, the first a multiple of 2^-42: k times it is exact
+    const double ln2h = 0x1.62e42fefa3800p-1, ln2l = 0x1.ef35793c76730p-45;
+    return fma(dk, ln2h, f - (h - fma(s, h + R, dk * ln2l)));
+}
+// x^e from L = log |x| as exp(e L), the product's rounding error put back
+// (exp would amplify it: |e L| is of order 10).
+__device__ __forceinline__ double exp_product(double e, double L)
+{
+    const double p = e * L;
+    const double r = exp(p);
+    return fma(r, fma(e, L, -p), r);
+}
+// pow's value at x <= 0, infinite and NaN x and at e = 0, r = |x|^e elsewhere.
+__device__ __forceinline__ double pow_special(double x, double e, double r)
+{
+    if (e == 0.0) return 1.0;
+    if (x != x || e != e) return x + e;
+    const double inf = HUGE_VAL;
+    if (x == 0.0) r = e > 0.0 ? 0.0 : inf;
+    if (fabs(x) == inf) r = e > 0.0 ? inf : 0.0;
+    if (x < 0.0) {
+        if (e != rint(e)) return x == -inf ? r : __longlong_as_double(0x7ff8000000000000ll);
+        if (0.5 * e != rint(0.5 * e)) r = -r;
+    }
+    return r;
+}
+// x^e1 and x^e2 of one base in FP64, within a few ulp of pow: the logarithm
+// shared, pow's special cases behind one branch.
 __device__ __forceinline__ void pow_pair(double x, double e1, double e2, double& r1, double& r2)
 {
-    if (x > 0.0 && e1 != 0.0 && e2 != 0.0) {
-        const double L = log(x);
-        r1 = exp(e1 * L);
-        r2 = exp(e2 * L);
-    } else {
-        r1 = pow(x, e1);
-        r2 = pow(x, e2);
+    const double L = log_positive(fabs(x));
+    r1 = exp_product(e1, L);
+    r2 = exp_product(e2, L);
+    if (!(x > 0.0 && x < HUGE_VAL && e1 != 0.0 && e2 != 0.0)) {
+        r1 = pow_special(x, e1, r1);
+        r2 = pow_special(x, e2, r2);
     }
 }
 // x^y for x >= 0 as 2^(y log2 x); a negative x gives NaN, as on the GPU
@@ -135,249 +180,105 @@ __device__ __forceinline__ void gstore(FT* p, unsigned boff, FT v)
     *reinterpret_cast<FT*>(reinterpret_cast<char*>(p) + boff) = v;
 }
 
-// ---------------------------------------------------------------- parameters
-
-// obme_npd_params converted to the arithmetic type.
-template <typename FT>
-struct NPDParams {
-    FT kNO3, kNH4, psi, kPAR, mu0, gamma, alpha_x, Q10;
-    FT mP, mZ, muZ, aP_solid, aZ_exc, pref, g, kG, aZ_ass, R, rho_c, R_chl;
-    FT nitrif, a_rem, s_rem, b_rem, d_rem, small_solid, Rd, rem, small_frac;
-    FT Rp, Rn;    // Oxygen(): respiration and nitrification O:N ratios (set from obme_oxygen)
-    int light_form, use_Q10, mort_form, graz_form;
-};
-
-template <typename FT>
-inline NPDParams<FT> convert_params(const obme_npd_params& p)
-{
-    NPDParams<FT> q;
-    q.Rp = q.Rn = FT(0);
-    q.kNO3 = (FT)p.nitrate_half_saturation;
-    q.kNH4 = (FT)p.ammonia_half_saturation;
-    q.psi = (FT)p.nitrate_ammonia_inhibition;
-    q.kPAR = (FT)p.light_half_saturation;
-    q.mu0 = (FT)p.phytoplankton_maximum_growth_rate;
-    q.gamma = (FT)p.phytoplankton_exudation_fraction;
-    q.alpha_x = (FT)p.ammonia_fraction_of_exudate;
-    q.Q10 = (FT)p.temperature_coefficient;
-    q.mP = (FT)p.phytoplankton_mortality_rate;
-    q.mZ = (FT)p.zooplankton_mortality_rate;
-    q.muZ = (FT)p.zooplankton_excretion_rate;
-    q.aP_solid = (FT)p.phytoplankton_solid_waste_fraction;
-    q.aZ_exc = (FT)p.excretion_inorganic_fraction;
-    q.pref = (FT)p.preference_for_phytoplankton;
-    q.g = (FT)p.maximum_grazing_rate;
-    q.kG = (FT)p.grazing_half_saturation;
-    q.aZ_ass = (FT)p.zooplankton_assimilation_fraction;
-    q.R = (FT)p.redfield_ratio;
-    q.rho_c = (FT)p.carbon_calcite_ratio;
-    q.R_chl = (FT)p.phytoplankton_chlorophyll_ratio;
-    q.nitrif = (FT)p.nitrification_rate;
-    q.a_rem = (FT)p.remineralisation_inorganic_fraction;
-    q.s_rem = (FT)p.small_remineralisation_rate;
-    q.b_rem = (FT)p.large_remineralisation_rate;
-    q.d_rem = (FT)p.dissolved_remineralisation_rate;
-    q.small_solid = (FT)p.small_solid_waste_fraction;
-    q.Rd = (FT)p.detritus_redfield_ratio;
-    q.rem = (FT)p.remineralisation_rate;
-    q.small_frac = (FT)p.small_particle_fraction;
-    q.light_form = p.light_limitation;
-    q.use_Q10 = p.use_temperature_coefficient;
-    q.mort_form = p.phytoplankton_mortality_formulation;
-    q.graz_form = p.grazing_concentration_formulation;
-    return q;
-}
-
 // ---------------------------------------------------------------- tendencies
 
-// Shared plankton terms (NutrientsPlanktonDetritus/plankton.jl).
+// The NutrientsPlanktonDetritus transitions in the arithmetic type FT.  The
+// products of parameters are formed once on the host in FP64 (the vector
+// ALUs do all float arithmetic: there is no scalar float ALU), and the
+// quotients are gathered: the Monod terms and the light limitation over one
+// reciprocal (FP64 two: the ammonia term apart), the grazing over one.  The
+// reference's expressions (plankton.jl, nutrients.jl, detritus.jl) hold 13
+// quotients per cell; FP64 agrees with them to rounding.
 template <typename FT>
-struct Grazing {
-    FT total, onP, onSmall;
-};
-
-template <typename FT>
-__device__ __forceinline__ FT light_limitation(const NPDParams<FT>& q, FT PAR)
-{   // plankton.jl:219-220
-    if (q.light_form == OBME_LIGHT_MONDO) return m_div(PAR, q.kPAR + PAR);
-    return m_div(PAR, m_sqrt(PAR * PAR + q.kPAR * q.kPAR));
-}
-
-template <typename FT>
-__device__ __forceinline__ Grazing<FT> grazing(const NPDParams<FT>& q, FT P, FT Z, FT sPOM)
-{   // total_grazing :118-135, grazing(Val{:P}) :352-369, grazing(Val{:sPOM}/Val{:D}) :371-389,
-    // weighted_phytoplankton_preference :393-397, concentration_limit :89-90
-    FT p = m_div(q.pref * P, q.pref * P + (FT(1) - q.pref) * sPOM + Tiny<FT>::eps0);
-    FT food = p * P + (FT(1) - p) * sPOM;
-    FT L = (q.graz_form == OBME_LINEAR) ? m_div(food, food + q.kG)
-                                        : m_div(food * food, food * food + q.kG * q.kG);
-    FT den = food + jeps(food);
-    Grazing<FT> G;
-    G.total = q.g * L * Z;
-    G.onP = m_div(q.g * p * L * P, den) * Z;
-    G.onSmall = m_div(q.g * (FT(1) - p) * L * sPOM, den) * Z;
-    return G;
-}
-
-template <typename FT>
-__device__ __forceinline__ FT mortality(const NPDParams<FT>& q, FT P)
-{   // plankton.jl:86-87
-    return q.mort_form == OBME_LINEAR ? q.mP * P : q.mP * (P * P);
-}
-
-// NPZD transitions (N, P, Z, D); T has zero tendency.  With dO2 the O2
-// transition of the Oxygen component's Nutrient method (oxygen.jl:35-46):
-// Rp μP - (Rp - Rn) respiration, where respiration is the plankton's
-// inorganic nitrogen waste alone (the line that adds the detritus waste,
-// oxygen.jl:42, begins with a unary + and is a separate, discarded
-// expression in Julia).
-template <typename FT>
-__device__ __forceinline__ void npzd_tendencies(const NPDParams<FT>& q, FT N, FT P, FT Z, FT T, FT D, FT PAR,
-                                                FT Lt, FT& dN, FT& dP, FT& dZ, FT& dD, FT* dO2 = nullptr)
-{
-    // phytoplankton_growth (plankton.jl:191-206), Nutrient limitation (:180-188)
-    FT Ln = m_div(N, N + q.kNO3);
-    FT Ll = light_limitation(q, PAR);
-    FT muP = q.mu0 * Ll * Ln * Lt * P;
-    FT sPOM = D * q.small_frac;  // detritus.jl:386-387
-    Grazing<FT> G = grazing(q, P, Z, sPOM);
-    FT nuP = mortality(q, P);
-    dP = (FT(1) - q.gamma) * muP - G.onP - nuP;                     // plankton.jl:92-105
-    dZ = q.aZ_ass * G.total - q.mZ * (Z * Z) - q.muZ * Z;          // :107-116
-    FT pinw = q.aZ_exc * q.muZ * Z + (FT(1) - q.aP_solid) * nuP;  // :292-306
-    FT dinw = D * q.rem;                                           // detritus.jl:389-390
-    FT uptake = muP * (FT(1) - q.alpha_x * q.gamma);               // plankton.jl:271-278
-    dN = pinw + dinw - uptake;                                     // nutrients.jl:86-90
-    FT ponw = (FT(1) - q.alpha_x) * q.gamma * muP + (FT(1) - q.aZ_exc) * q.muZ * Z;  // :312-325
-    FT solid = (FT(1) - q.aZ_ass) * G.total + q.aP_solid * nuP + q.mZ * (Z * Z);    // :330-346
-    dD = ponw + solid - G.onSmall - q.rem * D;                     // detritus.jl:373-379
-    if (dO2) *dO2 = q.Rp * muP - (q.Rp - q.Rn) * pinw;
-}
-
-// LOBSTER transitions; v/out in tracer order NO3, NH4, P, Z, sPOM, bPOM, DOM[, DIC, Alk][, O2].
-// CARB: bit 1 CarbonateSystem, bit 2 Oxygen.
-template <typename FT, int CARB>
-__device__ __forceinline__ void lobster_tendencies(const NPDParams<FT>& q, const FT* v, FT PAR, FT* out)
-{
-    FT NO3 = v[0], NH4 = v[1], P = v[2], Z = v[3], sPOM = v[4], bPOM = v[5], DOM = v[6];
-    // nitrogen_limitation (plankton.jl:150-166)
-    FT nl = m_div(NO3 * m_exp(-q.psi * NH4), NO3 + q.kNO3);
-    FT al = jmax(FT(0), m_div(NH4, q.kNH4 + NH4));
-    FT Ln = (nl + al) / FT(2);
-    FT Ll = light_limitation(q, PAR);
-    FT muP = q.mu0 * Ll * Ln * FT(1) * P;
-    Grazing<FT> G = grazing(q, P, Z, sPOM);
-    FT nuP = mortality(q, P);
-    FT nitrification = q.nitrif * NH4;                       // nutrients.jl:55
-    FT share = nl + al + Tiny<FT>::eps0;
-    FT up_NO3 = m_div(muP * nl, share);                     // plankton.jl:223-239
-    FT waste = q.alpha_x * q.gamma * muP;
-    FT up_NH4 = m_div(muP * al, share) - waste;             // :241-261
-    FT pinw = q.aZ_exc * q.muZ * Z + (FT(1) - q.aP_solid) * nuP;
-    FT dinw = (q.a_rem * (q.s_rem * sPOM + q.b_rem * bPOM) + q.d_rem * DOM);     // detritus.jl:252-263
-    FT ponw = (FT(1) - q.alpha_x) * q.gamma * muP + (FT(1) - q.aZ_exc) * q.muZ * Z;
-    FT donw = (FT(1) - q.a_rem) * (q.s_rem * sPOM + q.b_rem * bPOM);             // :265-274
-    FT solid = (FT(1) - q.aZ_ass) * G.total + q.aP_solid * nuP + q.mZ * (Z * Z);
-    FT dNO3 = nitrification - up_NO3;                        // nutrients.jl:57-60
-    FT dNH4 = pinw + dinw - nitrification - up_NH4;          // :62-67
-    out[0] = dNO3;
-    out[1] = dNH4;
-    out[2] = (FT(1) - q.gamma) * muP - G.onP - nuP;
-    out[3] = q.aZ_ass * G.total - q.mZ * (Z * Z) - q.muZ * Z;
-    out[4] = q.small_solid * solid - G.onSmall - q.s_rem * sPOM;       // detritus.jl:240-244
-    out[5] = (FT(1) - q.small_solid) * solid - q.b_rem * bPOM;        // :246-249
-    out[6] = ponw + donw - q.d_rem * DOM;                              // :234-238
-    if constexpr ((CARB & 1) != 0) {
-        FT pp = (FT(1) + q.rho_c * (FT(1) - q.gamma) - q.alpha_x * q.gamma) * muP * q.R;  // plankton.jl:280-290
-        FT picw = q.R * pinw;                                                           // :308-309
-        FT dicw = q.a_rem * (q.s_rem * (sPOM * q.Rd) + q.b_rem * (bPOM * q.Rd)) + q.d_rem * (DOM * q.Rd);
-        FT cdis = (G.onP + nuP) * q.rho_c * q.R;                                        // :429-441
-        FT cup = FT(2) * q.rho_c * muP * q.R;                                           // :443-450
-        out[7] = -pp + picw + dicw + cdis;                                              // carbonate_system.jl:50-55
-        out[8] = dNH4 * FT(0.9375) - dNO3 * FT(1.0625) - FT(2) * cup + FT(2) * cdis;    // :57-62
-    }
-    if constexpr ((CARB & 2) != 0) {
-        // oxygen.jl:21-31: the NH4 tendency stands for "nitrate_production"
-        out[(CARB & 1) ? 9 : 7] = q.Rp * muP - (q.Rp - q.Rn) * dNH4 - q.Rp * nitrification;
-    }
-}
-
-// ---------------------------------------------------------------- FP32 fast tendencies
-
-// Derived constants of the FP32-mixed path, formed once on the host in
-// FP64 and rounded: the vector ALUs of gfx950 do all float arithmetic
-// (there is no scalar float ALU), so uniform products are precomputed.
 struct FastParams {
-    float nPSI2;       // -psi * log2(e): exp(-psi NH4) = 2^(nPSI2 NH4)
-    float kNO3, kNH4, kPAR, kPAR2;
-    float mu0, mu0h;   // mu0, mu0/2 (LOBSTER's (L_NO3 + L_NH4)/2)
-    float pref, prefc; // pref, 1 - pref
-    float kG, kG2, g;
-    float mP, mZ, muZ;
-    float one_m_gamma, axg;
-    float nitrif;
-    float pinw_z;      // aZ_exc * muZ
-    float one_m_aPs, aPs;
-    float s_rem, b_rem, d_rem, a_rem, one_m_arem;
-    float ponw_mu;     // (1 - alpha_x) gamma
-    float ponw_z;      // (1 - aZ_exc) muZ
-    float one_m_aZass, aZass;
-    float ss, one_m_ss;
-    float ppc;         // (1 + rho (1-gamma) - alpha_x gamma) R
-    float R, Rd, rhoR2, rhoR4;  // R, Rd, 2 rho R, 4 rho R
-    float rem, small_frac, uptake_N;  // Detritus rate, fraction, (1 - alpha_x gamma)
-    float log2Q10_10;  // log2(Q10)/10: Q10^(T/10) = 2^(T log2Q10_10)
-    float oRp, oRpn;   // Oxygen(): Rp, Rp - Rn (set from obme_oxygen)
+    FT nPSI;           // FP32 -psi log2(e): exp(-psi NH4) = 2^(nPSI NH4); FP64 -psi
+    FT kNO3, kNH4, kPAR, kPAR2;
+    FT mu0h;           // mu0/2 (LOBSTER's (L_NO3 + L_NH4)/2)
+    FT pref, prefc;    // pref, 1 - pref
+    FT kGp, kGs, kG, kG2;   // kG pref, kG (1 - pref), kG, kG^2
+    FT g;
+    FT mP, mZ, muZ;
+    FT growP;          // (1 - gamma) mu0/2
+    FT axg;            // alpha_x gamma mu0/2
+    FT nitrif;
+    FT pinw_z;         // aZ_exc muZ
+    FT pinw_p, solid_p;   // (1 - aP) , aP: the mortality's inorganic and solid shares
+    FT s_rem, b_rem, d_rem, a_rem, one_m_arem;
+    FT ponw_mu;        // (1 - alpha_x) gamma mu0/2
+    FT ponw_z;         // (1 - aZ_exc) muZ
+    FT solid_g, gainZ; // (1 - aZ_ass) g, aZ_ass g
+    FT ss, one_m_ss;
+    FT ppc;            // (1 + rho (1-gamma) - alpha_x gamma) R mu0/2
+    FT R, Rd, rhoR, rhoRg, rhoR4;  // R, Rd, rho R, rho R g, 4 rho R mu0/2
+    FT rem, small_frac;           // Detritus rate and fraction
+    FT nGrowP, nUp, nPonw, nOx;   // NPZD: (1 - gamma) mu0, (1 - alpha_x gamma) mu0, (1 - alpha_x) gamma mu0, Rp mu0
+    FT logQ10_10, logQ10_10l;   // Q10^(T/10): FP32 log2(Q10)/10; FP64 ln(Q10)/10 and its rounding error
+    FT oRp, oRpn, oRpm;           // Oxygen(): Rp, Rp - Rn, Rp mu0/2
     int light_form, use_Q10, mort_form, graz_form;
 };
 
-inline FastParams make_fast_params(const obme_npd_params& p)
+template <typename FT>
+inline FastParams<FT> make_fast_params(const obme_npd_params& p, double Rp = 0.0, double Rn = 0.0)
 {
-    FastParams f;
-    f.oRp = f.oRpn = 0.0f;
+    FastParams<FT> f;
+    const bool F32 = sizeof(FT) == 4;
     const double LOG2E = 1.4426950408889634;
-    f.nPSI2 = (float)(-p.nitrate_ammonia_inhibition * LOG2E);
-    f.kNO3 = (float)p.nitrate_half_saturation;
-    f.kNH4 = (float)p.ammonia_half_saturation;
-    f.kPAR = (float)p.light_half_saturation;
-    f.kPAR2 = (float)(p.light_half_saturation * p.light_half_saturation);
-    f.mu0 = (float)p.phytoplankton_maximum_growth_rate;
-    f.mu0h = (float)(p.phytoplankton_maximum_growth_rate / 2);
-    f.pref = (float)p.preference_for_phytoplankton;
-    f.prefc = (float)(1 - p.preference_for_phytoplankton);
-    f.kG = (float)p.grazing_half_saturation;
-    f.kG2 = (float)(p.grazing_half_saturation * p.grazing_half_saturation);
-    f.g = (float)p.maximum_grazing_rate;
-    f.mP = (float)p.phytoplankton_mortality_rate;
-    f.mZ = (float)p.zooplankton_mortality_rate;
-    f.muZ = (float)p.zooplankton_excretion_rate;
-    f.one_m_gamma = (float)(1 - p.phytoplankton_exudation_fraction);
-    f.axg = (float)(p.ammonia_fraction_of_exudate * p.phytoplankton_exudation_fraction);
-    f.nitrif = (float)p.nitrification_rate;
-    f.pinw_z = (float)(p.excretion_inorganic_fraction * p.zooplankton_excretion_rate);
-    f.one_m_aPs = (float)(1 - p.phytoplankton_solid_waste_fraction);
-    f.aPs = (float)p.phytoplankton_solid_waste_fraction;
-    f.s_rem = (float)p.small_remineralisation_rate;
-    f.b_rem = (float)p.large_remineralisation_rate;
-    f.d_rem = (float)p.dissolved_remineralisation_rate;
-    f.a_rem = (float)p.remineralisation_inorganic_fraction;
-    f.one_m_arem = (float)(1 - p.remineralisation_inorganic_fraction);
-    f.ponw_mu = (float)((1 - p.ammonia_fraction_of_exudate) * p.phytoplankton_exudation_fraction);
-    f.ponw_z = (float)((1 - p.excretion_inorganic_fraction) * p.zooplankton_excretion_rate);
-    f.one_m_aZass = (float)(1 - p.zooplankton_assimilation_fraction);
-    f.aZass = (float)p.zooplankton_assimilation_fraction;
-    f.ss = (float)p.small_solid_waste_fraction;
-    f.one_m_ss = (float)(1 - p.small_solid_waste_fraction);
-    f.ppc = (float)((1 + p.carbon_calcite_ratio * (1 - p.phytoplankton_exudation_fraction)
-                     - p.ammonia_fraction_of_exudate * p.phytoplankton_exudation_fraction) * p.redfield_ratio);
-    f.R = (float)p.redfield_ratio;
-    f.Rd = (float)p.detritus_redfield_ratio;
-    f.rhoR2 = (float)(2 * p.carbon_calcite_ratio * p.redfield_ratio);
-    f.rhoR4 = (float)(4 * p.carbon_calcite_ratio * p.redfield_ratio);
-    f.rem = (float)p.remineralisation_rate;
-    f.small_frac = (float)p.small_particle_fraction;
-    f.uptake_N = (float)(1 - p.ammonia_fraction_of_exudate * p.phytoplankton_exudation_fraction);
-    f.log2Q10_10 = (float)(std::log2(p.temperature_coefficient > 0 ? p.temperature_coefficient : 1.0) / 10);
+    const double mu0 = p.phytoplankton_maximum_growth_rate, h = mu0 / 2;
+    const double gam = p.phytoplankton_exudation_fraction, ax = p.ammonia_fraction_of_exudate;
+    const double g = p.maximum_grazing_rate, kG = p.grazing_half_saturation, pr = p.preference_for_phytoplankton;
+    const double R = p.redfield_ratio, rho = p.carbon_calcite_ratio;
+    f.nPSI = (FT)(-p.nitrate_ammonia_inhibition * (F32 ? LOG2E : 1.0));
+    f.kNO3 = (FT)p.nitrate_half_saturation;
+    f.kNH4 = (FT)p.ammonia_half_saturation;
+    f.kPAR = (FT)p.light_half_saturation;
+    f.kPAR2 = (FT)(p.light_half_saturation * p.light_half_saturation);
+    f.mu0h = (FT)h;
+    f.pref = (FT)pr;
+    f.prefc = (FT)(1 - pr);
+    f.kGp = (FT)(kG * pr);
+    f.kGs = (FT)(kG * (1 - pr));
+    f.kG = (FT)kG;
+    f.kG2 = (FT)(kG * kG);
+    f.g = (FT)g;
+    f.mP = (FT)p.phytoplankton_mortality_rate;
+    f.mZ = (FT)p.zooplankton_mortality_rate;
+    f.muZ = (FT)p.zooplankton_excretion_rate;
+    f.growP = (FT)((1 - gam) * h);
+    f.axg = (FT)(ax * gam * h);
+    f.nitrif = (FT)p.nitrification_rate;
+    f.pinw_z = (FT)(p.excretion_inorganic_fraction * p.zooplankton_excretion_rate);
+    f.pinw_p = (FT)(1 - p.phytoplankton_solid_waste_fraction);
+    f.solid_p = (FT)p.phytoplankton_solid_waste_fraction;
+    f.s_rem = (FT)p.small_remineralisation_rate;
+    f.b_rem = (FT)p.large_remineralisation_rate;
+    f.d_rem = (FT)p.dissolved_remineralisation_rate;
+    f.a_rem = (FT)p.remineralisation_inorganic_fraction;
+    f.one_m_arem = (FT)(1 - p.remineralisation_inorganic_fraction);
+    f.ponw_mu = (FT)((1 - ax) * gam * h);
+    f.ponw_z = (FT)((1 - p.excretion_inorganic_fraction) * p.zooplankton_excretion_rate);
+    f.solid_g = (FT)((1 - p.zooplankton_assimilation_fraction) * g);
+    f.gainZ = (FT)(p.zooplankton_assimilation_fraction * g);
+    f.ss = (FT)p.small_solid_waste_fraction;
+    f.one_m_ss = (FT)(1 - p.small_solid_waste_fraction);
+    f.ppc = (FT)((1 + rho * (1 - gam) - ax * gam) * R * h);
+    f.R = (FT)R;
+    f.Rd = (FT)p.detritus_redfield_ratio;
+    f.rhoR = (FT)(rho * R);
+    f.rhoRg = (FT)(rho * R * g);
+    f.rhoR4 = (FT)(4 * rho * R * h);
+    f.rem = (FT)p.remineralisation_rate;
+    f.small_frac = (FT)p.small_particle_fraction;
+    f.nGrowP = (FT)((1 - gam) * mu0);
+    f.nUp = (FT)((1 - ax * gam) * mu0);
+    f.nPonw = (FT)((1 - ax) * gam * mu0);
+    f.nOx = (FT)(Rp * mu0);
+    const double Q = p.temperature_coefficient > 0 ? p.temperature_coefficient : 1.0;
+    const long double lnQ = std::log((long double)Q) / 10;
+    f.logQ10_10 = F32 ? (FT)(std::log2(Q) / 10) : (FT)lnQ;
+    f.logQ10_10l = F32 ? FT(0) : (FT)(lnQ - (long double)(double)lnQ);
+    f.oRp = (FT)Rp;
+    f.oRpn = (FT)(Rp - Rn);
+    f.oRpm = (FT)(Rp * h);
     f.light_form = p.light_limitation;
     f.use_Q10 = p.use_temperature_coefficient;
     f.mort_form = p.phytoplankton_mortality_formulation;
@@ -385,146 +286,179 @@ inline FastParams make_fast_params(const obme_npd_params& p)
     return f;
 }
 
-__device__ __forceinline__ float frcp(float x) { return __builtin_amdgcn_rcpf(x); }
-// max(0, x) that keeps a NaN x (Julia's max propagates NaN)
-__device__ __forceinline__ float fmax0(float x) { return (x < 0.0f) ? 0.0f : x; }
-constexpr float F_TINY = 1.17549435e-38f;  // smallest normal float
+// max(0, x).  (A NaN x gives 0 here: the nitrate uptake beside it is NaN then.)
+__device__ __forceinline__ float max0(float x) { return fmaxf(x, 0.0f); }
+__device__ __forceinline__ double max0(double x) { return fmax(x, 0.0); }
+// the smallest normal number: keeps 0/0 away as the reference's eps(food) does
+template <typename FT> struct Least;
+template <> struct Least<float> { static constexpr float v = 1.17549435e-38f; };
+template <> struct Least<double> { static constexpr double v = 2.2250738585072014e-308; };
 
-// Grazing of the PhytoZoo plankton (plankton.jl:118-135, :352-397) in FP32,
-// reformulated over n = pref P^2 + (1-pref) sPOM^2 and d = pref P + (1-pref) sPOM:
-// the preference-weighted food is n/d, so the total grazing is
-// g Z n^2 / (n^2 + kG^2 d^2) (quadratic) or g Z n / (n + kG d) (linear), and
-// the grazed fractions of the total are pref P^2 / n and (1-pref) sPOM^2 / n.
-// With fr = total / n = g Z n / (n^2 + kG^2 d^2) (or g Z / (n + kG d)) the
-// three terms are fr n, fr pref P^2 and fr (1-pref) sPOM^2: one reciprocal
-// instead of the reference's three divisions; F_TINY keeps 0/0 away as the
-// reference's eps(food) does.
-struct FGrazing {
-    float total, onP, onSmall;
-};
-// Formulation choices of the FP32 path: FM < 0 reads them from FastParams
-// at run time; otherwise they are compiled in, FM = light (bit 0: 0 Mondo,
-// 1 analytical) | phytoplankton mortality << 1 (0 linear, 1 quadratic) |
-// grazing concentration << 2 (0 linear, 1 quadratic) | Q10 in use << 3.
-template <int FM> __device__ __forceinline__ int fm_light(const FastParams& f) { if constexpr (FM < 0) return f.light_form; else return FM & 1; }
-template <int FM> __device__ __forceinline__ int fm_mort(const FastParams& f) { if constexpr (FM < 0) return f.mort_form; else return (FM >> 1) & 1; }
-template <int FM> __device__ __forceinline__ int fm_graz(const FastParams& f) { if constexpr (FM < 0) return f.graz_form; else return (FM >> 2) & 1; }
-template <int FM> __device__ __forceinline__ int fm_q10(const FastParams& f) { if constexpr (FM < 0) return f.use_Q10; else return (FM >> 3) & 1; }
-inline int fm_code(const FastParams& f)
+// Formulation choices: FM < 0 reads them from FastParams at run time;
+// otherwise they are compiled in, FM = light (bit 0: 0 Mondo, 1 analytical) |
+// phytoplankton mortality << 1 (0 linear, 1 quadratic) | grazing
+// concentration << 2 (0 linear, 1 quadratic) | Q10 in use << 3.
+template <int FM, typename FT> __device__ __forceinline__ int fm_light(const FastParams<FT>& f) { if constexpr (FM < 0) return f.light_form; else return FM & 1; }
+template <int FM, typename FT> __device__ __forceinline__ int fm_mort(const FastParams<FT>& f) { if constexpr (FM < 0) return f.mort_form; else return (FM >> 1) & 1; }
+template <int FM, typename FT> __device__ __forceinline__ int fm_graz(const FastParams<FT>& f) { if constexpr (FM < 0) return f.graz_form; else return (FM >> 2) & 1; }
+template <int FM, typename FT> __device__ __forceinline__ int fm_q10(const FastParams<FT>& f) { if constexpr (FM < 0) return f.use_Q10; else return (FM >> 3) & 1; }
+inline int fm_code(const FastParams<float>& f)
 {
     return (f.light_form & 1) | ((f.mort_form & 1) << 1) | ((f.graz_form & 1) << 2) | ((f.use_Q10 ? 1 : 0) << 3);
 }
 
-template <int FM = -1>
-__device__ __forceinline__ FGrazing fast_grazing(const FastParams& f, float P, float Z, float sPOM)
+// Q10^(T/10) (plankton.jl:210-214); FP64 with the product's low part put back.
+template <typename FT>
+__device__ __forceinline__ FT q10_factor(const FastParams<FT>& f, FT T)
 {
-    const float pP = f.pref * P;
-    const float cS = f.prefc * sPOM;
-    const float sS = cS * sPOM;
-    const float n = fmaf(pP, P, sS);
-    const float d = pP + cS;
-    const float gZ = f.g * Z;
-    float fr;
-    if (fm_graz<FM>(f) == OBME_LINEAR) fr = gZ * frcp(fmaf(f.kG, d, n) + F_TINY);
-    else {
-        const float kd = f.kG * d;
-        fr = (gZ * n) * frcp(fmaf(kd, kd, n * n) + F_TINY);
+    if constexpr (sizeof(FT) == 4) {
+        return m_exp2(T * f.logQ10_10);
+    } else {
+        const double p = T * f.logQ10_10;
+        const double e = exp(p);
+        return fma(e, fma(T, f.logQ10_10, -p) + T * f.logQ10_10l, e);
     }
-    FGrazing G;
+}
+
+// Grazing of the PhytoZoo plankton (plankton.jl:118-135, :352-397) without
+// the rate g: with n = pref P^2 + (1-pref) sPOM^2 and d = pref P + (1-pref)
+// sPOM the preference-weighted food is n/d, so the total grazing is
+// Z n^2 / (n^2 + kG^2 d^2) (quadratic) or Z n / (n + kG d) (linear), and the
+// grazed shares of the total are pref P^2 / n and (1-pref) sPOM^2 / n.  FP64
+// keeps the preference p = pref P / (d + ε) apart, as the reference has it: at
+// P = 0 with pref = 1 (a rescaled cell) n and d vanish and p = 0 leaves the
+// food to sPOM.
+template <typename FT>
+struct FGrazing {
+    FT total, onP, onSmall;
+};
+template <int FM, typename FT>
+__device__ __forceinline__ FGrazing<FT> fast_grazing(const FastParams<FT>& f, FT P2, FT P, FT Z, FT S)
+{
+    FGrazing<FT> G;
+    if constexpr (sizeof(FT) == 8) {
+        const FT pP = f.pref * P;
+        const FT p = pP * m_rcp(fma(f.prefc, S, pP) + Least<FT>::v);
+        const FT q = FT(1) - p;
+        const FT food = fma(p, P, q * S);
+        FT fr;
+        if (fm_graz<FM>(f) == OBME_LINEAR) fr = Z * m_rcp(food + f.kG);
+        else fr = (Z * food) * m_rcp(fma(food, food, f.kG2));
+        G.total = fr * food;
+        G.onP = fr * (p * P);
+        G.onSmall = fr * (q * S);
+        return G;
+    }
+    const FT onp = f.pref * P2, ons = f.prefc * (S * S);
+    const FT n = onp + ons;
+    const FT kd = fma(f.kGp, P, f.kGs * S);
+    FT fr;
+    if (fm_graz<FM>(f) == OBME_LINEAR) fr = Z * m_rcp(n + kd + Least<FT>::v);
+    else fr = (Z * n) * m_rcp(fma(kd, kd, fma(n, n, Least<FT>::v)));
     G.total = fr * n;
-    G.onP = fr * (pP * P);
-    G.onSmall = fr * sS;
+    G.onP = fr * onp;
+    G.onSmall = fr * ons;
     return G;
 }
 
-template <int FM = -1>
-__device__ __forceinline__ float fast_light(const FastParams& f, float PAR)
+// LOBSTER (+ CarbonateSystem, Oxygen) transitions; v/out in tracer order
+// NO3, NH4, P, Z, sPOM, bPOM, DOM[, DIC, Alk][, O2].  CARB: bit 1
+// CarbonateSystem, bit 2 Oxygen.  The nitrate and ammonia uptakes are mu0/2
+// L_PAR P times their own limitation (the reference forms them as fractions
+// of the total production, plankton.jl:223-261, which is the same product);
+// uN, uA and mu leave mu0/2 to the constants.
+template <int CARB, int FM = -1, typename FT>
+__device__ __forceinline__ void lobster_fast(const FastParams<FT>& f, const FT* v, FT PAR, FT* out)
 {
-    if (fm_light<FM>(f) == OBME_LIGHT_MONDO) return PAR * frcp(f.kPAR + PAR);
-    return PAR * __builtin_amdgcn_rsqf(fmaf(PAR, PAR, f.kPAR2));
-}
-
-// LOBSTER (+ CarbonateSystem) transitions in FP32; v/out in tracer order.
-// The nitrate and ammonia uptakes are mu0/2 L_PAR P times their own
-// limitation (the reference forms them as fractions of the total
-// production, plankton.jl:223-261, which is the same product).
-template <int CARB, int FM = -1>
-__device__ __forceinline__ void lobster_fast(const FastParams& f, const float* v, float PAR, float* out)
-{
-    const float NO3 = v[0], NH4 = v[1], P = v[2], Z = v[3], sPOM = v[4], bPOM = v[5], DOM = v[6];
-    const float a = NO3 + f.kNO3, b = f.kNH4 + NH4;
-    float up_NO3, muA;
-    if (fm_light<FM>(f) == OBME_LIGHT_MONDO) {
-        // one reciprocal for both Monod terms and the light limitation
-        // PAR / (kPAR + PAR): with c = kPAR + PAR > 0, 1/(a c) = b r and
-        // 1/(b c) = a r for r = 1/(a b c), and max(0, x / c) = max(0, x) / c
-        const float r = frcp((a * b) * (f.kPAR + PAR));
-        const float nlc = NO3 * __builtin_amdgcn_exp2f(f.nPSI2 * NH4) * (b * r);
-        const float alc = fmax0(NH4 * (a * r));
-        const float muLPc = f.mu0h * PAR * P;
-        up_NO3 = muLPc * nlc;
-        muA = muLPc * alc;
+    const FT NO3 = v[0], NH4 = v[1], P = v[2], Z = v[3], S = v[4], B = v[5], DOM = v[6];
+    const FT a = NO3 + f.kNO3, b = NH4 + f.kNH4;
+    FT inhibition;
+    if constexpr (sizeof(FT) == 4) inhibition = m_exp2(f.nPSI * NH4);
+    else inhibition = m_exp(f.nPSI * NH4);
+    const FT nl = NO3 * inhibition;
+    FT uN, uA;
+    if constexpr (sizeof(FT) == 8) {
+        const FT light = fm_light<FM>(f) == OBME_LIGHT_MONDO ? f.kPAR + PAR : FT(1);
+        const FT pp = fm_light<FM>(f) == OBME_LIGHT_MONDO ? PAR * P : PAR * P * m_rsqrt(fma(PAR, PAR, f.kPAR2));
+        const FT r = m_rcp(a * light);
+        uN = pp * nl * r;
+        uA = max0(NH4 * m_rcp(b)) * (pp * (a * r));
+    } else if (fm_light<FM>(f) == OBME_LIGHT_MONDO) {
+        // with c = kPAR + PAR > 0, 1/(a c) = b r and 1/(b c) = a r for
+        // r = 1/(a b c), and max(0, x / c) = max(0, x) / c
+        const FT r = m_rcp((a * b) * (f.kPAR + PAR));
+        const FT pp = PAR * P;
+        uN = nl * (b * (pp * r));
+        uA = max0(NH4 * (a * r)) * pp;
     } else {
-        // one reciprocal for both Monod terms
-        const float rab = frcp(a * b);
-        const float nl = NO3 * __builtin_amdgcn_exp2f(f.nPSI2 * NH4) * (b * rab);
-        const float al = fmax0(NH4 * (a * rab));
-        const float muLP = f.mu0h * fast_light<FM>(f, PAR) * P;
-        up_NO3 = muLP * nl;
-        muA = muLP * al;
+        const FT r = m_rcp(a * b);
+        const FT pp = PAR * P * m_rsqrt(fma(PAR, PAR, f.kPAR2));
+        uN = nl * (b * (pp * r));
+        uA = max0(NH4 * (a * r)) * pp;
     }
-    const float muP = up_NO3 + muA;
-    const FGrazing G = fast_grazing<FM>(f, P, Z, sPOM);
-    const float nuP = (fm_mort<FM>(f) == OBME_LINEAR) ? f.mP * P : f.mP * P * P;
-    const float nit = f.nitrif * NH4;
-    const float up_NH4 = fmaf(-f.axg, muP, muA);
-    const float pinw = fmaf(f.pinw_z, Z, f.one_m_aPs * nuP);
-    const float sb = fmaf(f.s_rem, sPOM, f.b_rem * bPOM);
-    const float dinw = fmaf(f.a_rem, sb, f.d_rem * DOM);
-    const float ponw = fmaf(f.ponw_mu, muP, f.ponw_z * Z);
-    const float Z2 = Z * Z;
-    const float solid = fmaf(f.one_m_aZass, G.total, fmaf(f.aPs, nuP, f.mZ * Z2));
-    const float dNO3 = nit - up_NO3;
-    const float dNH4 = pinw + dinw - nit - up_NH4;
+    const FT mu = uN + uA;
+    const FT P2 = P * P, Z2 = Z * Z;
+    const FGrazing<FT> G = fast_grazing<FM>(f, P2, P, Z, S);
+    const FT nuP = f.mP * (fm_mort<FM>(f) == OBME_LINEAR ? P : P2);
+    const FT nit = f.nitrif * NH4;
+    const FT sr = f.s_rem * S, br = f.b_rem * B, dd = f.d_rem * DOM;
+    const FT sb = sr + br;
+    const FT pinw = fma(f.pinw_z, Z, f.pinw_p * nuP);
+    const FT dinw = fma(f.a_rem, sb, dd);
+    const FT solid = fma(f.solid_g, G.total, fma(f.solid_p, nuP, f.mZ * Z2));
+    const FT dNO3 = fma(-f.mu0h, uN, nit);
+    const FT dNH4 = fma(f.axg, mu, fma(-f.mu0h, uA, (pinw + dinw) - nit));
     out[0] = dNO3;
     out[1] = dNH4;
-    out[2] = fmaf(f.one_m_gamma, muP, -G.onP) - nuP;
-    out[3] = fmaf(f.aZass, G.total, -f.mZ * Z2) - f.muZ * Z;
-    out[4] = fmaf(f.ss, solid, -G.onSmall) - f.s_rem * sPOM;
-    out[5] = fmaf(f.one_m_ss, solid, -f.b_rem * bPOM);
-    out[6] = fmaf(f.one_m_arem, sb, ponw) - f.d_rem * DOM;
+    out[2] = fma(f.growP, mu, fma(-f.g, G.onP, -nuP));
+    out[3] = fma(f.gainZ, G.total, fma(-f.mZ, Z2, -(f.muZ * Z)));
+    out[4] = fma(f.ss, solid, fma(-f.g, G.onSmall, -sr));
+    out[5] = fma(f.one_m_ss, solid, -br);
+    out[6] = fma(f.ponw_mu, mu, fma(f.ponw_z, Z, fma(f.one_m_arem, sb, -dd)));
     if constexpr ((CARB & 1) != 0) {
         // calcite dissolution (G_P + ν) ρ R (plankton.jl:429-441), uptake 2 ρ μP R (:443-450)
-        const float cdis2 = (G.onP + nuP) * f.rhoR2;            // 2 cdis
-        out[7] = fmaf(-f.ppc, muP, fmaf(f.R, pinw, fmaf(f.Rd, dinw, 0.5f * cdis2)));
-        out[8] = fmaf(0.9375f, dNH4, -1.0625f * dNO3) - f.rhoR4 * muP + cdis2;
+        const FT cdis = fma(f.rhoRg, G.onP, f.rhoR * nuP);
+        out[7] = fma(-f.ppc, mu, fma(f.R, pinw, fma(f.Rd, dinw, cdis)));
+        out[8] = fma(FT(0.9375), dNH4, fma(FT(-1.0625), dNO3, fma(-f.rhoR4, mu, cdis + cdis)));
     }
     if constexpr ((CARB & 2) != 0) {
-        // Rp (μP - nitrification) - (Rp - Rn) G_NH4 (oxygen.jl:21-31)
-        out[(CARB & 1) ? 9 : 7] = fmaf(f.oRp, muP - nit, -f.oRpn * dNH4);
+        // Rp (μP - nitrification) - (Rp - Rn) G_NH₄ (oxygen.jl:21-31: the NH₄
+        // tendency stands for "nitrate_production")
+        out[(CARB & 1) ? 9 : 7] = fma(f.oRpm, mu, fma(-f.oRp, nit, -(f.oRpn * dNH4)));
     }
 }
 
-// NPZD transitions in FP32 (N, P, Z, D); Lt = Q10^(T/10); dO2 as in npzd_tendencies.
-template <int FM = -1>
-__device__ __forceinline__ void npzd_fast(const FastParams& f, float N, float P, float Z, float D, float PAR,
-                                          float Lt, float& dN, float& dP, float& dZ, float& dD,
-                                          float* dO2 = nullptr)
+// NPZD transitions (N, P, Z, D); Lt = Q10^(T/10).  With dO2 the O2 transition
+// of the Oxygen component's Nutrient method (oxygen.jl:35-46): Rp μP -
+// (Rp - Rn) respiration, where respiration is the plankton's inorganic
+// nitrogen waste alone (the line that adds the detritus waste, oxygen.jl:42,
+// begins with a unary + and is a separate, discarded expression in Julia).
+template <int FM = -1, typename FT>
+__device__ __forceinline__ void npzd_fast(const FastParams<FT>& f, FT N, FT P, FT Z, FT D, FT PAR, FT Lt, FT& dN,
+                                          FT& dP, FT& dZ, FT& dD, FT* dO2 = nullptr)
 {
-    const float muP = f.mu0 * fast_light<FM>(f, PAR) * (N * frcp(N + f.kNO3)) * Lt * P;
-    const float sPOM = D * f.small_frac;
-    const FGrazing G = fast_grazing<FM>(f, P, Z, sPOM);
-    const float nuP = (fm_mort<FM>(f) == OBME_LINEAR) ? f.mP * P : f.mP * P * P;
-    const float Z2 = Z * Z;
-    dP = fmaf(f.one_m_gamma, muP, -G.onP) - nuP;
-    dZ = fmaf(f.aZass, G.total, -f.mZ * Z2) - f.muZ * Z;
-    const float pinw = fmaf(f.pinw_z, Z, f.one_m_aPs * nuP);
-    dN = fmaf(D, f.rem, pinw) - muP * f.uptake_N;
-    const float ponw = fmaf(f.ponw_mu, muP, f.ponw_z * Z);
-    const float solid = fmaf(f.one_m_aZass, G.total, fmaf(f.aPs, nuP, f.mZ * Z2));
-    dD = ponw + solid - G.onSmall - f.rem * D;
-    if (dO2) *dO2 = fmaf(f.oRp, muP, -f.oRpn * pinw);
+    const FT S = D * f.small_frac;
+    FT mu;   // without mu0
+    if (fm_light<FM>(f) == OBME_LIGHT_MONDO) mu = (N * Lt) * (PAR * P) * m_rcp((N + f.kNO3) * (f.kPAR + PAR));
+    else mu = (N * Lt) * (PAR * P) * (m_rcp(N + f.kNO3) * m_rsqrt(fma(PAR, PAR, f.kPAR2)));
+    const FT P2 = P * P, Z2 = Z * Z;
+    const FGrazing<FT> G = fast_grazing<FM>(f, P2, P, Z, S);
+    const FT nuP = f.mP * (fm_mort<FM>(f) == OBME_LINEAR ? P : P2);
+    const FT zz = f.mZ * Z2, rD = f.rem * D;
+    const FT pinw = fma(f.pinw_z, Z, f.pinw_p * nuP);
+    dP = fma(f.nGrowP, mu, fma(-f.g, G.onP, -nuP));
+    dZ = fma(f.gainZ, G.total, -zz) - f.muZ * Z;
+    dN = fma(-f.nUp, mu, rD + pinw);
+    const FT solid = fma(f.solid_g, G.total, fma(f.solid_p, nuP, zz));
+    dD = fma(f.nPonw, mu, fma(f.ponw_z, Z, solid)) - fma(f.g, G.onSmall, rD);
+    if (dO2) *dO2 = fma(f.nOx, mu, -f.oRpn * pinw);
 }
+
+}  // namespace obme
+
+#include "obme_sediment_order.h"
+
+namespace obme {
 
 // ScaleNegativeTracers groups for the kernels: members as bits of the
 // tracer index and a scalefactor per tracer index (obme_negative_scaling

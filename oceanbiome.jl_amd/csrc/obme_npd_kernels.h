@@ -2,8 +2,8 @@
 // LOBSTER biogeochemistry step on gfx950.
 //
 // Column sweep (column_lane): lane per water column.  A workgroup of NW
-// waves owns 64 NW consecutive i-columns of one j row; each lane walks its
-// column from the surface down, one level at a time, and runs the three RK3
+// waves owns 64 NW consecutive columns; each lane walks its column from the
+// surface down, one level at a time, and runs the three RK3
 // stages at each level before it moves on.  That order is legal because
 // stage s at level k reads only stage-s values of the levels above it:
 //  - the TwoBand chlorophyll integral (Light/2band.jl:18-32) is the running
@@ -161,7 +161,8 @@ struct StepArgs {
     int Nx, Ny, Nz;
     unsigned sx, sxy, base0;       // strides and interior origin offset
     unsigned field_bytes;          // byte size of one parent array
-    NPDParams<FT> q;
+    FastParams<FT> f;              // derived constants of the transitions
+    SedimentParams fs;             // FP32 with a sediment: the same, for its transitions
     FT kr, kb, xr, xb, er, eb, Rr;  // Rr = R_chl / r
     int surface_mode;
     FT surface_value;
@@ -169,7 +170,6 @@ struct StepArgs {
     FT dtf;                        // Δt in the arithmetic type
     FT dz_u, zc0_u, w0_u, w1_u;    // uniform grid: Δz, zc[0], sinking w
     FT invdz_u;                    // uniform grid: 1/Δz
-    FastParams f;                  // FP32 path: derived constants
     float rk_a[3], rk_b[3];        // FP32 path: Δt γ and Δt ζ per stage
     float kr2, kb2, xr2, xb2;      // FP32 path: attenuations × log2(e)
     float cr, cb;                  // FP32 path: e log2(R_chl / r) per band
@@ -223,9 +223,11 @@ struct StepArgs {
 };
 
 // Per-level geometry rows in `lev` (each Nz entries).
-enum { LEV_ZC = 0, LEV_UP, LEV_DN, LEV_INVDZ, LEV_COUNT };
+enum { LEV_ZC = 0, LEV_UP, LEV_DN, LEV_INVDZ, LEV_WR, LEV_WB, LEV_COUNT };
 // LEV_UP[k] = zc[k+1] - zf[k+1], LEV_DN[k] = zf[k+1] - zc[k] for k < Nz-1;
 // for k = Nz-1: LEV_UP = 0 and LEV_DN = zf[Nz] - zc[Nz-1] (the top half cell).
+// LEV_WR, LEV_WB: half the light left by the water alone at zc, exp(k zc) / 2
+// of the red and blue bands, formed in FP64.
 
 // Modes of the column sweep: the fused RK3 step, the tendencies (hook), the
 // PAR (hook), one RK3 stage with its substep (the step of the sinking schemes
@@ -291,9 +293,9 @@ __device__ __forceinline__ FT sink_face(int k, int Nz, FT cm2, FT cm1, FT c0, FT
 }
 
 // The column sweep.  Lane = water column: a workgroup of NW waves owns
-// NW*64 consecutive i-columns of one j row, so every load and store of a
-// level is one contiguous run of 64 values per wave (coalesced straight
-// from HBM, no staging).  Each lane walks its column from the surface down,
+// NW*64 consecutive columns of the flattened (i, j) order, so every load and
+// store of a level is one contiguous run of 64 values per wave, two where a
+// row ends in it (coalesced straight from HBM, no staging).  Each lane walks its column from the surface down,
 // one level at a time, and at each level runs the RK3 stages 1, 2, 3 in
 // turn: stage s at level k needs only stage-s values of the levels above
 // it (the chlorophyll integral, the upwind sinking inflow), which the lane
@@ -303,8 +305,8 @@ __device__ __forceinline__ FT sink_face(int k, int Nz, FT cm2, FT cm1, FT c0, FT
 // EXTRA (fused step only), a bit set: 1 negative scaling at the start of
 // every stage; 2 the CO2 flux computed here at the top level (with 1);
 // 4 the InstantRemineralisation sediment at the bottom level.  MASKX: some
-// lanes lie past the last column (Nx is not a multiple of the workgroup's
-// width); false compiles the stores without a mask.  PARK: the FP32
+// lanes lie past the last column (the columns are not a multiple of the
+// workgroup's width); false compiles the stores without a mask.  PARK: the FP32
 // chlorophyll integrals are Kahan-compensated running sums.  SCHEME: the
 // sinking face value, upwind (the fused step), or centred / WENO5, whose
 // face values need the levels below: those run one stage per launch
@@ -330,21 +332,21 @@ __device__ __forceinline__ void column_lane(const StepArgs<FT>& a, const int cw)
     static_assert(!WIN || MODE == TILE_STAGE || MODE == TILE_TENDENCY, "centred and WENO sinking: stage or hook mode");
     static_assert(!TS || WIN, "the stage mode serves the centred and WENO sinking");
 
-    const unsigned nbx = ((unsigned)a.Nx + (unsigned)cw - 1) / (unsigned)cw;
+    // the workgroup's columns: a run of the flattened (i, j) order, whatever the
+    // length of a row
+    const unsigned ncol2d = (unsigned)a.Nx * (unsigned)a.Ny;
     const unsigned tile = xcd_tile(blockIdx.x, gridDim.x);
-    const int j = (int)(tile / nbx);
-    const int i_raw = (int)(tile % nbx) * cw + (int)threadIdx.x;
+    const unsigned q_raw = tile * (unsigned)cw + threadIdx.x;
     // (MASKX false: the launch guarantees every lane holds a column)
-    const bool col_ok = !MASKX || i_raw < a.Nx;
+    const bool col_ok = !MASKX || q_raw < ncol2d;
     // a lane past the last column computes on the last column and stores nothing
-    const int i = col_ok ? i_raw : a.Nx - 1;
+    const unsigned col2d = col_ok ? q_raw : ncol2d - 1;
+    const unsigned j = col2d / (unsigned)a.Nx, i = col2d - j * (unsigned)a.Nx;
     const int Nz = a.Nz;
     const int ktop = Nz - 1;
     constexpr unsigned ES = sizeof(FT);
     const unsigned dk = a.sxy * ES;
-    const unsigned off_top = (a.base0 + (unsigned)i + a.sx * (unsigned)j + a.sxy * (unsigned)ktop) * ES;
-    const unsigned col2d = (unsigned)i + (unsigned)a.Nx * (unsigned)j;
-    const unsigned ncol2d = (unsigned)a.Nx * (unsigned)a.Ny;
+    const unsigned off_top = (a.base0 + i + a.sx * j + a.sxy * (unsigned)ktop) * ES;
     // byte offset of level k of this column in every parent array (the
     // same for all of them): a 32-bit per-lane offset from each array's
     // base address, which stays in two scalar registers
@@ -608,21 +610,21 @@ __device__ __forceinline__ void column_lane(const StepArgs<FT>& a, const int cw)
                 FT v[NT];
 #pragma unroll
                 for (int n = 0; n < NT; n++) v[n] = (CARB != 0 && n >= 7) ? FT(0) : X[n];
+                constexpr bool FIXED = F32 && (EXTRA & 4) != 0;
                 if constexpr (MODEL == OBME_NPZD) {
-                    if constexpr (F32) {
-                        const float Lt = fm_q10<FM>(a.f) ? m_exp2(v[3] * a.f.log2Q10_10) : 1.0f;
+                    FT Lt = FT(1);
+                    if (fm_q10<FM>(a.f)) Lt = q10_factor(a.f, v[3]);
+                    if constexpr (FIXED)
+                        npzd_sediment<FM>(a.fs, v[0], v[1], v[2], v[4], PARv, Lt, Gv[0], Gv[1], Gv[2], Gv[4],
+                                          (CARB & 2) ? &Gv[NT - 1] : nullptr);
+                    else
                         npzd_fast<FM>(a.f, v[0], v[1], v[2], v[4], PARv, Lt, Gv[0], Gv[1], Gv[2], Gv[4],
                                       (CARB & 2) ? &Gv[NT - 1] : nullptr);
-                    } else {
-                        FT Lt = FT(1);
-                        if (a.q.use_Q10) Lt = m_pow(a.q.Q10, v[3] / FT(10));
-                        npzd_tendencies(a.q, v[0], v[1], v[2], v[3], v[4], PARv, Lt, Gv[0], Gv[1], Gv[2], Gv[4],
-                                        (CARB & 2) ? &Gv[NT - 1] : nullptr);
-                    }
                     Gv[3] = FT(0);
+                } else if constexpr (FIXED) {
+                    lobster_sediment<CARB, FM>(a.fs, v, PARv, Gv);
                 } else {
-                    if constexpr (F32) lobster_fast<CARB, FM>(a.f, v, PARv, Gv);
-                    else lobster_tendencies<FT, CARB>(a.q, v, PARv, Gv);
+                    lobster_fast<CARB, FM>(a.f, v, PARv, Gv);
                 }
             }
             // minus the upwind drift flux divergence, w(face) c(upwind cell):
@@ -669,7 +671,7 @@ __device__ __forceinline__ void column_lane(const StepArgs<FT>& a, const int cw)
                 // the top-cell CO2 flux (GasExchange, gas_exchange.jl:26-38) of
                 // this stage's DIC and Alk, the surface kernel's expressions
                 if (top) {
-                    const unsigned tc = a.base0 + (unsigned)i + a.sx * (unsigned)j + a.sxy * (unsigned)ktop;
+                    const unsigned tc = a.base0 + i + a.sx * j + a.sxy * (unsigned)ktop;
                     const double T = a.T3 ? (double)a.T3[tc] : (a.Tprof ? a.Tprof[ktop] : a.Tconst);
                     const double S = a.S3 ? (double)a.S3[tc] : (a.Sprof ? a.Sprof[ktop] : a.Sconst);
                     SurfaceCarbon sc;
@@ -955,6 +957,7 @@ struct SurfaceArgs {
     const double* Tprof;
     const double* Sprof;
     double Tconst, Sconst;
+    int nsteps;                    // step mode: the steps recorded in srec, one after the other
     double* flux_out;              // optional diagnostics (last stage)
     double* pH_out;
     int Nx, Ny, Nz;
@@ -1048,34 +1051,44 @@ __global__ void __launch_bounds__(256) k_surface(SurfaceArgs<FT> a)
             // the increment starts from the residual the previous step left
             // (DIC = U + D carried to about twice FP32's precision in a call)
             float D = a.topres ? a.topres[col] : 0.0f;
+#pragma unroll 1
+            for (int sn = 0; sn < a.nsteps; sn++) {
+                const FT* rec = a.srec + (size_t)(sn * SURF_REC) * ncol + col;
+                Gm = FT(0);
 #pragma unroll
-            for (int st = 0; st < 3; st++) {
-                const float Gb = a.srec[st * ncol + col];
-                const float Alk = a.srec[(3 + st) * ncol + col];
-                F = surface_flux_warm(sc, a.solver, (double)U + (double)D, (double)Alk, a.co2.air_concentration,
-                                      a.mode, H, pH, ev, FP32_NEWTON_TOL);
-                const float G = Gb - (float)F * a.invdz_top;
-                D = fmaf(a.rk_a[st], G, fmaf(a.rk_b[st], Gm, D));
-                Gm = G;
+                for (int st = 0; st < 3; st++) {
+                    const float Gb = rec[(size_t)st * ncol];
+                    const float Alk = rec[(size_t)(3 + st) * ncol];
+                    F = surface_flux_warm(sc, a.solver, (double)U + (double)D, (double)Alk, a.co2.air_concentration,
+                                          a.mode, H, pH, ev, FP32_NEWTON_TOL);
+                    const float G = Gb - (float)F * a.invdz_top;
+                    D = fmaf(a.rk_a[st], G, fmaf(a.rk_b[st], Gm, D));
+                    Gm = G;
+                }
+                // U + D = s + e exactly (TwoSum): s stored, e to the next step
+                const float sum = U + D, dv = sum - U;
+                D = (U - (sum - dv)) + (D - dv);
+                U = sum;
             }
-            // U + D = s + e exactly (TwoSum): s stored, e to the next step
-            const float sum = U + D, dv = sum - U;
-            if (a.topres) a.topres[col] = (U - (sum - dv)) + (D - dv);
-            U = sum;
+            if (a.topres) a.topres[col] = D;
         } else {
             const FT g1 = FT(8.0 / 15.0), g2 = FT(5.0 / 12.0), g3 = FT(3.0 / 4.0);
             const FT z2 = FT(-17.0 / 60.0), z3 = FT(-5.0 / 12.0);
+#pragma unroll 1
+            for (int sn = 0; sn < a.nsteps; sn++) {
+                const FT* rec = a.srec + (size_t)(sn * SURF_REC) * ncol + col;
 #pragma unroll
-            for (int st = 0; st < 3; st++) {
-                FT Gb = a.srec[st * ncol + col];
-                FT Alk = a.srec[(3 + st) * ncol + col];
-                F = surface_flux_warm(sc, a.solver, (double)U, (double)Alk, a.co2.air_concentration, a.mode, H, pH,
-                                      ev);
-                FT G = Gb - (FT)F * a.invdz_top;
-                if (st == 0) U += a.dtf * g1 * G;
-                else if (st == 1) U += a.dtf * (g2 * G + z2 * Gm);
-                else U += a.dtf * (g3 * G + z3 * Gm);
-                Gm = G;
+                for (int st = 0; st < 3; st++) {
+                    FT Gb = rec[(size_t)st * ncol];
+                    FT Alk = rec[(size_t)(3 + st) * ncol];
+                    F = surface_flux_warm(sc, a.solver, (double)U, (double)Alk, a.co2.air_concentration, a.mode, H, pH,
+                                          ev);
+                    FT G = Gb - (FT)F * a.invdz_top;
+                    if (st == 0) U += a.dtf * g1 * G;
+                    else if (st == 1) U += a.dtf * (g2 * G + z2 * Gm);
+                    else U += a.dtf * (g3 * G + z3 * Gm);
+                    Gm = G;
+                }
             }
         }
         a.DIC[top] = U;
