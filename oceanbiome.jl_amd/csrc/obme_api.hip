@@ -792,10 +792,6 @@ static SurfaceArgs<FT> make_surface_args(const obme_handle* h, void* const* trac
     s.base0 = (unsigned)g.Hx + s.sx * (unsigned)g.Hy + s.sxy * (unsigned)g.Hz;
     s.invdz_top = (FT)(1.0 / h->dz[g.Nz - 1]);
     s.nsteps = 1;
-    // both precisions: Newton warm-started from the column's previous [H+]
-    // (FP32 to FP32_NEWTON_TOL, FP64 to a 1e-14 relative step), the
-    // reference's damped Newton as the fallback
-    s.mode = 1;
     s.co2 = c.co2;
     s.solver = c.solver;
     return s;

@@ -99,6 +99,40 @@ __device__ __forceinline__ double log_positive(double x)
     const double ln2h = 0x1.62e42fefa3800p-1, ln2l = 0x1.ef35793c76730p-45;
     return fma(dk, ln2h, f - (h - fma(s, h + R, dk * ln2l)));
 }
+// log x with log's values at x <= 0 (and NaN).
+__device__ __forceinline__ double m_log_any(double x)
+{
+    const double l = log_positive(x);
+    return x > 0.0 ? l : (x == 0.0 ? -HUGE_VAL : __longlong_as_double(0x7ff8000000000000ll));
+}
+// 10^x and log10 x through e, the products' rounding errors put back (about
+// 130 and 170 cycles of a wave; pow(10, x) takes 600, the library's log10 380).
+__device__ __forceinline__ double m_exp10(double x)
+{
+    const double c = 0x1.26bb1bbb55516p+1, cl = -0x1.f48ad494ea3e9p-53;   // ln 10
+    const double p = x * c;
+    const double r = exp(p);
+    return fma(r, fma(x, c, -p) + x * cl, r);
+}
+__device__ __forceinline__ double m_log10(double x)
+{
+    const double c = 0x1.bcb7b1526e50ep-2, cl = 0x1.95355baaafad3p-57;    // 1 / ln 10
+    const double L = m_log_any(x);
+    const double p = L * c;
+    return p + (fma(L, c, -p) + L * cl);
+}
+// Quotients by one denominator: its reciprocal once, then three instructions
+// each, with one correction (the rounded quotient; an IEEE quotient each
+// takes 13).  Denominators finite and not 0.
+struct Divisor {
+    double b, r;
+    __device__ __forceinline__ explicit Divisor(double x) : b(x), r(m_rcp(x)) {}
+    __device__ __forceinline__ double under(double a) const
+    {
+        const double q = a * r;
+        return fma(r, fma(-b, q, a), q);
+    }
+};
 // x^e from L = log |x| as exp(e L), the product's rounding error put back
 // (exp would amplify it: |e L| is of order 10).
 __device__ __forceinline__ double exp_product(double e, double L)
@@ -534,58 +568,43 @@ __device__ __forceinline__ double teos10_density(double T, double S, double Pbar
 }
 
 struct CarbonParams {
-    double DIC, Alk, boron, sulfate, fluoride, silicate, phosphate;
-    double K1, K2, KB, KW, KS, KF, KP1, KP2, KP3, KSi, K0, Tk;
+    double DIC, Alk, boron, sulfate, fluoride, silicate;
+    double K1, K2, KB, KW, KS, KF, KSi, K0, Tk;
 };
 
 // Equilibrium constants at the surface (P = nothing): CarbonChemistry/
 // equilibrium_constants.jl K0 :65-80, K1 :103-126, K2 :149-172, KB :202-250,
 // KW :279-313, IonicStrength :335-341, KS :366-419, KF :451-488,
-// KP1-3 :511-651, KSi :674-713.  log(T), √S, √Is are computed once.
-__device__ __forceinline__ double k0_constant(double T, double S, double lT)
+// KSi :674-713 (KP1-3 enter with phosphate, which is 0 here).  lT = log T, √S
+// and √Is are computed once; the quotients by T share its reciprocal.
+__device__ __forceinline__ double k0_constant(const Divisor& rT, double S, double lT)
 {
-    return exp(-60.2409 + (93.4517 * 100) / T + 23.3585 * (lT - log(100.0)) + 0.0 * (T * T)
+    const double T = rT.b;
+    return exp(-60.2409 + rT.under(93.4517 * 100) + 23.3585 * (lT - 4.605170185988092)
                + (0.023517 + (-0.023656 / 100) * T + (0.0047036 / 10000.0) * (T * T)) * S);
 }
 
-__device__ __forceinline__ void carbon_constants(double Tk, double S, CarbonParams& p)
+__device__ __forceinline__ void carbon_constants(const Divisor& rT, double lT, double S, CarbonParams& p)
 {
-    double lT = log(Tk);
+    const double Tk = rT.b;
+    auto over = [&](double a) { return rT.under(a); };
     double sS = sqrt(S);
     double Is = 19.924 * S / (1000.0 + -1.005 * S);
     double sIs = sqrt(Is);
-    p.K0 = k0_constant(Tk, S, lT);
-    p.K1 = pow(10.0, 61.2172 + -3633.86 / Tk + -9.67770 * lT + 0.011555 * S + -0.0001152 * (S * S));
-    p.K2 = pow(10.0, -25.9290 + -471.78 / Tk + 0.01781 * S + -0.0001122 * (S * S) + 3.16967 * lT);
-    p.KB = exp(148.0248 + (-8966.90 + -2890.53 * sS + -77.942 * S + 1.728 * pow(S, 1.5) + -0.0996 * (S * S)) / Tk
+    p.K0 = k0_constant(rT, S, lT);
+    p.K1 = m_exp10(61.2172 + over(-3633.86) + -9.67770 * lT + 0.011555 * S + -0.0001152 * (S * S));
+    p.K2 = m_exp10(-25.9290 + over(-471.78) + 0.01781 * S + -0.0001122 * (S * S) + 3.16967 * lT);
+    p.KB = exp(148.0248 + over(-8966.90 + -2890.53 * sS + -77.942 * S + 1.728 * (S * sS) + -0.0996 * (S * S))
                + 137.1942 * sS + 1.62142 * S + (-24.4344 + -25.085 * sS + -0.2474 * S) * lT + 0.053105 * sS * Tk);
-    p.KW = exp(148.9652 + -13847.26 / Tk + -23.6521 * lT + (-5.977 + 118.67 / Tk + 1.0495 * lT) * sS + -0.01615 * S);
-    double l1S = log(1 + -0.001005 * S);
-    p.KS = exp(141.328 + -4276.1 / Tk + -23.093 * lT + (324.57 + -13856.0 / Tk + -47.986 * lT) * sIs
-               + (-771.54 + 35474.0 / Tk + 114.723 * lT) * Is + -2698.0 * pow(Is, 1.5) / Tk
-               + 1776.0 * (Is * Is) / Tk + l1S);
-    p.KF = exp(-9.68 + 874.0 / Tk + 0.111 * sS + log(1 + 0.0 * S) + log(1 + 0.0 * S / p.KS));
-    p.KP1 = exp(115.525 + -4576.752 / Tk + -18.453 * lT + (0.69171 + -106.736 / Tk) * sS + (-0.01844 + -0.65643 / Tk) * S);
-    p.KP2 = exp(172.0883 + -8814.715 / Tk + -27.927 * lT + (1.3566 + -160.340 / Tk) * sS + (-0.05778 + 0.37335 / Tk) * S);
-    p.KP3 = exp(-18.141 + -3070.75 / Tk + 0.0 * lT + (2.81197 + 17.27039 / Tk) * sS + (-0.09984 + -44.99486 / Tk) * S);
-    p.KSi = exp(117.385 + -8904.2 / Tk + -19.334 * lT + (3.5913 + -458.79 / Tk) * sIs + (-1.5998 + 188.74 / Tk) * Is
-                + (0.07871 + -12.1652 / Tk) * (Is * Is) + l1S);
-}
-
-// Conversion of the functor's inputs (carbon_chemistry.jl:116-135): ρ at
-// Pbar = 1 (:123), kelvin, mmol/m³ → mol/kg.
-__device__ __forceinline__ void carbon_setup(double DIC, double Alk, double T, double S, CarbonParams& p)
-{
-    p.boron = 0.000232 / 10.811 * S / 1.80655;
-    p.sulfate = 0.14 / 96.06 * S / 1.80655;
-    p.fluoride = 0.000067 / 18.9984 * S / 1.80655;
-    double rho = teos10_density(T, S, 1.0);
-    p.Tk = T + 273.15;
-    p.Alk = Alk * (1e-3 / rho);
-    p.DIC = DIC * (1e-3 / rho);
-    p.phosphate = 0.0;
-    p.silicate = 0.0;
-    carbon_constants(p.Tk, S, p);
+    p.KW = exp(148.9652 + over(-13847.26) + -23.6521 * lT + (-5.977 + over(118.67) + 1.0495 * lT) * sS + -0.01615 * S);
+    double l1S = m_log_any(1 + -0.001005 * S);
+    p.KS = exp(141.328 + over(-4276.1) + -23.093 * lT + (324.57 + over(-13856.0) + -47.986 * lT) * sIs
+               + (-771.54 + over(35474.0) + 114.723 * lT) * Is + over(-2698.0 * (Is * sIs))
+               + over(1776.0 * (Is * Is)) + l1S);
+    // (the logarithms of 1 + 0 S and 1 + 0 S / KS of the form are 0)
+    p.KF = exp(-9.68 + over(874.0) + 0.111 * sS);
+    p.KSi = exp(117.385 + over(-8904.2) + -19.334 * lT + (3.5913 + over(-458.79)) * sIs + (-1.5998 + over(188.74)) * Is
+                + (0.07871 + over(-12.1652)) * (Is * Is) + l1S);
 }
 
 // alkalinity_residual / ∂ₕ (CarbonChemistry/alkalinity_residual.jl:18-75)
@@ -656,12 +675,18 @@ __device__ __forceinline__ double solve_for_H(const CarbonParams& p, const obme_
         double lb = (x - 0.0) / delta;
         lb = (lb < 0) ? 1.0 : lb;
         double lambda = jmin(1.0, lb);
-        double fnew = alk_residual<SI>(x - lambda * delta, p);
+        double trial = x - lambda * delta;
+        double fnew = alk_residual<SI>(trial, p);
         ne++;
         while ((fabs(fnew) >= fabs(fx) - s.armijo_constant * lambda * fx * jsign(fx)) && (lambda > s.min_damping)) {
             lambda *= s.damping;
-            fnew = alk_residual<SI>(x - lambda * delta, p);
-            ne++;
+            // (at the root the halved steps round to the same trial point)
+            const double t = x - lambda * delta;
+            if (t != trial) {
+                trial = t;
+                fnew = alk_residual<SI>(trial, p);
+                ne++;
+            }
         }
         double xn = x - lambda * delta;
         N += 1;
@@ -706,70 +731,68 @@ __device__ __forceinline__ float guess_H_fp32(const CarbonParams& p)
     return x;
 }
 
-// The residual and its derivative together for the refinement of the
-// mixed path: the same function as alk_residual / alk_residual_derivative,
-// each fraction rewritten over one reciprocal of its denominator
-// (bicarbonate + carbonate = DIC K1 (H + 2 K2) / cd, borate = boron KB /
-// (KB + H), ...), so 8 FP64 divisions instead of 24.  The FP64 path keeps the
-// reference's expressions.
-template <bool SI>
-__device__ __forceinline__ void alk_residual_and_derivative_fast(double H, const CarbonParams& p, double& f,
-                                                                 double& df)
-{
-    const double cd = H * H + p.K1 * H + p.K1 * p.K2;
-    const double rcd = 1.0 / cd;
-    const double sd = 1.0 + p.sulfate / p.KS;
-    const double rsd = 1.0 / sd;
-    const double rH = 1.0 / H;
-    const double rB = 1.0 / (p.KB + H);
-    const double KSsd = p.KS * sd;
-    const double rS = 1.0 / (H + KSsd);
-    const double rF = 1.0 / (H + p.KF);
-    const double DK1 = p.DIC * p.K1;
-    const double carb = DK1 * (H + 2.0 * p.K2) * rcd;
-    const double dcarb = DK1 * (cd - (H + 2.0 * p.K2) * (2.0 * H + p.K1)) * (rcd * rcd);
-    const double bor = p.boron * p.KB * rB;
-    const double dbor = -bor * rB;
-    const double hyd = p.KW * rH;
-    const double dhyd = -hyd * rH;
-    const double hso4 = p.sulfate * H * rS;
-    const double dhso4 = p.sulfate * KSsd * (rS * rS);
-    const double hf = p.fluoride * H * rF;
-    const double dhf = p.fluoride * p.KF * (rF * rF);
-    double acc = carb + bor + hyd;
-    double dacc = dcarb + dbor + dhyd;
-    if constexpr (SI) {
-        const double rSi = 1.0 / (p.KSi + H);
-        const double sil = p.silicate * p.KSi * rSi;
-        acc = acc + sil;
-        dacc = dacc - sil * rSi;
+// The residual and its derivative together for the refinement: the same
+// function as alk_residual / alk_residual_derivative, each fraction rewritten
+// over one reciprocal of its denominator (bicarbonate + carbonate =
+// DIC K1 (H + 2 K2) / cd, borate = boron KB / (KB + H), ...).  What does not
+// depend on H is formed once per solve.
+template <bool SI, typename FT = double>
+struct AlkResidual {
+    FT K1, K2, K12, KB, KW, KSsd, KF, KSi, DK1, bKB, sulfate, fluoride, sK, rsd, Alk;
+    __device__ __forceinline__ explicit AlkResidual(const CarbonParams& p)
+        : K1((FT)p.K1), K2((FT)(p.K2 + p.K2)), K12((FT)(p.K1 * p.K2)), KB((FT)p.KB), KW((FT)p.KW), KF((FT)p.KF),
+          KSi((FT)(SI ? p.KSi : 0.0)), DK1((FT)(p.DIC * p.K1)), bKB((FT)(p.boron * p.KB)), sulfate((FT)p.sulfate),
+          fluoride((FT)p.fluoride), sK((FT)(SI ? p.silicate * p.KSi : 0.0)), Alk((FT)p.Alk)
+    {
+        KSsd = (FT)(p.KS + p.sulfate);    // KS (1 + sulfate / KS)
+        rsd = (FT)p.KS * m_rcp(KSsd);
     }
-    f = acc - H * rsd - hso4 - hf - p.Alk;
-    df = dacc - rsd - dhso4 - dhf;
-}
+    __device__ __forceinline__ void operator()(FT H, FT& f, FT& df) const
+    {
+        const FT cd = fma(H, H + K1, K12);
+        const FT rcd = m_rcp(cd), rH = m_rcp(H), rB = m_rcp(KB + H), rS = m_rcp(H + KSsd), rF = m_rcp(H + KF);
+        const FT n = DK1 * rcd;
+        const FT h2 = H + K2;
+        const FT carb = n * h2;
+        const FT dcarb = n * fma(-h2 * rcd, H + H + K1, FT(1));
+        const FT bor = bKB * rB;
+        const FT hyd = KW * rH;
+        const FT qs = sulfate * rS, qf = fluoride * rF;
+        FT acc = carb + bor + hyd;
+        FT dacc = dcarb - bor * rB - hyd * rH;
+        if constexpr (SI) {
+            const FT rSi = m_rcp(KSi + H);
+            const FT sil = sK * rSi;
+            acc = acc + sil;
+            dacc = fma(-sil, rSi, dacc);
+        }
+        f = acc - H * (rsd + qs + qf) - Alk;
+        df = dacc - rsd - qs * (KSsd * rS) - qf * (KF * rF);
+    }
+};
 
 // Refinement of a close first guess by plain FP64 Newton on the same
 // residual; returns false when it has not converged after 6 steps.  It
 // stops after the step that is at most tol relative to the iterate: Newton
 // converges quadratically here, so the error left after a step of relative
-// size tol is of order tol^2 (tol = 1e-8 leaves ~1e-16, the FP64 rounding
-// of H; the default 1e-14 takes one confirming step more).
+// size tol is of order tol^2.
 // The stop of the FP32-mixed paths, whose [H+] feeds FP32 arithmetic: after
 // a step below 1e-4 relative, H is within ~1e-8 of the root (measured on
 // the CPU oracle from warm starts off by up to 1e-2: at most 9e-9).
 constexpr double FP32_NEWTON_TOL = 1e-4;
-// The stop of the FP64 warm-started refinements: a step below 1e-14
-// relative leaves H at the root to rounding.
-constexpr double FP64_NEWTON_TOL = 1e-14;
+// The stop of the FP64 refinements: after a step below 3e-9 relative the next
+// would be of order 1e-17, below the rounding of H.
+constexpr double FP64_NEWTON_TOL = 3e-9;
 template <bool SI = false>
-__device__ __forceinline__ bool refine_H(const CarbonParams& p, double& x, int& evals, double tol = 1e-14)
+__device__ __forceinline__ bool refine_H(const CarbonParams& p, double& x, int& evals, double tol = FP64_NEWTON_TOL)
 {
+    const AlkResidual<SI> residual(p);
 #pragma unroll 1
     for (int it = 0; it < 6; it++) {
         double f, df;
-        alk_residual_and_derivative_fast<SI>(x, p, f, df);
+        residual(x, f, df);
         evals++;
-        double d = f / df;
+        double d = f * m_rcp(df);
         double xn = x - d;
         if (!(xn > 0.0)) return false;
         x = xn;
@@ -781,22 +804,24 @@ __device__ __forceinline__ bool refine_H(const CarbonParams& p, double& x, int& 
 // pCO2 from H (carbon_chemistry.jl:160-162 and selected_output(::Val{:pCO₂}) :170-193).
 __device__ __forceinline__ double pco2_from_H(const CarbonParams& p, double H)
 {
-    double CO2 = p.DIC * (H * H) / (H * H + p.K1 * H + p.K1 * p.K2);
-    double fCO2 = (CO2 / p.K0) * 1e6;
+    double CO2 = p.DIC * (H * H) * m_rcp(H * H + p.K1 * H + p.K1 * p.K2);
+    double fCO2 = (CO2 * m_rcp(p.K0)) * 1e6;
     double P = 101325.0;
     double Tk = p.Tk;
     double B = (-1636.75 + 12.0408 * Tk + (-3.27957 * 1e-2) * (Tk * Tk) + (3.16528 * 1e-5) * (Tk * Tk * Tk)) * 1e-6;
     double dl = (57.7 + -0.118 * Tk) * 1e-6;
     fCO2 *= 0.09807;
-    double phi = 1.0;
-    double x = fCO2 / (phi * P);
+    // x = fCO2 / (φ P), φ = exp(...) from the x before: 1/φ is exp of minus it
+    const double c = P * m_rcp(8.31446261815324 * Tk);
+    const double fP = fCO2 / P;
+    double x = fP, rphi = 1.0;
+#pragma unroll
     for (int n = 0; n < 3; n++) {
-        double om = 1.0 - x;
-        phi = exp((B + 2.0 * (om * om) * dl) * P / (8.31446261815324 * Tk));
-        x = fCO2 / (phi * P);
+        const double om = 1.0 - x;
+        rphi = exp(-(B + 2.0 * (om * om) * dl) * c);
+        x = fP * rphi;
     }
-    double pCO2 = fCO2 / phi;
-    return pCO2 / 0.09807;
+    return fCO2 * rphi / 0.09807;
 }
 
 // Julia's literal x^4 (compensated power by squaring).
@@ -813,13 +838,13 @@ __device__ __forceinline__ double pow4_compensated(double x)
 
 // Gas transfer velocity (gas_transfer_velocity.jl:33-34, :61; schmidt
 // number gas_solubility.jl:211-212; solubility gas_solubility.jl:204).
-__device__ __forceinline__ double transfer_velocity(const obme_co2_exchange& g, double u10, double T, double S)
+// K0: the solubility at T and S.
+__device__ __forceinline__ double transfer_velocity(const obme_co2_exchange& g, double u10, double T, double S,
+                                                   double K0)
 {
     double k660 = g.transfer_velocity[0] + g.transfer_velocity[1] * u10 + g.transfer_velocity[2] * (u10 * u10);
     double sc = g.schmidt[0] + g.schmidt[1] * T + g.schmidt[2] * (T * T) + g.schmidt[3] * (T * T * T)
                 + g.schmidt[4] * pow4_compensated(T);
-    double Tk = T + 273.15;
-    double K0 = k0_constant(Tk, S, log(Tk));
     double sol = K0 * teos10_density(T, S, 0.0) / 1000.0;
     return k660 / sqrt(sc / 660.0) * sol;
 }
@@ -843,36 +868,66 @@ __device__ __forceinline__ void surface_carbon_setup(const obme_co2_exchange& g,
     double rho = teos10_density(T, S, 1.0);
     p.Tk = T + 273.15;
     sc.conv = 1e-3 / rho;
-    p.phosphate = 0.0;
     p.silicate = 0.0;
-    carbon_constants(p.Tk, S, p);
-    sc.k = transfer_velocity(g, u10, T, S);
+    carbon_constants(Divisor(p.Tk), m_log_any(p.Tk), S, p);
+    sc.k = transfer_velocity(g, u10, T, S, p.K0);
+}
+
+// Whether the damped Newton's settings are the reference's (solvers.jl:81-88):
+// it then ends at the root to rounding, and so does a refined guess.
+__device__ __forceinline__ bool reference_solver(const obme_carbon_solver& s)
+{
+    return s.max_iters == 100 && s.atol == 1e-20 && s.damping == 0.5 && s.armijo_constant == 0.5 &&
+           s.min_damping == 0.0009765625 && s.initial_pH_guess == 8.0;
+}
+// The damped Newton's root from its initial guess.  With the reference's
+// settings and DIC and silicate >= 0 (the residual then falls with H: one
+// root), an FP32 Newton from the same pH 8 refined in FP64 ends at the same
+// root in two FP64 iterations instead of 10 to 14, each a residual, a
+// derivative and a line search (4 10^6 points of the ocean's range, with the
+// constants: 1263 -> 151 us; 362 us with the guess in IEEE quotients to
+// 2e-7).  The damped Newton runs where the refinement
+// fails, and where the first step goes past 0 by more than 8 H: past
+// 1 / min_damping its line search cannot shorten a step onto 0, which ends in
+// NaN (hardly any salt or carbon under an ocean's alkalinity).
+template <bool SI = false>
+__device__ __forceinline__ double root_H(const CarbonParams& p, const obme_carbon_solver& s, int& evals)
+{
+    if (p.DIC >= 0.0 && reference_solver(s) && (!SI || p.silicate >= 0.0)) {
+        const AlkResidual<SI, float> residual(p);
+        float x = 1e-8f, step = 0.0f;
+#pragma unroll 1
+        for (int it = 0; it < 20; it++) {
+            float f, df;
+            residual(x, f, df);
+            const float d = f * m_rcp(df);
+            if (it == 0) step = d * 1e8f;
+            x = x - fminf(d, 0.5f * x);
+            if (fabsf(d) <= 1e-3f * x) break;     // the next would be of order 1e-6 x
+        }
+        double H = (double)x;
+        if (step < 8.0f && refine_H<SI>(p, H, evals)) return H;
+    }
+    return solve_for_H<SI>(p, s, pow(10.0, -s.initial_pH_guess), evals);
 }
 
 // Solve for H and return the flux F = k (pCO2_w - pCO2_air)
-// (GasExchange/gas_exchange.jl:26-38).  mode 0: the reference damped Newton
-// from 10^-initial_pH_guess; mode 1: FP32 first guess refined by FP64
-// Newton; with FALLBACK, a refinement that has not converged is redone
-// with the mode-0 solve (the fused step kernels omit the fallback to keep
-// their register budget; a non-converged refinement keeps its last iterate).
-template <bool FALLBACK = true>
+// (GasExchange/gas_exchange.jl:26-38).  mode 0: the reference damped Newton's
+// root; mode 1: FP32 first guess refined by FP64 Newton, whatever the
+// solver's settings, with the mode-0 solve where that has not converged.
 __device__ __forceinline__ double surface_flux(const SurfaceCarbon& sc, const obme_carbon_solver& s, double DIC,
-                                               double Alk, double pCO2_air, int mode, double& pH, int& evals)
+                                               double Alk, double pCO2_air, int mode, double& H, int& evals)
 {
     CarbonParams p = sc.p;
     p.Alk = Alk * sc.conv;
     p.DIC = DIC * sc.conv;
-    double H = 0.0;
     if (mode == 1) {
         H = (double)guess_H_fp32(p);
-        bool done = refine_H(p, H, evals);
-        if (FALLBACK && !done) H = solve_for_H(p, s, pow(10.0, -s.initial_pH_guess), evals);
+        if (!refine_H(p, H, evals)) H = solve_for_H(p, s, pow(10.0, -s.initial_pH_guess), evals);
     } else {
-        H = solve_for_H(p, s, pow(10.0, -s.initial_pH_guess), evals);
+        H = root_H(p, s, evals);
     }
-    pH = -log10(H);
-    double pCO2 = pco2_from_H(p, H);
-    return sc.k * (pCO2 - pCO2_air);
+    return sc.k * (pco2_from_H(p, H) - pCO2_air);
 }
 
 __device__ __forceinline__ double co2_flux(const obme_co2_exchange& g, const obme_carbon_solver& s, double DIC,
@@ -881,17 +936,19 @@ __device__ __forceinline__ double co2_flux(const obme_co2_exchange& g, const obm
 {
     SurfaceCarbon sc;
     surface_carbon_setup(g, T, S, u10, sc);
-    return surface_flux(sc, s, DIC, Alk, pCO2_air, mode, pH, evals);
+    double H;
+    const double F = surface_flux(sc, s, DIC, Alk, pCO2_air, mode, H, evals);
+    pH = -m_log10(H);
+    return F;
 }
 
-// Flux with the mixed path's warm start: H from the previous stage (or an
-// FP32 guess) refined by FP64 Newton (stopping after a step below tol
-// relative, see refine_H), with the reference solve as fallback.
+// Flux with a warm start: H from the previous stage (or an FP32 guess) refined
+// by FP64 Newton (stopping after a step below tol relative, see refine_H),
+// with the reference solve as fallback.
 __device__ __forceinline__ double surface_flux_warm(const SurfaceCarbon& sc, const obme_carbon_solver& s,
-                                                    double DIC, double Alk, double pCO2_air, int mode,
-                                                    double& H, double& pH, int& evals, double tol = 1e-14)
+                                                    double DIC, double Alk, double pCO2_air, double& H, int& evals,
+                                                    double tol = FP64_NEWTON_TOL)
 {
-    if (mode == 0) return surface_flux<true>(sc, s, DIC, Alk, pCO2_air, 0, pH, evals);
     CarbonParams p = sc.p;
     p.Alk = Alk * sc.conv;
     p.DIC = DIC * sc.conv;
@@ -903,7 +960,6 @@ __device__ __forceinline__ double surface_flux_warm(const SurfaceCarbon& sc, con
         if (!done) x = solve_for_H(p, s, pow(10.0, -s.initial_pH_guess), evals);
     }
     H = x;
-    pH = -log10(x);
     return sc.k * (pco2_from_H(p, x) - pCO2_air);
 }
 
@@ -939,14 +995,13 @@ __device__ __forceinline__ double o2_flux(const obme_o2_exchange& g, double O2, 
 }
 
 // SurfaceCarbon (without DIC and Alk) and the O2 coefficients of a column
-// as 21 doubles, for a stepper with T and S fixed.
-constexpr int SURF_PACK = 21;
+// as 17 doubles, for a stepper with T and S fixed.
+constexpr int SURF_PACK = 17;
 __device__ __forceinline__ void surface_pack(const SurfaceCarbon& sc, double kO2, double airO2, double* o)
 {
     const CarbonParams& p = sc.p;
-    const double f[SURF_PACK] = {p.boron, p.sulfate, p.fluoride, p.silicate, p.phosphate, p.K1, p.K2,
-                                 p.KB, p.KW, p.KS, p.KF, p.KP1, p.KP2, p.KP3, p.KSi, p.K0, p.Tk,
-                                 sc.conv, sc.k, kO2, airO2};
+    const double f[SURF_PACK] = {p.boron, p.sulfate, p.fluoride, p.silicate, p.K1, p.K2, p.KB, p.KW, p.KS,
+                                 p.KF, p.KSi, p.K0, p.Tk, sc.conv, sc.k, kO2, airO2};
 #pragma unroll
     for (int q = 0; q < SURF_PACK; q++) o[q] = f[q];
 }
@@ -959,23 +1014,19 @@ __device__ __forceinline__ void surface_unpack(const double* o, SurfaceCarbon& s
     p.sulfate = o[1];
     p.fluoride = o[2];
     p.silicate = o[3];
-    p.phosphate = o[4];
-    p.K1 = o[5];
-    p.K2 = o[6];
-    p.KB = o[7];
-    p.KW = o[8];
-    p.KS = o[9];
-    p.KF = o[10];
-    p.KP1 = o[11];
-    p.KP2 = o[12];
-    p.KP3 = o[13];
-    p.KSi = o[14];
-    p.K0 = o[15];
-    p.Tk = o[16];
-    sc.conv = o[17];
-    sc.k = o[18];
-    kO2 = o[19];
-    airO2 = o[20];
+    p.K1 = o[4];
+    p.K2 = o[5];
+    p.KB = o[6];
+    p.KW = o[7];
+    p.KS = o[8];
+    p.KF = o[9];
+    p.KSi = o[10];
+    p.K0 = o[11];
+    p.Tk = o[12];
+    sc.conv = o[13];
+    sc.k = o[14];
+    kO2 = o[15];
+    airO2 = o[16];
 }
 
 // ---- wave-level helpers (the column sweeps)

@@ -676,11 +676,10 @@ __device__ __forceinline__ void column_lane(const StepArgs<FT>& a, const int cw)
                     const double S = a.S3 ? (double)a.S3[tc] : (a.Sprof ? a.Sprof[ktop] : a.Sconst);
                     SurfaceCarbon sc;
                     surface_carbon_setup(a.co2, T, S, a.co2.wind_speed, sc);
-                    double pH = 0.0;
                     int ev = 0;
                     const double F = surface_flux_warm(sc, a.solver, (double)X[7], (double)X[8],
-                                                       a.co2.air_concentration, 1, Hc, pH, ev,
-                                                       F32 ? FP32_NEWTON_TOL : 1e-14);
+                                                       a.co2.air_concentration, Hc, ev,
+                                                       F32 ? FP32_NEWTON_TOL : FP64_NEWTON_TOL);
                     Gv[7] = Gv[7] - (FT)F * a.invdz_top;
                 }
             }
@@ -958,13 +957,11 @@ struct SurfaceArgs {
     const double* Sprof;
     double Tconst, Sconst;
     int nsteps;                    // step mode: the steps recorded in srec, one after the other
-    double* flux_out;              // optional diagnostics (last stage)
-    double* pH_out;
+    double* flux_out;              // the stage's flux (stage mode), or null
     int Nx, Ny, Nz;
     unsigned sx, sxy, base0;
     FT dtf, invdz_top;
     float rk_a[3], rk_b[3];        // FP32 path: Δt γ and Δt ζ per stage
-    int mode;                      // 0: reference damped Newton; 1: warm-started Newton (fallback: 0)
     obme_co2_exchange co2;
     obme_carbon_solver solver;
     // the stage mode (TILE_STAGE): the stage, and FP32 the step's increments so far
@@ -1018,11 +1015,11 @@ __global__ void __launch_bounds__(256) k_surface(SurfaceArgs<FT> a)
         surface_carbon_setup(a.co2, T, S, a.co2.wind_speed, sc);
     }
     double H = a.Hprev ? a.Hprev[col] : 0.0;
-    double pH = 0.0, F = 0.0;
+    double F = 0.0;
     int ev = 0;
     if constexpr (MODE == TILE_TENDENCY) {
-        F = surface_flux_warm(sc, a.solver, (double)a.DIC[top], (double)a.Alk[top], a.co2.air_concentration, a.mode,
-                              H, pH, ev, sizeof(FT) == 4 ? FP32_NEWTON_TOL : 1e-14);
+        F = surface_flux_warm(sc, a.solver, (double)a.DIC[top], (double)a.Alk[top], a.co2.air_concentration, H,
+                              ev, sizeof(FT) == 4 ? FP32_NEWTON_TOL : FP64_NEWTON_TOL);
         a.GDIC[top] = a.GDIC[top] - (FT)F * a.invdz_top;
     } else if constexpr (MODE == TILE_STAGE) {
         // the flux of the stage's top-cell DIC and Alk (FP32: U + D exactly;
@@ -1039,8 +1036,8 @@ __global__ void __launch_bounds__(256) k_surface(SurfaceArgs<FT> a)
                 alk += (double)a.topres[ncol + col];
             }
         }
-        F = surface_flux_warm(sc, a.solver, dic, alk, a.co2.air_concentration, a.mode, H, pH, ev,
-                              sizeof(FT) == 4 ? FP32_NEWTON_TOL : 1e-14);
+        F = surface_flux_warm(sc, a.solver, dic, alk, a.co2.air_concentration, H, ev,
+                              sizeof(FT) == 4 ? FP32_NEWTON_TOL : FP64_NEWTON_TOL);
     } else {
         // the identical update expressions of the sweep, with the flux term;
         // the step starts from the top-cell DIC the previous step's surface
@@ -1060,7 +1057,7 @@ __global__ void __launch_bounds__(256) k_surface(SurfaceArgs<FT> a)
                     const float Gb = rec[(size_t)st * ncol];
                     const float Alk = rec[(size_t)(3 + st) * ncol];
                     F = surface_flux_warm(sc, a.solver, (double)U + (double)D, (double)Alk, a.co2.air_concentration,
-                                          a.mode, H, pH, ev, FP32_NEWTON_TOL);
+                                          H, ev, FP32_NEWTON_TOL);
                     const float G = Gb - (float)F * a.invdz_top;
                     D = fmaf(a.rk_a[st], G, fmaf(a.rk_b[st], Gm, D));
                     Gm = G;
@@ -1081,8 +1078,7 @@ __global__ void __launch_bounds__(256) k_surface(SurfaceArgs<FT> a)
                 for (int st = 0; st < 3; st++) {
                     FT Gb = rec[(size_t)st * ncol];
                     FT Alk = rec[(size_t)(3 + st) * ncol];
-                    F = surface_flux_warm(sc, a.solver, (double)U, (double)Alk, a.co2.air_concentration, a.mode, H, pH,
-                                          ev);
+                    F = surface_flux_warm(sc, a.solver, (double)U, (double)Alk, a.co2.air_concentration, H, ev);
                     FT G = Gb - (FT)F * a.invdz_top;
                     if (st == 0) U += a.dtf * g1 * G;
                     else if (st == 1) U += a.dtf * (g2 * G + z2 * Gm);
@@ -1095,7 +1091,6 @@ __global__ void __launch_bounds__(256) k_surface(SurfaceArgs<FT> a)
     }
     if (a.Hprev) a.Hprev[col] = H;
     if (a.flux_out) a.flux_out[col] = F;
-    if (a.pH_out) a.pH_out[col] = pH;
 }
 
 }  // namespace obme

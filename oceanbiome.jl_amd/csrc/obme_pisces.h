@@ -535,13 +535,12 @@ __device__ __forceinline__ void pisces_tendencies(const FT* pp, const FT* v, con
 // ---------------------------------------------------------------- calcite saturation (FP64)
 
 // Millero (2007) pressure correction (equilibrium_constants.jl:29-38), a: a0 a1 a2 b0 b1
-__device__ __forceinline__ double pressure_correction(const double* a, double Tk, double P)
+// (as the exponent, under the reciprocal of R T)
+__device__ __forceinline__ double pressure_exponent(const double* a, double Tc, double P, double PRT)
 {
-    const double Tc = Tk - 273.15;
     const double dV = a[0] + a[1] * Tc + a[2] * (Tc * Tc);
     const double dk = a[3] + a[4] * Tc;
-    const double RT = 83.14472 * Tk;
-    return exp((-dV + 0.5 * dk * P) * P / RT);
+    return (-dV + 0.5 * dk * P) * PRT;
 }
 
 // Constants of the calcite saturation that depend only on T, S and the
@@ -579,18 +578,24 @@ __device__ __forceinline__ void omega_constants(double T, double S, double P, Om
     omega_salinity_terms(S, c);
     const double rho = teos10_density(T, S, P);
     const double Tk = T + 273.15;
+    const Divisor rT(Tk);
+    const double lT = m_log_any(Tk);
     c.conv = 1e-3 / rho;
-    carbon_constants(Tk, S, p);
-    c.K1 = p.K1 * pressure_correction(PC_K1, Tk, P);
-    c.K2 = p.K2 * pressure_correction(PC_K2, Tk, P);
-    c.KB = p.KB * pressure_correction(PC_KB, Tk, P);
-    c.KW = p.KW * pressure_correction(PC_KW, Tk, P);
-    c.KS = p.KS * pressure_correction(PC_KS, Tk, P);
-    c.KF = p.KF * pressure_correction(PC_KF, Tk, P);
+    carbon_constants(rT, lT, S, p);
+    const double Tc = Tk - 273.15;
+    const double PRT = P * m_rcp(83.14472 * Tk);
+    auto corrected = [&](double K, const double* a) { return K * exp(pressure_exponent(a, Tc, P, PRT)); };
+    c.K1 = corrected(p.K1, PC_K1);
+    c.K2 = corrected(p.K2, PC_K2);
+    c.KB = corrected(p.KB, PC_KB);
+    c.KW = corrected(p.KW, PC_KW);
+    c.KS = corrected(p.KS, PC_KS);
+    c.KF = corrected(p.KF, PC_KF);
     c.KSi = p.KSi;
-    const double lnK_therm = -171.9065 + -0.077993 * Tk + 2839.319 / Tk + 71.595 * log10(Tk);
-    const double lnK_sea = ((-0.77712 + 0.0028426 * Tk + 178.34 / Tk) * sqrt(S) + -0.07711 * S + 0.0041249 * pow(S, 1.5));
-    c.KSP = pressure_correction(PC_CAL, Tk, P) * pow(10.0, lnK_therm + lnK_sea);
+    const double sS = sqrt(S);
+    const double lnK_therm = -171.9065 + -0.077993 * Tk + rT.under(2839.319) + 71.595 * m_log10(Tk);
+    const double lnK_sea = ((-0.77712 + 0.0028426 * Tk + rT.under(178.34)) * sS + -0.07711 * S + 0.0041249 * (S * sS));
+    c.KSP = corrected(m_exp10(lnK_therm + lnK_sea), PC_CAL);
 }
 
 __device__ __forceinline__ CarbonParams omega_params(const OmegaConst& c, double DIC, double Alk, double Si)
@@ -601,7 +606,6 @@ __device__ __forceinline__ CarbonParams omega_params(const OmegaConst& c, double
     p.fluoride = c.fluoride;
     p.Alk = Alk * c.conv;
     p.DIC = DIC * c.conv;
-    p.phosphate = 0.0;
     p.silicate = Si * c.conv;
     p.K1 = c.K1;
     p.K2 = c.K2;
@@ -609,7 +613,6 @@ __device__ __forceinline__ CarbonParams omega_params(const OmegaConst& c, double
     p.KW = c.KW;
     p.KS = c.KS;
     p.KF = c.KF;
-    p.KP1 = p.KP2 = p.KP3 = 0.0;
     p.KSi = c.KSi;
     p.K0 = 0.0;
     p.Tk = 0.0;
@@ -626,14 +629,14 @@ __device__ __forceinline__ double omega_from_H(const OmegaConst& c, const Carbon
     return c.ca * co3 / c.KSP;
 }
 
-// The reference solve: damped Newton from 10^-pH₀.
+// The root of the reference solve, the damped Newton from 10^-pH₀.
 __device__ __forceinline__ double calcite_saturation(double DIC, double Alk, double T, double S, double Si, double P,
                                                      const obme_carbon_solver& s, int& evals)
 {
     OmegaConst c;
     omega_constants(T, S, P, c);
     const CarbonParams p = omega_params(c, DIC, Alk, Si);
-    const double H = solve_for_H<true>(p, s, pow(10.0, -s.initial_pH_guess), evals);
+    const double H = root_H<true>(p, s, evals);
     return omega_from_H(c, p, H);
 }
 

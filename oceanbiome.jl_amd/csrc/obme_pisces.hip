@@ -46,7 +46,7 @@ struct PiscesArgs {
     float* Hs;              // [ncell]: [H+] of the last stage (FP32-mixed warm start)
     int have_H;             // Hs holds the previous stage's [H+]
     double* sflux;          // [2][Nx*Ny]: top CO2 and O2 fluxes of the stage (gas exchange on)
-    double* Hsurf;          // [Nx*Ny]: [H+] of the surface pCO2 solve (FP32-mixed warm start)
+    double* Hsurf;          // [Nx*Ny]: [H+] of the surface pCO2 solve (warm start)
     obme_co2_exchange co2;
     obme_o2_exchange o2;
     FT* zeu;                // [Nx*Ny]
@@ -243,13 +243,17 @@ __global__ void __launch_bounds__(256) k_pisces_surface(PiscesArgs<FT> a)
     if (a.co2.enabled) {
         SurfaceCarbon sc;
         surface_carbon_setup(a.co2, T, S, a.co2.wind_speed, sc);
-        double H = (sizeof(FT) == 4) ? a.Hsurf[col] : 0.0;
-        double pH = 0.0;
+        const double DIC = (double)a.in[OBME_PI_DIC][p], Alk = (double)a.in[OBME_PI_ALK][p];
+        // FP64: the damped Newton's root, and in a stepper's call its
+        // refinement from the previous stage's
+        double H = (sizeof(FT) == 4 || a.have_H) ? a.Hsurf[col] : 0.0;
         int ev = 0;
-        Fc = surface_flux_warm(sc, a.solver, (double)a.in[OBME_PI_DIC][p], (double)a.in[OBME_PI_ALK][p],
-                               a.co2.air_concentration, sizeof(FT) == 4 ? 1 : 0, H, pH, ev,
-                               sizeof(FT) == 4 ? FP32_NEWTON_TOL : 1e-14);
-        if (sizeof(FT) == 4) a.Hsurf[col] = H;
+        if (sizeof(FT) == 8 && !(H > 0.0))
+            Fc = surface_flux(sc, a.solver, DIC, Alk, a.co2.air_concentration, 0, H, ev);
+        else
+            Fc = surface_flux_warm(sc, a.solver, DIC, Alk, a.co2.air_concentration, H, ev,
+                                   sizeof(FT) == 4 ? FP32_NEWTON_TOL : FP64_NEWTON_TOL);
+        a.Hsurf[col] = H;
     }
     if (a.o2.enabled) Fo = o2_flux(a.o2, (double)a.in[OBME_PI_O2][p], T, S);
     a.sflux[col] = Fc;
@@ -712,10 +716,10 @@ __global__ void __launch_bounds__(PF_WAVES * 64, OBME_PISCES_PF_OCC) k_pisces_fu
                 double kO2, airO2;
                 surface_unpack(s_surf[wv], scb, kO2, airO2);
                 if (a.co2.enabled) {
-                    double pH = 0.0, Hsurf = s_hsurf[wv];
+                    double Hsurf = s_hsurf[wv];
                     int ev = 0;
                     Fc = surface_flux_warm(scb, a.solver, (double)v[OBME_PI_DIC], (double)v[OBME_PI_ALK],
-                                           a.co2.air_concentration, 1, Hsurf, pH, ev, FP32_NEWTON_TOL);
+                                           a.co2.air_concentration, Hsurf, ev, FP32_NEWTON_TOL);
                     s_hsurf[wv] = Hsurf;
                 }
                 if (a.o2.enabled) Fo = kO2 * ((double)v[OBME_PI_O2] - airO2);

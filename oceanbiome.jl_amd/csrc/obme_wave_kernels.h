@@ -795,10 +795,9 @@ __device__ __forceinline__ void top_steps(const WaveArgs<FT>& w, FT* rec)
             rec[at] = X[PI];
             rec[at + w.ncol] = X[S0];
             rec[at + 2 * (size_t)w.ncol] = X[S1];
-            double pH = 0.0;
             int ev = 0;
-            const double F = surface_flux_warm(sc, a.solver, (double)X[7], (double)X[8], a.co2.air_concentration, 1, H,
-                                               pH, ev, F32 ? FP32_NEWTON_TOL : FP64_NEWTON_TOL);
+            const double F = surface_flux_warm(sc, a.solver, (double)X[7], (double)X[8], a.co2.air_concentration, H, ev,
+                                               F32 ? FP32_NEWTON_TOL : FP64_NEWTON_TOL);
             FT pr, pb, PAR;
             if constexpr (F32) {
                 const float lg = m_log2(X[PI]);
