@@ -38,8 +38,9 @@ struct PiscesArgs {
     const FT* in[NTR];      // stage input (parent arrays)
     FT* out[NW];            // stage output (parent arrays) or tendencies (TILE mode)
     FT* Gm;                 // previous-stage transitions [NW][ncell] (compact)
-    FT* PAR;                // [4][ncell] compact: total, band 1, 2, 3
-    FT* Omega;              // [ncell] compact
+    FT* PAR[4];             // total, band 1, 2, 3 (each may be null): [ncell] compact, or parent
+    FT* Omega;              // arrays, like Omega, where `parents` is set
+    int parents;
     const FT* oc;           // [OMEGA_CONST_FIELDS][ncell]: per-cell carbonate constants (the
                             // element type: FP32-mixed Ω solves in FP64 on FP32-rounded constants)
     FT* tfac;               // [TFAC_FIELDS][ncell]: temperature factors of the FP64 step, or null
@@ -86,98 +87,126 @@ __device__ __forceinline__ unsigned pidx(const PiscesArgs<FT>& a, int i, int j, 
     return a.base0 + (unsigned)i + a.sx * (unsigned)j + a.sxy * (unsigned)k;
 }
 
-// Thread per column: MultiBand PAR (multi_band.jl:147-165) top-down, the
-// euphotic depth (compute_euphotic_depth.jl:3-33, surface value = the
-// boundary value of PAR at z = 0) and the mixed-layer mean of the total PAR
-// (mean_mixed_layer_properties.jl:25-47) in the same sweep.
+// MultiBand PAR (multi_band.jl:147-165) top-down, the euphotic depth
+// (compute_euphotic_depth.jl:3-33, surface value = the boundary value of PAR
+// at z = 0) and the mixed-layer mean of the total PAR
+// (mean_mixed_layer_properties.jl:25-47).
+// A block takes CB columns that follow each other in x, in chunks of CL levels
+// from the top.  The loads, logarithms and exponentials go level by level over
+// all its threads (a row of CB cells is one segment of 64 or 128 B); what runs
+// down a column, in its order, goes through LDS: one lane per column and band
+// multiplies, one per column sums and looks for the euphotic crossing.  One
+// thread per column left the chip to Nx Ny / 64 waves, each a chain of Nz
+// logarithms and exponentials: 45 us at 128x96x64 in FP32 (now 17), 81 us
+// at 120x100x48 in FP64 (now 23).
+constexpr int CB = 16, CL = 64, COLUMN_THREADS = 256;
 template <typename FT>
-__global__ void __launch_bounds__(256) k_pisces_columns(PiscesArgs<FT> a)
+__global__ void __launch_bounds__(COLUMN_THREADS) k_pisces_columns(PiscesArgs<FT> a)
 {
-    const int col = blockIdx.x * blockDim.x + threadIdx.x;
-    if (col >= a.Nx * a.Ny) return;
-    const int i = col % a.Nx, j = col / a.Nx;
+    __shared__ FT s_band[3][CL][CB];
+    constexpr int LG = COLUMN_THREADS / CB;      // level rows in flight
+    const int c = threadIdx.x % CB, g = threadIdx.x / CB;
+    const int ncol = a.Nx * a.Ny;
+    const int col = blockIdx.x * CB + c;
+    const bool act = col < ncol;
+    const int i = act ? col % a.Nx : 0, j = act ? col / a.Nx : 0;
     const int Nz = a.Nz;
-    const long ncell = (long)a.Nx * a.Ny * Nz;
     const FT* zc = a.lev;
     const FT* zf = a.lev + Nz;
     const FT* sc = a.pp + OBME_PP_SCALARS;
     const FT zmxl = sc[OBME_PS_MIXED_LAYER_DEPTH];
-    const FT PAR0 = a.surf ? a.surf[col] : a.surface_PAR;
+    const FT PAR0 = a.surf ? a.surf[act ? col : 0] : a.surface_PAR;
     const FT thr = PAR0 * FT(1e-3);
-    const FT lthr = m_log(thr);
-    FT band[3] = {FT(0), FT(0), FT(0)};
-    FT acc = 0, depth = 0;
+    const long plane = (long)ncol;
+    // Chl^e of the three bands from one logarithm (FP64: exp(e ln Chl),
+    // within a few ulp of pow; pow for Chl <= 0 or a zero exponent)
+    const bool pw = !(a.e[0] != FT(0) && a.e[1] != FT(0) && a.e[2] != FT(0));
+    FT band = FT(0);                             // of lane (column c, band g < 3)
+    FT acc = 0, depth = 0;                       // of lane (column c, g = 0)
     FT PARup = 0;
     // the euphotic crossing: the first level below the top with PAR <= thr,
     // its PAR and the PAR of the level above (the logarithms after the walk)
     int kc = -1;
     FT Pc = FT(0), Pu = FT(0);
-    // Chl^e of the three bands from one logarithm (FP64: exp(e ln Chl),
-    // within a few ulp of pow; pow for Chl <= 0 or a zero exponent)
-    const bool pw = !(a.e[0] != FT(0) && a.e[1] != FT(0) && a.e[2] != FT(0));
-    const long plane = (long)a.Nx * a.Ny;
-    // One thread per column, one wave per SIMD: the walk goes in chunks of
-    // four levels, whose loads and logarithms and exponentials are
-    // independent of each other; only the bands' running products, the
-    // stores and the sums follow level by level.
-    constexpr int CH = 4;
-    for (int k0 = Nz - 1; k0 >= 0; k0 -= CH) {
-        FT E[CH][3];
+    for (int k0 = Nz - 1; k0 >= 0; k0 -= CL) {
+        const int nl = k0 + 1 < CL ? k0 + 1 : CL;
 #pragma unroll
-        for (int u = 0; u < CH; u++) {
-            const int k = k0 - u;
-            const int kk = k >= 0 ? k : 0;
-            const unsigned p = pidx(a, i, j, kk);
-            const FT Chl = a.in[OBME_PI_PCHL][p] + a.in[OBME_PI_DCHL][p];
-            const bool via_log = Chl > FT(0) && !pw;
-            const FT lChl = via_log ? m_log(Chl) : FT(0);
-            // the exponent increment from the level above (the top level:
-            // from the surface)
-            const FT dzl = (kk == Nz - 1) ? zc[kk] : zc[kk] - zc[kk + 1 < Nz ? kk + 1 : kk];
+        for (int u = 0; u < CL / LG; u++) {
+            const int l = g + u * LG, k = k0 - l;
+            if (l < nl && act) {
+                const unsigned p = pidx(a, i, j, k);
+                const FT Chl = a.in[OBME_PI_PCHL][p] + a.in[OBME_PI_DCHL][p];
+                const bool via_log = Chl > FT(0) && !pw;
+                const FT lChl = via_log ? m_log(Chl) : FT(0);
+                // the exponent increment from the level above (the top level:
+                // from the surface)
+                const FT dzl = (k == Nz - 1) ? zc[k] : zc[k] - zc[k + 1];
 #pragma unroll
-            for (int n = 0; n < 3; n++) {
-                const FT ce = via_log ? m_exp(a.e[n] * lChl) : m_pow(Chl, a.e[n]);
-                const FT att = a.kw[n] + a.chi[n] * ce;
-                E[u][n] = m_exp(dzl * att);
+                for (int n = 0; n < 3; n++) {
+                    const FT ce = via_log ? m_exp(a.e[n] * lChl) : m_pow(Chl, a.e[n]);
+                    const FT att = a.kw[n] + a.chi[n] * ce;
+                    s_band[n][l][c] = m_exp(dzl * att);
+                }
             }
         }
-#pragma unroll
-        for (int u = 0; u < CH; u++) {
-            const int k = k0 - u;
-            if (k < 0) break;
-#pragma unroll
-            for (int n = 0; n < 3; n++)
-                band[n] = (k == Nz - 1) ? PAR0 * a.division[n] * E[u][n] : band[n] * E[u][n];
-            const FT PAR = band[0] + band[1] + band[2];
-            const long c = (long)col + plane * k;
-            a.PAR[c] = PAR;
-            a.PAR[ncell + c] = band[0];
-            a.PAR[2 * ncell + c] = band[1];
-            a.PAR[3 * ncell + c] = band[2];
-            const bool cross = kc < 0 && k < Nz - 1 && PAR <= thr;
-            kc = cross ? k : kc;
-            Pc = cross ? PAR : Pc;
-            Pu = cross ? PARup : Pu;
-            PARup = PAR;
-            // mixed-layer integral, top cell first
-            const FT zk = zf[k];
-            const FT zk1 = (k + 1 < Nz) ? zf[k + 1] : FT(a.zf_top);
-            const FT dzk = zk1 - zk;
-            const FT dzk1 = (zk1 > zmxl) ? zk1 - zmxl : FT(0);
-            const FT dz = (zk >= zmxl) ? dzk : dzk1;
-            acc = acc + PAR * dz;
-            depth = depth + dz;
+        __syncthreads();
+        if (g < 3 && act) {
+            const FT share = g == 0 ? a.division[0] : (g == 1 ? a.division[1] : a.division[2]);
+            FT* E = &s_band[g][0][c];
+#pragma unroll 8
+            for (int l = 0; l < nl; l++) {
+                band = (k0 - l == Nz - 1) ? PAR0 * share * E[l * CB] : band * E[l * CB];
+                E[l * CB] = band;
+            }
         }
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < CL / LG; u++) {
+            const int l = g + u * LG, k = k0 - l;
+            if (l < nl && act) {
+                const FT b0 = s_band[0][l][c], b1 = s_band[1][l][c], b2 = s_band[2][l][c];
+                const FT PAR = b0 + b1 + b2;
+                const long q = a.parents ? (long)pidx(a, i, j, k) : (long)col + plane * k;
+                if (a.PAR[0]) a.PAR[0][q] = PAR;
+                if (a.PAR[1]) a.PAR[1][q] = b0;
+                if (a.PAR[2]) a.PAR[2][q] = b1;
+                if (a.PAR[3]) a.PAR[3][q] = b2;
+                s_band[0][l][c] = PAR;
+            }
+        }
+        __syncthreads();
+        if (g == 0 && act) {
+#pragma unroll 8
+            for (int l = 0; l < nl; l++) {
+                const int k = k0 - l;
+                const FT PAR = s_band[0][l][c];
+                const bool cross = kc < 0 && k < Nz - 1 && PAR <= thr;
+                kc = cross ? k : kc;
+                Pc = cross ? PAR : Pc;
+                Pu = cross ? PARup : Pu;
+                PARup = PAR;
+                // mixed-layer integral, top cell first
+                const FT zk = zf[k];
+                const FT zk1 = (k + 1 < Nz) ? zf[k + 1] : FT(a.zf_top);
+                const FT dzk = zk1 - zk;
+                const FT dzk1 = (zk1 > zmxl) ? zk1 - zmxl : FT(0);
+                const FT dz = (zk >= zmxl) ? dzk : dzk1;
+                acc = acc + PAR * dz;
+                depth = depth + dz;
+            }
+        }
+        if (k0 >= CL) __syncthreads();
     }
+    if (g != 0 || !act) return;
     // the euphotic depth, interpolated in log PAR with the level above
     FT zeu = FT(-INFINITY);
     if (kc >= 0) {
         const FT lPAR = m_log(Pc), lPARup = m_log(Pu);
-        zeu = zc[kc] + (lthr - lPAR) * (zc[kc] - zc[kc + 1]) / (lPAR - lPARup);
+        zeu = zc[kc] + (m_log(thr) - lPAR) * (zc[kc] - zc[kc + 1]) / (lPAR - lPARup);
     }
     if (!(zeu > FT(-INFINITY) && zeu < FT(INFINITY))) zeu = zc[0] - (Nz > 1 ? zc[1] - zc[0] : FT(1));
-    a.zeu[col] = zeu;
-    a.mlPAR[col] = acc / depth;
+    if (a.zeu) a.zeu[col] = zeu;
+    if (a.mlPAR) a.mlPAR[col] = acc / depth;
 }
 
 // Thread per cell: calcite saturation at the hydrostatic pressure
@@ -196,7 +225,7 @@ __global__ void __launch_bounds__(256) k_pisces_omega(PiscesArgs<FT> a)
     const double g = (double)a.pp[OBME_PP_SCALARS + OBME_PS_GRAVITY];
     const double P = fabs(z) * g * 1026 / 100000;
     int ev = 0;
-    a.Omega[c] = (FT)calcite_saturation((double)a.in[OBME_PI_DIC][p], (double)a.in[OBME_PI_ALK][p],
+    a.Omega[a.parents ? (long)p : c] = (FT)calcite_saturation((double)a.in[OBME_PI_DIC][p], (double)a.in[OBME_PI_ALK][p],
                                         (double)a.in[OBME_PI_T][p], (double)a.in[OBME_PI_S][p],
                                         (double)a.in[OBME_PI_SI][p], P, a.solver, ev);
 }
@@ -382,10 +411,10 @@ k_pisces_cell(PiscesArgs<FT> a)
     } else {
         A.Omega = a.Omega[c];
     }
-    A.PAR = a.PAR[c];
-    A.PAR1 = a.PAR[ncell + c];
-    A.PAR2 = a.PAR[2 * ncell + c];
-    A.PAR3 = a.PAR[3 * ncell + c];
+    A.PAR = a.PAR[0][c];
+    A.PAR1 = a.PAR[1][c];
+    A.PAR2 = a.PAR[2][c];
+    A.PAR3 = a.PAR[3][c];
     A.wPOCc = (wP[k] + wP[k + 1]) / 2;
     A.wGOCc = (wG[k] + wG[k + 1]) / 2;
     FT G[NW];
@@ -1076,7 +1105,7 @@ static PiscesArgs<FT> pisces_args(const obme_pisces* h, double t)
     PiscesArgs<FT> a;
     std::memset(&a, 0, sizeof(a));
     a.Gm = (FT*)h->d_Gm;
-    a.PAR = (FT*)h->d_PAR;
+    for (int n = 0; n < 4; n++) a.PAR[n] = (FT*)h->d_PAR + (size_t)n * h->ncell;
     a.Omega = (FT*)h->d_Omega;
     a.zeu = (FT*)h->d_zeu;
     a.mlPAR = (FT*)h->d_mlPAR;
@@ -1185,7 +1214,7 @@ static obme_status pisces_stage(obme_pisces* h, const void* const* in, void* con
         if (r != OBME_OK) return r;
     }
     const int bs = 256;
-    hipLaunchKernelGGL(k_pisces_columns<FT>, dim3((unsigned)((h->ncol + bs - 1) / bs)), dim3(bs), 0, s, a);
+    hipLaunchKernelGGL(k_pisces_columns<FT>, dim3((unsigned)((h->ncol + CB - 1) / CB)), dim3(COLUMN_THREADS), 0, s, a);
     OBME_HIP_TRY(hipGetLastError());
     if (a.sflux) {
         hipLaunchKernelGGL(k_pisces_surface<FT>, dim3((unsigned)((h->ncol + bs - 1) / bs)), dim3(bs), 0, s, a);
@@ -1253,33 +1282,33 @@ static obme_status pisces_stage_any(obme_pisces* h, const void* const* in, void*
                                   : pisces_stage<float>(h, in, out, t, dt, stage, mode, have_H, s);
 }
 
+// the auxiliary fields, straight into the caller's arrays (null: not wanted)
 template <typename FT>
-static obme_status pisces_copy_aux(obme_pisces* h, void* PAR, void* const* PARn, void* Omega, void* zeu,
-                                   void* mlPAR, hipStream_t s)
+static obme_status pisces_update(obme_pisces* h, const void* const* tracers, void* PAR, void* const* PARn,
+                                 void* Omega, void* zeu, void* mlPAR, double t, hipStream_t s)
 {
-    // compact interior -> parent layout for the 3-D outputs
-    const obme_grid& g = h->cfg.grid;
-    const size_t es = sizeof(FT);
-    const size_t sx = (size_t)(g.Nx + 2 * g.Hx), sxy = sx * (size_t)(g.Ny + 2 * g.Hy);
-    auto put3 = [&](void* dst, const char* src) -> obme_status {
-        if (!dst) return OBME_OK;
-        for (int k = 0; k < g.Nz; k++) {
-            char* d = (char*)dst + ((size_t)g.Hx + sx * (size_t)g.Hy + sxy * (size_t)(k + g.Hz)) * es;
-            const char* c = src + (size_t)k * g.Nx * g.Ny * es;
-            OBME_HIP_TRY(hipMemcpy2DAsync(d, sx * es, c, (size_t)g.Nx * es, (size_t)g.Nx * es, (size_t)g.Ny,
-                                          hipMemcpyDeviceToDevice, s));
-        }
-        return OBME_OK;
-    };
-    const char* P = (const char*)h->d_PAR;
-    obme_status st = put3(PAR, P);
-    for (int n = 0; n < 3 && st == OBME_OK; n++)
-        if (PARn) st = put3(PARn[n], P + (size_t)(n + 1) * h->ncell * es);
-    if (st == OBME_OK) st = put3(Omega, (const char*)h->d_Omega);
-    if (st == OBME_OK && zeu) OBME_HIP_TRY(hipMemcpyAsync(zeu, h->d_zeu, h->ncol * es, hipMemcpyDeviceToDevice, s));
-    if (st == OBME_OK && mlPAR)
-        OBME_HIP_TRY(hipMemcpyAsync(mlPAR, h->d_mlPAR, h->ncol * es, hipMemcpyDeviceToDevice, s));
-    return st;
+    // the modifiers first: the tracers are rescaled in place
+    obme_status r = pisces_scale<FT>(h, tracers, s);
+    if (r != OBME_OK) return r;
+    PiscesArgs<FT> a = pisces_args<FT>(h, t);
+    for (int n = 0; n < NTR; n++) a.in[n] = (const FT*)tracers[n];
+    a.parents = 1;
+    a.PAR[0] = (FT*)PAR;
+    for (int n = 0; n < 3; n++) a.PAR[n + 1] = PARn ? (FT*)PARn[n] : nullptr;
+    a.Omega = (FT*)Omega;
+    a.zeu = (FT*)zeu;
+    a.mlPAR = (FT*)mlPAR;
+    if (a.PAR[0] || a.PAR[1] || a.PAR[2] || a.PAR[3] || zeu || mlPAR) {
+        hipLaunchKernelGGL(k_pisces_columns<FT>, dim3((unsigned)((h->ncol + CB - 1) / CB)), dim3(COLUMN_THREADS), 0, s,
+                           a);
+        OBME_HIP_TRY(hipGetLastError());
+    }
+    if (Omega) {
+        const int bs = 256;
+        hipLaunchKernelGGL(k_pisces_omega<FT>, dim3((unsigned)((h->ncell + bs - 1) / bs)), dim3(bs), 0, s, a);
+        OBME_HIP_TRY(hipGetLastError());
+    }
+    return OBME_OK;
 }
 
 extern "C" obme_status obme_pisces_update_state(obme_pisces* h, const void* const* tracers, void* PAR,
@@ -1290,26 +1319,9 @@ extern "C" obme_status obme_pisces_update_state(obme_pisces* h, const void* cons
     for (int n = 0; n < NTR; n++)
         if (!tracers[n]) return obme_fail(OBME_ERR_INVALID, "null tracer pointer");
     hipStream_t s = (hipStream_t)stream;
-    const int bs = 256;
-    {
-        // the modifiers first: the tracers are rescaled in place
-        obme_status r = (h->prec == OBME_FP64) ? pisces_scale<double>(h, tracers, s) : pisces_scale<float>(h, tracers, s);
-        if (r != OBME_OK) return r;
-    }
-    if (h->prec == OBME_FP64) {
-        PiscesArgs<double> a = pisces_args<double>(h, t);
-        for (int n = 0; n < NTR; n++) a.in[n] = (const double*)tracers[n];
-        hipLaunchKernelGGL(k_pisces_columns<double>, dim3((unsigned)((h->ncol + bs - 1) / bs)), dim3(bs), 0, s, a);
-        hipLaunchKernelGGL(k_pisces_omega<double>, dim3((unsigned)((h->ncell + bs - 1) / bs)), dim3(bs), 0, s, a);
-        OBME_HIP_TRY(hipGetLastError());
-        return pisces_copy_aux<double>(h, PAR, PARn, Omega, euphotic_depth, mixed_layer_PAR, s);
-    }
-    PiscesArgs<float> a = pisces_args<float>(h, t);
-    for (int n = 0; n < NTR; n++) a.in[n] = (const float*)tracers[n];
-    hipLaunchKernelGGL(k_pisces_columns<float>, dim3((unsigned)((h->ncol + bs - 1) / bs)), dim3(bs), 0, s, a);
-    hipLaunchKernelGGL(k_pisces_omega<float>, dim3((unsigned)((h->ncell + bs - 1) / bs)), dim3(bs), 0, s, a);
-    OBME_HIP_TRY(hipGetLastError());
-    return pisces_copy_aux<float>(h, PAR, PARn, Omega, euphotic_depth, mixed_layer_PAR, s);
+    return (h->prec == OBME_FP64)
+               ? pisces_update<double>(h, tracers, PAR, PARn, Omega, euphotic_depth, mixed_layer_PAR, t, s)
+               : pisces_update<float>(h, tracers, PAR, PARn, Omega, euphotic_depth, mixed_layer_PAR, t, s);
 }
 
 extern "C" obme_status obme_pisces_add_tendencies(obme_pisces* h, const void* const* tracers, void* const* G,
