@@ -10,6 +10,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <algorithm>
+#include <climits>
 #include <cstring>
 #include <mutex>
 #include <string>
@@ -855,16 +856,23 @@ static WaveShape wave_shape(const obme_handle* h, int mode, int nsteps, bool gen
     // One step or a hook: the sweep moves a level's values in longer runs and
     // is the faster where its columns fill the chip.  On 64 levels, us per
     // step, sweep | this: FP32 16 384 columns 59 | 26, 65 536 64 | 81; FP64
-    // 180 | 65, 197 | 247; FP32 hooks 57 | 35, 110 | 158.  From two steps on,
-    // with the state in registers between them, this is the faster everywhere
+    // 180 | 65, 197 | 247; FP32 hooks 57 | 35, 110 | 158; FP64 hooks on 38 400
+    // 222 | 238.  The hooks of the centred and WENO schemes cross later (on
+    // 38 400 columns FP32 154 | 65, FP64 275 | 134).  From two steps on, with
+    // the state in registers between them, this is the faster everywhere
     // (262 144 columns, two steps: 507 | 486).  The centred and WENO steps and
     // the scaling and sediment variants are: a launch per stage and the flux
     // solve in the walk are what they replace.
-    if (ncol > 40960 && (mode != TILE_STEP || (nsteps < 2 && !general && !h->staged))) return best;
+    long most = LONG_MAX;
+    if (mode != TILE_STEP) most = !h->staged ? 32768 : (sizeof(FT) == 4 ? 131072 : 65536);
+    else if (nsteps < 2 && !general && !h->staged) most = 40960;
+    if (ncol > most) return best;
     double cost = 0.0;
     for (int i = 0; i < 4 && wave_levels<FT>(i); i++) {
         const int L = wave_levels<FT>(i);
         if (L > 2 && (mode != TILE_STEP || general || h->staged)) continue;
+        // (FP32 with a sediment: one level per lane, whose sinking rounds as the sweep's)
+        if (L > 1 && sizeof(FT) == 4 && mode == TILE_STEP && h->sediment) continue;
         const int lpc = (Nz + L - 1) / L;
         if (lpc > 64) continue;
         const int cpw = 64 / lpc;

@@ -510,9 +510,13 @@ __device__ __forceinline__ void column_wave(const WaveArgs<FT>& w, FT* lds)
                         x0 = I[S0][m];
                         x1 = I[S1][m];
                     }
-                const FT f = a.sed_w0 * x0 + a.sed_w1 * x1;
+                // (FP32: the product that the fused sum leaves unrounded is the
+                // one the sweep's compiled stages take, so that the FP64
+                // storage is the same to the bit from either kernel)
+                const bool second = F32 && st > 0 && ((CARB & 1) != 0) != (w.scale != 0);
+                const FT f = second ? fma(a.sed_w1, x1, a.sed_w0 * x0) : fma(a.sed_w0, x0, a.sed_w1 * x1);
                 const FT qf = f / (a.sed_k + f);
-                const FT e = a.sed_a + a.sed_b * (qf * qf);
+                const FT e = fma(a.sed_b, qf * qf, a.sed_a);
                 cpl = ((FT(1) - e) * f) / a.sed_dz0;
                 const double ge = (double)(e * f);
                 const bool init = a.sed_init && sn == 0;
@@ -672,9 +676,9 @@ __device__ __forceinline__ void column_wave(const WaveArgs<FT>& w, FT* lds)
                         x0 = U[S0][m];
                         x1 = U[S1][m];
                     }
-                const FT f = a.sed_w0 * x0 + a.sed_w1 * x1;
+                const FT f = fma(a.sed_w0, x0, a.sed_w1 * x1);
                 const FT qf = f / (a.sed_k + f);
-                const FT e = a.sed_a + a.sed_b * (qf * qf);
+                const FT e = fma(a.sed_b, qf * qf, a.sed_a);
                 if (a.storage) a.storage[qc] = sed_u;
                 a.sedG[qc] = (double)(e * f);
                 a.sedG[w.ncol + qc] = sed_ge;
