@@ -81,17 +81,54 @@ __device__ __forceinline__ double day_length(double t, double phi)
     return (24 - 24.0 / 180 * (acos(L) * (180.0 / 3.141592653589793))) * 3600.0;
 }
 
-// Per-stage uniform inputs of the transitions.
+// Per-stage uniform inputs of the transitions, from the day lengths
+// d = day_length(φ, t) (the argument order of growth_rate.jl:30) and
+// d' = day_length(t, φ) (growth_rate.jl:128).  There is no scalar float
+// arithmetic: what is the same for every cell is formed on the host (here, and
+// below what depends on the parameters alone).
 template <typename FT>
 struct StageConst {
-    FT dl_growth;   // day_length(φ, t): the argument order of growth_rate.jl:30
-    FT dl_chl;      // day_length(t, φ): growth_rate.jl:128
+    FT f1;          // f₁(d) = 1.5 d / (d + 1/2 day)
+    FT rl[2];       // 1 / (d (basal respiration + reference growth)): nanophytoplankton, diatoms
+    FT chl;         // d' / f₁(d')
 };
+
+// Combinations of the parameters, behind them in the device's array.
+enum {
+    PD_KSI_N, PD_KSI_D,        // 7 Sc² / (pk² + Sc²) of the half saturation for silicate
+    PD_RFE_N, PD_RFE_D,        // 1 / θFe optimum
+    PD_RKAPPA,                 // 1 / κ
+    PD_UTW,                    // m₀ / (1 - e₀) of the mesozooplankton
+    PD_UT_KEEP,                // 1 - e₀ - σ
+    PD_DOC_RATE,               // λ / Bact reference
+    PD_RFIX_E,                 // 1 / E fixation
+    PD_RAIN_ZM,                // min(1, -50 / zmxl)
+    PD_O2_N,                   // θ nitrification / θN
+    PD_COUNT
+};
+// (p: the OBME_PP_COUNT parameters)
+inline void derived_parameters(const double* p, double* d)
+{
+    const double *n = p + OBME_PP_NANO, *m = p + OBME_PP_DIATOMS, *z = p + OBME_PP_MESO, *s = p + OBME_PP_SCALARS;
+    const double c2 = s[OBME_PS_SILICATE_CLIMATOLOGY] * s[OBME_PS_SILICATE_CLIMATOLOGY];
+    d[PD_KSI_N] = 7 * c2 / (n[OBME_PH_PK] * n[OBME_PH_PK] + c2);
+    d[PD_KSI_D] = 7 * c2 / (m[OBME_PH_PK] * m[OBME_PH_PK] + c2);
+    d[PD_RFE_N] = 1 / n[OBME_PH_THETA_FE_OPT];
+    d[PD_RFE_D] = 1 / m[OBME_PH_THETA_FE_OPT];
+    d[PD_RKAPPA] = 1 / s[OBME_PS_KAPPA];
+    d[PD_UTW] = 1 / (1 - z[OBME_PZ_E0]) * z[OBME_PZ_M0];
+    d[PD_UT_KEEP] = 1 - z[OBME_PZ_E0] - z[OBME_PZ_SIGMA];
+    d[PD_DOC_RATE] = s[OBME_PS_DOC_LAMBDA] / s[OBME_PS_DOC_BACT_REF];
+    d[PD_RFIX_E] = 1 / s[OBME_PS_FIX_E];
+    const double q = -50 / s[OBME_PS_MIXED_LAYER_DEPTH];
+    d[PD_RAIN_ZM] = q < 1 ? q : 1;     // (the depth is below 0, checked at create)
+    d[PD_O2_N] = s[OBME_PS_O2_NITRIF] / s[OBME_PS_THETAN];
+}
 
 // Auxiliary values of one cell.
 template <typename FT>
 struct Aux {
-    FT z, zmxl, zeu, kappa, mlPAR, Omega, PAR, PAR1, PAR2, PAR3, wPOCc, wGOCc;
+    FT z, zmxl, zeu, mlPAR, Omega, PAR, PAR1, PAR2, PAR3, wPOCc, wGOCc;
 };
 
 // The factors of the transitions that depend on the temperature alone: the
@@ -152,7 +189,8 @@ __device__ __forceinline__ FT nitrogen_lim(FT N1, FT N2, FT K1, FT K2)
 // the growth rate (growth_rate.jl:3-47, GrowthRespirationLimitedProduction :104-111).
 template <typename FT>
 __device__ __forceinline__ void phyto_state(const FT* ph, const FT* sc, const FT* v, const Aux<FT>& A,
-                                            const StageConst<FT>& sk, FT btT, FT I, FT IChl, FT IFe, Phyto<FT>& s)
+                                            const StageConst<FT>& sk, const FT* pd, int cls, FT btT, FT I, FT IChl, FT IFe,
+                                            Phyto<FT>& s)
 {
     const FT NO3 = v[OBME_PI_NO3], NH4 = v[OBME_PI_NH4], PO4 = v[OBME_PI_PO4], Si = v[OBME_PI_SI];
     s.I = I;
@@ -170,25 +208,21 @@ __device__ __forceinline__ void phyto_state(const FT* ph, const FT* sc, const FT
     const FT thm = FT(1000) * (FT(0.0016) / FT(55.85) * FT(12) * thChl
                                + FT(1.5) * FT(1.21e-5) * FT(14) / (FT(55.85) * FT(7.625)) * s.LN
                                + FT(1.15e-4) * FT(14) / (FT(55.85) * FT(7.625)) * s.LNO3);
-    s.LFe = jmin(FT(1), jmax(FT(0), qdiv(thFe - thm, ph[OBME_PH_THETA_FE_OPT])));
-    const FT Sc = sc[OBME_PS_SILICATE_CLIMATOLOGY];
-    const FT pk = ph[OBME_PH_PK];
-    const FT KSi = Ksi + qdiv(7 * (Sc * Sc), pk * pk + Sc * Sc);
+    s.LFe = jmin(FT(1), jmax(FT(0), (thFe - thm) * pd[PD_RFE_N + cls]));
+    const FT KSi = Ksi + pd[PD_KSI_N + cls];
     FT LSi = qdiv(Si, Si + KSi);
     if (ph[OBME_PH_SI_LIMITED] == FT(0)) LSi = FT(INFINITY);
     s.L = jmin4(s.LN, s.LPO4, s.LFe, LSi);
     // growth rate μ(L)
     const FT PAR = ph[OBME_PH_BETA1] * A.PAR1 + ph[OBME_PH_BETA2] * A.PAR2 + ph[OBME_PH_BETA3] * A.PAR3;
-    const FT dl = sk.dl_growth;
     const FT d = jmax(FT(0), A.zeu - A.zmxl);
-    const FT drt = qdiv(d * d, A.kappa);
+    const FT drt = d * d * pd[PD_RKAPPA];
     const FT mui = ph[OBME_PH_MU0] * btT;
-    const FT f1 = qdiv(FT(1.5) * dl, dl + FT(0.5 * DAYS));
     const FT f2 = 1 - qdiv(drt, drt + ph[OBME_PH_DARK_TOLERANCE]);
     const FT alpha = ph[OBME_PH_ALPHA0] * (1 + ph[OBME_PH_BETA] * m_exp(-PAR));
     const FT theta = qdiv(IChl, 12 * I + eps0<FT>());
-    const FT fl = 1 - m_exp(qdiv(-alpha * theta * PAR, dl * (ph[OBME_PH_BASAL_RESPIRATION] + ph[OBME_PH_REFERENCE_GROWTH])));
-    s.mu = mui * f1 * f2 * fl * s.L;
+    const FT fl = 1 - m_exp(-alpha * theta * PAR * sk.rl[cls]);
+    s.mu = mui * sk.f1 * f2 * fl * s.L;
     s.muI = s.mu * I;
 }
 
@@ -211,9 +245,7 @@ __device__ __forceinline__ FT chlorophyll_growth(const FT* ph, const Phyto<FT>& 
                                                  const StageConst<FT>& sk)
 {
     const FT PAR = ph[OBME_PH_BETA1] * A.PAR1 + ph[OBME_PH_BETA2] * A.PAR2 + ph[OBME_PH_BETA3] * A.PAR3;
-    const FT dl = sk.dl_chl;
-    const FT f1 = qdiv(FT(1.5) * dl, dl + FT(0.5 * DAYS));
-    const FT mucheck = qdiv(s.mu, f1) * dl;
+    const FT mucheck = s.mu * sk.chl;
     const FT alpha = ph[OBME_PH_ALPHA0] * (1 + ph[OBME_PH_BETA] * m_exp(-PAR));
     const FT rho = qdiv(12 * mucheck * s.I, alpha * s.IChl * PAR + eps0<FT>()) * s.L;
     const FT th0 = ph[OBME_PH_CHL_MIN], th1 = ph[OBME_PH_CHL_MAX];
@@ -332,12 +364,13 @@ __device__ __forceinline__ void pisces_tendencies(const FT* pp, const FT* v, con
     const FT* zpZ = pp + OBME_PP_MICRO;
     const FT* zpM = pp + OBME_PP_MESO;
     const FT* sc = pp + OBME_PP_SCALARS;
+    const FT* pd = pp + OBME_PP_COUNT;
     const FT T = v[OBME_PI_T];
     const FT e0 = eps0<FT>();
 
     Phyto<FT> sP, sD;
-    phyto_state(phN, sc, v, A, sk, tf.btN, v[OBME_PI_P], v[OBME_PI_PCHL], v[OBME_PI_PFE], sP);
-    phyto_state(phD, sc, v, A, sk, tf.btD, v[OBME_PI_D], v[OBME_PI_DCHL], v[OBME_PI_DFE], sD);
+    phyto_state(phN, sc, v, A, sk, pd, 0, tf.btN, v[OBME_PI_P], v[OBME_PI_PCHL], v[OBME_PI_PFE], sP);
+    phyto_state(phD, sc, v, A, sk, pd, 1, tf.btD, v[OBME_PI_D], v[OBME_PI_DCHL], v[OBME_PI_DFE], sD);
     Zoo<FT> gZ, gM;
     const FT micro_iron = zpZ[OBME_PZ_IRON_RATIO];
     zoo_state<FT, 3>(zpZ, v, tf.bZ, micro_iron, A.wPOCc, A.wGOCc, v[OBME_PI_Z], gZ);
@@ -395,8 +428,8 @@ __device__ __forceinline__ void pisces_tendencies(const FT* pp, const FT* v, con
     const FT inorg_exc = zpZ[OBME_PZ_GAMMA] * excZ + zpM[OBME_PZ_GAMMA] * excM;
     const FT org_exc = (1 - zpZ[OBME_PZ_GAMMA]) * excZ + (1 - zpM[OBME_PZ_GAMMA]) * excM;
     // upper trophic waste of the meso class (mortality_waste.jl)
-    const FT utw = qdiv(FT(1), 1 - zpM[OBME_PZ_E0]) * zpM[OBME_PZ_M0] * gM.tf * (gM.I * gM.I);
-    const FT R_ut = (1 - zpM[OBME_PZ_E0] - zpM[OBME_PZ_SIGMA]) * utw;
+    const FT utw = pd[PD_UTW] * gM.tf * (gM.I * gM.I);
+    const FT R_ut = pd[PD_UT_KEEP] * utw;
     const FT fecal = zpM[OBME_PZ_SIGMA] * utw;
     const FT ut_excretion = (1 - zpM[OBME_PZ_GAMMA]) * R_ut;
     const FT ut_respiration = zpM[OBME_PZ_GAMMA] * R_ut;
@@ -413,7 +446,7 @@ __device__ __forceinline__ void pisces_tendencies(const FT* pp, const FT* v, con
                      * qdiv(DOC, DOC + sc[OBME_PS_K_DOC]);
 
     // DOC (dissolved_organic_carbon.jl:39-106)
-    const FT doc_deg = qdiv(sc[OBME_PS_DOC_LAMBDA] * tf.doc * LBact * Bact, sc[OBME_PS_DOC_BACT_REF]) * DOC;
+    const FT doc_deg = pd[PD_DOC_RATE] * tf.doc * LBact * Bact * DOC;
     const FT POC = v[OBME_PI_POC], GOC = v[OBME_PI_GOC];
     const FT Phi1 = shear_lt * (sc[OBME_PS_DOC_A1] * DOC + sc[OBME_PS_DOC_A2] * POC) * DOC;
     const FT Phi2 = shear_lt * (sc[OBME_PS_DOC_A3] * GOC) * DOC;
@@ -434,7 +467,7 @@ __device__ __forceinline__ void pisces_tendencies(const FT* pp, const FT* v, con
     const FT L_CaCO3 = jmin3(sP.LN, qdiv(Fe, Fe + FT(0.05)), sP.LPO4);
     const FT R = sc[OBME_PS_RAIN_RATIO] * L_CaCO3 * jmax(FT(1), v[OBME_PI_P] / 2)
                  * qdiv(jmax(FT(0), PAR - 1), 4 + PAR) * qdiv(FT(30), 30 + PAR) * jmax(FT(0), qdiv(T, T + FT(0.1)))
-                 * tf.rain * jmin(FT(1), qdiv(FT(-50), A.zmxl));
+                 * tf.rain * pd[PD_RAIN_ZM];
     const FT small_mort = (1 - R / 2) * (Plin + Pquad) + Dlin / 2;
     const FT large_mort = R / 2 * (Plin + Pquad) + Dlin / 2 + Dquad;
     const FT thP = qdiv(v[OBME_PI_PFE], v[OBME_PI_P] + e0);
@@ -497,7 +530,7 @@ __device__ __forceinline__ void pisces_tendencies(const FT* pp, const FT* v, con
     const FT mu_nano = phN[OBME_PH_MU0] * tf.btN;
     const FT growth_req = jmax(FT(0), mu_nano - FT(2.15));
     const FT nut_lim = jmin(qdiv(Fe, Fe + sc[OBME_PS_FIX_KFE]), qdiv(PO4, PO4 + sc[OBME_PS_FIX_KPO4]));
-    const FT light_lim = 1 - m_exp(qdiv(-PAR, sc[OBME_PS_FIX_E]));
+    const FT light_lim = 1 - m_exp(-PAR * pd[PD_RFIX_E]);
     const FT fixation = sc[OBME_PS_FIX_MAX] * growth_req * fix_limit * nut_lim * light_lim;
     const FT up_NO3 = qdiv(sP.muI * sP.LNO3, sP.LN + e0) + qdiv(sD.muI * sD.LNO3, sD.LN + e0);
     const FT up_NH4 = qdiv(sP.muI * sP.LNH4, sP.LN + e0) + qdiv(sD.muI * sD.LNH4, sD.LN + e0);
@@ -527,9 +560,9 @@ __device__ __forceinline__ void pisces_tendencies(const FT* pp, const FT* v, con
 
     // oxygen (oxygen.jl:30-50)
     const FT th_r = sc[OBME_PS_O2_RESP], th_n = sc[OBME_PS_O2_NITRIF];
-    G[OBME_PI_O2] = (th_r * up_NH4 + (th_r + th_n) * up_NO3 + qdiv(th_n * fixation, thN)
+    G[OBME_PI_O2] = (th_r * up_NH4 + (th_r + th_n) * up_NO3 + pd[PD_O2_N] * fixation
                      - ((th_r + th_n) * oxic + th_r * anoxic) - th_r * inorg_exc - th_r * ut_respiration
-                     - qdiv(th_n * nitrif, thN));
+                     - pd[PD_O2_N] * nitrif);
 }
 
 // ---------------------------------------------------------------- calcite saturation (FP64)
@@ -623,10 +656,9 @@ __device__ __forceinline__ CarbonParams omega_params(const OmegaConst& c, double
 // Ca·CO3/KSP).
 __device__ __forceinline__ double omega_from_H(const OmegaConst& c, const CarbonParams& p, double H)
 {
-    const double denom1 = (H * (H + p.K1));
-    const double denom2 = (1.0 + p.K1 * p.K2 / denom1);
-    const double co3 = p.DIC * p.K1 * p.K2 / denom1 / denom2;
-    return c.ca * co3 / c.KSP;
+    // DIC K1 K2 / (H (H + K1)) / (1 + K1 K2 / (H (H + K1))), over one denominator
+    const double K12 = p.K1 * p.K2;
+    return c.ca * p.DIC * K12 * m_rcp((H * (H + p.K1) + K12) * c.KSP);
 }
 
 // The root of the reference solve, the damped Newton from 10^-pH₀.

@@ -52,7 +52,7 @@ struct PiscesArgs {
     obme_o2_exchange o2;
     FT* zeu;                // [Nx*Ny]
     FT* mlPAR;              // [Nx*Ny]
-    const FT* pp;           // parameters (OBME_PP_*)
+    const FT* pp;           // parameters (OBME_PP_*), then their combinations (PD_*)
     const FT* lev;          // [4][Nz]: zc, zf (bottom face), dz, 1/dz
     const FT* w;            // [2][Nz+1]: POC and GOC face velocities
     double zf_top;          // top face position
@@ -375,7 +375,6 @@ k_pisces_cell(PiscesArgs<FT> a)
     A.z = a.lev[k];
     A.zmxl = sc[OBME_PS_MIXED_LAYER_DEPTH];
     A.zeu = a.zeu[col];
-    A.kappa = sc[OBME_PS_KAPPA];
     A.mlPAR = a.mlPAR[col];
     if constexpr (OM == 1) {
         OmegaConst o;
@@ -595,9 +594,11 @@ struct PiscesFused {
 #define OBME_PISCES_PF_WAVES 4
 #endif
 constexpr int PF_WAVES = OBME_PISCES_PF_WAVES;
-// waves per SIMD the register allocation is held to
+// waves per SIMD the register allocation is held to: 168 registers, without
+// spills now that the parameters are not kept in them (256x256x64, 10 steps:
+// two waves 4967 us, three 4375; with the parameters held, two 5780)
 #ifndef OBME_PISCES_PF_OCC
-#define OBME_PISCES_PF_OCC 2
+#define OBME_PISCES_PF_OCC 3
 #endif
 
 // the carbonate constants the fused step stages in (the indices of
@@ -734,7 +735,13 @@ __global__ void __launch_bounds__(PF_WAVES * 64, OBME_PISCES_PF_OCC) k_pisces_fu
         for (int n = 0; n < NW; n++) s_gm[n][tid] = FT(0);
 #pragma unroll 1
         for (int st = 0; st < 3; st++) {
-            const FT* pps = a.pp;
+            // the parameters again in every stage, by an offset the compiler
+            // cannot see through: a scalar load each, where it kept the whole
+            // array through the loop and its overflow in lanes of vector
+            // registers (180 of them, read back one instruction each)
+            int none;
+            asm("s_mov_b32 %0, 0" : "=s"(none) : "s"(st));
+            const FT* pps = a.pp + none;
             if constexpr (SCALE) scale_negatives_cell<NW>(f.ns, v);
 
             // the top boundary fluxes of DIC and O2 (the surface kernel's solve),
@@ -791,7 +798,6 @@ __global__ void __launch_bounds__(PF_WAVES * 64, OBME_PISCES_PF_OCC) k_pisces_fu
             A.z = zc;
             A.zmxl = zmxl;
             A.zeu = zeu;
-            A.kappa = pps[OBME_PP_SCALARS + OBME_PS_KAPPA];
             A.mlPAR = acc / depth;
             A.PAR = PAR;
             A.PAR1 = band[0];
@@ -943,8 +949,11 @@ static obme_status pisces_upload(obme_pisces* h)
 {
     const obme_pisces_config& c = h->cfg;
     const int Nz = c.grid.Nz;
-    std::vector<FT> pp(OBME_PP_COUNT);
+    std::vector<FT> pp(OBME_PP_COUNT + PD_COUNT);
+    double derived[PD_COUNT];
+    derived_parameters(c.params, derived);
     for (int n = 0; n < OBME_PP_COUNT; n++) pp[n] = (FT)c.params[n];
+    for (int n = 0; n < PD_COUNT; n++) pp[OBME_PP_COUNT + n] = (FT)derived[n];
     std::vector<FT> lev(4 * (size_t)Nz);
     for (int k = 0; k < Nz; k++) {
         lev[k] = (FT)h->zc[k];
@@ -1134,10 +1143,7 @@ static PiscesArgs<FT> pisces_args(const obme_pisces* h, double t)
         a.chi[n] = (FT)c.band_chi[n];
         a.division[n] = (FT)c.band_division[n];
     }
-    const double lat = c.params[OBME_PP_SCALARS + OBME_PS_LATITUDE];
     a.solver = c.solver;
-    (void)t;
-    (void)lat;
     if (h->sediment) {
         // -w of each listed tracer's bottom face (the face velocities the
         // sinking uses: w[0] of the POC or GOC profile)
@@ -1178,6 +1184,24 @@ static double host_day_length(double t, double phi)
     return (24 - 24.0 / 180 * (std::acos(L) * (180.0 / 3.141592653589793))) * 3600.0;
 }
 
+// the stage's uniform inputs at time t
+template <typename FT>
+static StageConst<FT> stage_const(const obme_pisces_config& c, double t)
+{
+    const double lat = c.params[OBME_PP_SCALARS + OBME_PS_LATITUDE];
+    const double d = host_day_length(lat, t);  // day_length(φ, t), growth_rate.jl:30
+    const double e = host_day_length(t, lat);  // day_length(t, φ), growth_rate.jl:128
+    auto f1 = [](double x) { return 1.5 * x / (x + 0.5 * 86400.0); };
+    StageConst<FT> k;
+    k.f1 = (FT)f1(d);
+    const int base[2] = {OBME_PP_NANO, OBME_PP_DIATOMS};
+    for (int q = 0; q < 2; q++)
+        k.rl[q] = (FT)(1 / (d * (c.params[base[q] + OBME_PH_BASAL_RESPIRATION] +
+                                 c.params[base[q] + OBME_PH_REFERENCE_GROWTH])));
+    k.chl = (FT)(e / f1(e));
+    return k;
+}
+
 template <typename FT>
 static obme_status pisces_scale(obme_pisces* h, const void* const* in, hipStream_t s);
 
@@ -1191,9 +1215,7 @@ static obme_status pisces_stage(obme_pisces* h, const void* const* in, void* con
     PiscesArgs<FT> a = pisces_args<FT>(h, t);
     for (int n = 0; n < NTR; n++) a.in[n] = (const FT*)in[n];
     for (int n = 0; n < NW; n++) a.out[n] = (FT*)out[n];
-    const double lat = h->cfg.params[OBME_PP_SCALARS + OBME_PS_LATITUDE];
-    a.sk.dl_growth = (FT)host_day_length(lat, t);  // day_length(φ, t), growth_rate.jl:30
-    a.sk.dl_chl = (FT)host_day_length(t, lat);     // day_length(t, φ), growth_rate.jl:128
+    a.sk = stage_const<FT>(h->cfg, t);
     a.dt = dt;
     a.stage = stage;
     if (h->sediment) {
@@ -1353,7 +1375,6 @@ static obme_status pisces_fused_steps(obme_pisces* h, void* const* tracers, int 
         f.B[q] = (float)(dt * zet[q]);
         f.div[q] = (float)h->cfg.band_division[q];
     }
-    const double lat = h->cfg.params[OBME_PP_SCALARS + OBME_PS_LATITUDE];
     if (h->cfg.co2.enabled || h->cfg.o2.enabled) {
         if (!h->d_surfc && hipMalloc(&h->d_surfc, (size_t)SURF_PACK * h->ncol * sizeof(double)) != hipSuccess)
             return obme_fail(OBME_ERR_NOMEM, "PISCES surface constants");
@@ -1370,8 +1391,7 @@ static obme_status pisces_fused_steps(obme_pisces* h, void* const* tracers, int 
             const double t = t0 + (s0 + sn) * dt;
             for (int q = 0; q < 3; q++) {
                 const double tq = t + cst[q] * dt;
-                f.sk[sn][q].dl_growth = (float)host_day_length(lat, tq);  // day_length(φ, t), growth_rate.jl:30
-                f.sk[sn][q].dl_chl = (float)host_day_length(tq, lat);     // day_length(t, φ), growth_rate.jl:128
+                f.sk[sn][q] = stage_const<float>(h->cfg, tq);
                 f.PAR0[sn][q] = (float)pisces_surface_value(h->cfg, tq);
             }
         }
