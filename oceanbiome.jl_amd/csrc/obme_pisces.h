@@ -584,7 +584,9 @@ __device__ __forceinline__ double pressure_exponent(const double* a, double Tc, 
 struct OmegaConst {
     double conv, K1, K2, KB, KW, KS, KF, KSi, boron, sulfate, fluoride, ca, KSP;
 };
-constexpr int OMEGA_CONST_FIELDS = 13;
+// stored per cell: conv to KSi and KSP (the salinity terms are formed from S,
+// four multiplications against 32 B to read)
+constexpr int OMEGA_CONST_FIELDS = 9;
 
 // The salinity totals and the calcium concentration (functions of S alone).
 __device__ __forceinline__ void omega_salinity_terms(double S, OmegaConst& c)

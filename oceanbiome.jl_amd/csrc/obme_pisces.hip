@@ -10,9 +10,9 @@
 // each RK3 stage is two launches: k_pisces_columns, then k_pisces_cell with
 // the calcite saturation solved inline from those constants, and the
 // substep.
-// The stage input is read and the stage output written to different
-// arrays (the caller's tracers and a library-owned copy, alternately), so
-// the sinking stencil's k+1 reads never race with the update.
+// The sinking stencil reads the cell above, so the six tracers that sink go
+// from the caller's arrays through two library-owned ones and back, one per
+// stage; the others are updated in place.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -308,8 +308,7 @@ __global__ void __launch_bounds__(256) k_pisces_prep(PiscesArgs<FT> a)
     OmegaConst o;
     omega_constants((double)a.in[OBME_PI_T][p], (double)a.in[OBME_PI_S][p], P, o);
     FT* out = const_cast<FT*>(a.oc);
-    const double f[OMEGA_CONST_FIELDS] = {o.conv, o.K1, o.K2, o.KB, o.KW, o.KS, o.KF, o.KSi,
-                                          o.boron, o.sulfate, o.fluoride, o.ca, o.KSP};
+    const double f[OMEGA_CONST_FIELDS] = {o.conv, o.K1, o.K2, o.KB, o.KW, o.KS, o.KF, o.KSi, o.KSP};
 #pragma unroll
     for (int n = 0; n < OMEGA_CONST_FIELDS; n++) out[(long)n * ncell + c] = (FT)f[n];
     if (a.tfac) {
@@ -387,11 +386,8 @@ k_pisces_cell(PiscesArgs<FT> a)
         o.KS = oc[5 * ncell];
         o.KF = oc[6 * ncell];
         o.KSi = oc[7 * ncell];
-        o.boron = oc[8 * ncell];
-        o.sulfate = oc[9 * ncell];
-        o.fluoride = oc[10 * ncell];
-        o.ca = oc[11 * ncell];
-        o.KSP = oc[12 * ncell];
+        o.KSP = oc[8 * ncell];
+        omega_salinity_terms((double)v[OBME_PI_S], o);
         const CarbonParams cp = omega_params(o, (double)v[OBME_PI_DIC], (double)v[OBME_PI_ALK], (double)v[OBME_PI_SI]);
         // Newton from the previous stage's [H+] (stored in FP32; the first
         // stage of a call from the FP32 guess), with the reference solve
@@ -410,10 +406,10 @@ k_pisces_cell(PiscesArgs<FT> a)
     } else {
         A.Omega = a.Omega[c];
     }
-    A.PAR = a.PAR[0][c];
     A.PAR1 = a.PAR[1][c];
     A.PAR2 = a.PAR[2][c];
     A.PAR3 = a.PAR[3][c];
+    A.PAR = A.PAR1 + A.PAR2 + A.PAR3;
     A.wPOCc = (wP[k] + wP[k + 1]) / 2;
     A.wGOCc = (wG[k] + wG[k + 1]) / 2;
     FT G[NW];
@@ -495,7 +491,7 @@ k_pisces_cell(PiscesArgs<FT> a)
                 u = u + fmaf(a.A, G[n], a.B * gm);
             }
             a.out[n][p] = u;
-            a.Gm[(long)n * ncell + c] = G[n];
+            if (a.stage != 2) a.Gm[(long)n * ncell + c] = G[n];
             if (SED && sed_cell && a.stage == 2 && a.sedw[n] != FT(0)) {
                 fnew = fnew_first ? a.sedw[n] * u : fnew + a.sedw[n] * u;
                 fnew_first = false;
@@ -601,13 +597,6 @@ constexpr int PF_WAVES = OBME_PISCES_PF_WAVES;
 #define OBME_PISCES_PF_OCC 3
 #endif
 
-// the carbonate constants the fused step stages in (the indices of
-// conv, K1, K2, KB, KW, KS, KF, KSi, KSP in k_pisces_prep's order); the
-// salinity terms are formed from S in the kernel (16 B less to read per
-// cell and step)
-constexpr int FUSED_OMEGA_FIELDS = 9;
-__device__ __forceinline__ constexpr int fused_omega_field(int q) { return q < 8 ? q : 12; }
-
 template <bool SCALE>
 __global__ void __launch_bounds__(PF_WAVES * 64, OBME_PISCES_PF_OCC) k_pisces_fused(PiscesArgs<float> a, PiscesFused f)
 {
@@ -636,7 +625,7 @@ __global__ void __launch_bounds__(PF_WAVES * 64, OBME_PISCES_PF_OCC) k_pisces_fu
     // previous stage's transitions live in LDS, each lane in its own slots,
     // to leave the registers to the state and the transitions
     // the constants that depend on T and P (the salinity terms come from S)
-    __shared__ float s_oc[FUSED_OMEGA_FIELDS][PF_WAVES * 64];
+    __shared__ float s_oc[OMEGA_CONST_FIELDS][PF_WAVES * 64];
     __shared__ FT s_gm[NW][PF_WAVES * 64];
     __shared__ FT s_ts[2][PF_WAVES * 64];
     __shared__ float s_h[PF_WAVES * 64];
@@ -658,10 +647,10 @@ __global__ void __launch_bounds__(PF_WAVES * 64, OBME_PISCES_PF_OCC) k_pisces_fu
         FT stg[NTR];
 #pragma unroll
         for (int n = 0; n < NTR; n++) stg[n] = tok ? a.in[n][pt] : FT(0);
-        float so[FUSED_OMEGA_FIELDS];
+        float so[OMEGA_CONST_FIELDS];
 #pragma unroll
-        for (int q = 0; q < FUSED_OMEGA_FIELDS; q++)
-            so[q] = tok ? (a.oc + (unsigned long)fused_omega_field(q) * ncell)[ct_cell] : 1.0f;
+        for (int q = 0; q < OMEGA_CONST_FIELDS; q++)
+            so[q] = tok ? (a.oc + (unsigned long)q * ncell)[ct_cell] : 1.0f;
         const float sh = (tok && f.have_H) ? a.Hs[ct_cell] : -1.0f;
         if (tok) {
 #pragma unroll
@@ -669,7 +658,7 @@ __global__ void __launch_bounds__(PF_WAVES * 64, OBME_PISCES_PF_OCC) k_pisces_fu
             s_ts[0][slot] = stg[OBME_PI_T];
             s_ts[1][slot] = stg[OBME_PI_S];
 #pragma unroll
-            for (int q = 0; q < FUSED_OMEGA_FIELDS; q++) s_oc[q][slot] = so[q];
+            for (int q = 0; q < OMEGA_CONST_FIELDS; q++) s_oc[q][slot] = so[q];
             s_h[slot] = sh;
         }
     }
@@ -911,7 +900,7 @@ struct obme_pisces {
     void* d_Hsurf = nullptr;
     void* d_surfc = nullptr;   // [SURF_PACK][Nx*Ny] surface constants of the fused step
     void* d_tfac = nullptr;    // [TFAC_FIELDS][ncell] temperature factors of the FP64 step
-    void* d_copy[NW] = {};
+    void* d_copy[2][6] = {};   // the sinking tracers between the stages
     size_t field_bytes = 0;
     std::vector<double> zc, zf, dz;
     std::vector<double> w_host;   // [2][Nz+1]: the POC and GOC face velocities (FP64)
@@ -936,8 +925,9 @@ extern "C" obme_status obme_pisces_destroy(obme_pisces* h)
     for (void* p : {h->d_pp, h->d_lev, h->d_w, h->d_PAR, h->d_Omega, h->d_zeu, h->d_mlPAR, h->d_Gm, h->d_oc, h->d_H,
                     h->d_sflux, h->d_Hsurf, h->d_surfc, h->d_tfac})
         if (p) (void)hipFree(p);
-    for (void* p : h->d_copy)
-        if (p) (void)hipFree(p);
+    for (auto& side : h->d_copy)
+        for (void* p : side)
+            if (p) (void)hipFree(p);
     if (h->d_sedGm) (void)hipFree(h->d_sedGm);
     if (h->d_sedGn) (void)hipFree(h->d_sedGn);
     delete h;
@@ -1069,7 +1059,7 @@ extern "C" obme_status obme_pisces_create(const obme_pisces_config* cfg, obme_pi
     auto alloc = [&](void** d, size_t bytes) {
         if (st == OBME_OK && hipMalloc(d, bytes) != hipSuccess) st = obme_fail(OBME_ERR_NOMEM, "PISCES buffers");
     };
-    alloc(&h->d_PAR, 4 * h->ncell * es);
+    alloc(&h->d_PAR, 3 * h->ncell * es);
     alloc(&h->d_Omega, h->ncell * es);
     alloc(&h->d_zeu, h->ncol * es);
     alloc(&h->d_mlPAR, h->ncol * es);
@@ -1114,7 +1104,8 @@ static PiscesArgs<FT> pisces_args(const obme_pisces* h, double t)
     PiscesArgs<FT> a;
     std::memset(&a, 0, sizeof(a));
     a.Gm = (FT*)h->d_Gm;
-    for (int n = 0; n < 4; n++) a.PAR[n] = (FT*)h->d_PAR + (size_t)n * h->ncell;
+    // (the total is the sum of the bands, formed where it is used)
+    for (int n = 1; n < 4; n++) a.PAR[n] = (FT*)h->d_PAR + (size_t)(n - 1) * h->ncell;
     a.Omega = (FT*)h->d_Omega;
     a.zeu = (FT*)h->d_zeu;
     a.mlPAR = (FT*)h->d_mlPAR;
@@ -1476,27 +1467,24 @@ static obme_status pisces_step(obme_pisces* h, void* const* tracers, double* sto
         if (r != OBME_OK) return r;
     }
     if (h->fused) return pisces_fused_steps(h, tracers, nsteps, dt, t0, s);
-    for (int n = 0; n < NW; n++)
-        if (!h->d_copy[n] && hipMalloc(&h->d_copy[n], h->field_bytes) != hipSuccess)
-            return obme_fail(OBME_ERR_NOMEM, "PISCES stage copy");
-    // Stage inputs and outputs alternate between the caller's arrays (U) and
-    // library copies (C), which start as full copies of U so that their halos
-    // match; the kernels write interiors only.  A step ends on the other side
-    // of where it started; an odd number of steps ends with a copy back.
-    for (int n = 0; n < NW; n++)
-        OBME_HIP_TRY(hipMemcpyAsync(h->d_copy[n], tracers[n], h->field_bytes, hipMemcpyDeviceToDevice, s));
-    const void* inU[NTR];
-    const void* inC[NTR];
-    void* outU[NW];
-    void* outC[NW];
-    for (int n = 0; n < NTR; n++) {
-        inU[n] = tracers[n];
-        inC[n] = (n < NW) ? h->d_copy[n] : tracers[n];
+    // The stages of a step go U -> C0 -> C1 -> U for the tracers that sink (U:
+    // the caller's arrays; the kernels read and write interiors only), and stay
+    // in U for the others.
+    const int sinking[6] = {OBME_PI_POC, OBME_PI_SFE, OBME_PI_GOC, OBME_PI_BFE, OBME_PI_PSI, OBME_PI_CACO3};
+    const void* in[3][NTR];
+    void* out[3][NW];
+    for (int q = 0; q < 3; q++) {
+        for (int n = 0; n < NTR; n++) in[q][n] = tracers[n];
+        for (int n = 0; n < NW; n++) out[q][n] = tracers[n];
     }
-    for (int n = 0; n < NW; n++) {
-        outU[n] = tracers[n];
-        outC[n] = h->d_copy[n];
-    }
+    for (int q = 0; q < 2; q++)
+        for (int m = 0; m < 6; m++) {
+            void*& copy = h->d_copy[q][m];
+            if (!copy && hipMalloc(&copy, h->field_bytes) != hipSuccess)
+                return obme_fail(OBME_ERR_NOMEM, "PISCES stage copy");
+            out[q][sinking[m]] = copy;
+            in[q + 1][sinking[m]] = copy;
+        }
     const double cst[3] = {0.0, 8.0 / 15.0, 2.0 / 3.0};
     // the sediment of this call: its first step ever (the lazy first
     // tendency) and whether the first sediment step repeats the previous Δt
@@ -1507,22 +1495,15 @@ static obme_status pisces_step(obme_pisces* h, void* const* tracers, double* sto
         ~CallSediment() { h->call_storage = nullptr; h->call_init = h->call_ab2 = 0; }
     } keep{h};
     h->call_storage = h->sediment ? storage : nullptr;
-    bool inCopy = false;  // where the current state lives
     for (int st = 0; st < nsteps; st++) {
         const double t = t0 + st * dt;
         h->call_init = (sed_init && st == 0) ? 1 : 0;
         h->call_ab2 = (sed_ab2 && st == 0) ? 1 : 0;
         for (int q = 0; q < 3; q++) {
-            const void* const* in = inCopy ? inC : inU;
-            void* const* out = inCopy ? outU : outC;
-            obme_status r = pisces_stage_any(h, in, out, t + cst[q] * dt, dt, q, 0, (st > 0 || q > 0) ? 1 : 0, s);
+            obme_status r = pisces_stage_any(h, in[q], out[q], t + cst[q] * dt, dt, q, 0, (st > 0 || q > 0) ? 1 : 0, s);
             if (r != OBME_OK) return r;
-            inCopy = !inCopy;
         }
     }
-    if (inCopy)
-        for (int n = 0; n < NW; n++)
-            OBME_HIP_TRY(hipMemcpyAsync(tracers[n], h->d_copy[n], h->field_bytes, hipMemcpyDeviceToDevice, s));
     if (h->sediment && storage) {
         // three sediment steps per step, the last of Δt (γ3 + ζ3)
         h->sed_iter += 3 * (long long)nsteps;
