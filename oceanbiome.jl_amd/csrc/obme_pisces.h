@@ -45,12 +45,11 @@ __device__ __forceinline__ FT qdiv(FT a, FT b)
     else return a * __builtin_amdgcn_rcpf(b);
 }
 
-// a / k for a constant k (FP32-mixed: times 1/k, folded at compile time).
+// a / k for a constant k: times 1/k, folded at compile time.
 template <typename FT>
 __device__ __forceinline__ FT qdivk(FT a, double k)
 {
-    if constexpr (sizeof(FT) == 8) return a / k;
-    else return a * (float)(1.0 / k);
+    return a * (FT)(1.0 / k);
 }
 
 template <typename FT>
@@ -61,7 +60,7 @@ __device__ __forceinline__ FT jmin4(FT a, FT b, FT c, FT d) { return jmin(jmin(j
 template <typename FT>
 __device__ __forceinline__ FT m_log(FT x)
 {
-    if constexpr (sizeof(FT) == 8) return log(x);
+    if constexpr (sizeof(FT) == 8) return m_log_any(x);
     else return __builtin_amdgcn_logf(x) * 0.693147180559945309f;
 }
 
@@ -137,13 +136,15 @@ struct Aux {
 // degradation (dissolved_organic_carbon.jl:62, two_size_class.jl:154), the
 // rain ratio's 1 + exp(-(T-10)²/25) (nano_diatom_coupling.jl), the ligand
 // constant of the free iron (iron/iron.jl:29), the silicate equilibrium
-// 10^(6.44 - 968/T_K) and (1 + T/400)^4 (silicate.jl:30-34).  The same
-// expressions whether evaluated per stage or once per stepper call.
+// 10^(6.44 - 968/T_K) and (1 + T/400)^4 (silicate.jl:30-34).  The rain ratio's
+// takes max(0, T / (T + 0.1)) with it, the silicate equilibrium enters as its
+// reciprocal and t15 is 0.225 (1 + T/15).  The same expressions whether
+// evaluated per stage or once per stepper call.
 template <typename FT>
 struct TFac {
-    FT btN, btD, bZ, bM, doc, pom, rain, kfe, eq, t4;
+    FT btN, btD, bZ, bM, doc, pom, rain, kfe, req, t4, t15;
 };
-constexpr int TFAC_FIELDS = 10;
+constexpr int TFAC_FIELDS = 11;
 
 template <typename FT>
 __device__ __forceinline__ void temperature_factors(const FT* pp, FT T, TFac<FT>& f)
@@ -156,10 +157,12 @@ __device__ __forceinline__ void temperature_factors(const FT* pp, FT T, TFac<FT>
     f.doc = m_pow(sc[OBME_PS_DOC_B], T);
     f.pom = m_pow(sc[OBME_PS_POM_B], T);
     const FT Tm = T - 10;
-    f.rain = 1 + m_exp(qdivk(-(Tm * Tm), 25));
+    f.rain = jmax(FT(0), qdiv(T, T + FT(0.1))) * (1 + m_exp(qdivk(-(Tm * Tm), 25)));
     f.kfe = m_exp(FT(16.27) - qdiv(FT(1565.7), jmax(T + FT(273.15), FT(5))));
-    f.eq = m_pow(FT(10), FT(6.44) - qdiv(FT(968), T + FT(273.15)));
-    f.t4 = m_pow(1 + qdivk(T, 400), FT(4));
+    f.req = m_pow(FT(10), qdiv(FT(968), T + FT(273.15)) - FT(6.44));
+    const FT t = 1 + qdivk(T, 400), t2 = t * t;
+    f.t4 = t2 * t2;
+    f.t15 = FT(0.225) * (1 + qdivk(T, 15));
 }
 
 // One phytoplankton class (parameters at block b of pp).
@@ -168,6 +171,7 @@ struct Phyto {
     FT I, IChl, IFe;
     FT L, LFe, LPO4, LN, LNO3, LNH4;
     FT mu, muI;
+    FT Kb, PAR, alpha;   // size factor, absorbed light, light sensitivity
 };
 
 template <typename FT>
@@ -199,6 +203,7 @@ __device__ __forceinline__ void phyto_state(const FT* ph, const FT* sc, const FT
     const FT thFe = (I == FT(0)) ? FT(0) : qdiv(IFe, I + eps0<FT>());
     const FT thChl = (I == FT(0)) ? FT(0) : qdiv(IChl, 12 * I + eps0<FT>());
     const FT Kb = size_factor(ph, I);
+    s.Kb = Kb;
     const FT Kno = ph[OBME_PH_KNO3] * Kb, Knh = ph[OBME_PH_KNH4] * Kb, Kp = ph[OBME_PH_KPO4] * Kb,
              Ksi = ph[OBME_PH_KSI_MIN] * Kb;
     s.LNO3 = nitrogen_lim(NO3, NH4, Kno, Knh);
@@ -220,6 +225,8 @@ __device__ __forceinline__ void phyto_state(const FT* ph, const FT* sc, const FT
     const FT mui = ph[OBME_PH_MU0] * btT;
     const FT f2 = 1 - qdiv(drt, drt + ph[OBME_PH_DARK_TOLERANCE]);
     const FT alpha = ph[OBME_PH_ALPHA0] * (1 + ph[OBME_PH_BETA] * m_exp(-PAR));
+    s.PAR = PAR;
+    s.alpha = alpha;
     const FT theta = qdiv(IChl, 12 * I + eps0<FT>());
     const FT fl = 1 - m_exp(-alpha * theta * PAR * sk.rl[cls]);
     s.mu = mui * sk.f1 * f2 * fl * s.L;
@@ -241,13 +248,10 @@ __device__ __forceinline__ void phyto_mortality(const FT* ph, const FT* sc, cons
 
 // chlorophyll growth (mixed_mondo.jl:84-97; growth_rate.jl:113-148)
 template <typename FT>
-__device__ __forceinline__ FT chlorophyll_growth(const FT* ph, const Phyto<FT>& s, const Aux<FT>& A,
-                                                 const StageConst<FT>& sk)
+__device__ __forceinline__ FT chlorophyll_growth(const FT* ph, const Phyto<FT>& s, const StageConst<FT>& sk)
 {
-    const FT PAR = ph[OBME_PH_BETA1] * A.PAR1 + ph[OBME_PH_BETA2] * A.PAR2 + ph[OBME_PH_BETA3] * A.PAR3;
     const FT mucheck = s.mu * sk.chl;
-    const FT alpha = ph[OBME_PH_ALPHA0] * (1 + ph[OBME_PH_BETA] * m_exp(-PAR));
-    const FT rho = qdiv(12 * mucheck * s.I, alpha * s.IChl * PAR + eps0<FT>()) * s.L;
+    const FT rho = qdiv(12 * mucheck * s.I, s.alpha * s.IChl * s.PAR + eps0<FT>()) * s.L;
     const FT th0 = ph[OBME_PH_CHL_MIN], th1 = ph[OBME_PH_CHL_MAX];
     return (1 - ph[OBME_PH_DELTA]) * 12 * (th0 + (th1 - th0) * rho) * s.mu * s.I;
 }
@@ -258,7 +262,7 @@ __device__ __forceinline__ FT iron_uptake(const FT* ph, const Phyto<FT>& s, FT b
 {
     const FT fe_max = ph[OBME_PH_FE_MAX];
     const FT mui = ph[OBME_PH_MU0] * btT;
-    const FT K = ph[OBME_PH_KFE_UPTAKE] * size_factor(ph, s.I);
+    const FT K = ph[OBME_PH_KFE_UPTAKE] * s.Kb;
     const FT L1 = qdiv(Fe, Fe + K + eps0<FT>());
     const FT L2 = 4 - qdiv(FT(4.5) * s.LFe, s.LFe + 1);
     // (1 - r) / (1.05 - r), r = θFe / θFe_max, θFe = IFe / (I + ε)
@@ -301,7 +305,7 @@ __device__ __forceinline__ FT silicate_uptake(const FT* ph, const FT* sc, const 
 // iron_grazing.jl:1-36); prey order P, D, POC (, Z for the meso class).
 template <typename FT>
 struct Zoo {
-    FT I, tsg, avail, gI, ge, gIFe, ff, ffFe, tf;
+    FT I, on, gI, ge, gIFe, ff, ffFe, tf;
 };
 
 template <typename FT, int NPREY>
@@ -328,13 +332,15 @@ __device__ __forceinline__ void zoo_state(const FT* zp, const FT* v, FT bT, FT m
         s = s + jmax(FT(0), food[n] - J) * pref[n] * iron[n];
     }
     const FT clg = jmax(FT(0), avail - jmin(avail / 2, zp[OBME_PZ_FOOD_THRESHOLD]));
-    g.tsg = qdiv(base * clg, zp[OBME_PZ_K] + total_food);
-    g.avail = avail;
-    const FT igr = qdiv(total_iron, zp[OBME_PZ_IRON_RATIO] * g.tsg + eps0<FT>());
+    const FT tsg = qdiv(base * clg, zp[OBME_PZ_K] + total_food);
+    const FT igr = qdiv(total_iron, zp[OBME_PZ_IRON_RATIO] * tsg + eps0<FT>());
     const FT fq = jmin(FT(1), igr);
     g.ge = fq * jmin(zp[OBME_PZ_E0], (1 - zp[OBME_PZ_SIGMA]) * igr);
-    g.gI = g.tsg * I;
-    g.gIFe = qdiv(s * g.tsg, avail + eps0<FT>()) * I;
+    g.gI = tsg * I;
+    // what is grazed per available prey: one quotient for every prey and its
+    // iron (avail = 0 has tsg = 0)
+    g.on = qdiv(g.gI, avail + eps0<FT>());
+    g.gIFe = s * g.on;
     // flux feeding on the sinking particles (food_quality_dependant.jl:185-199, iron_grazing.jl:38-53)
     const FT ffb = zp[OBME_PZ_FF] * g.tf;
     g.ff = ffb * (v[OBME_PI_POC] * wPOCc + v[OBME_PI_GOC] * wGOCc) * I;
@@ -345,7 +351,7 @@ __device__ __forceinline__ void zoo_state(const FT* zp, const FT* v, FT bT, FT m
 template <typename FT>
 __device__ __forceinline__ FT zoo_on(const FT* zp, const Zoo<FT>& g, FT pref, FT prey)
 {
-    return qdiv(pref * jmax(FT(0), prey - zp[OBME_PZ_J]) * g.tsg, g.avail + eps0<FT>()) * g.I;
+    return pref * jmax(FT(0), prey - zp[OBME_PZ_J]) * g.on;
 }
 
 template <typename FT>
@@ -354,8 +360,23 @@ __device__ __forceinline__ FT anoxia(const FT* sc, FT O2)
     return jmin(FT(1), jmax(FT(0), qdiv(FT(0.4) * (sc[OBME_PS_ANOXIA1] - O2), sc[OBME_PS_ANOXIA2] + O2)));
 }
 
-// The 24 transitions of one cell (v: tracers in OBME_PI order).
+// The parameters' pointer again, by an offset the compiler cannot see through
+// and only once `after` is known: what follows loads them anew.
 template <typename FT>
+__device__ __forceinline__ const FT* reread(const FT* pp, FT after)
+{
+    int none;
+    asm("s_mov_b32 %0, 0" : "=s"(none) : "v"(after));
+    return pp + none;
+}
+
+// The 24 transitions of one cell (v: tracers in OBME_PI order).  SECTIONS (the
+// fused step): each section loads its parameters anew, where the compiler keeps
+// what a later one uses again in lanes of vector registers (256x256x64, 10
+// steps: 4290 -> 4166 us).  Not in FP64, with two waves per SIMD to cover the
+// loads (238 lanes fewer, but 1146 -> 1236 us at 120x100x48), nor in the hook
+// (185 -> 192).
+template <bool SECTIONS = false, typename FT>
 __device__ __forceinline__ void pisces_tendencies(const FT* pp, const FT* v, const Aux<FT>& A,
                                                   const StageConst<FT>& sk, const TFac<FT>& tf, FT* G)
 {
@@ -365,16 +386,30 @@ __device__ __forceinline__ void pisces_tendencies(const FT* pp, const FT* v, con
     const FT* zpM = pp + OBME_PP_MESO;
     const FT* sc = pp + OBME_PP_SCALARS;
     const FT* pd = pp + OBME_PP_COUNT;
-    const FT T = v[OBME_PI_T];
     const FT e0 = eps0<FT>();
+
+    auto section = [&](FT after) {
+        if constexpr (SECTIONS) {
+            pp = reread(pp, after);
+            phN = pp + OBME_PP_NANO;
+            phD = pp + OBME_PP_DIATOMS;
+            zpZ = pp + OBME_PP_MICRO;
+            zpM = pp + OBME_PP_MESO;
+            sc = pp + OBME_PP_SCALARS;
+            pd = pp + OBME_PP_COUNT;
+        }
+    };
 
     Phyto<FT> sP, sD;
     phyto_state(phN, sc, v, A, sk, pd, 0, tf.btN, v[OBME_PI_P], v[OBME_PI_PCHL], v[OBME_PI_PFE], sP);
+    section(sP.muI);
     phyto_state(phD, sc, v, A, sk, pd, 1, tf.btD, v[OBME_PI_D], v[OBME_PI_DCHL], v[OBME_PI_DFE], sD);
+    section(sD.muI);
     Zoo<FT> gZ, gM;
     const FT micro_iron = zpZ[OBME_PZ_IRON_RATIO];
     zoo_state<FT, 3>(zpZ, v, tf.bZ, micro_iron, A.wPOCc, A.wGOCc, v[OBME_PI_Z], gZ);
     zoo_state<FT, 4>(zpM, v, tf.bM, micro_iron, A.wPOCc, A.wGOCc, v[OBME_PI_M], gM);
+    section(gM.gIFe);
     const FT O2 = v[OBME_PI_O2];
     const FT an = anoxia(sc, O2);
     // zooplankton mortality (food_quality_dependant.jl:201-227)
@@ -402,7 +437,7 @@ __device__ __forceinline__ void pisces_tendencies(const FT* pp, const FT* v, con
         const FT death = Plin + Pquad;
         G[OBME_PI_P] = (1 - phN[OBME_PH_DELTA]) * sP.muI - death - grazP;
         const FT thChl = qdiv(sP.IChl, 12 * sP.I + e0);
-        G[OBME_PI_PCHL] = chlorophyll_growth(phN, sP, A, sk) - (death + grazP) * thChl * 12;
+        G[OBME_PI_PCHL] = chlorophyll_growth(phN, sP, sk) - (death + grazP) * thChl * 12;
         const FT thFe = qdiv(sP.IFe, sP.I + e0);
         G[OBME_PI_PFE] = iron_uptake(phN, sP, tf.btN, v[OBME_PI_FE]) - (death + grazP) * thFe;
     }
@@ -410,7 +445,7 @@ __device__ __forceinline__ void pisces_tendencies(const FT* pp, const FT* v, con
         const FT death = Dlin + Dquad;
         G[OBME_PI_D] = (1 - phD[OBME_PH_DELTA]) * sD.muI - death - grazD;
         const FT thChl = qdiv(sD.IChl, 12 * sD.I + e0);
-        G[OBME_PI_DCHL] = chlorophyll_growth(phD, sD, A, sk) - (death + grazD) * thChl * 12;
+        G[OBME_PI_DCHL] = chlorophyll_growth(phD, sD, sk) - (death + grazD) * thChl * 12;
         const FT thFe = qdiv(sD.IFe, sD.I + e0);
         G[OBME_PI_DFE] = iron_uptake(phD, sD, tf.btD, v[OBME_PI_FE]) - (death + grazD) * thFe;
     }
@@ -418,6 +453,7 @@ __device__ __forceinline__ void pisces_tendencies(const FT* pp, const FT* v, con
     const FT thSi = qdiv(v[OBME_PI_DSI], v[OBME_PI_D] + e0);
     G[OBME_PI_DSI] = si_uptake - (Dlin + Dquad + grazD) * thSi;
 
+    section(G[OBME_PI_DFE]);
     // zooplankton (micro_and_meso.jl:36-48)
     G[OBME_PI_Z] = gZ.ge * (gZ.gI + gZ.ff) - mZ - zoo_on(zpM, gM, zpM[OBME_PZ_PREF_Z], v[OBME_PI_Z]);
     G[OBME_PI_M] = gM.ge * (gM.gI + gM.ff) - mM;
@@ -445,6 +481,7 @@ __device__ __forceinline__ void pisces_tendencies(const FT* pp, const FT* v, con
                            qdiv(PO4, PO4 + sc[OBME_PS_K_PO4_B]), qdiv(Fe, Fe + sc[OBME_PS_K_FE_B]))
                      * qdiv(DOC, DOC + sc[OBME_PS_K_DOC]);
 
+    section(LBact);
     // DOC (dissolved_organic_carbon.jl:39-106)
     const FT doc_deg = pd[PD_DOC_RATE] * tf.doc * LBact * Bact * DOC;
     const FT POC = v[OBME_PI_POC], GOC = v[OBME_PI_GOC];
@@ -466,8 +503,7 @@ __device__ __forceinline__ void pisces_tendencies(const FT* pp, const FT* v, con
     const FT PAR = A.PAR;
     const FT L_CaCO3 = jmin3(sP.LN, qdiv(Fe, Fe + FT(0.05)), sP.LPO4);
     const FT R = sc[OBME_PS_RAIN_RATIO] * L_CaCO3 * jmax(FT(1), v[OBME_PI_P] / 2)
-                 * qdiv(jmax(FT(0), PAR - 1), 4 + PAR) * qdiv(FT(30), 30 + PAR) * jmax(FT(0), qdiv(T, T + FT(0.1)))
-                 * tf.rain * pd[PD_RAIN_ZM];
+                 * qdiv(jmax(FT(0), PAR - 1), 4 + PAR) * qdiv(FT(30), 30 + PAR) * tf.rain * pd[PD_RAIN_ZM];
     const FT small_mort = (1 - R / 2) * (Plin + Pquad) + Dlin / 2;
     const FT large_mort = R / 2 * (Plin + Pquad) + Dlin / 2 + Dquad;
     const FT thP = qdiv(v[OBME_PI_PFE], v[OBME_PI_P] + e0);
@@ -484,6 +520,7 @@ __device__ __forceinline__ void pisces_tendencies(const FT* pp, const FT* v, con
     G[OBME_PI_GOC] = (sigM * (gM.gI + gM.ff) + large_mort + linM + fecal + pom_agg + Phi2
                       - tot_graz_GOC - lam_pom * GOC);
 
+    section(G[OBME_PI_GOC]);
     // iron in particles (iron.jl:2-89) with the free iron of SimpleIron (iron/iron.jl:25-37)
     const FT ligands = jmax(FT(0.6), FT(0.09) * (DOC + 40) - 3);
     const FT Kfe = tf.kfe;
@@ -504,14 +541,14 @@ __device__ __forceinline__ void pisces_tendencies(const FT* pp, const FT* v, con
                       + fecal * zpM[OBME_PZ_IRON_RATIO] + lamFe * GOC * Fef + sc[OBME_PS_LARGE_BACT_FE] * BactFe
                       + CgFe2 + pom_agg * thS - tot_graz_GOC * thB - lam_pom * v[OBME_PI_BFE]);
 
+    section(G[OBME_PI_BFE]);
     // particulate silicate (silicate.jl:1-48)
     const FT chi = sc[OBME_PS_CHI0] * ((A.z >= zm) ? FT(1)
                                                    : m_exp(qdiv((sc[OBME_PS_SI_FAST] - sc[OBME_PS_SI_SLOW]) * (zm - A.z), A.wGOCc)));
     const FT lam0 = chi * sc[OBME_PS_SI_FAST] + (1 - chi) * sc[OBME_PS_SI_SLOW];
-    const FT eq = tf.eq;
-    const FT sat = qdiv(eq - v[OBME_PI_SI], eq);
-    const FT t4 = tf.t4;
-    const FT lam_si = lam0 * (FT(0.225) * (1 + qdivk(T, 15)) * sat + FT(0.775) * m_pow(t4 * sat, FT(9)));
+    const FT sat = 1 - v[OBME_PI_SI] * tf.req;
+    const FT ts = tf.t4 * sat, ts2 = ts * ts, ts4 = ts2 * ts2;
+    const FT lam_si = lam0 * (tf.t15 * sat + FT(0.775) * (ts4 * ts4 * ts));
     const FT si_diss = lam_si * v[OBME_PI_PSI];
     G[OBME_PI_PSI] = (grazD + Dlin + Dquad) * thSi - si_diss;
 
@@ -523,6 +560,7 @@ __device__ __forceinline__ void pisces_tendencies(const FT* pp, const FT* v, con
                          * v[OBME_PI_CACO3];
     G[OBME_PI_CACO3] = calc_prod - calc_diss;
 
+    section(G[OBME_PI_CACO3]);
     // nitrogen (nitrogen/nitrate_ammonia.jl:22-88)
     const FT thN = sc[OBME_PS_THETAN];
     const FT nitrif = qdiv(sc[OBME_PS_NITRIF] * NH4, 1 + A.mlPAR) * (1 - an);
@@ -532,8 +570,10 @@ __device__ __forceinline__ void pisces_tendencies(const FT* pp, const FT* v, con
     const FT nut_lim = jmin(qdiv(Fe, Fe + sc[OBME_PS_FIX_KFE]), qdiv(PO4, PO4 + sc[OBME_PS_FIX_KPO4]));
     const FT light_lim = 1 - m_exp(-PAR * pd[PD_RFIX_E]);
     const FT fixation = sc[OBME_PS_FIX_MAX] * growth_req * fix_limit * nut_lim * light_lim;
-    const FT up_NO3 = qdiv(sP.muI * sP.LNO3, sP.LN + e0) + qdiv(sD.muI * sD.LNO3, sD.LN + e0);
-    const FT up_NH4 = qdiv(sP.muI * sP.LNH4, sP.LN + e0) + qdiv(sD.muI * sD.LNH4, sD.LN + e0);
+    // (L <= LN: no uptake where LN = 0)
+    const FT upP = qdiv(sP.muI, sP.LN + e0), upD = qdiv(sD.muI, sD.LN + e0);
+    const FT up_NO3 = upP * sP.LNO3 + upD * sD.LNO3;
+    const FT up_NH4 = upP * sP.LNH4 + upD * sD.LNH4;
     G[OBME_PI_NO3] = nitrif + thN * (oxic - up_NO3);
     G[OBME_PI_NH4] = fixation + thN * (anoxic + inorg_exc + ut_respiration - up_NH4) - nitrif;
 

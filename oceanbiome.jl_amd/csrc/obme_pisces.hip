@@ -315,7 +315,7 @@ __global__ void __launch_bounds__(256) k_pisces_prep(PiscesArgs<FT> a)
         // the temperature factors of the transitions, with T fixed
         TFac<FT> t;
         temperature_factors(a.pp, a.in[OBME_PI_T][p], t);
-        const FT tv[TFAC_FIELDS] = {t.btN, t.btD, t.bZ, t.bM, t.doc, t.pom, t.rain, t.kfe, t.eq, t.t4};
+        const FT tv[TFAC_FIELDS] = {t.btN, t.btD, t.bZ, t.bM, t.doc, t.pom, t.rain, t.kfe, t.req, t.t4, t.t15};
 #pragma unroll
         for (int n = 0; n < TFAC_FIELDS; n++) a.tfac[(long)n * ncell + c] = tv[n];
     }
@@ -426,8 +426,9 @@ k_pisces_cell(PiscesArgs<FT> a)
         tf.pom = t[5 * ncell];
         tf.rain = t[6 * ncell];
         tf.kfe = t[7 * ncell];
-        tf.eq = t[8 * ncell];
+        tf.req = t[8 * ncell];
         tf.t4 = t[9 * ncell];
+        tf.t15 = t[10 * ncell];
     } else {
         temperature_factors(a.pp, v[OBME_PI_T], tf);
     }
@@ -674,7 +675,7 @@ __global__ void __launch_bounds__(PF_WAVES * 64, OBME_PISCES_PF_OCC) k_pisces_fu
         // the temperature factors, once per step
         TFac<FT> t;
         temperature_factors(a.pp, v[OBME_PI_T], t);
-        const FT tv[TFAC_FIELDS] = {t.btN, t.btD, t.bZ, t.bM, t.doc, t.pom, t.rain, t.kfe, t.eq, t.t4};
+        const FT tv[TFAC_FIELDS] = {t.btN, t.btD, t.bZ, t.bM, t.doc, t.pom, t.rain, t.kfe, t.req, t.t4, t.t15};
 #pragma unroll
         for (int q = 0; q < TFAC_FIELDS; q++) s_tf[q][tid] = tv[q];
     }
@@ -824,9 +825,10 @@ __global__ void __launch_bounds__(PF_WAVES * 64, OBME_PISCES_PF_OCC) k_pisces_fu
             tf.pom = s_tf[5][tid];
             tf.rain = s_tf[6][tid];
             tf.kfe = s_tf[7][tid];
-            tf.eq = s_tf[8][tid];
+            tf.req = s_tf[8][tid];
             tf.t4 = s_tf[9][tid];
-            pisces_tendencies(pps, v, A, f.sk[sn][st], tf, G);
+            tf.t15 = s_tf[10][tid];
+            pisces_tendencies<true>(pps, v, A, f.sk[sn][st], tf, G);
             // flux-form upwind sinking: (w(k+1) c(k+1) - w(k) c(k)) / dz, the
             // level above from lane r - 1, w = 0 on the top face
             auto sink = [&](int n, FT wlo, FT whi) {
