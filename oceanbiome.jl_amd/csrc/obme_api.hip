@@ -1622,10 +1622,16 @@ extern "C" obme_status obme_kernel_timing(obme_handle* h, int32_t which, double*
 
 // ------------------------------------------------------------------ batched ensemble
 
-template <typename FT, int L, int CPW, int NW, bool SED = false>
-__global__ void __launch_bounds__(NW * 64, (SED && sizeof(FT) == 4 && L == 2) ? 5 : 1) k_batch(BatchArgs<FT> a)
+template <int L, int CPW, int NW>
+__global__ void __launch_bounds__(NW * 64, L == 2 ? 5 : 1) k_batch(BatchArgs<float> a)
 {
-    batch_columns<FT, L, CPW, NW, SED>(a);
+    batch_columns<float, L, CPW, NW, true>(a);
+}
+constexpr int RAGGED_WAVES = 4;   // waves per workgroup
+template <typename FT, int L, int FM, bool SED>
+__global__ void __launch_bounds__(RAGGED_WAVES * 64) k_batch_ragged(BatchArgs<FT> a)
+{
+    batch_ragged<FT, L, FM, SED>(a);
 }
 
 // Tile shapes of the ensemble kernel: capacity L*64/CPW levels per column.
@@ -1656,6 +1662,11 @@ struct obme_batch {
     int steps_per_launch = 0;             // 0: every step of a call in one launch per class
     std::vector<int> class_tile, class_n; // per class of the plan
     std::vector<int*> class_cols;
+    // the ragged packing (all but FP32 with a sediment): per levels per lane
+    // of the plan's classes, the lanes' table and its waves
+    bool default_forms = false;
+    std::vector<int*> group_lanes;
+    std::vector<int> group_L, group_waves;
     // captured multi-launch step
     hipStream_t cap_stream = nullptr;
     hipGraphExec_t graph = nullptr;
@@ -1680,6 +1691,41 @@ static void batch_free_classes(obme_batch* b)
     b->class_cols.clear();
     b->class_tile.clear();
     b->class_n.clear();
+    for (int* p : b->group_lanes)
+        if (p) (void)hipFree(p);
+    b->group_lanes.clear();
+    b->group_L.clear();
+    b->group_waves.clear();
+}
+
+// The ragged packing of the columns with L levels per lane, each lane's column
+// or -1: longest first, each into the wave with the least room that still
+// holds it.
+static std::vector<int> pack_ragged(const obme_batch* b, const std::vector<int>& cols, int L)
+{
+    std::vector<int> by_lanes[65];
+    for (int c : cols) by_lanes[(b->offsets[c + 1] - b->offsets[c] + L - 1) / L].push_back(c);
+    std::vector<int> lanes;
+    std::vector<int> room[65];        // waves by their free lanes
+    for (int n = 64; n >= 1; n--)
+        for (int c : by_lanes[n]) {
+            int f = n, w;
+            while (f <= 64 && room[f].empty()) f++;
+            if (f > 64) {
+                f = 64;
+                w = (int)(lanes.size() / 64);
+                lanes.resize(lanes.size() + 64, -1);
+            } else {
+                w = room[f].back();
+                room[f].pop_back();
+            }
+            std::fill_n(lanes.begin() + ((size_t)w * 64 + (64 - f)), n, c);
+            if (f > n) room[f - n].push_back(w);
+        }
+    // whole workgroups
+    const size_t wg = 64 * RAGGED_WAVES;
+    lanes.resize((lanes.size() + wg - 1) / wg * wg, -1);
+    return lanes;
 }
 
 static void batch_drop_graph(obme_batch* b)
@@ -1690,7 +1736,8 @@ static void batch_drop_graph(obme_batch* b)
 }
 
 // Sorts the columns into the classes of plan p (smallest capacity that holds
-// the column), deepest columns first within a class.
+// the column): packed by levels per lane, or, FP32 with a sediment, class by
+// class, deepest columns first.
 static obme_status batch_apply_plan(obme_batch* b, int p)
 {
     if (p < 0 || p >= (int)BATCH_PLANS.size()) return fail(OBME_ERR_INVALID, "unknown packing plan");
@@ -1707,9 +1754,28 @@ static obme_status batch_apply_plan(obme_batch* b, int p)
     }
     batch_free_classes(b);
     batch_drop_graph(b);
+    const bool ragged = !(b->sediment && b->prec != OBME_FP64);
+    if (ragged) {
+        for (int L : {1, 2, 4}) {
+            std::vector<int> cols;
+            for (size_t t = 0; t < tiles.size(); t++)
+                if (BATCH_TILES[tiles[t]].L == L) cols.insert(cols.end(), lists[t].begin(), lists[t].end());
+            const std::vector<int> lanes = pack_ragged(b, cols, L);
+            if (lanes.empty()) continue;
+            int* d = nullptr;
+            HIP_TRY(hipMalloc((void**)&d, lanes.size() * sizeof(int)));
+            b->group_lanes.push_back(d);
+            b->group_L.push_back(L);
+            b->group_waves.push_back((int)(lanes.size() / 64));
+            HIP_TRY(hipMemcpy(d, lanes.data(), lanes.size() * sizeof(int), hipMemcpyHostToDevice));
+        }
+    }
     for (size_t t = 0; t < tiles.size(); t++) {
         std::vector<int>& l = lists[t];
         if (l.empty()) continue;
+        b->class_tile.push_back(tiles[t]);
+        b->class_n.push_back((int)l.size());
+        if (ragged) continue;
         std::stable_sort(l.begin(), l.end(), [&](int x, int y) {
             return b->offsets[x + 1] - b->offsets[x] > b->offsets[y + 1] - b->offsets[y];
         });
@@ -1717,8 +1783,6 @@ static obme_status batch_apply_plan(obme_batch* b, int p)
         HIP_TRY(hipMalloc((void**)&d, l.size() * sizeof(int)));
         HIP_TRY(hipMemcpy(d, l.data(), l.size() * sizeof(int), hipMemcpyHostToDevice));
         b->class_cols.push_back(d);
-        b->class_tile.push_back(tiles[t]);
-        b->class_n.push_back((int)l.size());
     }
     b->plan = p;
     return OBME_OK;
@@ -1759,8 +1823,7 @@ static BatchArgs<FT> batch_args(const obme_batch* b, void* const* tracers, doubl
     return a;
 }
 
-template <typename FT>
-static obme_status batch_launch_class(const obme_batch* b, int q, BatchArgs<FT> a, int nsteps, hipStream_t s)
+static obme_status batch_launch_class(const obme_batch* b, int q, BatchArgs<float> a, int nsteps, hipStream_t s)
 {
     a.cols = b->class_cols[q];
     a.ncols = b->class_n[q];
@@ -1768,23 +1831,57 @@ static obme_status batch_launch_class(const obme_batch* b, int q, BatchArgs<FT> 
     const BatchTile& t = BATCH_TILES[b->class_tile[q]];
     const int per_wg = t.NW * t.CPW;
     dim3 grid((a.ncols + per_wg - 1) / per_wg), block(t.NW * 64);
-    using Kernel = void (*)(BatchArgs<FT>);
+    using Kernel = void (*)(BatchArgs<float>);
     Kernel k = nullptr;
-#define OBME_BATCH_KERNEL(L_, CPW_) (b->sediment ? k_batch<FT, L_, CPW_, 4, true> : k_batch<FT, L_, CPW_, 4, false>)
     switch (b->class_tile[q]) {
-    case 0: k = OBME_BATCH_KERNEL(1, 4); break;
-    case 1: k = OBME_BATCH_KERNEL(2, 4); break;
-    case 2: k = OBME_BATCH_KERNEL(1, 2); break;
-    case 3: k = OBME_BATCH_KERNEL(2, 2); break;
-    case 4: k = OBME_BATCH_KERNEL(1, 1); break;
-    case 5: k = OBME_BATCH_KERNEL(2, 1); break;
-    case 6: k = OBME_BATCH_KERNEL(4, 2); break;
-    case 7: k = OBME_BATCH_KERNEL(4, 4); break;
+    case 0: k = k_batch<1, 4, 4>; break;
+    case 1: k = k_batch<2, 4, 4>; break;
+    case 2: k = k_batch<1, 2, 4>; break;
+    case 3: k = k_batch<2, 2, 4>; break;
+    case 4: k = k_batch<1, 1, 4>; break;
+    case 5: k = k_batch<2, 1, 4>; break;
+    case 6: k = k_batch<4, 2, 4>; break;
+    case 7: k = k_batch<4, 4, 4>; break;
     default: return fail(OBME_ERR_INVALID, "bad batch tile");
     }
-#undef OBME_BATCH_KERNEL
     hipLaunchKernelGGL(k, grid, block, 0, s, a);
     HIP_TRY(hipGetLastError());
+    return OBME_OK;
+}
+
+template <typename FT, bool SED>
+static void (*ragged_kernel(int L, bool default_forms))(BatchArgs<FT>)
+{
+    constexpr int FM = default_fm<OBME_NPZD>();
+    switch (L) {
+    case 1: return default_forms ? k_batch_ragged<FT, 1, FM, SED> : k_batch_ragged<FT, 1, -1, SED>;
+    case 2: return default_forms ? k_batch_ragged<FT, 2, FM, SED> : k_batch_ragged<FT, 2, -1, SED>;
+    default: return default_forms ? k_batch_ragged<FT, 4, FM, SED> : k_batch_ragged<FT, 4, -1, SED>;
+    }
+}
+
+// One launch per levels per lane, or per class.
+template <typename FT>
+static obme_status batch_launch(const obme_batch* b, BatchArgs<FT> a, int nsteps, hipStream_t s)
+{
+    if constexpr (sizeof(FT) == 4) {
+        if (b->sediment) {
+            for (size_t q = 0; q < b->class_tile.size(); q++) {
+                obme_status r = batch_launch_class(b, (int)q, a, nsteps, s);
+                if (r != OBME_OK) return r;
+            }
+            return OBME_OK;
+        }
+    }
+    a.nsteps = nsteps;
+    for (size_t q = 0; q < b->group_L.size(); q++) {
+        a.cols = b->group_lanes[q];
+        void (*k)(BatchArgs<FT>) = ragged_kernel<FT, false>(b->group_L[q], b->default_forms);
+        if constexpr (sizeof(FT) == 8)
+            if (b->sediment) k = ragged_kernel<FT, true>(b->group_L[q], b->default_forms);
+        hipLaunchKernelGGL(k, dim3((unsigned)(b->group_waves[q] / RAGGED_WAVES)), dim3(RAGGED_WAVES * 64), 0, s, a);
+        HIP_TRY(hipGetLastError());
+    }
     return OBME_OK;
 }
 
@@ -1843,10 +1940,8 @@ static obme_status batch_enqueue(const obme_batch* b, void* const* tracers, int 
         a.c_out = (done + n < nsteps && b->d_comp) ? 1 : 0;
         a.sed_init = (done == 0) ? sc.init : 0;
         a.sed_ab2 = (done == 0) ? sc.ab2 : 0;
-        for (size_t q = 0; q < b->class_tile.size(); q++) {
-            obme_status r = batch_launch_class<FT>(b, (int)q, a, n, s);
-            if (r != OBME_OK) return r;
-        }
+        obme_status r = batch_launch<FT>(b, a, n, s);
+        if (r != OBME_OK) return r;
     }
     return OBME_OK;
 }
@@ -1964,6 +2059,8 @@ extern "C" obme_status obme_batch_create(const obme_config* cfg, int32_t n_colum
         q.zooplankton_assimilation_fraction = get(OBME_BP_ZOO_ASSIMILATION_FRACTION, q.zooplankton_assimilation_fraction);
         q.remineralisation_rate = get(OBME_BP_REMINERALISATION_RATE, q.remineralisation_rate);
         q.small_particle_fraction = get(OBME_BP_SMALL_PARTICLE_FRACTION, q.small_particle_fraction);
+        // (the formulations are the configuration's, the same for every column)
+        if (c == 0) b->default_forms = (fm_code(make_fast_params<float>(q)) == default_fm<OBME_NPZD>());
         if (f64) dpar[c] = make_fast_params<double>(q);
         else fpar[c] = make_fast_params<float>(q);
         if (fixed) spar[c] = make_sediment_params(q);

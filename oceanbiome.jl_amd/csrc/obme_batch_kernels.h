@@ -18,15 +18,20 @@
 // once, at the end of the call.
 //
 // Layout: tracer n (N, P, Z, D) is one packed array; column c occupies
-// [offsets[c], offsets[c+1]) with k = 0 at the bottom.  Columns are packed
-// into wave segments of LPC = 64/CPW lanes, lane r of a segment holding the
-// L levels counted from the top, j = r*L + m (k = Nz_c - 1 - j).  The host
-// sorts columns into classes by depth (capacity L*LPC >= Nz_c) and launches
-// one persistent kernel per class over that class's column list.  Cell
-// centres depend only on j: zc = -(j + 1/2) dz.
+// [offsets[c], offsets[c+1]) with k = 0 at the bottom.  Lane r of a column
+// holds the L levels counted from the top, j = r*L + m (k = Nz_c - 1 - j).
+// Cell centres depend only on j: zc = -(j + 1/2) dz.  The host sorts columns
+// into classes by depth; what becomes of them on the lanes:
+//  - batch_ragged: a column takes ceil(Nz_c / L) lanes and a wave as many
+//    columns as fit into its 64 lanes, of every class with the same L; the
+//    sums down a column are masked to its lanes;
+//  - batch_columns (FP32 with a sediment): a class's columns in segments of
+//    LPC = 64/CPW lanes (capacity L*LPC >= Nz_c), one persistent kernel per
+//    class.  The sediment's storage is FP64, and a sum down a column in
+//    another order moves it.
 #pragma once
 
-#include "obme_npd_kernels.h"
+#include "obme_wave_kernels.h"
 
 namespace obme {
 
@@ -43,8 +48,8 @@ struct BatchArgs {
     FT* C[4];                       // FP32: the residuals of U, packed alike (launch to launch)
     int c_in, c_out;                // FP32: start from the stored residuals; store them at the end
     const int* offsets;             // [n_columns + 1]
-    const int* cols;                // this class's column list
-    int ncols;                      // entries of `cols`
+    const int* cols;                // this class's column list; batch_ragged: each lane's column (or -1)
+    int ncols;                      // entries of `cols` (batch_columns)
     const FastParams<FT>* fpar;     // per-column derived constants
     const SedimentParams* fsed;     // FP32 with a sediment: the same, for its transitions
     const BatchColumn* bcol;        // per-column constants
@@ -312,6 +317,202 @@ __device__ __forceinline__ void batch_columns(const BatchArgs<FT>& a)
                     }
                 }
     }
+}
+
+// The ragged packing: the lane's column from the host's table.
+// What bounds it is the instructions of the transitions (four waves per SIMD,
+// nothing read or written between the first step and the last), so lanes
+// without a level are time lost: segments of 32 and 64 lanes held 72 % levels
+// where columns have 16 to 128, in two launches of one wave's length each
+// (8192 such columns, 50 steps in FP32: 404 us; this 269).  FM: the
+// default formulations compiled in, or < 0 (fm_light).
+template <typename FT, int L, int FM, bool SED>
+__device__ __forceinline__ void batch_ragged(const BatchArgs<FT>& a)
+{
+    constexpr bool F32 = sizeof(FT) == 4;
+    static_assert(!(F32 && SED), "FP32 with a sediment: batch_columns");
+    const int lane = threadIdx.x & 63;
+    const int at = a.cols[blockIdx.x * blockDim.x + threadIdx.x];
+    const bool ok = at >= 0;
+    const int col = ok ? at : 0;
+    // the lane's place in its column: from the last lane at or before it whose
+    // predecessor has another (a lane without a column stands alone)
+    const int before = __shfl_up(at, 1, 64);   // (by every lane)
+    const unsigned long long starts = __ballot(lane == 0 || !ok || before != at);
+    const int r = lane - (63 - __clzll((long long)(starts & (~0ull >> (63 - lane)))));
+    const int off = a.offsets[col];
+    const int Nzc = ok ? a.offsets[col + 1] - off : 0;
+    auto has = [&](int m) -> bool { return r * L + m < Nzc; };
+    auto idx = [&](int m) -> int { return off + Nzc - 1 - (r * L + m); };
+    const ColumnMasks cm = column_masks<0>(lane, r);
+
+    // (a lane's levels below the bottom hold 1: they feed no other lane or
+    // level, and their powers are ordinary ones)
+    FT U[4][L], D[F32 ? 4 : 1][L], Gm[4][L];
+#pragma unroll
+    for (int n = 0; n < 4; n++)
+#pragma unroll
+        for (int m = 0; m < L; m++) {
+            U[n][m] = has(m) ? a.U[n][idx(m)] : FT(1);
+            if constexpr (F32) D[n][m] = (a.c_in && has(m)) ? a.C[n][idx(m)] : FT(0);
+        }
+    const BatchColumn bc = a.bcol[col];
+    const FT Lt = (FT)bc.Lt;
+    const FT wiP = (FT)(bc.wP / (double)a.dz), wiD = (FT)(bc.wD / (double)a.dz);
+    const FastParams<FT> fp = a.fpar[col];
+
+    // the sediment of the column, held by the lane of its bottom cell
+    const int jb = Nzc - 1, mb = jb % L;
+    const bool sed = SED && ok && r == jb / L;
+    double sed_u = 0.0, sed_ge = 0.0;
+    if (sed) {
+        sed_u = a.storage ? a.storage[col] : 0.0;
+        sed_ge = (a.storage && a.sed_ab2) ? a.sedGm[col] : 0.0;
+    }
+
+    // the surface light left by the water alone at the own levels, halved
+    FT wr[L], wb[L];
+#pragma unroll
+    for (int m = 0; m < L; m++) {
+        const double zc = -((double)(r * L + m) + 0.5) * (double)a.dz, h = 0.5 * (ok ? bc.PAR0 : 0.0);
+        wr[m] = (FT)(h * exp(a.kr * zc));
+        wb[m] = (FT)(h * exp(a.kb * zc));
+    }
+    const double g2 = 5.0 / 12.0, g3 = 3.0 / 4.0, z2 = -17.0 / 60.0, z3 = -5.0 / 12.0;
+    const FT hr = F32 ? (FT)a.xr2h : (FT)(a.xr * (0.5 * (double)a.dz));
+    const FT hb = F32 ? (FT)a.xb2h : (FT)(a.xb * (0.5 * (double)a.dz));
+
+#pragma unroll 1
+    for (int s = 0; s < a.nsteps; s++) {
+        auto stage = [&](auto st_c) {
+            constexpr int st = decltype(st_c)::value;
+            FT X[4][L];
+#pragma unroll
+            for (int n = 0; n < 4; n++)
+#pragma unroll
+                for (int m = 0; m < L; m++) {
+                    if constexpr (F32) X[n][m] = U[n][m] + D[n][m];
+                    else X[n][m] = U[n][m];
+                }
+            // the light: the integral to level j is, in half cells, twice the
+            // sum over the levels above and the level's own
+            FT pr[L], pb[L];
+            FT totr = FT(0), totb = FT(0);
+#pragma unroll
+            for (int m = 0; m < L; m++) {
+                if constexpr (F32) {
+                    const float lg = m_log2(X[1][m]);
+                    pr[m] = m_exp2(fmaf(a.er_f, lg, a.cr));
+                    pb[m] = m_exp2(fmaf(a.eb_f, lg, a.cb));
+                } else {
+                    pow_pair(X[1][m] * a.Rr, a.er, a.eb, pr[m], pb[m]);
+                }
+                totr = m == 0 ? pr[m] : totr + pr[m];
+                totb = m == 0 ? pb[m] : totb + pb[m];
+            }
+            FT runr = lane_above<0>(column_prefix<0>(totr, cm), cm);
+            FT runb = lane_above<0>(column_prefix<0>(totb, cm), cm);
+            const FT cP_up = lane_above<0>(X[1][L - 1], cm), cD_up = lane_above<0>(X[3][L - 1], cm);
+            FT PARv[L];
+#pragma unroll
+            for (int m = 0; m < L; m++) {
+                const FT Ir = fma(FT(2), runr, pr[m]), Ib = fma(FT(2), runb, pb[m]);
+                runr = runr + pr[m];
+                runb = runb + pb[m];
+                if constexpr (F32) PARv[m] = fma(wr[m], m_exp2(-hr * Ir), wb[m] * m_exp2(-hb * Ib));
+                else PARv[m] = wr[m] * m_exp(-hr * Ir) + wb[m] * m_exp(-hb * Ib);
+            }
+            // the sediment: the bottom cell's flux and burial, the receiver's
+            // coupled tendency, the sediment step
+            FT cpl = FT(0);
+            if constexpr (SED) {
+                if (sed) {
+                    FT Pb = X[1][0], Db = X[3][0];
+#pragma unroll
+                    for (int m = 1; m < L; m++)
+                        if (m == mb) {
+                            Pb = X[1][m];
+                            Db = X[3][m];
+                        }
+                    const FT f = a.sedP * (-bc.wP) * Pb + a.sedD * (-bc.wD) * Db;
+                    const FT qf = f / (a.sed_k + f);
+                    const FT e = a.sed_a + a.sed_b * (qf * qf);
+                    cpl = ((FT(1) - e) * f) / a.dz;
+                    const double ge = (double)(e * f);
+                    const bool init = a.sed_init && s == 0;
+                    if (st == 0) {
+                        if (!init)
+                            sed_u += a.sed_dt[0] * (a.sed_ab2 && s == 0 ? a.sed_cn * ge - a.sed_cm * sed_ge : ge);
+                    } else {
+                        if (st == 1 && init) sed_u += a.sed_dt[0] * ge;
+                        sed_u += a.sed_dt[st] * ge;
+                    }
+                    sed_ge = ge;
+                }
+            }
+            // tendencies, sinking, RK3 substep
+#pragma unroll
+            for (int m = 0; m < L; m++) {
+                FT G[4];
+                npzd_fast<FM>(fp, X[0][m], X[1][m], X[2][m], X[3][m], PARv[m], Lt, G[0], G[1], G[2], G[3]);
+                // (the lane above the top one gives 0)
+                const FT cPn = m == 0 ? cP_up : X[1][m > 0 ? m - 1 : 0];
+                const FT cDn = m == 0 ? cD_up : X[3][m > 0 ? m - 1 : 0];
+                G[1] = fma(-wiP, cPn - X[1][m], G[1]);
+                G[3] = fma(-wiD, cDn - X[3][m], G[3]);
+                if constexpr (SED) {
+                    if (sed && m == mb) {
+#pragma unroll
+                        for (int n = 0; n < 4; n++)
+                            if (n == a.sed_recv) G[n] = G[n] + cpl;
+                    }
+                }
+#pragma unroll
+                for (int n = 0; n < 4; n++) {
+                    if constexpr (F32) {
+                        if constexpr (st == 0) D[n][m] = fmaf(a.rk_a[0], G[n], D[n][m]);
+                        else D[n][m] = fmaf(a.rk_a[st], G[n], fmaf(a.rk_b[st], Gm[n][m], D[n][m]));
+                    } else {
+                        if constexpr (st == 0) U[n][m] += (a.dtf * (8.0 / 15.0)) * G[n];
+                        else U[n][m] += a.dtf * ((st == 1 ? g2 : g3) * G[n] + (st == 1 ? z2 : z3) * Gm[n][m]);
+                    }
+                    Gm[n][m] = G[n];
+                }
+            }
+        };
+        stage(std::integral_constant<int, 0>{});
+        stage(std::integral_constant<int, 1>{});
+        stage(std::integral_constant<int, 2>{});
+        if constexpr (F32) {
+            // U + D = s + e exactly (TwoSum): U = s, and e carries on
+#pragma unroll
+            for (int n = 0; n < 4; n++)
+#pragma unroll
+                for (int m = 0; m < L; m++) {
+                    const float u = U[n][m], d = D[n][m];
+                    const float sum = u + d;
+                    const float dv = sum - u;
+                    D[n][m] = (u - (sum - dv)) + (d - dv);
+                    U[n][m] = sum;
+                }
+        }
+    }
+    if constexpr (SED) {
+        if (sed && a.storage) {
+            a.storage[col] = sed_u;
+            a.sedGm[col] = sed_ge;
+        }
+    }
+#pragma unroll
+    for (int n = 0; n < 4; n++)
+#pragma unroll
+        for (int m = 0; m < L; m++)
+            if (has(m)) {
+                a.U[n][idx(m)] = U[n][m];
+                if constexpr (F32) {
+                    if (a.c_out) a.C[n][idx(m)] = D[n][m];
+                }
+            }
 }
 
 }  // namespace obme
