@@ -1068,7 +1068,17 @@ static obme_status run_typed(obme_handle* h, void* const* tracers, void* const* 
     }
     obme_status r = OBME_OK;
     WaveShape ws;
-    if constexpr (MODE == TILE_TENDENCY || MODE == TILE_PAR) ws = wave_shape<FT>(h, MODE, 1, false);
+    if constexpr (MODE == TILE_TENDENCY) ws = wave_shape<FT>(h, MODE, 1, false);
+    if constexpr (MODE == TILE_PAR) {
+        using Shape = LightShape<FT>;
+        const unsigned ncol = (unsigned)(a.Nx * a.Ny);
+        if (ncol <= Shape::MOST_COLUMNS) {
+            hipLaunchKernelGGL(k_light<FT>, dim3((ncol + Shape::COLS - 1) / Shape::COLS), dim3(Shape::THREADS), 0, s, a,
+                               (const FT*)tracers[h->cfg.model == OBME_NPZD ? 1 : 2], ncol);
+            HIP_TRY(hipGetLastError());
+            return OBME_OK;
+        }
+    }
     if (ws.levels) {
         WaveArgs<FT> w;
         std::memset(&w, 0, sizeof(w));

@@ -229,9 +229,10 @@ enum { LEV_ZC = 0, LEV_UP, LEV_DN, LEV_INVDZ, LEV_WR, LEV_WB, LEV_COUNT };
 // LEV_WR, LEV_WB: half the light left by the water alone at zc, exp(k zc) / 2
 // of the red and blue bands, formed in FP64.
 
-// Modes of the column sweep: the fused RK3 step, the tendencies (hook), the
-// PAR (hook), one RK3 stage with its substep (the step of the sinking schemes
-// whose face values need the levels below).
+// What a launch does: the fused RK3 step, the tendencies (hook), the PAR (hook;
+// k_light, and the sweep for many columns in FP64), one RK3 stage with its
+// substep (the step of the sinking schemes whose face values need the levels
+// below).
 enum { TILE_STEP = 0, TILE_TENDENCY = 1, TILE_PAR = 2, TILE_STAGE = 3 };
 
 // The value at face k of a sinking tracer reconstructed from above (w <= 0:
@@ -969,6 +970,127 @@ struct SurfaceArgs {
     const FT* Dsc;
     unsigned ncell;
 };
+
+// The light hook: TwoBand PAR (Light/2band.jl:18-32) of P into the parent array.
+// A block takes COLS columns that follow each other, in chunks of up to ROWS x
+// LEVELS levels from the top: a thread works n = ceil(Nz / ROWS) <= LEVELS
+// levels of its column, and the integral above them is the sum of the rows
+// above (PAR = PAR0 (e^(kr zc - χr ∫r) + e^(kb zc - χb ∫b)) / 2).  What bounds it is
+// reading P and writing PAR; one lane per column walked its levels one load
+// after the other (384x384x64 in FP32: 40 us, 1.9 TB/s; this 24).  FP64: what
+// bounds it are the powers (260 instructions a level), whose code is too long
+// to unroll (eight levels: 27 us of fetching it on 17x76x58, 8 with a loop);
+// its levels wait in LDS.  Above 65536 columns FP64 takes the sweep, which keeps
+// the powers' constants in registers down the column (500x300x40: 50 us | 60;
+// with the tendencies 256x256x64 221 | 215, 333x187x20 65.6 | 65.1).
+template <typename FT>
+struct LightShape {
+    static constexpr int COLS = sizeof(FT) == 4 ? 64 : 32;
+    static constexpr int ROWS = 8, LEVELS = 8, THREADS = COLS * ROWS;
+    static constexpr unsigned MOST_COLUMNS = sizeof(FT) == 4 ? ~0u : 65536u;
+};
+template <typename FT>
+__global__ void __launch_bounds__(LightShape<FT>::THREADS, 4) k_light(StepArgs<FT> a, const FT* P, unsigned ncol)
+{
+    constexpr bool F32 = sizeof(FT) == 4;
+    constexpr int COLS = LightShape<FT>::COLS, ROWS = LightShape<FT>::ROWS, LEVELS = LightShape<FT>::LEVELS;
+    constexpr int UNROLL = F32 ? LEVELS : 1;
+    // a chunk's levels: the thickness from zf(k+1) to zc(k), the whole level's
+    // and the light left by the water alone in both bands
+    struct alignas(4 * sizeof(FT)) Level {
+        FT above, whole, wr, wb;
+    };
+    __shared__ Level s_level[ROWS * LEVELS];
+    __shared__ FT s_row[2][ROWS][COLS];
+    __shared__ FT s_power[F32 ? 1 : 2][F32 ? 1 : LEVELS][F32 ? 1 : ROWS * COLS];
+    const int c = threadIdx.x % COLS, g = threadIdx.x / COLS;
+    const unsigned q = blockIdx.x * COLS + c;
+    const bool ok = q < ncol;
+    const unsigned base = a.base0 + (ok ? q % (unsigned)a.Nx + a.sx * (q / (unsigned)a.Nx) : 0u);
+    const int Nz = a.Nz;
+    const int n = min((Nz + ROWS - 1) / ROWS, LEVELS), chunk = n * ROWS;
+    const rsrc_t out = make_rsrc(a.PAR, a.field_bytes);
+    FT PAR0 = a.surface_mode == OBME_SURFACE_DIURNAL ? a.PAR0_stage[0] : a.surface_value;
+    if (a.surface_mode == OBME_SURFACE_ARRAY) PAR0 = a.surf[ok ? q : 0];
+    FT pr[LEVELS], pb[LEVELS];          // FP32: the levels' powers
+    auto power = [&](int band, int u) -> FT& {
+        if constexpr (F32) return band ? pb[u] : pr[u];
+        else return s_power[band][u][threadIdx.x];
+    };
+    FT Cr = FT(0), Cb = FT(0);          // the integrals over the chunks above
+#pragma unroll 1
+    for (int k0 = Nz - 1; k0 >= 0; k0 -= chunk) {
+        const int kt = k0 - g * n;
+        // (levels below the bottom: the bottom one again, of no thickness)
+        FT x[LEVELS];
+#pragma unroll
+        for (int u = 0; u < LEVELS; u++)
+            if (u < n) x[u] = P[base + a.sxy * (unsigned)max(kt - u, 0)];
+        if (threadIdx.x < chunk) {
+            const int k = k0 - (int)threadIdx.x;
+            Level v = {FT(0), FT(0), FT(0), FT(0)};
+            if (k >= 0) {
+                v.above = a.lev[LEV_DN * Nz + k];
+                v.whole = v.above + (k > 0 ? a.lev[LEV_UP * Nz + k - 1] : FT(0));
+                v.wr = a.lev[LEV_WR * Nz + k];
+                v.wb = a.lev[LEV_WB * Nz + k];
+            }
+            s_level[threadIdx.x] = v;
+        }
+#pragma unroll
+        for (int u = 0; u < LEVELS; u++)
+            if (u < n) power(0, u) = x[u];
+        __syncthreads();
+        FT Sr = FT(0), Sb = FT(0);
+#pragma unroll UNROLL
+        for (int u = 0; u < LEVELS; u++) {
+            if (u >= n) break;
+            const FT p = power(0, u);
+            FT r, b;
+            if constexpr (F32) {
+                const float lg = m_log2(p);
+                r = m_exp2(fmaf(a.er, lg, a.cr));
+                b = m_exp2(fmaf(a.eb, lg, a.cb));
+            } else {
+                pow_pair(p * a.Rr, a.er, a.eb, r, b);
+            }
+            power(0, u) = r;
+            power(1, u) = b;
+            const FT w = s_level[g * n + u].whole;
+            Sr = fma(w, r, Sr);
+            Sb = fma(w, b, Sb);
+        }
+        s_row[0][g][c] = Sr;
+        s_row[1][g][c] = Sb;
+        __syncthreads();
+        FT Ir = Cr, Ib = Cb;
+#pragma unroll
+        for (int m = 0; m < ROWS; m++) {
+            const FT sr = s_row[0][m][c], sb = s_row[1][m][c];
+            if (m < g) {
+                Ir += sr;
+                Ib += sb;
+            }
+            Cr += sr;
+            Cb += sb;
+        }
+#pragma unroll UNROLL
+        for (int u = 0; u < LEVELS; u++) {
+            if (u >= n) break;
+            const Level v = s_level[g * n + u];
+            const FT r = power(0, u), b = power(1, u);
+            const FT Jr = fma(v.above, r, Ir), Jb = fma(v.above, b, Ib);
+            FT PAR;
+            if constexpr (F32) PAR = PAR0 * fmaf(v.wr, m_exp2(-a.xr2 * Jr), v.wb * m_exp2(-a.xb2 * Jb));
+            else PAR = PAR0 * (v.wr * m_exp(-a.xr * Jr) + v.wb * m_exp(-a.xb * Jb));
+            const unsigned off = (base + a.sxy * (unsigned)max(kt - u, 0)) * (unsigned)sizeof(FT);
+            buf_store(out, ok && u <= kt ? off : a.field_bytes, PAR);
+            Ir = fma(v.whole, r, Ir);
+            Ib = fma(v.whole, b, Ib);
+        }
+        if (k0 >= chunk) __syncthreads();
+    }
+}
 
 // The surface constants of every column (T and S of the top cell), once per
 // stepper call, for k_surface: a.surfc_cols columns (one where T and S do

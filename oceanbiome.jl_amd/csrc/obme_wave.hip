@@ -37,7 +37,6 @@ static WaveKernel<FT> wave_kernel_levels(int mode, bool uniform, int lpc, bool g
         if (mode == TILE_TENDENCY)
             return win ? k_column_wave<MODEL, CARB, FT, TILE_TENDENCY, false, L, false, true, FM>
                        : k_column_wave<MODEL, CARB, FT, TILE_TENDENCY, false, L, false, false, FM>;
-        if (mode == TILE_PAR) return k_column_wave<MODEL, CARB, FT, TILE_PAR, false, L, false, false, FM>;
     }
     return nullptr;
 }

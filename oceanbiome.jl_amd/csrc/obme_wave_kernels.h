@@ -188,7 +188,7 @@ __device__ __forceinline__ const FastParams<FT>& transition_params(const WaveArg
     return *(const FastParams<FT>*)(Shared)(unsigned long long)p;
 }
 
-// MODE: TILE_STEP, TILE_TENDENCY or TILE_PAR.  UNI: uniform grid with
+// MODE: TILE_STEP or TILE_TENDENCY.  UNI: uniform grid with
 // constant sinking speeds (FP32 folds the half cell into the attenuation).
 // GEN (step): the negative scaling, the sediment and the recorded top cell,
 // chosen at run time.  WIN: the centred and WENO face values.
@@ -209,7 +209,7 @@ __device__ __forceinline__ void column_wave(const WaveArgs<FT>& w, FT* lds)
     // registers than there are, and kept through the loop they are moved from
     // vector lanes (180 of 1000 vector instructions of a stage); with two
     // levels the vector registers have no room for the reads
-    constexpr bool SHARED = !F32 && L == 1 && MODE != TILE_PAR;
+    constexpr bool SHARED = !F32 && L == 1;
     const StepArgs<FT>& a = w.a;
 
     const int tid = threadIdx.x, T = blockDim.x;
@@ -241,7 +241,6 @@ __device__ __forceinline__ void column_wave(const WaveArgs<FT>& w, FT* lds)
         return io_slot0 + (jt % L) * 64 + jt / L;
     };
     auto reads = [&](int n) -> bool {
-        if (MODE == TILE_PAR) return n == PI;
         if (MODE == TILE_TENDENCY && CARB != 0 && n >= 7 && MODEL == OBME_LOBSTER)
             return (CARB & 2) != 0 && n == OX && a.o2_on;
         if (MODE == TILE_TENDENCY && MODEL == OBME_NPZD && (CARB & 2) != 0 && n == OX) return false;
@@ -309,7 +308,7 @@ __device__ __forceinline__ void column_wave(const WaveArgs<FT>& w, FT* lds)
             whi[m][1] = a.wsink[(Nz + 1) + k + 1];
         }
         Lt[m] = FT(1);
-        if constexpr (MODEL == OBME_NPZD && MODE != TILE_PAR) {
+        if constexpr (MODEL == OBME_NPZD) {
             // Q10^(T/10): T is fixed
             if (fm_q10<FM>(a.f)) Lt[m] = q10_factor(a.f, U[3][m]);
         }
@@ -319,7 +318,7 @@ __device__ __forceinline__ void column_wave(const WaveArgs<FT>& w, FT* lds)
     if (a.surface_mode == OBME_SURFACE_ARRAY) PAR0col = a.surf[qc];
     // LOBSTER's O2 exchange at the top cell
     FT o2k = FT(0), o2air = FT(0);
-    if constexpr ((CARB & 2) != 0 && MODE != TILE_PAR) {
+    if constexpr ((CARB & 2) != 0) {
         if (a.o2_on && top) {
             o2k = (FT)a.o2c[2 * qc];
             o2air = (FT)a.o2c[2 * qc + 1];
@@ -454,7 +453,6 @@ __device__ __forceinline__ void column_wave(const WaveArgs<FT>& w, FT* lds)
                 PARv[m] = PAR0 * (wr[m] * m_exp(-(a.xr * h) * Ir) + wb[m] * m_exp(-(a.xb * h) * Ib));
             }
         }
-        if constexpr (MODE == TILE_PAR) return;
 
         // ---- sinking: the values above (and for WIN below) of the two tracers
         FT fx[2][L], fxu[2][L];         // the face value below each cell, and of the face above
@@ -690,12 +688,10 @@ __device__ __forceinline__ void column_wave(const WaveArgs<FT>& w, FT* lds)
     __syncthreads();
 #pragma unroll
     for (int m = 0; m < L; m++) {
-        if constexpr (MODE != TILE_PAR) {
 #pragma unroll
-            for (int n = 0; n < NT; n++)
-                if (n != RO) lds[n * TL + own + 64 * m] = U[n][m];
-        }
-        if constexpr (!STEP) lds[(MODE == TILE_PAR ? 0 : NT) * TL + own + 64 * m] = PARv[m];
+        for (int n = 0; n < NT; n++)
+            if (n != RO) lds[n * TL + own + 64 * m] = U[n][m];
+        if constexpr (!STEP) lds[NT * TL + own + 64 * m] = PARv[m];
     }
     __syncthreads();
 #pragma unroll
@@ -705,9 +701,7 @@ __device__ __forceinline__ void column_wave(const WaveArgs<FT>& w, FT* lds)
         const unsigned off = (io_base + a.sxy * (unsigned)k) * (unsigned)sizeof(FT);
         const int sl = io_slot(k);
         const bool ktop = k == Nz - 1;
-        if constexpr (MODE == TILE_PAR) {
-            gstore(a.PAR, off, lds[sl]);
-        } else if constexpr (MODE == TILE_TENDENCY) {
+        if constexpr (MODE == TILE_TENDENCY) {
             FT g0[NT];
 #pragma unroll
             for (int n = 0; n < NT; n++)
