@@ -1073,9 +1073,11 @@ static obme_status run_typed(obme_handle* h, void* const* tracers, void* const* 
         using Shape = LightShape<FT>;
         const unsigned ncol = (unsigned)(a.Nx * a.Ny);
         if (ncol <= Shape::MOST_COLUMNS) {
+            LaunchTimer tm(h, OBME_KERNEL_SWEEP, s);
             hipLaunchKernelGGL(k_light<FT>, dim3((ncol + Shape::COLS - 1) / Shape::COLS), dim3(Shape::THREADS), 0, s, a,
                                (const FT*)tracers[h->cfg.model == OBME_NPZD ? 1 : 2], ncol);
             HIP_TRY(hipGetLastError());
+            tm.done();
             return OBME_OK;
         }
     }

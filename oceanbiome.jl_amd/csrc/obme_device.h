@@ -709,38 +709,6 @@ __device__ __forceinline__ double solve_for_H(const CarbonParams& p, const obme_
     return x;
 }
 
-// FP32 first guess for [H+]: Newton on the residual in FP32 from pH 8, each
-// step limited to half the distance to the bound H = 0, at most 16 steps.
-__device__ __forceinline__ float guess_H_fp32(const CarbonParams& p)
-{
-    float K1 = (float)p.K1, K2 = (float)p.K2, KB = (float)p.KB, KW = (float)p.KW, KS = (float)p.KS,
-          KF = (float)p.KF, DIC = (float)p.DIC, Alk = (float)p.Alk, boron = (float)p.boron,
-          sulfate = (float)p.sulfate, fluoride = (float)p.fluoride;
-    float sd = 1.0f + sulfate / KS;
-    float rsd = 1.0f / sd;
-    float K12 = K1 * K2;
-    float x = 1e-8f;
-#pragma unroll 1
-    for (int it = 0; it < 16; it++) {
-        float rx = 1.0f / x;
-        float cd = x * x + K1 * x + K12;
-        float rcd = 1.0f / cd;
-        float rbd = 1.0f / (1.0f + x / KB);
-        float rhsd = 1.0f / (1.0f + KS * rx * sd);
-        float rfd = 1.0f / (1.0f + KF * rx);
-        float f = (K1 * x + 2.0f * K12) * DIC * rcd + boron * rbd + KW * rx - x * rsd - sulfate * rhsd
-                  - fluoride * rfd - Alk;
-        float df = K1 * DIC * (K12 - x * x) * rcd * rcd - (2.0f * x + K1) * 2.0f * DIC * K12 * rcd * rcd
-                   - boron * rbd * rbd / KB - KW * rx * rx - rsd - sulfate * rhsd * rhsd * KS * rx * rx * sd
-                   - fluoride * rfd * rfd * KF * rx * rx;
-        float d = f / df;
-        float lam = (d > 0.0f) ? fminf(1.0f, 0.5f * x / d) : 1.0f;
-        x = x - lam * d;
-        if (fabsf(d) <= 2e-7f * x) break;
-    }
-    return x;
-}
-
 // The residual and its derivative together for the refinement: the same
 // function as alk_residual / alk_residual_derivative, each fraction rewritten
 // over one reciprocal of its denominator (bicarbonate + carbonate =
@@ -780,6 +748,34 @@ struct AlkResidual {
         df = dacc - rsd - qs * (KSsd * rS) - qf * (KF * rF);
     }
 };
+
+// FP32 first guess for [H+]: Newton on the residual in FP32 from pH 8, each
+// step limited to half the distance to the bound H = 0, to a step of 1e-3 (the
+// next would be of order 1e-6).  first_step: the first step before the limit,
+// in units of its H (positive towards 0).
+template <bool SI = false>
+__device__ __forceinline__ float guess_H_fp32(const CarbonParams& p, float& first_step)
+{
+    const AlkResidual<SI, float> residual(p);
+    float x = 1e-8f;
+    first_step = 0.0f;
+#pragma unroll 1
+    for (int it = 0; it < 20; it++) {
+        float f, df;
+        residual(x, f, df);
+        const float d = f * m_rcp(df);
+        if (it == 0) first_step = d * 1e8f;
+        x = x - fminf(d, 0.5f * x);
+        if (fabsf(d) <= 1e-3f * x) break;
+    }
+    return x;
+}
+template <bool SI = false>
+__device__ __forceinline__ float guess_H_fp32(const CarbonParams& p)
+{
+    float first_step;
+    return guess_H_fp32<SI>(p, first_step);
+}
 
 // Refinement of a close first guess by plain FP64 Newton on the same
 // residual; returns false when it has not converged after 6 steps.  It
@@ -904,18 +900,8 @@ template <bool SI = false>
 __device__ __forceinline__ double root_H(const CarbonParams& p, const obme_carbon_solver& s, int& evals)
 {
     if (p.DIC >= 0.0 && reference_solver(s) && (!SI || p.silicate >= 0.0)) {
-        const AlkResidual<SI, float> residual(p);
-        float x = 1e-8f, step = 0.0f;
-#pragma unroll 1
-        for (int it = 0; it < 20; it++) {
-            float f, df;
-            residual(x, f, df);
-            const float d = f * m_rcp(df);
-            if (it == 0) step = d * 1e8f;
-            x = x - fminf(d, 0.5f * x);
-            if (fabsf(d) <= 1e-3f * x) break;     // the next would be of order 1e-6 x
-        }
-        double H = (double)x;
+        float step;
+        double H = (double)guess_H_fp32<SI>(p, step);
         if (step < 8.0f && refine_H<SI>(p, H, evals)) return H;
     }
     return solve_for_H<SI>(p, s, pow(10.0, -s.initial_pH_guess), evals);

@@ -403,7 +403,7 @@ k_pisces_cell(PiscesArgs<FT> a)
         // reference solve from pH 8 also ends, after many more iterations
         // (and a wave waits for its slowest lane)
         int ev = 0;
-        double H = a.have_H ? (double)a.Hs[c] : (double)guess_H_fp32(cp);
+        double H = a.have_H ? (double)a.Hs[c] : (double)guess_H_fp32<true>(cp);
         if (!refine_H<true>(cp, H, ev, sizeof(FT) == 8 ? FP64_NEWTON_TOL : FP32_NEWTON_TOL))
             H = solve_for_H<true>(cp, a.solver, pow(10.0, -a.solver.initial_pH_guess), ev);
         a.Hs[c] = (float)H;
@@ -816,7 +816,7 @@ __global__ void __launch_bounds__(PF_WAVES * 64, OBME_PISCES_PF_OCC) k_pisces_fu
                 const CarbonParams cp =
                     omega_params(o, (double)v[OBME_PI_DIC], (double)v[OBME_PI_ALK], (double)v[OBME_PI_SI]);
                 int ev = 0;
-                if (H < 0) H = (double)guess_H_fp32(cp);
+                if (H < 0) H = (double)guess_H_fp32<true>(cp);
                 if (!refine_H<true>(cp, H, ev, FP32_NEWTON_TOL)) H = solve_for_H<true>(cp, a.solver, pow(10.0, -a.solver.initial_pH_guess), ev);
                 A.Omega = (FT)omega_from_H(o, cp, H);
             }
