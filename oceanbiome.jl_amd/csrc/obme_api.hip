@@ -211,6 +211,7 @@ struct obme_handle {
     bool o2c_ready = false;    // d_o2c holds the current obme_step call's coefficients
     double* d_Hprev = nullptr; // Nx*Ny warm starts of [H+]
     float* d_topres = nullptr; // 2*Nx*Ny residuals of the top-cell DIC and Alk (mixed path, CO2 exchange)
+    bool carry_top = true;     // the current call passes them from launch to launch (one step: nothing to pass)
     double* d_surfc = nullptr; // [SURF_PACK][surfc_cols] surface constants of the current stepper call
     int surfc_cols = 0;        // Nx*Ny, or 1 when the call's T and S are the same in every column
     bool surfc_ready = false;  // d_surfc holds the constants of this call's T and S
@@ -1026,7 +1027,8 @@ static obme_status run_typed(obme_handle* h, void* const* tracers, void* const* 
         a.sflux = h->d_sflux;
     }
     // the top-cell DIC and Alk residuals (FP32 fused step, CO2 by the surface kernel)
-    float* topres = ((MODE == TILE_STEP && a.co2_on) || (MODE == TILE_STAGE && a.co2_stage)) ? h->d_topres : nullptr;
+    float* topres = ((MODE == TILE_STEP && a.co2_on && h->carry_top) || (MODE == TILE_STAGE && a.co2_stage))
+                        ? h->d_topres : nullptr;
     a.topres = topres;
     if (MODE != TILE_PAR && a.o2_on && !h->o2c_ready) {
         // the O2 exchange coefficients of this call's surface T and S (once
@@ -1131,7 +1133,7 @@ static obme_status run_wave_steps(obme_handle* h, const WaveShape& ws, void* con
     w.rk_c[1] = (float)(dt * (5.0 / 12.0 - 5.0 / 12.0));
     a.T3 = (const FT*)T;
     a.S3 = (const FT*)S;
-    a.topres = a.co2_on ? h->d_topres : nullptr;
+    a.topres = (a.co2_on && h->carry_top) ? h->d_topres : nullptr;
     w.scale = h->scaling;
     w.sed = h->sediment;
     w.scheme = h->scheme;
@@ -1272,8 +1274,9 @@ extern "C" obme_status obme_step_with_sediment(obme_handle* h, void* const* trac
         HIP_TRY(hipGetLastError());
         h->surfc_ready = true;
     }
-    if (nsteps > 0 && h->d_topres && c.model == OBME_LOBSTER && c.carbonate_system && c.co2.enabled &&
-        !h->co2_inline) {
+    h->carry_top = nsteps > 1 || h->staged;
+    if (nsteps > 0 && h->carry_top && h->d_topres && c.model == OBME_LOBSTER && c.carbonate_system &&
+        c.co2.enabled && !h->co2_inline) {
         // the top-cell DIC and Alk residuals start at zero in every call
         const size_t ncol = (size_t)c.grid.Nx * c.grid.Ny;
         hipLaunchKernelGGL(k_zero_f64, dim3((unsigned)((ncol + 255) / 256)), dim3(256), 0, s, (double*)h->d_topres,
