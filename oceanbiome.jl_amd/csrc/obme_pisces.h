@@ -5,7 +5,7 @@
 // sinking of the particle tracers.
 //
 // Kernels (one RK3 stage each):
-//   k_pisces_columns  thread per water column: MultiBand PAR from the surface
+//   k_pisces_columns  blocks of water columns: MultiBand PAR from the surface
 //                     down (multi_band.jl:147-165), euphotic depth
 //                     (compute_euphotic_depth.jl:3-33), mixed-layer mean PAR
 //                     (mean_mixed_layer_properties.jl:25-47);

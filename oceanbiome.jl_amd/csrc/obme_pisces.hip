@@ -399,7 +399,7 @@ k_pisces_cell(PiscesArgs<FT> a)
         // for a cell whose refinement fails.  FP32-mixed stops after a step
         // below 1e-4 relative: quadratic convergence leaves H within ~1e-8 of
         // the root, below the FP32 rounding of Ω.  FP64 stops after a step
-        // below 1e-14 relative: H at the root to rounding, where the
+        // below 3e-9 relative: H at the root to rounding, where the
         // reference solve from pH 8 also ends, after many more iterations
         // (and a wave waits for its slowest lane)
         int ev = 0;
