@@ -579,7 +579,7 @@ struct PiscesFused {
 };
 
 // The fused FP32-mixed PISCES step: one wave per water column, lane r
-// holding level k = Nz - 1 - r (r = 0 at the top; Nz <= 64, lanes r >= Nz
+// holding level k = Nz - 1 - r (r = 0 at the top; Nz <= 64 W, lanes r >= Nz
 // idle), the three RK3 stages in registers, one read and one write of each
 // tracer per step, in place.  Per stage, as the per-stage kernels do:
 // the scaling modifier (SCALE); the MultiBand PAR as an inclusive prefix
@@ -592,6 +592,10 @@ struct PiscesFused {
 // 24 transitions; the upwind sinking with the value of the level above
 // from the neighbouring lane; the substep.  The workgroup's PF_WAVES
 // columns are neighbours along i, in the XCD-aware tile order.
+// W = 2: columns of 65 to 128 levels on two waves, the lower's level above and
+// the column's sums through LDS, two barriers a stage (100x80x90, three steps:
+// the per-stage kernels 985 us, this 587; one step 332 | 292, on 66 levels
+// 266 | 268).
 #ifndef OBME_PISCES_PF_WAVES
 #define OBME_PISCES_PF_WAVES 4
 #endif
@@ -603,19 +607,31 @@ constexpr int PF_WAVES = OBME_PISCES_PF_WAVES;
 #define OBME_PISCES_PF_OCC 3
 #endif
 
-template <bool SCALE>
-__global__ void __launch_bounds__(PF_WAVES * 64, OBME_PISCES_PF_OCC) k_pisces_fused(PiscesArgs<float> a, PiscesFused f)
+// what a wave of a column of two leaves for the other, in a stage
+struct PiscesHalf {
+    float total[3], above[6];       // the light's sums, the sinking tracers of its last level
+    float mixed;                    // its part of the mixed layer's light
+    float zk, lk, zu, lu;           // where its light first falls below the threshold
+    float zlast, llast;             // its last level
+    int found, first;               // it does; in its first lane
+};
+
+template <bool SCALE, int W>
+__global__ void __launch_bounds__(PF_WAVES * 64, W == 1 ? OBME_PISCES_PF_OCC : 2) k_pisces_fused(PiscesArgs<float> a, PiscesFused f)
 {
     using FT = float;
-    const int r = threadIdx.x & 63;
+    constexpr int COLS = PF_WAVES / W;      // columns of the workgroup
     // the wave's column, as a scalar: the values derived from it (the column
     // index, its surface PAR and gas constants) stay out of the vector registers
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const unsigned nbx = ((unsigned)a.Nx + PF_WAVES - 1) / PF_WAVES;
+    const int half = W == 1 ? 0 : wv % W;
+    const int lane = threadIdx.x & 63;
+    const int r = half * 64 + lane;         // levels from the top
+    const unsigned nbx = ((unsigned)a.Nx + COLS - 1) / COLS;
     const unsigned tile = xcd_tile(blockIdx.x, gridDim.x);
     const int j = (int)(tile / nbx);
-    const int ib = (int)(tile % nbx) * PF_WAVES;
-    const int i = ib + wv;
+    const int ib = (int)(tile % nbx) * COLS;
+    const int i = ib + wv / W;
     // a wave past the last column computes on zeros and stores nothing
     // (it stays for the workgroup barriers)
     const bool colok = i < a.Nx;
@@ -638,13 +654,15 @@ __global__ void __launch_bounds__(PF_WAVES * 64, OBME_PISCES_PF_OCC) k_pisces_fu
     __shared__ double s_surf[PF_WAVES][SURF_PACK];   // the top lane's surface constants
     __shared__ double s_hsurf[PF_WAVES];             // and its [H+] warm start (not held in registers)
     __shared__ float s_tf[TFAC_FIELDS][PF_WAVES * 64];   // the lane's temperature factors (T is fixed)
+    // (by the stage's parity: a wave may be a stage ahead of the other's last reads)
+    __shared__ PiscesHalf s_half[W == 1 ? 1 : 2][W == 1 ? 1 : PF_WAVES];
 
-    // stage in: thread t takes level kt = t / PF_WAVES of column ct = t %
-    // PF_WAVES (PF_WAVES neighbouring values along i per level: coalesced)
+    // stage in: thread t takes level kt = t / COLS of column ct = t %
+    // COLS (COLS neighbouring values along i per level: coalesced)
     // and puts it into the LDS slot of the lane that owns that cell
-    const int kt = tid / PF_WAVES, ct = tid % PF_WAVES;
+    const int kt = tid / COLS, ct = tid % COLS;
     const bool tok = kt < Nz && ib + ct < a.Nx;
-    const int slot = ct * 64 + (Nz - 1 - (kt < Nz ? kt : 0));
+    const int slot = ct * (64 * W) + (Nz - 1 - (kt < Nz ? kt : 0));
     const unsigned pt = pidx(a, tok ? ib + ct : 0, j, tok ? kt : 0);
     // (32-bit: a field holds fewer than 2^31 cells, checked at create)
     const unsigned ct_cell = (unsigned)(tok ? ib + ct : 0) + (unsigned)a.Nx * (unsigned)j +
@@ -705,7 +723,14 @@ __global__ void __launch_bounds__(PF_WAVES * 64, OBME_PISCES_PF_OCC) k_pisces_fu
         const FT dzk1 = (zk1 > zmxl) ? zk1 - zmxl : FT(0);
         wml = act ? ((zk >= zmxl) ? dzk : dzk1) : FT(0);
     }
-    const FT depth = __builtin_bit_cast(FT, __builtin_amdgcn_readlane(__builtin_bit_cast(int, seg_prefix<64>(wml)), 63));
+    FT depth = __builtin_bit_cast(FT, __builtin_amdgcn_readlane(__builtin_bit_cast(int, seg_prefix<64>(wml)), 63));
+    if constexpr (W == 2) {
+        if (lane == 0) s_half[0][wv].mixed = depth;
+        __syncthreads();
+        depth = s_half[0][wv & ~1].mixed + s_half[0][wv | 1].mixed;
+        __syncthreads();
+    }
+    int parity = 0;
     // the column's surface PAR: a 2-D array, or per stage from the host
     const FT PAR0col = a.surf ? a.surf[col] : FT(0);
     FT zeu_none;
@@ -763,12 +788,32 @@ __global__ void __launch_bounds__(PF_WAVES * 64, OBME_PISCES_PF_OCC) k_pisces_fu
             const FT Chl = v[OBME_PI_PCHL] + v[OBME_PI_DCHL];
             const FT lChl = m_log2(Chl);   // Chl^e = 2^(e log2 Chl), one logarithm for the three bands
             FT band[3];
+            FT S[3];
 #pragma unroll
             for (int n = 0; n < 3; n++) {
                 const FT att = a.kw[n] + a.chi[n] * m_exp2(a.e[n] * lChl);
-                const FT S = seg_prefix<64>(act ? dzl * att : FT(0));
-                band[n] = (PAR0 * f.div[n]) * m_exp(S);
+                S[n] = seg_prefix<64>(act ? dzl * att : FT(0));
             }
+            if constexpr (W == 2) {
+                parity ^= 1;
+                if (half == 0 && lane == 63) {
+                    PiscesHalf& h = s_half[parity][wv];
+#pragma unroll
+                    for (int n = 0; n < 3; n++) h.total[n] = S[n];
+                    h.above[0] = v[OBME_PI_POC];
+                    h.above[1] = v[OBME_PI_SFE];
+                    h.above[2] = v[OBME_PI_GOC];
+                    h.above[3] = v[OBME_PI_BFE];
+                    h.above[4] = v[OBME_PI_PSI];
+                    h.above[5] = v[OBME_PI_CACO3];
+                }
+                __syncthreads();
+                if (half == 1)
+#pragma unroll
+                    for (int n = 0; n < 3; n++) S[n] += s_half[parity][wv - 1].total[n];
+            }
+#pragma unroll
+            for (int n = 0; n < 3; n++) band[n] = (PAR0 * f.div[n]) * m_exp(S[n]);
             const FT PAR = band[0] + band[1] + band[2];
 
             // euphotic depth: the first level below the top cell, from the top,
@@ -776,18 +821,47 @@ __global__ void __launch_bounds__(PF_WAVES * 64, OBME_PISCES_PF_OCC) k_pisces_fu
             const FT lPAR = m_log(PAR);
             const unsigned long long cand = __ballot(act && r >= 1 && PAR <= thr);
             FT zeu = zeu_none;
-            if (cand) {
-                const int rs = __ffsll((long long)cand) - 1;
-                const FT zk = __builtin_bit_cast(FT, __builtin_amdgcn_readlane(__builtin_bit_cast(int, zc), rs));
-                const FT zu = __builtin_bit_cast(FT, __builtin_amdgcn_readlane(__builtin_bit_cast(int, zc), rs - 1));
-                const FT lk = __builtin_bit_cast(FT, __builtin_amdgcn_readlane(__builtin_bit_cast(int, lPAR), rs));
-                const FT lu = __builtin_bit_cast(FT, __builtin_amdgcn_readlane(__builtin_bit_cast(int, lPAR), rs - 1));
+            bool found = cand != 0;
+            FT zk = FT(0), zu = FT(0), lk = FT(0), lu = FT(0);
+            const int rs = found ? __ffsll((long long)cand) - 1 : 1, ra = rs > 0 ? rs - 1 : 0;
+            if (found) {
+                zk = __builtin_bit_cast(FT, __builtin_amdgcn_readlane(__builtin_bit_cast(int, zc), rs));
+                zu = __builtin_bit_cast(FT, __builtin_amdgcn_readlane(__builtin_bit_cast(int, zc), ra));
+                lk = __builtin_bit_cast(FT, __builtin_amdgcn_readlane(__builtin_bit_cast(int, lPAR), rs));
+                lu = __builtin_bit_cast(FT, __builtin_amdgcn_readlane(__builtin_bit_cast(int, lPAR), ra));
+            }
+            // mixed-layer mean of the total PAR
+            FT acc =
+                __builtin_bit_cast(FT, __builtin_amdgcn_readlane(__builtin_bit_cast(int, seg_prefix<64>(PAR * wml)), 63));
+            if constexpr (W == 2) {
+                if (lane == 63) {
+                    PiscesHalf& h = s_half[parity][wv];
+                    h.mixed = acc;
+                    h.found = found ? 1 : 0;
+                    h.first = rs == 0 ? 1 : 0;
+                    h.zk = zk;
+                    h.lk = lk;
+                    h.zu = zu;
+                    h.lu = lu;
+                    h.zlast = zc;
+                    h.llast = lPAR;
+                }
+                __syncthreads();
+                const PiscesHalf &up = s_half[parity][wv & ~1], &low = s_half[parity][wv | 1];
+                acc = up.mixed + low.mixed;
+                const PiscesHalf& at = up.found ? up : low;
+                found = up.found || low.found;
+                zk = at.zk;
+                lk = at.lk;
+                // (the lower wave's first level lies below the upper's last)
+                const bool across = !up.found && low.first;
+                zu = across ? up.zlast : at.zu;
+                lu = across ? up.llast : at.lu;
+            }
+            if (found) {
                 zeu = zk + (lthr - lk) * (zk - zu) / (lk - lu);
                 if (!(zeu > FT(-INFINITY) && zeu < FT(INFINITY))) zeu = zeu_none;
             }
-            // mixed-layer mean of the total PAR
-            const FT acc =
-                __builtin_bit_cast(FT, __builtin_amdgcn_readlane(__builtin_bit_cast(int, seg_prefix<64>(PAR * wml)), 63));
 
             Aux<FT> A;
             A.z = zc;
@@ -836,16 +910,19 @@ __global__ void __launch_bounds__(PF_WAVES * 64, OBME_PISCES_PF_OCC) k_pisces_fu
             pisces_tendencies<true>(pps, v, A, f.sk[sn][st], tf, G);
             // flux-form upwind sinking: (w(k+1) c(k+1) - w(k) c(k)) / dz, the
             // level above from lane r - 1, w = 0 on the top face
-            auto sink = [&](int n, FT wlo, FT whi) {
-                const FT cu = lane_shr1(v[n]);
+            auto sink = [&](int n, int m, FT wlo, FT whi) {
+                FT cu = lane_shr1(v[n]);
+                if constexpr (W == 2) {
+                    if (half == 1 && lane == 0) cu = s_half[parity][wv - 1].above[m];
+                }
                 G[n] = G[n] - (whi * cu - wlo * v[n]) * idz;
             };
-            sink(OBME_PI_POC, wPlo, wPhi);
-            sink(OBME_PI_SFE, wPlo, wPhi);
-            sink(OBME_PI_GOC, wGlo, wGhi);
-            sink(OBME_PI_BFE, wGlo, wGhi);
-            sink(OBME_PI_PSI, wGlo, wGhi);
-            sink(OBME_PI_CACO3, wGlo, wGhi);
+            sink(OBME_PI_POC, 0, wPlo, wPhi);
+            sink(OBME_PI_SFE, 1, wPlo, wPhi);
+            sink(OBME_PI_GOC, 2, wGlo, wGhi);
+            sink(OBME_PI_BFE, 3, wGlo, wGhi);
+            sink(OBME_PI_PSI, 4, wGlo, wGhi);
+            sink(OBME_PI_CACO3, 5, wGlo, wGhi);
             if (top) {
                 G[OBME_PI_DIC] = G[OBME_PI_DIC] - (FT)Fc * idz;
                 G[OBME_PI_O2] = G[OBME_PI_O2] - (FT)Fo * idz;
@@ -874,9 +951,9 @@ __global__ void __launch_bounds__(PF_WAVES * 64, OBME_PISCES_PF_OCC) k_pisces_fu
         // the stage loop
         int t2 = tid;
         asm volatile("" : "+v"(t2));
-        const int kt2 = t2 / PF_WAVES, ct2 = t2 % PF_WAVES;
+        const int kt2 = t2 / COLS, ct2 = t2 % COLS;
         if (kt2 < Nz && ib + ct2 < a.Nx) {
-            const int slot2 = ct2 * 64 + (Nz - 1 - kt2);
+            const int slot2 = ct2 * (64 * W) + (Nz - 1 - kt2);
             const unsigned pt2 = pidx(a, ib + ct2, j, kt2);
 #pragma unroll
             for (int n = 0; n < NW; n++) a.out[n][pt2] = s_gm[n][slot2];
@@ -912,7 +989,7 @@ struct obme_pisces {
     std::vector<double> zc, zf, dz;
     std::vector<double> w_host;   // [2][Nz+1]: the POC and GOC face velocities (FP64)
     bool scaling = false;
-    bool fused = false;        // FP32-mixed with Nz <= 64: k_pisces_fused (OBME_PISCES_FUSED=0 turns it off)
+    bool fused = false;        // FP32-mixed with Nz <= 128: k_pisces_fused (OBME_PISCES_FUSED=0 turns it off)
     int fused_steps = PF_MAX_STEPS;   // steps per fused launch (OBME_PISCES_FUSED_STEPS sets 1 .. 16)
     // an InstantRemineralisation sediment under every column (cfg.sediment)
     bool sediment = false;
@@ -1054,9 +1131,9 @@ extern "C" obme_status obme_pisces_create(const obme_pisces_config* cfg, obme_pi
     h->cfg.grid.zc = h->cfg.grid.zf = h->cfg.grid.dz = nullptr;
     h->scaling = cfg->scaling.n_groups > 0;
     h->sediment = cfg->sediment.model == OBME_SEDIMENT_INSTANT_REMINERALISATION;
-    // the fused step: FP32-mixed, one wave per column of at most 64 levels
-    // (with a sediment, the per-stage kernels)
-    h->fused = h->prec == OBME_FP32_MIXED && g.Nz <= 64 && !h->sediment;
+    // the fused step: FP32-mixed, one wave per column of at most 64 levels, two
+    // of at most 128 (with a sediment, the per-stage kernels)
+    h->fused = h->prec == OBME_FP32_MIXED && g.Nz <= 128 && !h->sediment;
     if (const char* e = std::getenv("OBME_PISCES_FUSED")) h->fused = h->fused && std::atoi(e) != 0;
     if (const char* e = std::getenv("OBME_PISCES_FUSED_STEPS")) {
         const int n = std::atoi(e);
@@ -1381,7 +1458,8 @@ static obme_status pisces_fused_steps(obme_pisces* h, void* const* tracers, int 
         OBME_HIP_TRY(hipGetLastError());
         f.surf = (const double*)h->d_surfc;
     }
-    const unsigned nbx = (unsigned)((h->cfg.grid.Nx + PF_WAVES - 1) / PF_WAVES);
+    const int W = h->cfg.grid.Nz <= 64 ? 1 : 2, cols = PF_WAVES / W;
+    const unsigned nbx = (unsigned)((h->cfg.grid.Nx + cols - 1) / cols);
     const unsigned nb = nbx * (unsigned)h->cfg.grid.Ny;
     for (int s0 = 0; s0 < nsteps; s0 += h->fused_steps) {
         f.nsteps = std::min(h->fused_steps, nsteps - s0);
@@ -1394,10 +1472,9 @@ static obme_status pisces_fused_steps(obme_pisces* h, void* const* tracers, int 
             }
         }
         f.have_H = s0 > 0 ? 1 : 0;
-        if (h->scaling)
-            hipLaunchKernelGGL(k_pisces_fused<true>, dim3(nb), dim3(PF_WAVES * 64), 0, s, a, f);
-        else
-            hipLaunchKernelGGL(k_pisces_fused<false>, dim3(nb), dim3(PF_WAVES * 64), 0, s, a, f);
+        auto k = W == 1 ? (h->scaling ? k_pisces_fused<true, 1> : k_pisces_fused<false, 1>)
+                        : (h->scaling ? k_pisces_fused<true, 2> : k_pisces_fused<false, 2>);
+        hipLaunchKernelGGL(k, dim3(nb), dim3(PF_WAVES * 64), 0, s, a, f);
         OBME_HIP_TRY(hipGetLastError());
     }
     return OBME_OK;
