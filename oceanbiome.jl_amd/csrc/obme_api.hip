@@ -1637,10 +1637,10 @@ extern "C" obme_status obme_kernel_timing(obme_handle* h, int32_t which, double*
 
 // ------------------------------------------------------------------ batched ensemble
 
-template <int L, int CPW, int NW>
+template <int L, int CPW, int NW, int FM>
 __global__ void __launch_bounds__(NW * 64, L == 2 ? 5 : 1) k_batch(BatchArgs<float> a)
 {
-    batch_columns<float, L, CPW, NW, true>(a);
+    batch_columns<L, CPW, NW, FM>(a);
 }
 constexpr int RAGGED_WAVES = 4;   // waves per workgroup
 template <typename FT, int L, int FM, bool SED>
@@ -1846,17 +1846,18 @@ static obme_status batch_launch_class(const obme_batch* b, int q, BatchArgs<floa
     const BatchTile& t = BATCH_TILES[b->class_tile[q]];
     const int per_wg = t.NW * t.CPW;
     dim3 grid((a.ncols + per_wg - 1) / per_wg), block(t.NW * 64);
-    using Kernel = void (*)(BatchArgs<float>);
-    Kernel k = nullptr;
+    constexpr int FM = default_fm<OBME_NPZD>();
+    const bool d = b->default_forms;
+    void (*k)(BatchArgs<float>) = nullptr;
     switch (b->class_tile[q]) {
-    case 0: k = k_batch<1, 4, 4>; break;
-    case 1: k = k_batch<2, 4, 4>; break;
-    case 2: k = k_batch<1, 2, 4>; break;
-    case 3: k = k_batch<2, 2, 4>; break;
-    case 4: k = k_batch<1, 1, 4>; break;
-    case 5: k = k_batch<2, 1, 4>; break;
-    case 6: k = k_batch<4, 2, 4>; break;
-    case 7: k = k_batch<4, 4, 4>; break;
+    case 0: k = d ? k_batch<1, 4, 4, FM> : k_batch<1, 4, 4, -1>; break;
+    case 1: k = d ? k_batch<2, 4, 4, FM> : k_batch<2, 4, 4, -1>; break;
+    case 2: k = d ? k_batch<1, 2, 4, FM> : k_batch<1, 2, 4, -1>; break;
+    case 3: k = d ? k_batch<2, 2, 4, FM> : k_batch<2, 2, 4, -1>; break;
+    case 4: k = d ? k_batch<1, 1, 4, FM> : k_batch<1, 1, 4, -1>; break;
+    case 5: k = d ? k_batch<2, 1, 4, FM> : k_batch<2, 1, 4, -1>; break;
+    case 6: k = d ? k_batch<4, 2, 4, FM> : k_batch<4, 2, 4, -1>; break;
+    case 7: k = d ? k_batch<4, 4, 4, FM> : k_batch<4, 4, 4, -1>; break;
     default: return fail(OBME_ERR_INVALID, "bad batch tile");
     }
     hipLaunchKernelGGL(k, grid, block, 0, s, a);
@@ -1932,7 +1933,6 @@ static obme_status batch_enqueue(const obme_batch* b, void* const* tracers, int 
         for (int n = 0; n < 4; n++) a.C[n] = (FT*)(b->d_comp + n * ncell);
     if (b->sediment) {
         const obme_sediment& sd = b->cfg.sediment;
-        a.sed_on = 1;
         a.storage = sc.storage;
         a.sedGm = sc.Gm;
         a.sed_recv = b->sed_recv;

@@ -59,14 +59,13 @@ struct BatchArgs {
     // TwoBand coefficients: FP64 reference form and FP32 log2-scaled form
     double kr, kb, xr, xb, er, eb, Rr;
     float kr2, kb2, er_f, eb_f, cr, cb, xr2h, xb2h;
-    // InstantRemineralisation sediment under every column (sed_on; storage
+    // InstantRemineralisation sediment under every column (storage
     // null: the coupling alone, the storage not advanced).  The flux through
     // the bottom face f = sedP (-wP) P + sedD (-wD) D
     // of the bottom cell, burial e = a + b (f / (k + f))^2, the receiver's
     // coupled tendency (1 - e) f / dz; after each stage's substep the storage
     // steps by the stage Δt with the tendency e f of the stage's start
     // (update_state.jl:6-17; instant_remineralisation.jl:101-123).
-    int sed_on;
     double* storage;                // [n_columns] or null
     double* sedGm;                  // [n_columns] G⁻: the tendency of the sediment's last step
     int sed_init;                   // the sediment's first step ever is this launch's first step
@@ -78,14 +77,16 @@ struct BatchArgs {
     FT sedP, sedD;                  // 1 where P / D is one of the sinking tracers, else 0
 };
 
-// One persistent workgroup loops over tiles of NW*CPW columns.  SED: the
-// sediment's code compiled in (the ensemble without one keeps its registers).
-template <typename FT, int L, int CPW, int NW, bool SED>
-__device__ __forceinline__ void batch_columns(const BatchArgs<FT>& a)
+// FP32 with a sediment: one persistent workgroup loops over tiles of NW*CPW
+// columns.  FM: the default formulations compiled in, or < 0 (fm_light): they
+// are read per lane, and each choice is a branch over the lanes (8192 columns
+// of 16 to 128 levels, 50 steps: 478 us so, 463 compiled in; 307 of 34 to 79,
+// 20 steps: 97.7 and 92.8), with the same roundings.
+template <int L, int CPW, int NW, int FM>
+__device__ __forceinline__ void batch_columns(const BatchArgs<float>& a)
 {
     constexpr int LPC = 64 / CPW;
     static_assert(LPC == 16 || LPC == 32 || LPC == 64, "segments of 16, 32 or 64 lanes");
-    constexpr bool F32 = sizeof(FT) == 4;
     const int lane = threadIdx.x & 63;
     const int w = threadIdx.x >> 6;
     const int r = lane % LPC;
@@ -102,37 +103,30 @@ __device__ __forceinline__ void batch_columns(const BatchArgs<FT>& a)
         auto has = [&](int m) -> bool { return r * L + m < Nzc; };
         auto idx = [&](int m) -> int { return off + Nzc - 1 - (r * L + m); };
 
-        FT U[4][L], D[F32 ? 4 : 1][L], Gm[4][L];
+        float U[4][L], D[4][L], Gm[4][L];
 #pragma unroll
         for (int n = 0; n < 4; n++)
 #pragma unroll
             for (int m = 0; m < L; m++) {
-                U[n][m] = has(m) ? a.U[n][idx(m)] : FT(0);
-                Gm[n][m] = FT(0);
-                if constexpr (F32) D[n][m] = (a.c_in && has(m)) ? a.C[n][idx(m)] : FT(0);
+                U[n][m] = has(m) ? a.U[n][idx(m)] : 0.0f;
+                Gm[n][m] = 0.0f;
+                D[n][m] = (a.c_in && has(m)) ? a.C[n][idx(m)] : 0.0f;
             }
-        auto val = [&](int n, int m) -> FT {
-            if constexpr (F32) return U[n][m] + D[n][m];
-            else return U[n][m];
-        };
+        auto val = [&](int n, int m) -> float { return U[n][m] + D[n][m]; };
 
         // column constants (every lane of a segment reads the same entry)
         const int cc = (col >= 0) ? col : 0;
         const BatchColumn bc = a.bcol[cc];
-        const FT PAR0 = (FT)bc.PAR0;
-        const FT Lt = (FT)bc.Lt;
-        const FT wP = (FT)bc.wP, wD = (FT)bc.wD;
-        constexpr bool FIXED = F32 && SED;
-        using Params = std::conditional_t<FIXED, SedimentParams, FastParams<FT>>;
-        Params fp;
-        if constexpr (FIXED) fp = a.fsed[cc];
-        else fp = a.fpar[cc];
+        const float PAR0 = (float)bc.PAR0;
+        const float Lt = (float)bc.Lt;
+        const float wP = (float)bc.wP, wD = (float)bc.wD;
+        const SedimentParams fp = a.fsed[cc];
         const float wiP = (float)(bc.wP / (double)a.dz), wiD = (float)(bc.wD / (double)a.dz);
 
         // the sediment of this column, held by the lane of its bottom cell
         // (j = Nzc - 1: lane rb, level mb)
         const int jb = Nzc - 1;
-        const bool sed = SED && a.sed_on && col >= 0 && r == jb / L;
+        const bool sed = col >= 0 && r == jb / L;
         const int mb = jb % L;
         // the storage and the last tendency in LDS, one slot per segment
         // (not held in registers through the launch)
@@ -144,99 +138,73 @@ __device__ __forceinline__ void batch_columns(const BatchArgs<FT>& a)
 
         // water terms of the own levels
         float ezr[L], ezb[L];
-        FT zc[L];
 #pragma unroll
         for (int m = 0; m < L; m++) {
-            zc[m] = -(FT(r * L + m) + FT(0.5)) * a.dz;
-            if constexpr (F32) {
-                ezr[m] = a.kr2 * zc[m];
-                ezb[m] = a.kb2 * zc[m];
-            }
+            const float zc = -((float)(r * L + m) + 0.5f) * a.dz;
+            ezr[m] = a.kr2 * zc;
+            ezb[m] = a.kb2 * zc;
         }
-        const double g1 = 8.0 / 15.0, g2 = 5.0 / 12.0, g3 = 3.0 / 4.0, z2 = -17.0 / 60.0, z3 = -5.0 / 12.0;
 
 #pragma unroll 1
         for (int s = 0; s < a.nsteps; s++) {
 #pragma unroll 1
             for (int st = 0; st < 3; st++) {
                 // chlorophyll terms and the light integral (as in the sweep)
-                FT pr[L], pb[L];
+                float pr[L], pb[L];
 #pragma unroll
                 for (int m = 0; m < L; m++) {
-                    if constexpr (F32) {
-                        const float lg = m_log2(val(1, m));
-                        pr[m] = m_exp2(fmaf(a.er_f, lg, a.cr));
-                        pb[m] = m_exp2(fmaf(a.eb_f, lg, a.cb));
-                    } else {
-                        const double x = val(1, m) * a.Rr;
-                        pow_pair(x, a.er, a.eb, pr[m], pb[m]);
-                    }
+                    const float lg = m_log2(val(1, m));
+                    pr[m] = m_exp2(fmaf(a.er_f, lg, a.cr));
+                    pb[m] = m_exp2(fmaf(a.eb_f, lg, a.cb));
                 }
-                const FT pr_up = lane_shr1(pr[L - 1]);
-                const FT pb_up = lane_shr1(pb[L - 1]);
-                const FT cP_up = lane_shr1(val(1, L - 1));
-                const FT cD_up = lane_shr1(val(3, L - 1));
-                FT incr[L], incb[L];
-                FT totr = FT(0), totb = FT(0);
+                const float pr_up = lane_shr1(pr[L - 1]);
+                const float pb_up = lane_shr1(pb[L - 1]);
+                const float cP_up = lane_shr1(val(1, L - 1));
+                const float cD_up = lane_shr1(val(3, L - 1));
+                float incr[L], incb[L];
+                float totr = 0.0f, totb = 0.0f;
 #pragma unroll
                 for (int m = 0; m < L; m++) {
                     const bool top = (m == 0) && (r == 0);
-                    const FT prn = (m == 0) ? pr_up : pr[m > 0 ? m - 1 : 0];
-                    const FT pbn = (m == 0) ? pb_up : pb[m > 0 ? m - 1 : 0];
-                    FT ir, ib;
-                    if constexpr (F32) {
-                        ir = top ? pr[m] : prn + pr[m];
-                        ib = top ? pb[m] : pbn + pb[m];
-                    } else {
-                        const double h = a.dz / 2;
-                        ir = top ? h * pr[m] : h * prn + h * pr[m];
-                        ib = top ? h * pb[m] : h * pbn + h * pb[m];
-                    }
-                    incr[m] = has(m) ? ir : FT(0);
-                    incb[m] = has(m) ? ib : FT(0);
+                    const float prn = (m == 0) ? pr_up : pr[m > 0 ? m - 1 : 0];
+                    const float pbn = (m == 0) ? pb_up : pb[m > 0 ? m - 1 : 0];
+                    const float ir = top ? pr[m] : prn + pr[m];
+                    const float ib = top ? pb[m] : pbn + pb[m];
+                    incr[m] = has(m) ? ir : 0.0f;
+                    incb[m] = has(m) ? ib : 0.0f;
                     totr = totr + incr[m];
                     totb = totb + incb[m];
                 }
-                FT runr = lane_shr1(seg_prefix<LPC>(totr));
-                FT runb = lane_shr1(seg_prefix<LPC>(totb));
+                float runr = lane_shr1(seg_prefix<LPC>(totr));
+                float runb = lane_shr1(seg_prefix<LPC>(totb));
                 if (r == 0) {
-                    runr = FT(0);
-                    runb = FT(0);
+                    runr = 0.0f;
+                    runb = 0.0f;
                 }
-                FT PARv[L];
+                float PARv[L];
 #pragma unroll
                 for (int m = 0; m < L; m++) {
                     runr = runr + incr[m];
                     runb = runb + incb[m];
-                    if constexpr (F32)
-                        PARv[m] = (PAR0 * 0.5f) * (m_exp2(fmaf(-a.xr2h, runr, ezr[m])) +
-                                                   m_exp2(fmaf(-a.xb2h, runb, ezb[m])));
-                    else
-                        PARv[m] = PAR0 * (m_exp(a.kr * zc[m] - a.xr * runr) + m_exp(a.kb * zc[m] - a.xb * runb)) / 2;
+                    PARv[m] = (PAR0 * 0.5f) * (m_exp2(fmaf(-a.xr2h, runr, ezr[m])) +
+                                               m_exp2(fmaf(-a.xb2h, runb, ezb[m])));
                 }
                 // the sediment: the bottom cell's flux and burial, the
                 // receiver's coupled tendency, the sediment step
-                FT cpl = FT(0);
+                float cpl = 0.0f;
                 if (sed) {
-                    FT Pb = val(1, 0), Db = val(3, 0);
+                    float Pb = val(1, 0), Db = val(3, 0);
 #pragma unroll
                     for (int m = 1; m < L; m++)
                         if (m == mb) {
                             Pb = val(1, m);
                             Db = val(3, m);
                         }
-                    const FT f = a.sedP * (-wP) * Pb + a.sedD * (-wD) * Db;
-                    FT qf, e;
-                    if constexpr (F32) {
-                        // FP32-mixed: the hardware reciprocal (1 ulp) and 1/Δz
-                        qf = f * __builtin_amdgcn_rcpf(a.sed_k + f);
-                        e = a.sed_a + a.sed_b * (qf * qf);
-                        cpl = ((FT(1) - e) * f) * a.invdz;
-                    } else {
-                        qf = f / (a.sed_k + f);
-                        e = a.sed_a + a.sed_b * (qf * qf);
-                        cpl = ((FT(1) - e) * f) / a.dz;
-                    }
+                    const float f = a.sedP * (-wP) * Pb + a.sedD * (-wD) * Db;
+                    // the hardware reciprocal (1 ulp) and 1/Δz
+                    const float qf = f * __builtin_amdgcn_rcpf(a.sed_k + f);
+                    const float e = a.sed_a + a.sed_b * (qf * qf);
+                    cpl = ((1.0f - e) * f) * a.invdz;
                     const double ge = (double)(e * f);
                     const bool init = a.sed_init && s == 0;
                     if (st == 0) {
@@ -254,20 +222,13 @@ __device__ __forceinline__ void batch_columns(const BatchArgs<FT>& a)
 #pragma unroll
                 for (int m = L - 1; m >= 0; m--) {
                     const bool top = (m == 0) && (r == 0);
-                    const FT N = val(0, m), P = val(1, m), Z = val(2, m), Dd = val(3, m);
-                    FT G[4];
-                    if constexpr (FIXED) npzd_sediment(fp, N, P, Z, Dd, PARv[m], Lt, G[0], G[1], G[2], G[3]);
-                    else npzd_fast(fp, N, P, Z, Dd, PARv[m], Lt, G[0], G[1], G[2], G[3]);
-                    const FT cPn = (m == 0) ? cP_up : val(1, m > 0 ? m - 1 : 0);
-                    const FT cDn = (m == 0) ? cD_up : val(3, m > 0 ? m - 1 : 0);
-                    if constexpr (F32) {
-                        G[1] = fmaf(-wiP, (top ? 0.0f : cPn) - P, G[1]);
-                        G[3] = fmaf(-wiD, (top ? 0.0f : cDn) - Dd, G[3]);
-                    } else {
-                        const double FhiP = top ? 0.0 : wP * cPn, FhiD = top ? 0.0 : wD * cDn;
-                        G[1] = G[1] - (FhiP - wP * P) * a.invdz;
-                        G[3] = G[3] - (FhiD - wD * Dd) * a.invdz;
-                    }
+                    const float N = val(0, m), P = val(1, m), Z = val(2, m), Dd = val(3, m);
+                    float G[4];
+                    npzd_sediment<FM>(fp, N, P, Z, Dd, PARv[m], Lt, G[0], G[1], G[2], G[3]);
+                    const float cPn = (m == 0) ? cP_up : val(1, m > 0 ? m - 1 : 0);
+                    const float cDn = (m == 0) ? cD_up : val(3, m > 0 ? m - 1 : 0);
+                    G[1] = fmaf(-wiP, (top ? 0.0f : cPn) - P, G[1]);
+                    G[3] = fmaf(-wiD, (top ? 0.0f : cDn) - Dd, G[3]);
                     if (sed && m == mb) {
 #pragma unroll
                         for (int n = 0; n < 4; n++)
@@ -275,32 +236,24 @@ __device__ __forceinline__ void batch_columns(const BatchArgs<FT>& a)
                     }
 #pragma unroll
                     for (int n = 0; n < 4; n++) {
-                        if constexpr (F32) {
-                            const float A = (st == 0) ? a.rk_a[0] : (st == 1 ? a.rk_a[1] : a.rk_a[2]);
-                            const float B = (st == 0) ? a.rk_b[0] : (st == 1 ? a.rk_b[1] : a.rk_b[2]);
-                            D[n][m] = fmaf(A, G[n], fmaf(B, Gm[n][m], D[n][m]));
-                        } else {
-                            const double gs = (st == 1) ? g2 : g3;
-                            const double zs = (st == 1) ? z2 : z3;
-                            U[n][m] += (st == 0) ? (a.dtf * g1) * G[n] : a.dtf * (gs * G[n] + zs * Gm[n][m]);
-                        }
+                        const float A = (st == 0) ? a.rk_a[0] : (st == 1 ? a.rk_a[1] : a.rk_a[2]);
+                        const float B = (st == 0) ? a.rk_b[0] : (st == 1 ? a.rk_b[1] : a.rk_b[2]);
+                        D[n][m] = fmaf(A, G[n], fmaf(B, Gm[n][m], D[n][m]));
                         Gm[n][m] = G[n];
                     }
                 }
             }
-            if constexpr (F32) {
-                // U + D = s + e exactly (TwoSum): U = s, and e carries on
+            // U + D = s + e exactly (TwoSum): U = s, and e carries on
 #pragma unroll
-                for (int n = 0; n < 4; n++)
+            for (int n = 0; n < 4; n++)
 #pragma unroll
-                    for (int m = 0; m < L; m++) {
-                        const float u = U[n][m], d = D[n][m];
-                        const float sum = u + d;
-                        const float dv = sum - u;
-                        D[n][m] = (u - (sum - dv)) + (d - dv);
-                        U[n][m] = sum;
-                    }
-            }
+                for (int m = 0; m < L; m++) {
+                    const float u = U[n][m], d = D[n][m];
+                    const float sum = u + d;
+                    const float dv = sum - u;
+                    D[n][m] = (u - (sum - dv)) + (d - dv);
+                    U[n][m] = sum;
+                }
         }
         if (sed && a.storage) {
             a.storage[col] = s_sed[0][seg];
@@ -312,9 +265,7 @@ __device__ __forceinline__ void batch_columns(const BatchArgs<FT>& a)
             for (int m = 0; m < L; m++)
                 if (has(m)) {
                     a.U[n][idx(m)] = U[n][m];
-                    if constexpr (F32) {
-                        if (a.c_out) a.C[n][idx(m)] = D[n][m];
-                    }
+                    if (a.c_out) a.C[n][idx(m)] = D[n][m];
                 }
     }
 }

@@ -208,7 +208,7 @@ __device__ __forceinline__ void npzd_sediment(const SedimentParams& f, float N, 
     const float muP = f.mu0 * sediment_light<FM>(f, PAR) * (N * frcp(N + f.kNO3)) * Lt * P;
     const float sPOM = D * f.small_frac;
     const SGrazing G = sediment_grazing<FM>(f, P, Z, sPOM);
-    const float nuP = (fm_mort<FM>(f) == OBME_LINEAR) ? f.mP * P : f.mP * P * P;
+    float nuP = (fm_mort<FM>(f) == OBME_LINEAR) ? f.mP * P : f.mP * P * P;
     const float Z2 = Z * Z;
     dP = fmaf(f.one_m_gamma, muP, -G.onP) - nuP;
     dZ = fmaf(f.aZass, G.total, -f.mZ * Z2) - f.muZ * Z;
