@@ -1637,16 +1637,17 @@ extern "C" obme_status obme_kernel_timing(obme_handle* h, int32_t which, double*
 
 // ------------------------------------------------------------------ batched ensemble
 
-template <int L, int CPW, int NW, int FM>
-__global__ void __launch_bounds__(NW * 64, L == 2 ? 5 : 1) k_batch(BatchArgs<float> a)
-{
-    batch_columns<L, CPW, NW, FM>(a);
-}
-constexpr int RAGGED_WAVES = 4;   // waves per workgroup
 template <typename FT, int L, int FM, bool SED>
-__global__ void __launch_bounds__(RAGGED_WAVES * 64) k_batch_ragged(BatchArgs<FT> a)
+__global__ void __launch_bounds__(RAGGED_WAVES * 64, sizeof(FT) == 4 && SED && L == 2 ? 5 : 1)
+    k_batch_ragged(BatchArgs<FT> a)
 {
-    batch_ragged<FT, L, FM, SED>(a);
+    if constexpr (sizeof(FT) == 4 && SED) batch_ragged_sediment<L, FM, false>(a);
+    else batch_ragged<FT, L, FM, SED>(a);
+}
+template <int L, int FM>
+__global__ void __launch_bounds__(RAGGED_WAVES * 64, L == 2 ? 5 : 1) k_batch_rows(BatchArgs<float> a)
+{
+    batch_ragged_sediment<L, FM, true>(a);
 }
 
 // Tile shapes of the ensemble kernel: capacity L*64/CPW levels per column.
@@ -1670,18 +1671,17 @@ struct obme_batch {
     double dz, T;
     int* d_offsets = nullptr;
     void* d_fpar = nullptr;               // per-column derived constants, FastParams of the element type
-    SedimentParams* d_fsed = nullptr;     // FP32 with a sediment: its transitions' constants
+    SedimentParams* d_fsed = nullptr;     // (FP32 with a sediment: in its transitions' own form)
     BatchColumn* d_bcol = nullptr;
     float* d_comp = nullptr;              // FP32: the residual arrays, 4 x offsets[n_columns]
     int plan = -1;
     int steps_per_launch = 0;             // 0: every step of a call in one launch per class
     std::vector<int> class_tile, class_n; // per class of the plan
-    std::vector<int*> class_cols;
-    // the ragged packing (all but FP32 with a sediment): per levels per lane
+    // the ragged packing: per levels per lane
     // of the plan's classes, the lanes' table and its waves
     bool default_forms = false;
     std::vector<int*> group_lanes;
-    std::vector<int> group_L, group_waves;
+    std::vector<int> group_L, group_waves, group_rows;
     // captured multi-launch step
     hipStream_t cap_stream = nullptr;
     hipGraphExec_t graph = nullptr;
@@ -1701,9 +1701,6 @@ struct obme_batch {
 
 static void batch_free_classes(obme_batch* b)
 {
-    for (int* p : b->class_cols)
-        if (p) (void)hipFree(p);
-    b->class_cols.clear();
     b->class_tile.clear();
     b->class_n.clear();
     for (int* p : b->group_lanes)
@@ -1711,15 +1708,20 @@ static void batch_free_classes(obme_batch* b)
     b->group_lanes.clear();
     b->group_L.clear();
     b->group_waves.clear();
+    b->group_rows.clear();
 }
 
 // The ragged packing of the columns with L levels per lane, each lane's column
 // or -1: longest first, each into the wave with the least room that still
-// holds it.
-static std::vector<int> pack_ragged(const obme_batch* b, const std::vector<int>& cols, int L)
+// holds it.  A column takes a multiple of `unit` lanes (16: whole rows, those
+// of three or four from a wave's first).
+static std::vector<int> pack_ragged(const obme_batch* b, const std::vector<int>& cols, int L, int unit)
 {
     std::vector<int> by_lanes[65];
-    for (int c : cols) by_lanes[(b->offsets[c + 1] - b->offsets[c] + L - 1) / L].push_back(c);
+    for (int c : cols) {
+        const int n = (b->offsets[c + 1] - b->offsets[c] + L - 1) / L;
+        by_lanes[(n + unit - 1) / unit * unit].push_back(c);
+    }
     std::vector<int> lanes;
     std::vector<int> room[65];        // waves by their free lanes
     for (int n = 64; n >= 1; n--)
@@ -1751,8 +1753,7 @@ static void batch_drop_graph(obme_batch* b)
 }
 
 // Sorts the columns into the classes of plan p (smallest capacity that holds
-// the column): packed by levels per lane, or, FP32 with a sediment, class by
-// class, deepest columns first.
+// the column) and packs them by levels per lane.
 static obme_status batch_apply_plan(obme_batch* b, int p)
 {
     if (p < 0 || p >= (int)BATCH_PLANS.size()) return fail(OBME_ERR_INVALID, "unknown packing plan");
@@ -1769,35 +1770,38 @@ static obme_status batch_apply_plan(obme_batch* b, int p)
     }
     batch_free_classes(b);
     batch_drop_graph(b);
-    const bool ragged = !(b->sediment && b->prec != OBME_FP64);
-    if (ragged) {
-        for (int L : {1, 2, 4}) {
-            std::vector<int> cols;
-            for (size_t t = 0; t < tiles.size(); t++)
-                if (BATCH_TILES[tiles[t]].L == L) cols.insert(cols.end(), lists[t].begin(), lists[t].end());
-            const std::vector<int> lanes = pack_ragged(b, cols, L);
-            if (lanes.empty()) continue;
-            int* d = nullptr;
-            HIP_TRY(hipMalloc((void**)&d, lanes.size() * sizeof(int)));
-            b->group_lanes.push_back(d);
-            b->group_L.push_back(L);
-            b->group_waves.push_back((int)(lanes.size() / 64));
-            HIP_TRY(hipMemcpy(d, lanes.data(), lanes.size() * sizeof(int), hipMemcpyHostToDevice));
+    for (int L : {1, 2, 4}) {
+        std::vector<int> cols;
+        for (size_t t = 0; t < tiles.size(); t++)
+            if (BATCH_TILES[tiles[t]].L == L) cols.insert(cols.end(), lists[t].begin(), lists[t].end());
+        std::vector<int> lanes = pack_ragged(b, cols, L, 1);
+        // FP32 with a sediment: whole rows where they take no more waves per
+        // SIMD (1024 of them).  A launch is as long as its busiest SIMD, and
+        // row shifts are the faster sums: 46 against 63 us at one wave per
+        // SIMD, 65 and 74 at two, 110 and 118 at four (20 steps), but a
+        // column takes more lanes: 86 against 76 us where the rows need three
+        // waves per SIMD and the closer packing two.
+        bool rows = false;
+        if (b->sediment && b->prec != OBME_FP64) {
+            std::vector<int> in_rows = pack_ragged(b, cols, L, 16);
+            const size_t simds = 1024 * 64;
+            rows = (in_rows.size() + simds - 1) / simds <= (lanes.size() + simds - 1) / simds;
+            if (rows) lanes.swap(in_rows);
         }
+        if (lanes.empty()) continue;
+        int* d = nullptr;
+        HIP_TRY(hipMalloc((void**)&d, lanes.size() * sizeof(int)));
+        b->group_lanes.push_back(d);
+        b->group_L.push_back(L);
+        b->group_rows.push_back(rows ? 1 : 0);
+        b->group_waves.push_back((int)(lanes.size() / 64));
+        HIP_TRY(hipMemcpy(d, lanes.data(), lanes.size() * sizeof(int), hipMemcpyHostToDevice));
     }
     for (size_t t = 0; t < tiles.size(); t++) {
         std::vector<int>& l = lists[t];
         if (l.empty()) continue;
         b->class_tile.push_back(tiles[t]);
         b->class_n.push_back((int)l.size());
-        if (ragged) continue;
-        std::stable_sort(l.begin(), l.end(), [&](int x, int y) {
-            return b->offsets[x + 1] - b->offsets[x] > b->offsets[y + 1] - b->offsets[y];
-        });
-        int* d = nullptr;
-        HIP_TRY(hipMalloc((void**)&d, l.size() * sizeof(int)));
-        HIP_TRY(hipMemcpy(d, l.data(), l.size() * sizeof(int), hipMemcpyHostToDevice));
-        b->class_cols.push_back(d);
     }
     b->plan = p;
     return OBME_OK;
@@ -1838,33 +1842,6 @@ static BatchArgs<FT> batch_args(const obme_batch* b, void* const* tracers, doubl
     return a;
 }
 
-static obme_status batch_launch_class(const obme_batch* b, int q, BatchArgs<float> a, int nsteps, hipStream_t s)
-{
-    a.cols = b->class_cols[q];
-    a.ncols = b->class_n[q];
-    a.nsteps = nsteps;
-    const BatchTile& t = BATCH_TILES[b->class_tile[q]];
-    const int per_wg = t.NW * t.CPW;
-    dim3 grid((a.ncols + per_wg - 1) / per_wg), block(t.NW * 64);
-    constexpr int FM = default_fm<OBME_NPZD>();
-    const bool d = b->default_forms;
-    void (*k)(BatchArgs<float>) = nullptr;
-    switch (b->class_tile[q]) {
-    case 0: k = d ? k_batch<1, 4, 4, FM> : k_batch<1, 4, 4, -1>; break;
-    case 1: k = d ? k_batch<2, 4, 4, FM> : k_batch<2, 4, 4, -1>; break;
-    case 2: k = d ? k_batch<1, 2, 4, FM> : k_batch<1, 2, 4, -1>; break;
-    case 3: k = d ? k_batch<2, 2, 4, FM> : k_batch<2, 2, 4, -1>; break;
-    case 4: k = d ? k_batch<1, 1, 4, FM> : k_batch<1, 1, 4, -1>; break;
-    case 5: k = d ? k_batch<2, 1, 4, FM> : k_batch<2, 1, 4, -1>; break;
-    case 6: k = d ? k_batch<4, 2, 4, FM> : k_batch<4, 2, 4, -1>; break;
-    case 7: k = d ? k_batch<4, 4, 4, FM> : k_batch<4, 4, 4, -1>; break;
-    default: return fail(OBME_ERR_INVALID, "bad batch tile");
-    }
-    hipLaunchKernelGGL(k, grid, block, 0, s, a);
-    HIP_TRY(hipGetLastError());
-    return OBME_OK;
-}
-
 template <typename FT, bool SED>
 static void (*ragged_kernel(int L, bool default_forms))(BatchArgs<FT>)
 {
@@ -1876,25 +1853,27 @@ static void (*ragged_kernel(int L, bool default_forms))(BatchArgs<FT>)
     }
 }
 
-// One launch per levels per lane, or per class.
+static void (*rows_kernel(int L, bool default_forms))(BatchArgs<float>)
+{
+    constexpr int FM = default_fm<OBME_NPZD>();
+    switch (L) {
+    case 1: return default_forms ? k_batch_rows<1, FM> : k_batch_rows<1, -1>;
+    case 2: return default_forms ? k_batch_rows<2, FM> : k_batch_rows<2, -1>;
+    default: return default_forms ? k_batch_rows<4, FM> : k_batch_rows<4, -1>;
+    }
+}
+
+// One launch per levels per lane.
 template <typename FT>
 static obme_status batch_launch(const obme_batch* b, BatchArgs<FT> a, int nsteps, hipStream_t s)
 {
-    if constexpr (sizeof(FT) == 4) {
-        if (b->sediment) {
-            for (size_t q = 0; q < b->class_tile.size(); q++) {
-                obme_status r = batch_launch_class(b, (int)q, a, nsteps, s);
-                if (r != OBME_OK) return r;
-            }
-            return OBME_OK;
-        }
-    }
     a.nsteps = nsteps;
     for (size_t q = 0; q < b->group_L.size(); q++) {
         a.cols = b->group_lanes[q];
-        void (*k)(BatchArgs<FT>) = ragged_kernel<FT, false>(b->group_L[q], b->default_forms);
-        if constexpr (sizeof(FT) == 8)
-            if (b->sediment) k = ragged_kernel<FT, true>(b->group_L[q], b->default_forms);
+        void (*k)(BatchArgs<FT>) = b->sediment ? ragged_kernel<FT, true>(b->group_L[q], b->default_forms)
+                                               : ragged_kernel<FT, false>(b->group_L[q], b->default_forms);
+        if constexpr (sizeof(FT) == 4)
+            if (b->group_rows[q]) k = rows_kernel(b->group_L[q], b->default_forms);
         hipLaunchKernelGGL(k, dim3((unsigned)(b->group_waves[q] / RAGGED_WAVES)), dim3(RAGGED_WAVES * 64), 0, s, a);
         HIP_TRY(hipGetLastError());
     }
@@ -2077,8 +2056,8 @@ extern "C" obme_status obme_batch_create(const obme_config* cfg, int32_t n_colum
         // (the formulations are the configuration's, the same for every column)
         if (c == 0) b->default_forms = (fm_code(make_fast_params<float>(q)) == default_fm<OBME_NPZD>());
         if (f64) dpar[c] = make_fast_params<double>(q);
+        else if (fixed) spar[c] = make_sediment_params(q);
         else fpar[c] = make_fast_params<float>(q);
-        if (fixed) spar[c] = make_sediment_params(q);
         BatchColumn& bc = bcol[c];
         bc.PAR0 = get(OBME_BP_SURFACE_PAR, cfg->par.surface_value);
         bc.wP = -get(OBME_BP_P_SINKING_SPEED, cfg->sinking.speed[1]);
@@ -2095,9 +2074,9 @@ extern "C" obme_status obme_batch_create(const obme_config* cfg, int32_t n_colum
     };
     bool ok = up((void**)&b->d_offsets, b->offsets.data(), b->offsets.size() * sizeof(int)) &&
               up((void**)&b->d_bcol, bcol.data(), bcol.size() * sizeof(BatchColumn));
-    if (ok) ok = f64 ? up(&b->d_fpar, dpar.data(), dpar.size() * sizeof(dpar[0]))
-                     : up(&b->d_fpar, fpar.data(), fpar.size() * sizeof(fpar[0]));
-    if (ok && fixed) ok = up((void**)&b->d_fsed, spar.data(), spar.size() * sizeof(spar[0]));
+    if (ok) ok = f64     ? up(&b->d_fpar, dpar.data(), dpar.size() * sizeof(dpar[0]))
+                 : fixed ? up((void**)&b->d_fsed, spar.data(), spar.size() * sizeof(spar[0]))
+                         : up(&b->d_fpar, fpar.data(), fpar.size() * sizeof(fpar[0]));
     if (ok && b->prec != OBME_FP64)
         ok = hipMalloc((void**)&b->d_comp, 4 * (size_t)b->offsets[n_columns] * sizeof(float)) == hipSuccess;
     if (ok && cfg->sediment.model == OBME_SEDIMENT_INSTANT_REMINERALISATION) {

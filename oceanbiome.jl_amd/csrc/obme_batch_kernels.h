@@ -20,15 +20,12 @@
 // Layout: tracer n (N, P, Z, D) is one packed array; column c occupies
 // [offsets[c], offsets[c+1]) with k = 0 at the bottom.  Lane r of a column
 // holds the L levels counted from the top, j = r*L + m (k = Nz_c - 1 - j).
-// Cell centres depend only on j: zc = -(j + 1/2) dz.  The host sorts columns
-// into classes by depth; what becomes of them on the lanes:
-//  - batch_ragged: a column takes ceil(Nz_c / L) lanes and a wave as many
-//    columns as fit into its 64 lanes, of every class with the same L; the
-//    sums down a column are masked to its lanes;
-//  - batch_columns (FP32 with a sediment): a class's columns in segments of
-//    LPC = 64/CPW lanes (capacity L*LPC >= Nz_c), one persistent kernel per
-//    class.  The sediment's storage is FP64, and a sum down a column in
-//    another order moves it.
+// Cell centres depend only on j: zc = -(j + 1/2) dz.  A column takes
+// ceil(Nz_c / L) lanes and a wave as many columns as fit into its 64 lanes,
+// of every class with the same L (the host sorts columns into classes by
+// depth); the sums down a column are masked to its lanes.  FP32 with a
+// sediment is a kernel of its own (batch_ragged_sediment): the sediment's
+// storage is FP64, and a sum down a column in another order moves it.
 #pragma once
 
 #include "obme_wave_kernels.h"
@@ -48,10 +45,9 @@ struct BatchArgs {
     FT* C[4];                       // FP32: the residuals of U, packed alike (launch to launch)
     int c_in, c_out;                // FP32: start from the stored residuals; store them at the end
     const int* offsets;             // [n_columns + 1]
-    const int* cols;                // this class's column list; batch_ragged: each lane's column (or -1)
-    int ncols;                      // entries of `cols` (batch_columns)
+    const int* cols;                // each lane's column (or -1)
     const FastParams<FT>* fpar;     // per-column derived constants
-    const SedimentParams* fsed;     // FP32 with a sediment: the same, for its transitions
+    const SedimentParams* fsed;     // FP32 with a sediment: these instead, for its transitions
     const BatchColumn* bcol;        // per-column constants
     int nsteps;
     FT dtf, dz, invdz;
@@ -77,197 +73,271 @@ struct BatchArgs {
     FT sedP, sedD;                  // 1 where P / D is one of the sinking tracers, else 0
 };
 
-// FP32 with a sediment: one persistent workgroup loops over tiles of NW*CPW
-// columns.  FM: the default formulations compiled in, or < 0 (fm_light): they
-// are read per lane, and each choice is a branch over the lanes (8192 columns
-// of 16 to 128 levels, 50 steps: 478 us so, 463 compiled in; 307 of 34 to 79,
-// 20 steps: 97.7 and 92.8), with the same roundings.
-template <int L, int CPW, int NW, int FM>
-__device__ __forceinline__ void batch_columns(const BatchArgs<float>& a)
+constexpr int RAGGED_WAVES = 4;   // waves per workgroup
+
+// The lane's place in its column: from the last lane at or before it whose
+// predecessor has another (a lane without a column stands alone).
+__device__ __forceinline__ int column_lane(int lane, int at)
 {
-    constexpr int LPC = 64 / CPW;
-    static_assert(LPC == 16 || LPC == 32 || LPC == 64, "segments of 16, 32 or 64 lanes");
+    const int before = __shfl_up(at, 1, 64);   // (by every lane)
+    const unsigned long long starts = __ballot(lane == 0 || at < 0 || before != at);
+    return lane - (63 - __clzll((long long)(starts & (~0ull >> (63 - lane)))));
+}
+
+// The sum over the column's lanes from the top to this one, rounded as
+// seg_prefix rounds it in a segment of its own: steps of 1, 2, 4 and 8 lanes
+// within the column's groups of 16, then the group before, then the second
+// group's last lane.  (column_prefix groups by the wave's rows of 16: its last
+// bits depend on where the packing puts a column.)
+struct FixedPrefix {
+    bool b1, b2, b4, b8, odd, far, any_odd, any_far;
+    int lane4, before4, l31;
+    __device__ __forceinline__ FixedPrefix(int lane, int r)
+    {
+        const int g = r & 15;
+        b1 = g >= 1;
+        b2 = g >= 2;
+        b4 = g >= 4;
+        b8 = g >= 8;
+        odd = (r & 16) != 0;
+        far = r >= 32;
+        any_odd = __any(odd);
+        any_far = __any(far);
+        lane4 = lane * 4;
+        before4 = (lane - g - 1) * 4;
+        l31 = (lane - r + 31) * 4;
+    }
+    __device__ __forceinline__ static float from(int lane4, float x)
+    {
+        return __int_as_float(__builtin_amdgcn_ds_bpermute(lane4, __float_as_int(x)));
+    }
+    __device__ __forceinline__ float operator()(float x) const
+    {
+        float y = lane_shr1(x);
+        x = x + (b1 ? y : 0.0f);
+        y = lane_shr1(lane_shr1(x));
+        x = x + (b2 ? y : 0.0f);
+        y = from(lane4 - 16, x);
+        x = x + (b4 ? y : 0.0f);
+        y = from(lane4 - 32, x);
+        x = x + (b8 ? y : 0.0f);
+        if (any_odd) {
+            y = from(before4, x);
+            x = x + (odd ? y : 0.0f);
+        }
+        if (any_far) {
+            y = from(l31, x);
+            x = x + (far ? y : 0.0f);
+        }
+        return x;
+    }
+};
+
+// The same sums where every column starts at a row of 16 lanes (and a column of
+// three or four rows at row 0): the wave's rows are the column's groups.
+struct RowPrefix {
+    int mA, mB;
+    __device__ __forceinline__ RowPrefix(int lane, int r)
+    {
+        // (a column of two rows may start at row 2, one of three at row 0 only)
+        mA = (r & 16) ? -1 : 0;
+        mB = r >= 32 ? -1 : 0;
+    }
+    __device__ __forceinline__ float operator()(float x) const
+    {
+        x = seg_prefix<16>(x);
+        x = x + lane_and(dpp<0x142, 0xf, true>(x), mA);
+        x = x + lane_and(dpp<0x143, 0xf, true>(x), mB);
+        return x;
+    }
+};
+
+// FP32 with a sediment, in the ragged packing (ROWS: in whole rows of lanes).
+// What bounds it is what bounds batch_ragged, and with a wave or two per SIMD
+// the sums' latency.  In segments of 32 and 64 lanes per class, a launch each:
+// 8192 columns of 16 to 128 levels, 50 steps, 463 us; this 340 (307 of 34 to
+// 79 levels, 20 steps: 92.8 and 46).  FM: the default formulations compiled
+// in, or < 0 (fm_light): they are read per lane, and each choice is a branch
+// over the lanes (478 against 463 us), with the same roundings.
+template <int L, int FM, bool ROWS>
+__device__ __forceinline__ void batch_ragged_sediment(const BatchArgs<float>& a)
+{
     const int lane = threadIdx.x & 63;
-    const int w = threadIdx.x >> 6;
-    const int r = lane % LPC;
-    const int seg = w * CPW + lane / LPC;
-    const int ntiles = (a.ncols + NW * CPW - 1) / (NW * CPW);
+    const int at = a.cols[blockIdx.x * blockDim.x + threadIdx.x];
+    const int col = at;
+    const int r = column_lane(lane, at);
+    const int off = (col >= 0) ? a.offsets[col] : 0;
+    const int Nzc = (col >= 0) ? a.offsets[col + 1] - off : 0;
+    const std::conditional_t<ROWS, RowPrefix, FixedPrefix> prefix(lane, r);
+    // level m of this lane: j = r*L + m from the top, k = Nzc-1-j
+    auto has = [&](int m) -> bool { return r * L + m < Nzc; };
+    auto idx = [&](int m) -> int { return off + Nzc - 1 - (r * L + m); };
+
+    float U[4][L], D[4][L], Gm[4][L];
+#pragma unroll
+    for (int n = 0; n < 4; n++)
+#pragma unroll
+        for (int m = 0; m < L; m++) {
+            U[n][m] = has(m) ? a.U[n][idx(m)] : 0.0f;
+            Gm[n][m] = 0.0f;
+            D[n][m] = (a.c_in && has(m)) ? a.C[n][idx(m)] : 0.0f;
+        }
+    auto val = [&](int n, int m) -> float { return U[n][m] + D[n][m]; };
+
+    // column constants (every lane of a column reads the same entry)
+    const int cc = (col >= 0) ? col : 0;
+    const BatchColumn bc = a.bcol[cc];
+    const float PAR0 = (float)bc.PAR0;
+    const float Lt = (float)bc.Lt;
+    const float wP = (float)bc.wP, wD = (float)bc.wD;
+    const SedimentParams fp = a.fsed[cc];
+    const float wiP = (float)(bc.wP / (double)a.dz), wiD = (float)(bc.wD / (double)a.dz);
+
+    // the sediment of this column, held by the lane of its bottom cell
+    // (j = Nzc - 1: lane rb, level mb)
+    const int jb = Nzc - 1;
+    const bool sed = col >= 0 && r == jb / L;
+    const int mb = jb % L;
+    // the storage and the last tendency in LDS (not held in registers
+    // through the launch)
+    __shared__ double s_sed[2][RAGGED_WAVES * 64];
+    const int seg = threadIdx.x;
+    if (sed) {
+        s_sed[0][seg] = a.storage ? a.storage[col] : 0.0;
+        s_sed[1][seg] = (a.storage && a.sed_ab2) ? a.sedGm[col] : 0.0;
+    }
+
+    // water terms of the own levels
+    float ezr[L], ezb[L];
+#pragma unroll
+    for (int m = 0; m < L; m++) {
+        const float zc = -((float)(r * L + m) + 0.5f) * a.dz;
+        ezr[m] = a.kr2 * zc;
+        ezb[m] = a.kb2 * zc;
+    }
 
 #pragma unroll 1
-    for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        const int g = tile * (NW * CPW) + seg;
-        const int col = (g < a.ncols) ? a.cols[g] : -1;
-        const int off = (col >= 0) ? a.offsets[col] : 0;
-        const int Nzc = (col >= 0) ? a.offsets[col + 1] - off : 0;
-        // level m of this lane: j = r*L + m from the top, k = Nzc-1-j
-        auto has = [&](int m) -> bool { return r * L + m < Nzc; };
-        auto idx = [&](int m) -> int { return off + Nzc - 1 - (r * L + m); };
-
-        float U[4][L], D[4][L], Gm[4][L];
+    for (int s = 0; s < a.nsteps; s++) {
+#pragma unroll 1
+        for (int st = 0; st < 3; st++) {
+            // chlorophyll terms and the light integral (as in the sweep)
+            float pr[L], pb[L];
+#pragma unroll
+            for (int m = 0; m < L; m++) {
+                const float lg = m_log2(val(1, m));
+                pr[m] = m_exp2(fmaf(a.er_f, lg, a.cr));
+                pb[m] = m_exp2(fmaf(a.eb_f, lg, a.cb));
+            }
+            const float pr_up = lane_shr1(pr[L - 1]);
+            const float pb_up = lane_shr1(pb[L - 1]);
+            const float cP_up = lane_shr1(val(1, L - 1));
+            const float cD_up = lane_shr1(val(3, L - 1));
+            float incr[L], incb[L];
+            float totr = 0.0f, totb = 0.0f;
+#pragma unroll
+            for (int m = 0; m < L; m++) {
+                const bool top = (m == 0) && (r == 0);
+                const float prn = (m == 0) ? pr_up : pr[m > 0 ? m - 1 : 0];
+                const float pbn = (m == 0) ? pb_up : pb[m > 0 ? m - 1 : 0];
+                const float ir = top ? pr[m] : prn + pr[m];
+                const float ib = top ? pb[m] : pbn + pb[m];
+                incr[m] = has(m) ? ir : 0.0f;
+                incb[m] = has(m) ? ib : 0.0f;
+                totr = totr + incr[m];
+                totb = totb + incb[m];
+            }
+            float runr = lane_shr1(prefix(totr));
+            float runb = lane_shr1(prefix(totb));
+            if (r == 0) {
+                runr = 0.0f;
+                runb = 0.0f;
+            }
+            float PARv[L];
+#pragma unroll
+            for (int m = 0; m < L; m++) {
+                runr = runr + incr[m];
+                runb = runb + incb[m];
+                PARv[m] = (PAR0 * 0.5f) * (m_exp2(fmaf(-a.xr2h, runr, ezr[m])) +
+                                           m_exp2(fmaf(-a.xb2h, runb, ezb[m])));
+            }
+            // the sediment: the bottom cell's flux and burial, the
+            // receiver's coupled tendency, the sediment step
+            float cpl = 0.0f;
+            if (sed) {
+                float Pb = val(1, 0), Db = val(3, 0);
+#pragma unroll
+                for (int m = 1; m < L; m++)
+                    if (m == mb) {
+                        Pb = val(1, m);
+                        Db = val(3, m);
+                    }
+                const float f = a.sedP * (-wP) * Pb + a.sedD * (-wD) * Db;
+                // the hardware reciprocal (1 ulp) and 1/Δz
+                const float qf = f * __builtin_amdgcn_rcpf(a.sed_k + f);
+                const float e = a.sed_a + a.sed_b * (qf * qf);
+                cpl = ((1.0f - e) * f) * a.invdz;
+                const double ge = (double)(e * f);
+                const bool init = a.sed_init && s == 0;
+                if (st == 0) {
+                    if (!init) {
+                        const bool ab2 = a.sed_ab2 && s == 0;
+                        s_sed[0][seg] += a.sed_dt[0] * (ab2 ? a.sed_cn * ge - a.sed_cm * s_sed[1][seg] : ge);
+                    }
+                } else {
+                    if (st == 1 && init) s_sed[0][seg] += a.sed_dt[0] * ge;
+                    s_sed[0][seg] += a.sed_dt[st] * ge;
+                }
+                s_sed[1][seg] = ge;
+            }
+            // tendencies bottom-up within the lane, sinking, RK3 substep
+#pragma unroll
+            for (int m = L - 1; m >= 0; m--) {
+                const bool top = (m == 0) && (r == 0);
+                const float N = val(0, m), P = val(1, m), Z = val(2, m), Dd = val(3, m);
+                float G[4];
+                npzd_sediment<FM>(fp, N, P, Z, Dd, PARv[m], Lt, G[0], G[1], G[2], G[3]);
+                const float cPn = (m == 0) ? cP_up : val(1, m > 0 ? m - 1 : 0);
+                const float cDn = (m == 0) ? cD_up : val(3, m > 0 ? m - 1 : 0);
+                G[1] = fmaf(-wiP, (top ? 0.0f : cPn) - P, G[1]);
+                G[3] = fmaf(-wiD, (top ? 0.0f : cDn) - Dd, G[3]);
+                if (sed && m == mb) {
+#pragma unroll
+                    for (int n = 0; n < 4; n++)
+                        if (n == a.sed_recv) G[n] = G[n] + cpl;
+                }
+#pragma unroll
+                for (int n = 0; n < 4; n++) {
+                    const float A = (st == 0) ? a.rk_a[0] : (st == 1 ? a.rk_a[1] : a.rk_a[2]);
+                    const float B = (st == 0) ? a.rk_b[0] : (st == 1 ? a.rk_b[1] : a.rk_b[2]);
+                    D[n][m] = fmaf(A, G[n], fmaf(B, Gm[n][m], D[n][m]));
+                    Gm[n][m] = G[n];
+                }
+            }
+        }
+        // U + D = s + e exactly (TwoSum): U = s, and e carries on
 #pragma unroll
         for (int n = 0; n < 4; n++)
 #pragma unroll
             for (int m = 0; m < L; m++) {
-                U[n][m] = has(m) ? a.U[n][idx(m)] : 0.0f;
-                Gm[n][m] = 0.0f;
-                D[n][m] = (a.c_in && has(m)) ? a.C[n][idx(m)] : 0.0f;
+                const float u = U[n][m], d = D[n][m];
+                const float sum = u + d;
+                const float dv = sum - u;
+                D[n][m] = (u - (sum - dv)) + (d - dv);
+                U[n][m] = sum;
             }
-        auto val = [&](int n, int m) -> float { return U[n][m] + D[n][m]; };
-
-        // column constants (every lane of a segment reads the same entry)
-        const int cc = (col >= 0) ? col : 0;
-        const BatchColumn bc = a.bcol[cc];
-        const float PAR0 = (float)bc.PAR0;
-        const float Lt = (float)bc.Lt;
-        const float wP = (float)bc.wP, wD = (float)bc.wD;
-        const SedimentParams fp = a.fsed[cc];
-        const float wiP = (float)(bc.wP / (double)a.dz), wiD = (float)(bc.wD / (double)a.dz);
-
-        // the sediment of this column, held by the lane of its bottom cell
-        // (j = Nzc - 1: lane rb, level mb)
-        const int jb = Nzc - 1;
-        const bool sed = col >= 0 && r == jb / L;
-        const int mb = jb % L;
-        // the storage and the last tendency in LDS, one slot per segment
-        // (not held in registers through the launch)
-        __shared__ double s_sed[2][NW * CPW];
-        if (sed) {
-            s_sed[0][seg] = a.storage ? a.storage[col] : 0.0;
-            s_sed[1][seg] = (a.storage && a.sed_ab2) ? a.sedGm[col] : 0.0;
-        }
-
-        // water terms of the own levels
-        float ezr[L], ezb[L];
-#pragma unroll
-        for (int m = 0; m < L; m++) {
-            const float zc = -((float)(r * L + m) + 0.5f) * a.dz;
-            ezr[m] = a.kr2 * zc;
-            ezb[m] = a.kb2 * zc;
-        }
-
-#pragma unroll 1
-        for (int s = 0; s < a.nsteps; s++) {
-#pragma unroll 1
-            for (int st = 0; st < 3; st++) {
-                // chlorophyll terms and the light integral (as in the sweep)
-                float pr[L], pb[L];
-#pragma unroll
-                for (int m = 0; m < L; m++) {
-                    const float lg = m_log2(val(1, m));
-                    pr[m] = m_exp2(fmaf(a.er_f, lg, a.cr));
-                    pb[m] = m_exp2(fmaf(a.eb_f, lg, a.cb));
-                }
-                const float pr_up = lane_shr1(pr[L - 1]);
-                const float pb_up = lane_shr1(pb[L - 1]);
-                const float cP_up = lane_shr1(val(1, L - 1));
-                const float cD_up = lane_shr1(val(3, L - 1));
-                float incr[L], incb[L];
-                float totr = 0.0f, totb = 0.0f;
-#pragma unroll
-                for (int m = 0; m < L; m++) {
-                    const bool top = (m == 0) && (r == 0);
-                    const float prn = (m == 0) ? pr_up : pr[m > 0 ? m - 1 : 0];
-                    const float pbn = (m == 0) ? pb_up : pb[m > 0 ? m - 1 : 0];
-                    const float ir = top ? pr[m] : prn + pr[m];
-                    const float ib = top ? pb[m] : pbn + pb[m];
-                    incr[m] = has(m) ? ir : 0.0f;
-                    incb[m] = has(m) ? ib : 0.0f;
-                    totr = totr + incr[m];
-                    totb = totb + incb[m];
-                }
-                float runr = lane_shr1(seg_prefix<LPC>(totr));
-                float runb = lane_shr1(seg_prefix<LPC>(totb));
-                if (r == 0) {
-                    runr = 0.0f;
-                    runb = 0.0f;
-                }
-                float PARv[L];
-#pragma unroll
-                for (int m = 0; m < L; m++) {
-                    runr = runr + incr[m];
-                    runb = runb + incb[m];
-                    PARv[m] = (PAR0 * 0.5f) * (m_exp2(fmaf(-a.xr2h, runr, ezr[m])) +
-                                               m_exp2(fmaf(-a.xb2h, runb, ezb[m])));
-                }
-                // the sediment: the bottom cell's flux and burial, the
-                // receiver's coupled tendency, the sediment step
-                float cpl = 0.0f;
-                if (sed) {
-                    float Pb = val(1, 0), Db = val(3, 0);
-#pragma unroll
-                    for (int m = 1; m < L; m++)
-                        if (m == mb) {
-                            Pb = val(1, m);
-                            Db = val(3, m);
-                        }
-                    const float f = a.sedP * (-wP) * Pb + a.sedD * (-wD) * Db;
-                    // the hardware reciprocal (1 ulp) and 1/Δz
-                    const float qf = f * __builtin_amdgcn_rcpf(a.sed_k + f);
-                    const float e = a.sed_a + a.sed_b * (qf * qf);
-                    cpl = ((1.0f - e) * f) * a.invdz;
-                    const double ge = (double)(e * f);
-                    const bool init = a.sed_init && s == 0;
-                    if (st == 0) {
-                        if (!init) {
-                            const bool ab2 = a.sed_ab2 && s == 0;
-                            s_sed[0][seg] += a.sed_dt[0] * (ab2 ? a.sed_cn * ge - a.sed_cm * s_sed[1][seg] : ge);
-                        }
-                    } else {
-                        if (st == 1 && init) s_sed[0][seg] += a.sed_dt[0] * ge;
-                        s_sed[0][seg] += a.sed_dt[st] * ge;
-                    }
-                    s_sed[1][seg] = ge;
-                }
-                // tendencies bottom-up within the lane, sinking, RK3 substep
-#pragma unroll
-                for (int m = L - 1; m >= 0; m--) {
-                    const bool top = (m == 0) && (r == 0);
-                    const float N = val(0, m), P = val(1, m), Z = val(2, m), Dd = val(3, m);
-                    float G[4];
-                    npzd_sediment<FM>(fp, N, P, Z, Dd, PARv[m], Lt, G[0], G[1], G[2], G[3]);
-                    const float cPn = (m == 0) ? cP_up : val(1, m > 0 ? m - 1 : 0);
-                    const float cDn = (m == 0) ? cD_up : val(3, m > 0 ? m - 1 : 0);
-                    G[1] = fmaf(-wiP, (top ? 0.0f : cPn) - P, G[1]);
-                    G[3] = fmaf(-wiD, (top ? 0.0f : cDn) - Dd, G[3]);
-                    if (sed && m == mb) {
-#pragma unroll
-                        for (int n = 0; n < 4; n++)
-                            if (n == a.sed_recv) G[n] = G[n] + cpl;
-                    }
-#pragma unroll
-                    for (int n = 0; n < 4; n++) {
-                        const float A = (st == 0) ? a.rk_a[0] : (st == 1 ? a.rk_a[1] : a.rk_a[2]);
-                        const float B = (st == 0) ? a.rk_b[0] : (st == 1 ? a.rk_b[1] : a.rk_b[2]);
-                        D[n][m] = fmaf(A, G[n], fmaf(B, Gm[n][m], D[n][m]));
-                        Gm[n][m] = G[n];
-                    }
-                }
-            }
-            // U + D = s + e exactly (TwoSum): U = s, and e carries on
-#pragma unroll
-            for (int n = 0; n < 4; n++)
-#pragma unroll
-                for (int m = 0; m < L; m++) {
-                    const float u = U[n][m], d = D[n][m];
-                    const float sum = u + d;
-                    const float dv = sum - u;
-                    D[n][m] = (u - (sum - dv)) + (d - dv);
-                    U[n][m] = sum;
-                }
-        }
-        if (sed && a.storage) {
-            a.storage[col] = s_sed[0][seg];
-            a.sedGm[col] = s_sed[1][seg];
-        }
-#pragma unroll
-        for (int n = 0; n < 4; n++)
-#pragma unroll
-            for (int m = 0; m < L; m++)
-                if (has(m)) {
-                    a.U[n][idx(m)] = U[n][m];
-                    if (a.c_out) a.C[n][idx(m)] = D[n][m];
-                }
     }
+    if (sed && a.storage) {
+        a.storage[col] = s_sed[0][seg];
+        a.sedGm[col] = s_sed[1][seg];
+    }
+#pragma unroll
+    for (int n = 0; n < 4; n++)
+#pragma unroll
+        for (int m = 0; m < L; m++)
+            if (has(m)) {
+                a.U[n][idx(m)] = U[n][m];
+                if (a.c_out) a.C[n][idx(m)] = D[n][m];
+            }
 }
 
 // The ragged packing: the lane's column from the host's table.
@@ -281,16 +351,12 @@ template <typename FT, int L, int FM, bool SED>
 __device__ __forceinline__ void batch_ragged(const BatchArgs<FT>& a)
 {
     constexpr bool F32 = sizeof(FT) == 4;
-    static_assert(!(F32 && SED), "FP32 with a sediment: batch_columns");
+    static_assert(!(F32 && SED), "FP32 with a sediment: batch_ragged_sediment");
     const int lane = threadIdx.x & 63;
     const int at = a.cols[blockIdx.x * blockDim.x + threadIdx.x];
     const bool ok = at >= 0;
     const int col = ok ? at : 0;
-    // the lane's place in its column: from the last lane at or before it whose
-    // predecessor has another (a lane without a column stands alone)
-    const int before = __shfl_up(at, 1, 64);   // (by every lane)
-    const unsigned long long starts = __ballot(lane == 0 || !ok || before != at);
-    const int r = lane - (63 - __clzll((long long)(starts & (~0ull >> (63 - lane)))));
+    const int r = column_lane(lane, at);
     const int off = a.offsets[col];
     const int Nzc = ok ? a.offsets[col + 1] - off : 0;
     auto has = [&](int m) -> bool { return r * L + m < Nzc; };

@@ -1,8 +1,9 @@
 """FP32 ensembles with a sediment: the default formulations (compiled in) and
 others (chosen at run time), in every plan and at the depths where the packing
-has its edges, against the oracle's column runs; the bounds are those of the
-other FP32 ensemble tests (1e-5, ten times that per column), and the storage's
-is the tracers'."""
+has its edges, in whole rows of lanes and, with many short columns, lane by
+lane, against the oracle's column runs; the bounds are those of the other FP32
+ensemble tests (1e-5, ten times that per column), and the storage's is the
+tracers'."""
 import pytest
 
 import oracle as O
@@ -14,14 +15,16 @@ from test_gpu_batch_packing import DEPTHS, _ensemble
 
 pytestmark = pytest.mark.gpu
 TOL = 1e-5
+# (in whole rows: over 1024 waves; lane by lane: far fewer)
+CASES = dict(DEPTHS, many=[1, 2, 3, 5, 8, 13, 21] * 650 + [128, 127, 97, 65, 64, 63, 62, 33, 31])
 
 
 @pytest.mark.parametrize("forms", ["default", "other"])
-@pytest.mark.parametrize("name", DEPTHS)
+@pytest.mark.parametrize("name", CASES)
 def test_forms(name, forms):
     import torch
     print("case batch sediment", name, forms, flush=True)
-    depths = DEPTHS[name]
+    depths = CASES[name]
     wl = _ensemble(depths, seed=5)
     if forms == "other":
         wl.bgc.plankton.phytoplankton_mortality_formulation = Quadratic
