@@ -202,7 +202,7 @@ struct obme_handle {
     int ntracers;
     int prec;
     std::vector<double> zc, zf, dz, Tprof, Sprof;
-    void* d_lev = nullptr;     // LEV_COUNT * Nz of FT
+    void* d_lev = nullptr;     // LEV_COUNT * Nz of FT; d_wsink and d_fast lie in its allocation
     void* d_wsink = nullptr;   // MAX_SINK * (Nz+1) of FT
     double* d_Tprof = nullptr;
     double* d_Sprof = nullptr;
@@ -347,6 +347,9 @@ static int ntracers_of(const obme_config& c)
 }
 
 template <typename FT>
+static StepArgs<FT> make_args(const obme_handle* h, void* const* tracers);
+
+template <typename FT>
 static obme_status upload_geometry(obme_handle* h)
 {
     const int Nz = h->cfg.grid.Nz;
@@ -364,8 +367,6 @@ static obme_status upload_geometry(obme_handle* h)
         lev[LEV_WR * Nz + k] = (FT)(0.5 * std::exp(h->cfg.par.water_red_attenuation * h->zc[k]));
         lev[LEV_WB * Nz + k] = (FT)(0.5 * std::exp(h->cfg.par.water_blue_attenuation * h->zc[k]));
     }
-    HIP_TRY(hipMalloc(&h->d_lev, lev.size() * sizeof(FT)));
-    HIP_TRY(hipMemcpy(h->d_lev, lev.data(), lev.size() * sizeof(FT), hipMemcpyHostToDevice));
     // drift velocities (Utils/sinking_velocity_fields.jl:10-35), faces 1..Nz+1
     std::vector<FT> w((size_t)MAX_SINK * (Nz + 1), (FT)0);
     const obme_sinking& sk = h->cfg.sinking;
@@ -377,8 +378,21 @@ static obme_status upload_geometry(obme_handle* h)
             w[(size_t)s * (Nz + 1) + (k - 1)] = (FT)(-speed * (sk.open_bottom ? 1.0 : (1 - std::exp((1 - k) / d))));
         w[(size_t)s * (Nz + 1) + Nz] = (FT)0;
     }
-    HIP_TRY(hipMalloc(&h->d_wsink, w.size() * sizeof(FT)));
-    HIP_TRY(hipMemcpy(h->d_wsink, w.data(), w.size() * sizeof(FT), hipMemcpyHostToDevice));
+    // one allocation and one copy for the tables: the levels, the drift
+    // velocities and, FP64, the transitions' constants
+    const size_t lev_bytes = lev.size() * sizeof(FT), w_bytes = w.size() * sizeof(FT);
+    const size_t fast_at = (lev_bytes + w_bytes + 15) / 16 * 16;
+    std::vector<char> all(fast_at + (sizeof(FT) == 8 ? sizeof(FastParams<FT>) : 0));
+    std::memcpy(all.data(), lev.data(), lev_bytes);
+    std::memcpy(all.data() + lev_bytes, w.data(), w_bytes);
+    if constexpr (sizeof(FT) == 8) {
+        const FastParams<FT> f = make_args<FT>(h, nullptr).f;
+        std::memcpy(all.data() + fast_at, &f, sizeof(f));
+    }
+    HIP_TRY(hipMalloc(&h->d_lev, all.size()));
+    HIP_TRY(hipMemcpy(h->d_lev, all.data(), all.size(), hipMemcpyHostToDevice));
+    h->d_wsink = (char*)h->d_lev + lev_bytes;
+    if constexpr (sizeof(FT) == 8) h->d_fast = (char*)h->d_lev + fast_at;
 
     // Uniform-grid fast path: the kernel forms zc = zc[0] + k dz, the half
     // cells dz/2, 1/dz and constant face velocities itself.  Taken only when
@@ -443,9 +457,6 @@ static int steps_within(size_t bytes, size_t per_step)
 {
     return (int)std::max<size_t>(1, std::min<size_t>(WAVE_MAX_STEPS, bytes / std::max<size_t>(1, per_step)));
 }
-
-template <typename FT>
-static StepArgs<FT> make_args(const obme_handle* h, void* const* tracers);
 
 extern "C" obme_status obme_create(const obme_config* cfg, obme_handle** out)
 {
@@ -527,14 +538,6 @@ extern "C" obme_status obme_create(const obme_config* cfg, obme_handle** out)
         obme_destroy(h);
         return st;
     }
-    if (h->prec == OBME_FP64) {
-        const FastParams<double> f = make_args<double>(h, nullptr).f;
-        if (hipMalloc(&h->d_fast, sizeof(f)) != hipSuccess ||
-            hipMemcpy(h->d_fast, &f, sizeof(f), hipMemcpyHostToDevice) != hipSuccess) {
-            obme_destroy(h);
-            return fail(OBME_ERR_NOMEM, "constants");
-        }
-    }
     h->sweep_waves = default_sweep_waves((size_t)g.Nx * g.Ny);
     if (const char* e = std::getenv("OBME_SWEEP_WAVES")) {
         const int nw = std::atoi(e);
@@ -600,12 +603,10 @@ extern "C" obme_status obme_destroy(obme_handle* h)
 {
     if (!h) return OBME_OK;
     if (h->d_lev) (void)hipFree(h->d_lev);
-    if (h->d_wsink) (void)hipFree(h->d_wsink);
     if (h->d_Tprof) (void)hipFree(h->d_Tprof);
     if (h->d_Sprof) (void)hipFree(h->d_Sprof);
     if (h->d_srec) (void)hipFree(h->d_srec);
     if (h->d_toprec) (void)hipFree(h->d_toprec);
-    if (h->d_fast) (void)hipFree(h->d_fast);
     if (h->d_Hprev) (void)hipFree(h->d_Hprev);
     if (h->d_topres) (void)hipFree(h->d_topres);
     if (h->d_o2c) (void)hipFree(h->d_o2c);
