@@ -847,8 +847,12 @@ static WaveShape wave_shape(const obme_handle* h, int mode, int nsteps, bool gen
     const long ncol = (long)h->cfg.grid.Nx * h->cfg.grid.Ny;
     if (Nz < 2 || !h->default_forms) return best;
     // (FP32 takes the logarithm of the chlorophyll attenuation)
-    if (sizeof(FT) == 4 && !(h->cfg.par.chlorophyll_red_attenuation >= 0 && h->cfg.par.chlorophyll_blue_attenuation >= 0))
-        return best;
+    const obme_two_band_par& par = h->cfg.par;
+    if (sizeof(FT) == 4 && !(par.chlorophyll_red_attenuation >= 0 && par.chlorophyll_blue_attenuation >= 0)) return best;
+    // exponents of 0 to 1: the powers of finite tracers are finite, and a level's
+    // own can be taken off the sum that includes it
+    auto tame = [](double e) { return e >= 0 && e <= 1; };
+    if (!tame(par.chlorophyll_red_exponent) || !tame(par.chlorophyll_blue_exponent)) return best;
     if (mode == TILE_STEP && h->sediment) {
         if (h->cfg.sediment.model == OBME_SEDIMENT_SIMPLE_MULTI_G) return best;
         // NPZD's sinking P takes the light's rounding into the FP64 storage

@@ -115,7 +115,8 @@ __device__ __forceinline__ double m_exp10(double x)
     const double c = 0x1.26bb1bbb55516p+1, cl = -0x1.f48ad494ea3e9p-53;   // ln 10
     const double p = x * c;
     const double r = exp(p);
-    return fma(r, fma(x, c, -p) + x * cl, r);
+    const double q = fma(r, fma(x, c, -p) + x * cl, r);
+    return q < HUGE_VAL ? q : r;    // (overflow: the correction is inf * 0)
 }
 __device__ __forceinline__ double m_log10(double x)
 {
@@ -137,19 +138,23 @@ struct Divisor {
     }
 };
 // x^e from L = log |x| as exp(e L), the product's rounding error put back
-// (exp would amplify it: |e L| is of order 10).
+// (exp would amplify it: |e L| is of order 10).  Where the power overflows or e
+// is infinite it is not below infinity (NaN: infinity times a correction of 0),
+// and pow_special takes it.
 __device__ __forceinline__ double exp_product(double e, double L)
 {
     const double p = e * L;
     const double r = exp(p);
     return fma(r, fma(e, L, -p), r);
 }
-// pow's value at x <= 0, infinite and NaN x and at e = 0, r = |x|^e elsewhere.
+// pow's value at x <= 0, infinite and NaN x, at e = 0 and where it overflows,
+// r = |x|^e elsewhere.
 __device__ __forceinline__ double pow_special(double x, double e, double r)
 {
     if (e == 0.0) return 1.0;
     if (x != x || e != e) return x + e;
     const double inf = HUGE_VAL;
+    if (!(r < inf)) r = fabs(x) == 1.0 ? 1.0 : ((e > 0.0) == (fabs(x) > 1.0) ? inf : 0.0);
     if (x == 0.0) r = e > 0.0 ? 0.0 : inf;
     if (fabs(x) == inf) r = e > 0.0 ? inf : 0.0;
     if (x < 0.0) {
@@ -165,7 +170,7 @@ __device__ __forceinline__ void pow_pair(double x, double e1, double e2, double&
     const double L = log_positive(fabs(x));
     r1 = exp_product(e1, L);
     r2 = exp_product(e2, L);
-    if (!(x > 0.0 && x < HUGE_VAL && e1 != 0.0 && e2 != 0.0)) {
+    if (!(x > 0.0 && x < HUGE_VAL && e1 != 0.0 && e2 != 0.0 && r1 < HUGE_VAL && r2 < HUGE_VAL)) {
         r1 = pow_special(x, e1, r1);
         r2 = pow_special(x, e2, r2);
     }
@@ -174,7 +179,7 @@ __device__ __forceinline__ void pow_pair(double x, double e1, double e2, double&
 __device__ __forceinline__ double m_pow(double x, double y)
 {
     double r = exp_product(y, log_positive(fabs(x)));
-    if (!(x > 0.0 && x < HUGE_VAL && y != 0.0)) r = pow_special(x, y, r);
+    if (!(x > 0.0 && x < HUGE_VAL && y != 0.0 && r < HUGE_VAL)) r = pow_special(x, y, r);
     return r;
 }
 // x^y for x >= 0 as 2^(y log2 x); a negative x gives NaN, as on the GPU
