@@ -261,7 +261,8 @@ struct FastParams {
     FT R, Rd, rhoR, rhoRg, rhoR4;  // R, Rd, rho R, rho R g, 4 rho R mu0/2
     FT rem, small_frac;           // Detritus rate and fraction
     FT nGrowP, nUp, nPonw, nOx;   // NPZD: (1 - gamma) mu0, (1 - alpha_x gamma) mu0, (1 - alpha_x) gamma mu0, Rp mu0
-    FT logQ10_10, logQ10_10l;   // Q10^(T/10): FP32 log2(Q10)/10; FP64 ln(Q10)/10 and its rounding error
+    FT logQ10_10, logQ10_10l;   // Q10^(T/10): FP32 log2(Q10)/10; FP64 ln|Q10|/10 and its rounding error
+    FT Q10;                     // (FP64)
     FT oRp, oRpn, oRpm;           // Oxygen(): Rp, Rp - Rn, Rp mu0/2
     int light_form, use_Q10, mort_form, graz_form;
 };
@@ -321,10 +322,13 @@ inline FastParams<FT> make_fast_params(const obme_npd_params& p, double Rp = 0.0
     f.nUp = (FT)((1 - ax * gam) * mu0);
     f.nPonw = (FT)((1 - ax) * gam * mu0);
     f.nOx = (FT)(Rp * mu0);
-    const double Q = p.temperature_coefficient > 0 ? p.temperature_coefficient : 1.0;
+    // (a Q10 of 0 or less: FP32 none, FP64 pow's values)
+    const double Q = F32 ? (p.temperature_coefficient > 0 ? p.temperature_coefficient : 1.0)
+                         : std::fabs(p.temperature_coefficient);
     const long double lnQ = std::log((long double)Q) / 10;
     f.logQ10_10 = F32 ? (FT)(std::log2(Q) / 10) : (FT)lnQ;
     f.logQ10_10l = F32 ? FT(0) : (FT)(lnQ - (long double)(double)lnQ);
+    f.Q10 = (FT)p.temperature_coefficient;
     f.oRp = (FT)Rp;
     f.oRpn = (FT)(Rp - Rn);
     f.oRpm = (FT)(Rp * h);
@@ -365,7 +369,10 @@ __device__ __forceinline__ FT q10_factor(const FastParams<FT>& f, FT T)
     } else {
         const double p = T * f.logQ10_10;
         const double e = exp(p);
-        return fma(e, fma(T, f.logQ10_10, -p) + T * f.logQ10_10l, e);
+        double r = fma(e, fma(T, f.logQ10_10, -p) + T * f.logQ10_10l, e);
+        r = r < HUGE_VAL ? r : e;       // (overflow: the correction is inf * 0)
+        if (!(f.Q10 > 0)) r = pow_special(f.Q10, T / 10, r);
+        return r;
     }
 }
 

@@ -1,7 +1,8 @@
 """FP64 powers past the range of doubles: the chlorophyll power of the light
 with exponents that take it to infinity (no light is left) or to 0 (the water's
-light is left), in the light hook, the tendencies and the step, against the
-oracle's pow."""
+light is left), in the light hook, the tendencies and the step; and the
+temperature factor Q10^(T/10) where it overflows, underflows and for a Q10 of 0
+or less; against the oracle's pow."""
 import numpy as np
 import pytest
 
@@ -65,3 +66,37 @@ def test_chlorophyll_power_past_the_range(e, P, Nz):
         torch.cuda.synchronize()
         for a, b in zip(to_host(tr), step):
             assert rel_l2(g.interior(a), g.interior(b)) <= 1e-12
+
+
+# T = 0 and a multiple of 10 among the levels
+@pytest.mark.parametrize("Q10, T", [(0.0, 12.0), (0.0, 0.0), (-2.0, 10.0), (-2.0, 20.0), (-2.0, 12.0), (1.88, -2e5),
+                                    (1.88, 12.0)], ids=str)
+@pytest.mark.parametrize("Nz", [6, 300])
+def test_temperature_factor(Q10, T, Nz):
+    import torch
+    print("case Q10", Q10, T, Nz, flush=True)
+    bgc, g, fields = _npzd(Nz, 0.629, True)
+    bgc.plankton.temperature_coefficient = Q10
+    g.interior(fields[3])[...] = T
+    cfg = bgc.config(abi.OBME_FP64)
+    dev = HIPBiogeochemistry(bgc, "fp64")
+    tr = to_device(fields, dev.dtype)
+    G = [torch.zeros_like(t) for t in tr]
+    dev.update_tendencies(tr, G)
+    want = [g.new_field() for _ in fields]
+    O.grid_tendencies(cfg, fields, want)
+    torch.cuda.synchronize()
+    for n in (0, 1, 2, 4):
+        a, b = g.interior(G[n].cpu().numpy()), g.interior(want[n])
+        assert np.array_equal(np.isnan(a), np.isnan(b)), n
+        ok = ~np.isnan(b)
+        assert rel_l2(a[ok], b[ok]) <= 1e-12, n
+    step = [f.copy() for f in fields]
+    O.grid_run(cfg, step, 2, 60.0)
+    dev.step(tr, 2, 60.0)
+    torch.cuda.synchronize()
+    for n, (x, y) in enumerate(zip(to_host(tr), step)):
+        a, b = g.interior(x), g.interior(y)
+        assert np.array_equal(np.isnan(a), np.isnan(b)), n
+        ok = ~np.isnan(b)
+        assert rel_l2(a[ok], b[ok]) <= 1e-12, n
