@@ -339,7 +339,7 @@ inline FastParams<FT> make_fast_params(const obme_npd_params& p, double Rp = 0.0
     return f;
 }
 
-// max(0, x).  (A NaN x gives 0 here: the nitrate uptake beside it is NaN then.)
+// max(0, x), 0 for a NaN x.
 __device__ __forceinline__ float max0(float x) { return fmaxf(x, 0.0f); }
 __device__ __forceinline__ double max0(double x) { return fmax(x, 0.0); }
 // the smallest normal number: keeps 0/0 away as the reference's eps(food) does
@@ -435,7 +435,11 @@ __device__ __forceinline__ void lobster_fast(const FastParams<FT>& f, const FT* 
     FT uN, uA;
     if constexpr (sizeof(FT) == 8) {
         const FT light = fm_light<FM>(f) == OBME_LIGHT_MONDO ? f.kPAR + PAR : FT(1);
-        const FT pp = fm_light<FM>(f) == OBME_LIGHT_MONDO ? PAR * P : PAR * P * m_rsqrt(fma(PAR, PAR, f.kPAR2));
+        FT pp = fm_light<FM>(f) == OBME_LIGHT_MONDO ? PAR * P : PAR * P * m_rsqrt(fma(PAR, PAR, f.kPAR2));
+        // an infinite NH4 has no limitation (infinity over infinity): NaN to
+        // both uptakes.  (A NaN of max0's is then a denominator of 0 under a
+        // negative NH4, whose quotient is -infinity.)
+        pp = fma(FT(0), NH4, pp);
         const FT r = m_rcp(a * light);
         uN = pp * nl * r;
         uA = max0(NH4 * m_rcp(b)) * (pp * (a * r));
