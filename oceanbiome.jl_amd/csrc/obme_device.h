@@ -21,23 +21,15 @@ namespace obme {
 
 // ---------------------------------------------------------------- scalars
 
-// Julia Base min/max for IEEE floats (NaN propagates; -0 < 0).  FP32: the
-// hardware's minimum/maximum of IEEE 754-2019, which is just that, in one
-// instruction (a difference, its sign and two selects take five: a third of
-// the PISCES transitions' comparisons and selects).  FP64 has none: a
-// comparison that keeps a NaN x, and y where it is chosen.
+// Julia Base min/max for IEEE floats (NaN propagates; -0 < 0): the minimum and
+// maximum of IEEE 754-2019.  FP32: one hardware instruction (a difference, its
+// sign and two selects take five: a third of the PISCES transitions'
+// comparisons and selects).  FP64: the hardware's minimum, which orders the
+// zeros, a comparison and two selects for NaN.
 template <typename FT>
-__device__ __forceinline__ FT jmin(FT x, FT y)
-{
-    if constexpr (sizeof(FT) == 4) return __builtin_elementwise_minimum(x, y);
-    else return (x <= y || __builtin_isnan(x)) ? x : y;
-}
+__device__ __forceinline__ FT jmin(FT x, FT y) { return __builtin_elementwise_minimum(x, y); }
 template <typename FT>
-__device__ __forceinline__ FT jmax(FT x, FT y)
-{
-    if constexpr (sizeof(FT) == 4) return __builtin_elementwise_maximum(x, y);
-    else return (x >= y || __builtin_isnan(x)) ? x : y;
-}
+__device__ __forceinline__ FT jmax(FT x, FT y) { return __builtin_elementwise_maximum(x, y); }
 
 // Precision-dispatched math.  FP64: the accurate device library.  FP32:
 // the hardware instructions v_exp_f32 (2^x), v_log_f32 (log2 x),
