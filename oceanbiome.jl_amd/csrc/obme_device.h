@@ -156,13 +156,16 @@ __device__ __forceinline__ double pow_special(double x, double e, double r)
     return r;
 }
 // x^e1 and x^e2 of one base in FP64, within a few ulp of pow: the logarithm
-// shared, pow's special cases behind one branch.
+// shared, pow's special cases behind one branch.  TAME: exponents of 0 to 1,
+// with which a power of a finite base does not overflow (LOBSTER's FP64 step
+// on 256x256x64, four steps: 628 us, 640 with the comparisons).
+template <bool TAME = false>
 __device__ __forceinline__ void pow_pair(double x, double e1, double e2, double& r1, double& r2)
 {
     const double L = log_positive(fabs(x));
     r1 = exp_product(e1, L);
     r2 = exp_product(e2, L);
-    if (!(x > 0.0 && x < HUGE_VAL && e1 != 0.0 && e2 != 0.0 && r1 < HUGE_VAL && r2 < HUGE_VAL)) {
+    if (!(x > 0.0 && x < HUGE_VAL && e1 != 0.0 && e2 != 0.0) || !(TAME || (r1 < HUGE_VAL && r2 < HUGE_VAL))) {
         r1 = pow_special(x, e1, r1);
         r2 = pow_special(x, e2, r2);
     }

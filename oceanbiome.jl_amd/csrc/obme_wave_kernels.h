@@ -415,7 +415,7 @@ __device__ __forceinline__ void column_wave(const WaveArgs<FT>& w, FT* lds)
                 pr[m] = m_exp2(fmaf(a.er, lg, w.cr));
                 pb[m] = m_exp2(fmaf(a.eb, lg, w.cb));
             } else {
-                pow_pair(I[PI][m] * a.Rr, a.er, a.eb, pr[m], pb[m]);
+                pow_pair<true>(I[PI][m] * a.Rr, a.er, a.eb, pr[m], pb[m]);
             }
         }
         // the integral to level j: with c = the half cells either side of the
@@ -804,7 +804,7 @@ __device__ __forceinline__ void top_steps(const WaveArgs<FT>& w, FT* rec)
                 const float h = w.uniform ? 1.0f : (float)dn;   // (a uniform grid's half cell is in cr, cb)
                 PAR = PAR0 * fmaf(wr, m_exp2(-(h * pr)), wb * m_exp2(-(h * pb)));
             } else {
-                pow_pair(X[PI] * a.Rr, a.er, a.eb, pr, pb);
+                pow_pair<true>(X[PI] * a.Rr, a.er, a.eb, pr, pb);
                 PAR = PAR0 * (wr * m_exp(-a.xr * (dn * pr)) + wb * m_exp(-a.xb * (dn * pb)));
             }
             FT Gv[NT], v[NT];
