@@ -202,7 +202,7 @@ struct obme_handle {
     int ntracers;
     int prec;
     std::vector<double> zc, zf, dz, Tprof, Sprof;
-    void* d_lev = nullptr;     // LEV_COUNT * Nz of FT; d_wsink and d_fast lie in its allocation
+    void* d_lev = nullptr;     // LEV_COUNT * Nz of FT; d_wsink, d_fast and d_light lie in its allocation
     void* d_wsink = nullptr;   // MAX_SINK * (Nz+1) of FT
     double* d_Tprof = nullptr;
     double* d_Sprof = nullptr;
@@ -217,6 +217,7 @@ struct obme_handle {
     bool surfc_ready = false;  // d_surfc holds the constants of this call's T and S
     int srec_steps = 1;        // steps of surface records that d_srec holds
     void* d_fast = nullptr;    // FP64: the transitions' constants (FastParams<double>)
+    const double* d_light = nullptr;   // FP32: the levels' chlorophyll attenuations (LIGHT_*)
     void* d_toprec = nullptr;  // the top cells' records of k_top_steps (scaling with the CO2 flux)
     int toprec_steps = 0;      // steps of them that d_toprec holds
     bool default_forms = false;   // the model's default formulations (the FP32 kernels' compiled-in choices)
@@ -379,20 +380,39 @@ static obme_status upload_geometry(obme_handle* h)
         w[(size_t)s * (Nz + 1) + Nz] = (FT)0;
     }
     // one allocation and one copy for the tables: the levels, the drift
-    // velocities and, FP64, the transitions' constants
+    // velocities and, FP64, the transitions' constants, FP32 the levels'
+    // chlorophyll attenuations
     const size_t lev_bytes = lev.size() * sizeof(FT), w_bytes = w.size() * sizeof(FT);
-    const size_t fast_at = (lev_bytes + w_bytes + 15) / 16 * 16;
-    std::vector<char> all(fast_at + (sizeof(FT) == 8 ? sizeof(FastParams<FT>) : 0));
+    const size_t more_at = (lev_bytes + w_bytes + 15) / 16 * 16;
+    std::vector<char> all(more_at + (sizeof(FT) == 8 ? sizeof(FastParams<FT>) : LIGHT_COUNT * (size_t)Nz * sizeof(double)));
     std::memcpy(all.data(), lev.data(), lev_bytes);
     std::memcpy(all.data() + lev_bytes, w.data(), w_bytes);
     if constexpr (sizeof(FT) == 8) {
         const FastParams<FT> f = make_args<FT>(h, nullptr).f;
-        std::memcpy(all.data() + fast_at, &f, sizeof(f));
+        std::memcpy(all.data() + more_at, &f, sizeof(f));
+    } else {
+        double* light = (double*)(all.data() + more_at);
+        const obme_two_band_par& p = h->cfg.par;
+        const double log2e = 1.4426950408889634, lRr = std::log2(p.phytoplankton_chlorophyll_ratio / p.pigment_ratio);
+        auto per_power = [&](double attenuation, double exponent) {
+            const double c = exponent * lRr, lost = c - (float)c;
+            return attenuation * log2e * (std::isfinite(lost) ? std::exp2(lost) : 1.0);
+        };
+        const double x[2] = {per_power(p.chlorophyll_red_attenuation, p.chlorophyll_red_exponent),
+                             per_power(p.chlorophyll_blue_attenuation, p.chlorophyll_blue_exponent)};
+        for (int k = 0; k < Nz; k++) {
+            const double above = h->zf[k + 1] - h->zc[k], below = k > 0 ? h->zc[k] - h->zf[k] : 0.0;
+            for (int q = 0; q < 2; q++) {
+                light[(LIGHT_ABOVE_R + q) * (size_t)Nz + k] = x[q] * above;
+                light[(LIGHT_WHOLE_R + q) * (size_t)Nz + k] = x[q] * (above + below);
+            }
+        }
     }
     HIP_TRY(hipMalloc(&h->d_lev, all.size()));
     HIP_TRY(hipMemcpy(h->d_lev, all.data(), all.size(), hipMemcpyHostToDevice));
     h->d_wsink = (char*)h->d_lev + lev_bytes;
-    if constexpr (sizeof(FT) == 8) h->d_fast = (char*)h->d_lev + fast_at;
+    if constexpr (sizeof(FT) == 8) h->d_fast = (char*)h->d_lev + more_at;
+    else h->d_light = (const double*)((char*)h->d_lev + more_at);
 
     // Uniform-grid fast path: the kernel forms zc = zc[0] + k dz, the half
     // cells dz/2, 1/dz and constant face velocities itself.  Taken only when
@@ -748,11 +768,14 @@ static StepArgs<FT> make_args(const obme_handle* h, void* const* tracers)
         const double log2e = 1.4426950408889634;
         a.kr2 = (float)(c.par.water_red_attenuation * log2e);
         a.kb2 = (float)(c.par.water_blue_attenuation * log2e);
+        a.light = h->d_light;
         a.xr2 = (float)(c.par.chlorophyll_red_attenuation * log2e);
         a.xb2 = (float)(c.par.chlorophyll_blue_attenuation * log2e);
         const double lRr = std::log2(c.par.phytoplankton_chlorophyll_ratio / c.par.pigment_ratio);
         a.cr = (float)(c.par.chlorophyll_red_exponent * lRr);
         a.cb = (float)(c.par.chlorophyll_blue_exponent * lRr);
+        a.erl = (float)(c.par.chlorophyll_red_exponent - (float)c.par.chlorophyll_red_exponent);
+        a.ebl = (float)(c.par.chlorophyll_blue_exponent - (float)c.par.chlorophyll_blue_exponent);
         a.xr2h = (float)(c.par.chlorophyll_red_attenuation * log2e * h->dz_u / 2);
         a.xb2h = (float)(c.par.chlorophyll_blue_attenuation * log2e * h->dz_u / 2);
         a.wi0 = (float)(h->w0_u / h->dz_u);

@@ -172,6 +172,8 @@ struct StepArgs {
     FT invdz_u;                    // uniform grid: 1/Δz
     float rk_a[3], rk_b[3];        // FP32 path: Δt γ and Δt ζ per stage
     float kr2, kb2, xr2, xb2;      // FP32 path: attenuations × log2(e)
+    const double* light;           // FP32 path: [LIGHT_COUNT][Nz], the levels' chlorophyll attenuations
+    float erl, ebl;                // FP32 path: what er and eb lost to rounding
     float cr, cb;                  // FP32 path: e log2(R_chl / r) per band
     float xr2h, xb2h;              // FP32 uniform grid: xr2 dz/2, xb2 dz/2
     float wi0, wi1;                // FP32 uniform grid: w / dz of the two sinking tracers
@@ -228,6 +230,11 @@ enum { LEV_ZC = 0, LEV_UP, LEV_DN, LEV_INVDZ, LEV_WR, LEV_WB, LEV_COUNT };
 // for k = Nz-1: LEV_UP = 0 and LEV_DN = zf[Nz] - zc[Nz-1] (the top half cell).
 // LEV_WR, LEV_WB: half the light left by the water alone at zc, exp(k zc) / 2
 // of the red and blue bands, formed in FP64.
+
+// FP32: the rows of `light`, in powers of 2 per unit of the band's chlorophyll
+// power (and times what the rounding of cr or cb took from the power): the attenuation from the face above a level to its centre, and the
+// whole of its cell's (from its centre up and down; the bottom level: above).
+enum { LIGHT_ABOVE_R = 0, LIGHT_ABOVE_B, LIGHT_WHOLE_R, LIGHT_WHOLE_B, LIGHT_COUNT };
 
 // What a launch does: the fused RK3 step, the tendencies (hook), the PAR (hook;
 // k_light, and the sweep for many columns in FP64), one RK3 stage with its
@@ -971,23 +978,46 @@ struct SurfaceArgs {
     unsigned ncell;
 };
 
+// FP32: the chlorophyll powers of both bands as the light hooks take them, the
+// exponents' rounding errors put back (they would be a bias of the integral).
+template <typename FT>
+__device__ __forceinline__ void chlorophyll_powers(const StepArgs<FT>& a, float P, float& r, float& b)
+{
+    const float lg = m_log2(P), l = __builtin_amdgcn_fmed3f(lg, -200.0f, 200.0f);
+    r = m_exp2(fmaf((float)a.er, lg, fmaf(a.erl, l, a.cr)));
+    b = m_exp2(fmaf((float)a.eb, lg, fmaf(a.ebl, l, a.cb)));
+}
+
 // The light hook: TwoBand PAR (Light/2band.jl:18-32) of P into the parent array.
 // A block takes COLS columns that follow each other, in chunks of up to ROWS x
 // LEVELS levels from the top: a thread works n = ceil(Nz / ROWS) <= LEVELS
 // levels of its column, and the integral above them is the sum of the rows
 // above (PAR = PAR0 (e^(kr zc - χr ∫r) + e^(kb zc - χb ∫b)) / 2).  What bounds it is
 // reading P and writing PAR; one lane per column walked its levels one load
-// after the other (384x384x64 in FP32: 40 us, 1.9 TB/s; this 24).  FP64: what
+// after the other (384x384x64 in FP32: 25.3 us, 3.0 TB/s; this 21.5).  FP64: what
 // bounds it are the powers (260 instructions a level), whose code is too long
 // to unroll (eight levels: 27 us of fetching it on 17x76x58, 8 with a loop);
 // its levels wait in LDS.  Above 65536 columns FP64 takes the sweep, which keeps
 // the powers' constants in registers down the column (500x300x40: 50 us | 60;
 // with the tendencies 256x256x64 221 | 215, 333x187x20 65.6 | 65.1).
+// FP32: the integral is summed in FP64 (which takes as long as FP32 and a
+// conversion) and its exponent rounded once, as the sweep's compensated sums
+// are: largest error on 64 levels of P about 0.1 1.4e-6 (the sweep 1.9e-6; with
+// sums in FP32 3.8e-6), on 400 of P about 3 5.7e-6 (9.3e-6; 3.0e-5).  With them
+// 384x384x64 took 20.1 us, 512x512x30 17.5 (now 18.9).
 template <typename FT>
 struct LightShape {
     static constexpr int COLS = sizeof(FT) == 4 ? 64 : 32;
     static constexpr int ROWS = 8, LEVELS = 8, THREADS = COLS * ROWS;
     static constexpr unsigned MOST_COLUMNS = sizeof(FT) == 4 ? ~0u : 65536u;
+};
+// A level: the thickness from zf(k+1) to zc(k) and the whole level's (FP32:
+// times the band's attenuation, see `light`), the light left by the water
+// alone, of both bands.
+template <typename FT>
+struct alignas(16) LightLevel {
+    double above[sizeof(FT) == 4 ? 2 : 1], whole[sizeof(FT) == 4 ? 2 : 1];
+    FT wr, wb;
 };
 template <typename FT>
 __global__ void __launch_bounds__(LightShape<FT>::THREADS, 4) k_light(StepArgs<FT> a, const FT* P, unsigned ncol)
@@ -995,15 +1025,14 @@ __global__ void __launch_bounds__(LightShape<FT>::THREADS, 4) k_light(StepArgs<F
     constexpr bool F32 = sizeof(FT) == 4;
     constexpr int COLS = LightShape<FT>::COLS, ROWS = LightShape<FT>::ROWS, LEVELS = LightShape<FT>::LEVELS;
     constexpr int UNROLL = F32 ? LEVELS : 1;
-    // a chunk's levels: the thickness from zf(k+1) to zc(k), the whole level's
-    // and the light left by the water alone in both bands
-    struct alignas(4 * sizeof(FT)) Level {
-        FT above, whole, wr, wb;
-    };
+    constexpr int B = F32 ? 1 : 0;      // the blue band's thicknesses
+    using Level = LightLevel<FT>;
     __shared__ Level s_level[ROWS * LEVELS];
-    __shared__ FT s_row[2][ROWS][COLS];
+    __shared__ double s_row[2][ROWS][COLS];
     __shared__ FT s_power[F32 ? 1 : 2][F32 ? 1 : LEVELS][F32 ? 1 : ROWS * COLS];
-    const int c = threadIdx.x % COLS, g = threadIdx.x / COLS;
+    // (FP32: a wave is one row)
+    const int c = threadIdx.x % COLS;
+    const int g = F32 ? __builtin_amdgcn_readfirstlane(threadIdx.x / COLS) : threadIdx.x / COLS;
     const unsigned q = blockIdx.x * COLS + c;
     const bool ok = q < ncol;
     const unsigned base = a.base0 + (ok ? q % (unsigned)a.Nx + a.sx * (q / (unsigned)a.Nx) : 0u);
@@ -1017,7 +1046,7 @@ __global__ void __launch_bounds__(LightShape<FT>::THREADS, 4) k_light(StepArgs<F
         if constexpr (F32) return band ? pb[u] : pr[u];
         else return s_power[band][u][threadIdx.x];
     };
-    FT Cr = FT(0), Cb = FT(0);          // the integrals over the chunks above
+    double Cr = 0.0, Cb = 0.0;          // the integrals over the chunks above
 #pragma unroll 1
     for (int k0 = Nz - 1; k0 >= 0; k0 -= chunk) {
         const int kt = k0 - g * n;
@@ -1028,10 +1057,17 @@ __global__ void __launch_bounds__(LightShape<FT>::THREADS, 4) k_light(StepArgs<F
             if (u < n) x[u] = P[base + a.sxy * (unsigned)max(kt - u, 0)];
         if (threadIdx.x < chunk) {
             const int k = k0 - (int)threadIdx.x;
-            Level v = {FT(0), FT(0), FT(0), FT(0)};
+            Level v = {};
             if (k >= 0) {
-                v.above = a.lev[LEV_DN * Nz + k];
-                v.whole = v.above + (k > 0 ? a.lev[LEV_UP * Nz + k - 1] : FT(0));
+                if constexpr (F32) {
+                    v.above[0] = a.light[LIGHT_ABOVE_R * Nz + k];
+                    v.above[B] = a.light[LIGHT_ABOVE_B * Nz + k];
+                    v.whole[0] = a.light[LIGHT_WHOLE_R * Nz + k];
+                    v.whole[B] = a.light[LIGHT_WHOLE_B * Nz + k];
+                } else {
+                    v.above[0] = a.lev[LEV_DN * Nz + k];
+                    v.whole[0] = v.above[0] + (k > 0 ? a.lev[LEV_UP * Nz + k - 1] : FT(0));
+                }
                 v.wr = a.lev[LEV_WR * Nz + k];
                 v.wb = a.lev[LEV_WB * Nz + k];
             }
@@ -1041,52 +1077,54 @@ __global__ void __launch_bounds__(LightShape<FT>::THREADS, 4) k_light(StepArgs<F
         for (int u = 0; u < LEVELS; u++)
             if (u < n) power(0, u) = x[u];
         __syncthreads();
-        FT Sr = FT(0), Sb = FT(0);
+        double Sr = 0.0, Sb = 0.0;
 #pragma unroll UNROLL
         for (int u = 0; u < LEVELS; u++) {
             if (u >= n) break;
             const FT p = power(0, u);
             FT r, b;
             if constexpr (F32) {
-                const float lg = m_log2(p);
-                r = m_exp2(fmaf(a.er, lg, a.cr));
-                b = m_exp2(fmaf(a.eb, lg, a.cb));
+                chlorophyll_powers(a, p, r, b);
             } else {
                 pow_pair(p * a.Rr, a.er, a.eb, r, b);
             }
             power(0, u) = r;
             power(1, u) = b;
-            const FT w = s_level[g * n + u].whole;
-            Sr = fma(w, r, Sr);
-            Sb = fma(w, b, Sb);
+            const Level& v = s_level[g * n + u];
+            Sr = fma(v.whole[0], (double)r, Sr);
+            Sb = fma(v.whole[B], (double)b, Sb);
         }
         s_row[0][g][c] = Sr;
         s_row[1][g][c] = Sb;
         __syncthreads();
-        FT Ir = Cr, Ib = Cb;
+        double Ir = Cr, Ib = Cb;
 #pragma unroll
-        for (int m = 0; m < ROWS; m++) {
-            const FT sr = s_row[0][m][c], sb = s_row[1][m][c];
+        for (int m = 0; m < ROWS - 1; m++) {
             if (m < g) {
-                Ir += sr;
-                Ib += sb;
+                Ir += s_row[0][m][c];
+                Ib += s_row[1][m][c];
             }
-            Cr += sr;
-            Cb += sb;
+        }
+        if (k0 >= chunk) {
+#pragma unroll
+            for (int m = 0; m < ROWS; m++) {
+                Cr += s_row[0][m][c];
+                Cb += s_row[1][m][c];
+            }
         }
 #pragma unroll UNROLL
         for (int u = 0; u < LEVELS; u++) {
             if (u >= n) break;
             const Level v = s_level[g * n + u];
             const FT r = power(0, u), b = power(1, u);
-            const FT Jr = fma(v.above, r, Ir), Jb = fma(v.above, b, Ib);
+            const FT Jr = (FT)fma(v.above[0], (double)r, Ir), Jb = (FT)fma(v.above[B], (double)b, Ib);
             FT PAR;
-            if constexpr (F32) PAR = PAR0 * fmaf(v.wr, m_exp2(-a.xr2 * Jr), v.wb * m_exp2(-a.xb2 * Jb));
+            if constexpr (F32) PAR = PAR0 * fmaf(v.wr, m_exp2(-Jr), v.wb * m_exp2(-Jb));
             else PAR = PAR0 * (v.wr * m_exp(-a.xr * Jr) + v.wb * m_exp(-a.xb * Jb));
             const unsigned off = (base + a.sxy * (unsigned)max(kt - u, 0)) * (unsigned)sizeof(FT);
             buf_store(out, ok && u <= kt ? off : a.field_bytes, PAR);
-            Ir = fma(v.whole, r, Ir);
-            Ib = fma(v.whole, b, Ib);
+            Ir = fma(v.whole[0], (double)r, Ir);
+            Ib = fma(v.whole[B], (double)b, Ib);
         }
         if (k0 >= chunk) __syncthreads();
     }

@@ -405,52 +405,80 @@ __device__ __forceinline__ void column_wave(const WaveArgs<FT>& w, FT* lds)
         }
 
         // ---- TwoBand PAR (Light/2band.jl:18-32)
-        FT pr[L], pb[L];
+        if constexpr (F32 && !STEP) {
+            // the hook's PAR is a result: its sums go in FP64, as in k_light, and
+            // the attenuations stay out of the powers' constants (64 levels of P
+            // about 0.1: rms error 3.8e-7, summed as the step's 1.2e-6; a step's
+            // tracers are no nearer the FP64 ones for it)
+            FT pr[L], pb[L];
+            double above[2][L], whole[2][L], Ir = 0.0, Ib = 0.0;
 #pragma unroll
-        for (int m = 0; m < L; m++) {
-            if constexpr (F32) {
-                // the attenuation (and, on a uniform grid, the half cell) is
-                // part of the power's constant
-                const float lg = m_log2(I[PI][m]);
-                pr[m] = m_exp2(fmaf(a.er, lg, w.cr));
-                pb[m] = m_exp2(fmaf(a.eb, lg, w.cb));
-            } else {
-                pow_pair<true>(I[PI][m] * a.Rr, a.er, a.eb, pr[m], pb[m]);
+            for (int m = 0; m < L; m++) {
+                chlorophyll_powers(a, I[PI][m], pr[m], pb[m]);
+                above[0][m] = a.light[LIGHT_ABOVE_R * Nz + lk[m]];
+                above[1][m] = a.light[LIGHT_ABOVE_B * Nz + lk[m]];
+                whole[0][m] = a.light[LIGHT_WHOLE_R * Nz + lk[m]];
+                whole[1][m] = a.light[LIGHT_WHOLE_B * Nz + lk[m]];
+                Ir = fma(whole[0][m], (double)pr[m], Ir);
+                Ib = fma(whole[1][m], (double)pb[m], Ib);
             }
-        }
-        // the integral to level j: with c = the half cells either side of the
-        // levels above, Σ c p over them, plus the half cell down to j (uniform:
-        // in half cells, 2 Σ p + p_j); one level per lane takes it from the
-        // inclusive sum
-        FT totr = FT(0), totb = FT(0);
+            Ir = lane_above<SEG>(column_prefix<SEG>(Ir, cm), cm);
+            Ib = lane_above<SEG>(column_prefix<SEG>(Ib, cm), cm);
 #pragma unroll
-        for (int m = 0; m < L; m++) {
-            const FT cr_ = UNI ? pr[m] : cw[m] * pr[m], cb_ = UNI ? pb[m] : cw[m] * pb[m];
-            totr = m == 0 ? cr_ : totr + cr_;
-            totb = m == 0 ? cb_ : totb + cb_;
-        }
-        FT runr = column_prefix<SEG>(totr, cm), runb = column_prefix<SEG>(totb, cm);
-        if constexpr (L > 1) {
-            runr = lane_above<SEG>(runr, cm);
-            runb = lane_above<SEG>(runb, cm);
-        }
-#pragma unroll
-        for (int m = 0; m < L; m++) {
-            FT Ir, Ib;
-            if constexpr (L == 1) {
-                Ir = UNI ? fma(FT(2), runr, -pr[0]) : fma(dn[0] - cw[0], pr[0], runr);
-                Ib = UNI ? fma(FT(2), runb, -pb[0]) : fma(dn[0] - cw[0], pb[0], runb);
-            } else {
-                Ir = UNI ? fma(FT(2), runr, pr[m]) : fma(dn[m], pr[m], runr);
-                Ib = UNI ? fma(FT(2), runb, pb[m]) : fma(dn[m], pb[m], runb);
-                runr = UNI ? runr + pr[m] : fma(cw[m], pr[m], runr);
-                runb = UNI ? runb + pb[m] : fma(cw[m], pb[m], runb);
+            for (int m = 0; m < L; m++) {
+                const float Jr = (float)fma(above[0][m], (double)pr[m], Ir), Jb = (float)fma(above[1][m], (double)pb[m], Ib);
+                PARv[m] = PAR0 * fmaf(wr[m], m_exp2(-Jr), wb[m] * m_exp2(-Jb));
+                Ir = fma(whole[0][m], (double)pr[m], Ir);
+                Ib = fma(whole[1][m], (double)pb[m], Ib);
             }
-            if constexpr (F32) {
-                PARv[m] = PAR0 * fmaf(wr[m], m_exp2(-Ir), wb[m] * m_exp2(-Ib));
-            } else {
-                const FT h = UNI ? a.dz_u * FT(0.5) : FT(1);
-                PARv[m] = PAR0 * (wr[m] * m_exp(-(a.xr * h) * Ir) + wb[m] * m_exp(-(a.xb * h) * Ib));
+        } else {
+            FT pr[L], pb[L];
+#pragma unroll
+            for (int m = 0; m < L; m++) {
+                if constexpr (F32) {
+                    // the attenuation (and, on a uniform grid, the half cell) is
+                    // part of the power's constant
+                    const float lg = m_log2(I[PI][m]);
+                    pr[m] = m_exp2(fmaf(a.er, lg, w.cr));
+                    pb[m] = m_exp2(fmaf(a.eb, lg, w.cb));
+                } else {
+                    pow_pair<true>(I[PI][m] * a.Rr, a.er, a.eb, pr[m], pb[m]);
+                }
+            }
+            // the integral to level j: with c = the half cells either side of the
+            // levels above, Σ c p over them, plus the half cell down to j (uniform:
+            // in half cells, 2 Σ p + p_j); one level per lane takes it from the
+            // inclusive sum
+            FT totr = FT(0), totb = FT(0);
+#pragma unroll
+            for (int m = 0; m < L; m++) {
+                const FT cr_ = UNI ? pr[m] : cw[m] * pr[m], cb_ = UNI ? pb[m] : cw[m] * pb[m];
+                totr = m == 0 ? cr_ : totr + cr_;
+                totb = m == 0 ? cb_ : totb + cb_;
+            }
+            FT runr = column_prefix<SEG>(totr, cm), runb = column_prefix<SEG>(totb, cm);
+            if constexpr (L > 1) {
+                runr = lane_above<SEG>(runr, cm);
+                runb = lane_above<SEG>(runb, cm);
+            }
+#pragma unroll
+            for (int m = 0; m < L; m++) {
+                FT Ir, Ib;
+                if constexpr (L == 1) {
+                    Ir = UNI ? fma(FT(2), runr, -pr[0]) : fma(dn[0] - cw[0], pr[0], runr);
+                    Ib = UNI ? fma(FT(2), runb, -pb[0]) : fma(dn[0] - cw[0], pb[0], runb);
+                } else {
+                    Ir = UNI ? fma(FT(2), runr, pr[m]) : fma(dn[m], pr[m], runr);
+                    Ib = UNI ? fma(FT(2), runb, pb[m]) : fma(dn[m], pb[m], runb);
+                    runr = UNI ? runr + pr[m] : fma(cw[m], pr[m], runr);
+                    runb = UNI ? runb + pb[m] : fma(cw[m], pb[m], runb);
+                }
+                if constexpr (F32) {
+                    PARv[m] = PAR0 * fmaf(wr[m], m_exp2(-Ir), wb[m] * m_exp2(-Ib));
+                } else {
+                    const FT h = UNI ? a.dz_u * FT(0.5) : FT(1);
+                    PARv[m] = PAR0 * (wr[m] * m_exp(-(a.xr * h) * Ir) + wb[m] * m_exp(-(a.xb * h) * Ib));
+                }
             }
         }
 
