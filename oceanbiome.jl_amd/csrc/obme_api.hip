@@ -1116,6 +1116,7 @@ static obme_status run_typed(obme_handle* h, void* const* tracers, void* const* 
         std::memset(&w, 0, sizeof(w));
         w.a = a;
         wave_light<FT>(h, false, w);
+        w.uniform = h->uniform && !h->staged;
         w.nsteps = 1;
         w.scheme = h->scheme;
         w.PAR0s[0][0] = a.surface_mode == OBME_SURFACE_DIURNAL ? a.PAR0_stage[0] : a.surface_value;

@@ -58,7 +58,7 @@ struct WaveArgs {
     // (in powers of 2), on a uniform grid times Δz / 2
     float cr, cb;
     const FastParams<FT>* fpar;         // FP64: the transitions' constants in device memory
-    int uniform;                        // uniform grid, constant sinking speeds (k_top_steps)
+    int uniform;                        // uniform grid, constant sinking speeds (k_top_steps, the hook)
     int scale;                          // negative scaling at the start of every stage
     int sed;                            // InstantRemineralisation sediment under the column
     int scheme;                         // the sinking face value
@@ -581,6 +581,12 @@ __device__ __forceinline__ void column_wave(const WaveArgs<FT>& w, FT* lds)
             if constexpr (F32 && UNI && !WIN) {
                 Gv[S0] = fmaf(-a.wi0, fxu[0][m] - fx[0][m], Gv[S0]);
                 Gv[S1] = fmaf(-a.wi1, fxu[1][m] - fx[1][m], Gv[S1]);
+            } else if (F32 && !STEP && !WIN && w.uniform) {
+                // (the hook has one kernel for every grid: with constant speeds
+                // the difference first, which the flux of either face would
+                // round away)
+                Gv[S0] = fma((FT)-a.wi0, fxu[0][m] - fx[0][m], Gv[S0]);
+                Gv[S1] = fma((FT)-a.wi1, fxu[1][m] - fx[1][m], Gv[S1]);
             } else {
                 // (no flux through the surface)
                 const FT h0 = (top && m == 0) ? FT(0) : whi[m][0] * fxu[0][m];
