@@ -1163,7 +1163,11 @@ static obme_status run_wave_steps(obme_handle* h, const WaveShape& ws, void* con
     a.T3 = (const FT*)T;
     a.S3 = (const FT*)S;
     a.topres = (a.co2_on && h->carry_top) ? h->d_topres : nullptr;
-    w.scale = h->scaling;
+    // (FP64: with a factor below 0 the sum can be negative where no member is)
+    w.scale = h->scaling ? 1 : 0;
+    for (int g = 0; g < h->cfg.scaling.n_groups; g++)
+        for (int m = 0; m < h->cfg.scaling.n_members[g]; m++)
+            if (!(h->cfg.scaling.scalefactor[g][m] >= 0)) w.scale = 2;
     w.sed = h->sediment;
     w.scheme = h->scheme;
     const bool general = h->scaling || h->sediment;

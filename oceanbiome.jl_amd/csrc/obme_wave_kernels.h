@@ -59,7 +59,7 @@ struct WaveArgs {
     float cr, cb;
     const FastParams<FT>* fpar;         // FP64: the transitions' constants in device memory
     int uniform;                        // uniform grid, constant sinking speeds (k_top_steps, the hook)
-    int scale;                          // negative scaling at the start of every stage
+    int scale;                          // negative scaling at the start of every stage (2: of every cell)
     int sed;                            // InstantRemineralisation sediment under the column
     int scheme;                         // the sinking face value
     // the top cell is stepped by k_top_steps (scaling with the CO2 flux): its
@@ -375,7 +375,7 @@ __device__ __forceinline__ void column_wave(const WaveArgs<FT>& w, FT* lds)
 #pragma unroll
                 for (int m = 0; m < L; m++) {
                     FT x[NT];
-                    bool need = false;
+                    bool need = !F32 && w.scale == 2;
 #pragma unroll
                     for (int n = 0; n < NT; n++) {
                         x[n] = I[n][m];
@@ -807,7 +807,7 @@ __device__ __forceinline__ void top_steps(const WaveArgs<FT>& w, FT* rec)
 #pragma unroll 1
         for (int st = 0; st < 3; st++) {
             FT PAR0 = a.surface_mode == OBME_SURFACE_ARRAY ? a.surf[q] : w.PAR0s[sn][st];
-            bool need = false;
+            bool need = !F32 && w.scale == 2;
             FT x[NT];
 #pragma unroll
             for (int n = 0; n < NT; n++) {
