@@ -242,6 +242,38 @@ enum { LIGHT_ABOVE_R = 0, LIGHT_ABOVE_B, LIGHT_WHOLE_R, LIGHT_WHOLE_B, LIGHT_COU
 // below).
 enum { TILE_STEP = 0, TILE_TENDENCY = 1, TILE_PAR = 2, TILE_STAGE = 3 };
 
+// The InstantRemineralisation sediment's arithmetic, the same in every kernel of
+// the fused step: its storage is an FP64 sum, in which a last bit of the FP32
+// flux that rounds the other way is far above the rounding of the sum itself.
+// So the fused products are spelled out.  The flux through the bottom face,
+// f = Σ -w c of the two sinking tracers: the one of them whose product is not
+// rounded by itself (FP32; a handle's configuration decides, so that its storage
+// is the same to the bit from whichever kernel serves a call).
+template <int CARB>
+__device__ __forceinline__ constexpr bool sediment_second(bool scaling, int stage)
+{
+    return stage > 0 && ((CARB & 1) != 0) != scaling;
+}
+template <typename FT>
+__device__ __forceinline__ FT sediment_flux(const StepArgs<FT>& a, FT x0, FT x1, bool second)
+{
+    return second ? fma(a.sed_w1, x1, a.sed_w0 * x0) : fma(a.sed_w0, x0, a.sed_w1 * x1);
+}
+// The burial efficiency e = a + b (f / (k + f))^2.
+template <typename FT>
+__device__ __forceinline__ FT sediment_burial(const StepArgs<FT>& a, FT f)
+{
+    const FT qf = f / (a.sed_k + f);
+    return fma(a.sed_b, qf * qf, a.sed_a);
+}
+// The storage u after a sediment step of stage st's Δt with the tendency ge (ab2:
+// χ-weighted with the previous one).
+template <typename FT>
+__device__ __forceinline__ double sediment_step(const StepArgs<FT>& a, int st, double u, double ge, int ab2, double gm)
+{
+    return fma(a.sed_dt[st], ab2 ? fma(a.sed_cn, ge, -(a.sed_cm * gm)) : ge, u);
+}
+
 // The value at face k of a sinking tracer reconstructed from above (w <= 0:
 // the upwind cell is k): fifth-order WENO from the cells k-2 .. k+2, third
 // order from k-1 .. k+1, with WENO-Z weights (Borges et al. 2008) on the
@@ -752,9 +784,9 @@ __device__ __forceinline__ void column_lane(const StepArgs<FT>& a, const int cw)
                         sed_ge[q] = G[q];
                     }
                 } else if (bot) {
-                    const FT f = a.sed_w0 * X[S0] + a.sed_w1 * X[S1];
-                    const FT qf = f / (a.sed_k + f);
-                    const FT e = a.sed_a + a.sed_b * (qf * qf);
+                    const bool second = F32 && sediment_second<CARB>((EXTRA & 1) != 0, st);
+                    const FT f = sediment_flux(a, X[S0], X[S1], second);
+                    const FT e = sediment_burial(a, f);
                     const FT cpl = ((FT(1) - e) * f) / a.sed_dz0;
 #pragma unroll
                     for (int n = 0; n < NT; n++)
@@ -767,11 +799,10 @@ __device__ __forceinline__ void column_lane(const StepArgs<FT>& a, const int cw)
                     // second stage start serves both.
                     const double ge = (double)(e * f);
                     if (st == 0) {
-                        if (!a.sed_init)
-                            sed_u[0] += a.sed_dt[0] * (a.sed_ab2 ? a.sed_cn * ge - a.sed_cm * sed_gm[0] : ge);
+                        if (!a.sed_init) sed_u[0] = sediment_step(a, 0, sed_u[0], ge, a.sed_ab2, sed_gm[0]);
                     } else {
-                        if (st == 1 && a.sed_init) sed_u[0] += a.sed_dt[0] * ge;
-                        sed_u[0] += a.sed_dt[st] * ge;
+                        if (st == 1 && a.sed_init) sed_u[0] = sediment_step(a, 0, sed_u[0], ge, 0, 0.0);
+                        sed_u[0] = sediment_step(a, st, sed_u[0], ge, 0, 0.0);
                     }
                     sed_ge[0] = ge;
                 }
@@ -877,7 +908,7 @@ __device__ __forceinline__ void column_lane(const StepArgs<FT>& a, const int cw)
                 if (bot && col_ok) {
                     const FT x0 = F32 ? U[S0] + D[F32 ? S0 : 0] : U[S0];
                     const FT x1 = F32 ? U[S1] + D[F32 ? S1 : 0] : U[S1];
-                    const FT f = a.sed_w0 * x0 + a.sed_w1 * x1;
+                    const FT f = sediment_flux(a, x0, x1, false);
                     if (a.sed_model == OBME_SEDIMENT_SIMPLE_MULTI_G) {
                         double G[3];
                         smg_tendencies(a.smg, sed_u, (double)f, G);
@@ -888,10 +919,8 @@ __device__ __forceinline__ void column_lane(const StepArgs<FT>& a, const int cw)
                             a.sedG[(3 + q) * ncol2d + col2d] = sed_ge[q];
                         }
                     } else {
-                        const FT qf = f / (a.sed_k + f);
-                        const FT e = a.sed_a + a.sed_b * (qf * qf);
                         if (a.storage) a.storage[col2d] = sed_u[0];
-                        a.sedG[col2d] = (double)(e * f);
+                        a.sedG[col2d] = (double)(sediment_burial(a, f) * f);
                         a.sedG[ncol2d + col2d] = sed_ge[0];
                     }
                 }

@@ -536,22 +536,17 @@ __device__ __forceinline__ void column_wave(const WaveArgs<FT>& w, FT* lds)
                         x0 = I[S0][m];
                         x1 = I[S1][m];
                     }
-                // (FP32: the product that the fused sum leaves unrounded is the
-                // one the sweep's compiled stages take, so that the FP64
-                // storage is the same to the bit from either kernel)
-                const bool second = F32 && st > 0 && ((CARB & 1) != 0) != (w.scale != 0);
-                const FT f = second ? fma(a.sed_w1, x1, a.sed_w0 * x0) : fma(a.sed_w0, x0, a.sed_w1 * x1);
-                const FT qf = f / (a.sed_k + f);
-                const FT e = fma(a.sed_b, qf * qf, a.sed_a);
+                const bool second = F32 && sediment_second<CARB>(w.scale != 0, st);
+                const FT f = sediment_flux(a, x0, x1, second);
+                const FT e = sediment_burial(a, f);
                 cpl = ((FT(1) - e) * f) / a.sed_dz0;
                 const double ge = (double)(e * f);
                 const bool init = a.sed_init && sn == 0;
                 if (st == 0) {
-                    if (!init)
-                        sed_u += a.sed_dt[0] * ((a.sed_ab2 && sn == 0) ? a.sed_cn * ge - a.sed_cm * sed_gm : ge);
+                    if (!init) sed_u = sediment_step(a, 0, sed_u, ge, a.sed_ab2 && sn == 0, sed_gm);
                 } else {
-                    if (st == 1 && init) sed_u += a.sed_dt[0] * ge;
-                    sed_u += a.sed_dt[st] * ge;
+                    if (st == 1 && init) sed_u = sediment_step(a, 0, sed_u, ge, 0, 0.0);
+                    sed_u = sediment_step(a, st, sed_u, ge, 0, 0.0);
                 }
                 sed_ge = ge;
             }
@@ -708,11 +703,9 @@ __device__ __forceinline__ void column_wave(const WaveArgs<FT>& w, FT* lds)
                         x0 = U[S0][m];
                         x1 = U[S1][m];
                     }
-                const FT f = fma(a.sed_w0, x0, a.sed_w1 * x1);
-                const FT qf = f / (a.sed_k + f);
-                const FT e = fma(a.sed_b, qf * qf, a.sed_a);
+                const FT f = sediment_flux(a, x0, x1, false);
                 if (a.storage) a.storage[qc] = sed_u;
-                a.sedG[qc] = (double)(e * f);
+                a.sedG[qc] = (double)(sediment_burial(a, f) * f);
                 a.sedG[w.ncol + qc] = sed_ge;
             }
         }
