@@ -862,6 +862,17 @@ struct WaveShape {
     int levels = 0, lpc = 0, cpw = 0, nw = 0;
 };
 
+// The steps of a launch of run_wave_steps, of a call of nsteps: as many as the
+// handle has records for.
+static int launch_steps(const obme_handle* h, int nsteps)
+{
+    int n = std::min(nsteps, WAVE_MAX_STEPS);
+    const bool co2 = h->cfg.model == OBME_LOBSTER && h->cfg.carbonate_system && h->cfg.co2.enabled;
+    if (co2) n = std::min(n, h->co2_inline ? h->toprec_steps : h->srec_steps);
+    return n;
+}
+
+// nsteps: of a launch
 template <typename FT>
 static WaveShape wave_shape(const obme_handle* h, int mode, int nsteps, bool general)
 {
@@ -887,8 +898,8 @@ static WaveShape wave_shape(const obme_handle* h, int mode, int nsteps, bool gen
     // step, sweep | this: FP32 16 384 columns 59 | 26, 65 536 64 | 81; FP64
     // 180 | 65, 197 | 247; FP32 hooks 57 | 35, 110 | 158; FP64 hooks on 38 400
     // 222 | 238.  The hooks of the centred and WENO schemes cross later (on
-    // 38 400 columns FP32 154 | 65, FP64 275 | 134).  From two steps on, with
-    // the state in registers between them, this is the faster everywhere
+    // 38 400 columns FP32 154 | 65, FP64 275 | 134).  From two steps of a launch
+    // on, with the state in registers between them, this is the faster everywhere
     // (262 144 columns, two steps: 507 | 486).  The centred and WENO steps and
     // the scaling and sediment variants are: a launch per stage and the flux
     // solve in the walk are what they replace.
@@ -1178,9 +1189,7 @@ static obme_status run_wave_steps(obme_handle* h, const WaveShape& ws, void* con
         obme_status r = prepare_o2<FT>(h, a, s);
         if (r != OBME_OK) return r;
     }
-    int chunk = WAVE_MAX_STEPS;
-    if (a.co2_on) chunk = std::min(chunk, h->srec_steps);
-    if (h->co2_inline) chunk = std::min(chunk, h->toprec_steps);
+    const int chunk = launch_steps(h, nsteps);
     for (int s0 = 0; s0 < nsteps; s0 += chunk) {
         w.nsteps = std::min(chunk, nsteps - s0);
         for (int q = 0; q < w.nsteps; q++)
@@ -1321,9 +1330,10 @@ extern "C" obme_status obme_step_with_sediment(obme_handle* h, void* const* trac
     {
         const bool general = h->scaling || h->sediment;
         const bool f64 = h->prec == OBME_FP64;
-        const WaveShape ws = f64 ? wave_shape<double>(h, TILE_STEP, nsteps, general)
-                                 : wave_shape<float>(h, TILE_STEP, nsteps, general);
-        if (ws.levels && nsteps > 0 && (!h->co2_inline || h->toprec_steps > 0)) {
+        const int steps = launch_steps(h, nsteps);
+        const WaveShape ws = f64 ? wave_shape<double>(h, TILE_STEP, steps, general)
+                                 : wave_shape<float>(h, TILE_STEP, steps, general);
+        if (ws.levels && steps > 0) {
             r = f64 ? run_wave_steps<double>(h, ws, tracers, T, S, storage, nsteps, t0, dt, s)
                     : run_wave_steps<float>(h, ws, tracers, T, S, storage, nsteps, t0, dt, s);
             h->surfc_ready = false;
