@@ -367,7 +367,10 @@ int32_t obme_sweep_waves(const obme_handle* h);
 /* No counterpart in the reference: the sweep's autotuner.  Times obme_step
  * (one warm-up step, then trial_steps steps, best of two rounds) with every
  * launch shape on a scratch copy of `tracers`, which are only read (T and S
- * as in obme_step), and keeps the fastest.  The handle's carried state (the
+ * as in obme_step), and keeps the fastest.  The trials run the sweep, one
+ * launch per step, whatever kernel obme_step itself would take: the shape
+ * serves the calls that reach the sweep (one step of a large grid, the
+ * tendency hook of one).  The handle's carried state (the
  * sediment stepper's history, the [H+] warm starts, the kernel-timing
  * records) is left as it was.  Allocates the scratch copy; synchronises the
  * stream. */

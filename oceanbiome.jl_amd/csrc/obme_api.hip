@@ -223,6 +223,7 @@ struct obme_handle {
     bool default_forms = false;   // the model's default formulations (the FP32 kernels' compiled-in choices)
     int sink_idx[MAX_SINK];
     int sweep_waves;           // waves per workgroup of the sweep (1, 2, 4 or 8)
+    bool sweep_only = false;   // obme_autotune's trials: every step by the sweep
     bool uniform;
     bool scaling;              // ScaleNegativeTracers groups configured
     bool co2_inline;           // scaling with the CO2 flux: the flux is computed in the sweep
@@ -879,7 +880,7 @@ static WaveShape wave_shape(const obme_handle* h, int mode, int nsteps, bool gen
     WaveShape best;
     const int Nz = h->cfg.grid.Nz;
     const long ncol = (long)h->cfg.grid.Nx * h->cfg.grid.Ny;
-    if (Nz < 2 || !h->default_forms) return best;
+    if (Nz < 2 || !h->default_forms || h->sweep_only) return best;
     // (FP32 takes the logarithm of the chlorophyll attenuation)
     const obme_two_band_par& par = h->cfg.par;
     if (sizeof(FT) == 4 && !(par.chlorophyll_red_attenuation >= 0 && par.chlorophyll_blue_attenuation >= 0)) return best;
@@ -1506,7 +1507,9 @@ extern "C" obme_status obme_sweep_configure(obme_handle* h, int32_t waves)
 extern "C" int32_t obme_sweep_waves(const obme_handle* h) { return h ? h->sweep_waves : -1; }
 
 // Times obme_step with every launch shape on a scratch copy of the state and
-// keeps the fastest.  The buffers a step carries forward in the handle (the
+// keeps the fastest.  Every trial step is the sweep's, also where obme_step
+// would take a kernel that has no such shape: the shape serves the calls that
+// do reach the sweep.  The buffers a step carries forward in the handle (the
 // sediment stepper's G, the [H+] warm starts) are swapped for scratch ones
 // during the trials, so the next real step sees them as they were.
 extern "C" obme_status obme_autotune(obme_handle* h, void* const* tracers, const void* T, const void* S,
@@ -1540,12 +1543,14 @@ extern "C" obme_status obme_autotune(obme_handle* h, void* const* tracers, const
             h->sed_last_dt = sed_last_dt;
             h->timing = timing;
             h->sweep_waves = waves;
+            h->sweep_only = false;
             for (void* p : owned) (void)hipFree(p);
             if (e0) (void)hipEventDestroy(e0);
             if (e1) (void)hipEventDestroy(e1);
         }
     } keep{h, h->d_Hprev, h->d_sedG, h->sed_iter, h->sed_last_dt, h->timing, h->sweep_waves, {}};
     h->timing = false;
+    h->sweep_only = true;
     auto alloc = [&](size_t b, void** p) -> bool {
         if (hipMalloc(p, b) != hipSuccess) return false;
         keep.owned.push_back(*p);
