@@ -502,14 +502,16 @@ obme_status obme_batch_step(obme_batch* b, void* const* tracers, int32_t nsteps,
  * leaves the storage alone, as obme_step does. */
 obme_status obme_batch_step_with_sediment(obme_batch* b, void* const* tracers, double* storage, int32_t nsteps,
                                           double dt, double t0, void* stream);
-/* Column packing: plan = index of a set of tile shapes (columns go to the
- * smallest tile that holds them), steps_per_launch as above. */
+/* Column packing: plan = 0 .. 6, how many levels a lane of a wave holds by the
+ * depth of the column, steps_per_launch as above. */
 obme_status obme_batch_configure(obme_batch* b, int32_t plan, int32_t steps_per_launch);
-/* Times every packing plan and steps-per-launch choice for trial_steps steps
- * on a scratch copy of `tracers` (left unchanged) and keeps the fastest. */
+/* Times every packing plan that packs the ensemble in its own way, with every
+ * steps-per-launch choice, for trial_steps steps on a scratch copy of
+ * `tracers` (left unchanged) and keeps the fastest. */
 obme_status obme_batch_autotune(obme_batch* b, void* const* tracers, int32_t trial_steps, double dt,
                                 void* stream);
-/* Text description of the current packing; returns its length or < 0. */
+/* Text description of the current packing, launch by launch; returns its
+ * length or < 0. */
 int32_t obme_batch_describe(const obme_batch* b, char* buf, int32_t cap);
 
 

@@ -1698,18 +1698,33 @@ __global__ void __launch_bounds__(RAGGED_WAVES * 64, L == 2 ? 5 : 1) k_batch_row
     batch_ragged_sediment<L, FM, true>(a);
 }
 
-// Tile shapes of the ensemble kernel: capacity L*64/CPW levels per column.
-struct BatchTile {
-    int L, CPW, NW;
+// Depth classes of the ensemble: the levels per lane of columns of up to
+// `capacity` levels.
+struct BatchClass {
+    int L, capacity;
 };
-static const BatchTile BATCH_TILES[] = {
-    {1, 4, 4}, {2, 4, 4}, {1, 2, 4}, {2, 2, 4}, {1, 1, 4}, {2, 1, 4}, {4, 2, 4}, {4, 4, 4},
+static const BatchClass BATCH_CLASSES[] = {
+    {1, 16}, {2, 32}, {1, 32}, {2, 64}, {1, 64}, {2, 128}, {4, 128}, {4, 64},
 };
-static int batch_capacity(int t) { return BATCH_TILES[t].L * 64 / BATCH_TILES[t].CPW; }
-// Packing plans: the tile shapes a plan sorts columns into, by capacity.
+// Packing plans: the classes a plan sorts columns into.  (The packing itself
+// goes by levels per lane, so plans 0, 1 and 2 are the same, and 4 and 6.)
 static const std::vector<std::vector<int>> BATCH_PLANS = {
     {5}, {3, 5}, {1, 3, 5}, {0, 1, 3, 5}, {2, 4, 5}, {7, 6}, {0, 2, 4, 5},
 };
+// The levels per lane of a column of nz levels in plan p: of the smallest class
+// that holds it; 0: none does.
+static int plan_levels(int p, int nz)
+{
+    int best = 0, capacity = INT_MAX;
+    for (int q : BATCH_PLANS[p]) {
+        const BatchClass& c = BATCH_CLASSES[q];
+        if (nz <= c.capacity && c.capacity < capacity) {
+            capacity = c.capacity;
+            best = c.L;
+        }
+    }
+    return best;
+}
 
 struct obme_batch {
     obme_config cfg;
@@ -1723,13 +1738,12 @@ struct obme_batch {
     BatchColumn* d_bcol = nullptr;
     float* d_comp = nullptr;              // FP32: the residual arrays, 4 x offsets[n_columns]
     int plan = -1;
-    int steps_per_launch = 0;             // 0: every step of a call in one launch per class
-    std::vector<int> class_tile, class_n; // per class of the plan
+    int steps_per_launch = 0;             // 0: every step of a call in one launch (per levels per lane)
     // the ragged packing: per levels per lane
-    // of the plan's classes, the lanes' table and its waves
+    // of the plan's classes, its columns, the lanes' table and its waves
     bool default_forms = false;
     std::vector<int*> group_lanes;
-    std::vector<int> group_L, group_waves, group_rows;
+    std::vector<int> group_L, group_n, group_waves, group_rows;
     // captured multi-launch step
     hipStream_t cap_stream = nullptr;
     hipGraphExec_t graph = nullptr;
@@ -1749,12 +1763,11 @@ struct obme_batch {
 
 static void batch_free_classes(obme_batch* b)
 {
-    b->class_tile.clear();
-    b->class_n.clear();
     for (int* p : b->group_lanes)
         if (p) (void)hipFree(p);
     b->group_lanes.clear();
     b->group_L.clear();
+    b->group_n.clear();
     b->group_waves.clear();
     b->group_rows.clear();
 }
@@ -1800,28 +1813,20 @@ static void batch_drop_graph(obme_batch* b)
     b->g_nsteps = -1;
 }
 
-// Sorts the columns into the classes of plan p (smallest capacity that holds
-// the column) and packs them by levels per lane.
+// Packs the columns by the levels per lane that plan p gives them.
 static obme_status batch_apply_plan(obme_batch* b, int p)
 {
     if (p < 0 || p >= (int)BATCH_PLANS.size()) return fail(OBME_ERR_INVALID, "unknown packing plan");
-    std::vector<int> tiles = BATCH_PLANS[p];
-    std::sort(tiles.begin(), tiles.end(), [](int x, int y) { return batch_capacity(x) < batch_capacity(y); });
-    std::vector<std::vector<int>> lists(tiles.size());
+    std::vector<int> lists[5];      // by levels per lane
     for (int c = 0; c < b->n_columns; c++) {
-        const int nz = b->offsets[c + 1] - b->offsets[c];
-        int q = -1;
-        for (size_t t = 0; t < tiles.size() && q < 0; t++)
-            if (nz <= batch_capacity(tiles[t])) q = (int)t;
-        if (q < 0) return fail(OBME_ERR_UNSUPPORTED, "a column is deeper than the plan's largest tile");
-        lists[q].push_back(c);
+        const int L = plan_levels(p, b->offsets[c + 1] - b->offsets[c]);
+        if (!L) return fail(OBME_ERR_UNSUPPORTED, "a column is deeper than the plan's deepest class");
+        lists[L].push_back(c);
     }
     batch_free_classes(b);
     batch_drop_graph(b);
     for (int L : {1, 2, 4}) {
-        std::vector<int> cols;
-        for (size_t t = 0; t < tiles.size(); t++)
-            if (BATCH_TILES[tiles[t]].L == L) cols.insert(cols.end(), lists[t].begin(), lists[t].end());
+        const std::vector<int>& cols = lists[L];
         std::vector<int> lanes = pack_ragged(b, cols, L, 1);
         // FP32 with a sediment: whole rows where they take no more waves per
         // SIMD (1024 of them).  A launch is as long as its busiest SIMD, and
@@ -1841,15 +1846,10 @@ static obme_status batch_apply_plan(obme_batch* b, int p)
         HIP_TRY(hipMalloc((void**)&d, lanes.size() * sizeof(int)));
         b->group_lanes.push_back(d);
         b->group_L.push_back(L);
+        b->group_n.push_back((int)cols.size());
         b->group_rows.push_back(rows ? 1 : 0);
         b->group_waves.push_back((int)(lanes.size() / 64));
         HIP_TRY(hipMemcpy(d, lanes.data(), lanes.size() * sizeof(int), hipMemcpyHostToDevice));
-    }
-    for (size_t t = 0; t < tiles.size(); t++) {
-        std::vector<int>& l = lists[t];
-        if (l.empty()) continue;
-        b->class_tile.push_back(tiles[t]);
-        b->class_n.push_back((int)l.size());
     }
     b->plan = p;
     return OBME_OK;
@@ -1948,7 +1948,7 @@ static BatchSedimentCall batch_sediment_call(const obme_batch* b, double* storag
 }
 
 // All launches of nsteps steps: per chunk of steps_per_launch steps, one
-// launch per class.
+// launch per levels per lane.
 template <typename FT>
 static obme_status batch_enqueue(const obme_batch* b, void* const* tracers, int nsteps, double dt, hipStream_t s,
                                  const BatchSedimentCall& sc)
@@ -2285,7 +2285,16 @@ extern "C" obme_status obme_batch_autotune(obme_batch* b, void* const* tracers, 
     int best_plan = keep_plan, best_spl = keep_spl;
     float best_ms = 1e30f;
     std::vector<int> spls = {0, 1, 10};
+    bool depths[129] = {};      // columns have at most 128 levels (obme_batch_create)
+    for (int c = 0; c < b->n_columns; c++) depths[b->offsets[c + 1] - b->offsets[c]] = true;
     for (int p = 0; p < (int)BATCH_PLANS.size() && st == OBME_OK; p++) {
+        // (a plan that packs these columns as an earlier one does is that one)
+        bool known = false;
+        for (int q = 0; q < p && !known; q++) {
+            known = true;
+            for (int nz = 1; nz <= 128 && known; nz++) known = !depths[nz] || plan_levels(p, nz) == plan_levels(q, nz);
+        }
+        if (known) continue;
         if (batch_apply_plan(b, p) != OBME_OK) continue;  // a plan that cannot hold the deepest column
         for (int spl : spls) {
             b->steps_per_launch = spl;
@@ -2316,17 +2325,17 @@ extern "C" obme_status obme_batch_autotune(obme_batch* b, void* const* tracers, 
     return st != OBME_OK ? st : r;
 }
 
-// "plan P steps_per_launch K classes: L,CPW,NW:count ..." (returns length or < 0)
+// "plan P steps_per_launch K launches: L per lane, C columns in W waves; ..."
+// (returns length or < 0)
 extern "C" int32_t obme_batch_describe(const obme_batch* b, char* buf, int32_t cap)
 {
     if (!b || !buf || cap < 1) return -1;
     std::string s = "plan " + std::to_string(b->plan) + " steps_per_launch " + std::to_string(b->steps_per_launch) +
-                    " classes:";
-    for (size_t q = 0; q < b->class_tile.size(); q++) {
-        const BatchTile& t = BATCH_TILES[b->class_tile[q]];
-        s += " " + std::to_string(t.L) + "," + std::to_string(t.CPW) + "," + std::to_string(t.NW) + ":" +
-             std::to_string(b->class_n[q]);
-    }
+                    " launches:";
+    for (size_t q = 0; q < b->group_L.size(); q++)
+        s += std::string(q ? ";" : "") + " " + std::to_string(b->group_L[q]) + " per lane, " +
+             std::to_string(b->group_n[q]) + " columns in " + std::to_string(b->group_waves[q]) + " waves" +
+             (b->group_rows[q] ? " by rows" : "");
     std::snprintf(buf, cap, "%s", s.c_str());
     return (int32_t)s.size();
 }
