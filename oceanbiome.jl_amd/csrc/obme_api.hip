@@ -2103,9 +2103,9 @@ extern "C" obme_status obme_batch_create(const obme_config* cfg, int32_t n_colum
         q.small_particle_fraction = get(OBME_BP_SMALL_PARTICLE_FRACTION, q.small_particle_fraction);
         // (the formulations are the configuration's, the same for every column)
         if (c == 0) b->default_forms = (fm_code(make_fast_params<float>(q)) == default_fm<OBME_NPZD>());
-        if (f64) dpar[c] = make_fast_params<double>(q);
+        if (f64) dpar[c] = make_fast_params<double>(q, 0.0, 0.0, false);
         else if (fixed) spar[c] = make_sediment_params(q);
-        else fpar[c] = make_fast_params<float>(q);
+        else fpar[c] = make_fast_params<float>(q, 0.0, 0.0, false);
         BatchColumn& bc = bcol[c];
         bc.PAR0 = get(OBME_BP_SURFACE_PAR, cfg->par.surface_value);
         bc.wP = -get(OBME_BP_P_SINKING_SPEED, cfg->sinking.speed[1]);

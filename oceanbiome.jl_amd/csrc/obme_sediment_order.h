@@ -30,9 +30,8 @@ struct SedimentParams {
     float ppc;         // (1 + rho (1-gamma) - alpha_x gamma) R
     float R, Rd, rhoR2, rhoR4;  // R, Rd, 2 rho R, 4 rho R
     float rem, small_frac, uptake_N;  // Detritus rate, fraction, (1 - alpha_x gamma)
-    float log2Q10_10;  // log2(Q10)/10: Q10^(T/10) = 2^(T log2Q10_10)
     float oRp, oRpn;   // Oxygen(): Rp, Rp - Rn (set from obme_oxygen)
-    int light_form, use_Q10, mort_form, graz_form;
+    int light_form, mort_form, graz_form;
 };
 
 inline SedimentParams make_sediment_params(const obme_npd_params& p)
@@ -81,9 +80,7 @@ inline SedimentParams make_sediment_params(const obme_npd_params& p)
     f.rem = (float)p.remineralisation_rate;
     f.small_frac = (float)p.small_particle_fraction;
     f.uptake_N = (float)(1 - p.ammonia_fraction_of_exudate * p.phytoplankton_exudation_fraction);
-    f.log2Q10_10 = (float)(std::log2(p.temperature_coefficient > 0 ? p.temperature_coefficient : 1.0) / 10);
     f.light_form = p.light_limitation;
-    f.use_Q10 = p.use_temperature_coefficient;
     f.mort_form = p.phytoplankton_mortality_formulation;
     f.graz_form = p.grazing_concentration_formulation;
     return f;
