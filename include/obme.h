@@ -339,7 +339,7 @@ obme_status obme_step(obme_handle* h, void* const* tracers,
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc).  obme_step with its per-call scratch (surface records,
  * [H+] warm starts, surface constants, O2 exchange coefficients, top-cell
- * DIC and Alk residuals) in a static
+ * DIC and Alk residuals, the top cells' records of negative scaling) in a static
  * device array of 64 MiB per device instead of buffers the library
  * allocates; it calls no hipMalloc or hipFree (the handle itself comes from
  * obme_create).  A grid whose scratch exceeds 64 MiB is rejected with
@@ -347,8 +347,10 @@ obme_status obme_step(obme_handle* h, void* const* tracers,
  * 40 B per column, about 1.6 million columns).  The warm starts begin at
  * zero on every call: where obme_step's handle carries warm starts from
  * earlier calls, results differ from it within the root solve's tolerance
- * (a relative Newton step of 1e-4 FP32-mixed, 1e-14 FP64); on a fresh
- * handle FP64 results are the same.  Every call on a
+ * (a relative Newton step of 1e-4 FP32-mixed, 3e-9 FP64, whose square is
+ * what is left); on a fresh handle FP64 results are the same, to rounding
+ * where the array has room for fewer steps per launch than obme_step takes.
+ * Every call on a
  * device shares that device's array: calls that overlap on one device race.
  * Must be called on the device the handle was created on. */
 obme_status obme_step_noalloc(obme_handle* h, void* const* tracers, const void* T, const void* S,

@@ -216,10 +216,16 @@ struct obme_handle {
     int surfc_cols = 0;        // Nx*Ny, or 1 when the call's T and S are the same in every column
     bool surfc_ready = false;  // d_surfc holds the constants of this call's T and S
     int srec_steps = 1;        // steps of surface records that d_srec holds
+    // Records of several steps, allocated by the first call whose launches take
+    // several and kept until the handle goes (a captured graph may hold them).
+    // A call of one step has d_srec.
+    void* d_srecs = nullptr;
+    int srecs_steps = 0;
+    bool noalloc = false;      // within obme_step_noalloc
     void* d_fast = nullptr;    // FP64: the transitions' constants (FastParams<double>)
     const double* d_light = nullptr;   // FP32: the levels' chlorophyll attenuations (LIGHT_*)
-    void* d_toprec = nullptr;  // the top cells' records of k_top_steps (scaling with the CO2 flux)
-    int toprec_steps = 0;      // steps of them that d_toprec holds
+    void* d_toprec = nullptr;  // the top cells' records of k_top_steps (scaling with the CO2 flux; as d_srecs)
+    int toprec_steps = 0;      // steps of them that d_toprec holds (0: none, the sweep solves the flux)
     bool default_forms = false;   // the model's default formulations (the FP32 kernels' compiled-in choices)
     int sink_idx[MAX_SINK];
     int sweep_waves;           // waves per workgroup of the sweep (1, 2, 4 or 8)
@@ -470,8 +476,8 @@ static int default_sweep_waves(size_t ncol)
     return best;
 }
 
-// Steps of per-column records of a launch that a handle keeps room for: as
-// many as fit RECORD_BYTES, 1 to WAVE_MAX_STEPS.
+// Steps of per-column records of a launch that a handle keeps room for, once a
+// call takes several steps: as many as fit RECORD_BYTES, 1 to WAVE_MAX_STEPS.
 constexpr size_t RECORD_BYTES = (size_t)128 << 20;
 constexpr int TOP_REC = 9;   // k_top_steps: three values per stage
 static int steps_within(size_t bytes, size_t per_step)
@@ -582,16 +588,7 @@ extern "C" obme_status obme_create(const obme_config* cfg, obme_handle** out)
     if (cfg->model == OBME_LOBSTER && cfg->carbonate_system && cfg->co2.enabled) {
         size_t ncol = (size_t)g.Nx * g.Ny;
         size_t es = (h->prec == OBME_FP64) ? 8 : 4;
-        // the records of several steps, for the launches that take several
-        h->srec_steps = h->co2_inline ? 1 : steps_within(RECORD_BYTES, SURF_REC * ncol * es);
-        hipError_t e1 = hipMalloc(&h->d_srec, h->srec_steps * SURF_REC * ncol * es);
-        if (h->co2_inline) {
-            h->toprec_steps = steps_within(RECORD_BYTES, TOP_REC * ncol * es);
-            if (hipMalloc(&h->d_toprec, h->toprec_steps * TOP_REC * ncol * es) != hipSuccess) {
-                obme_destroy(h);
-                return fail(OBME_ERR_NOMEM, "top-cell records");
-            }
-        }
+        hipError_t e1 = hipMalloc(&h->d_srec, SURF_REC * ncol * es);
         hipError_t e2 = hipMalloc((void**)&h->d_Hprev, ncol * sizeof(double));
         hipError_t e3 = (h->prec == OBME_FP64) ? hipSuccess : hipMalloc((void**)&h->d_topres, 2 * ncol * sizeof(float));
         if (e1 != hipSuccess || e2 != hipSuccess || e3 != hipSuccess) {
@@ -627,6 +624,7 @@ extern "C" obme_status obme_destroy(obme_handle* h)
     if (h->d_Tprof) (void)hipFree(h->d_Tprof);
     if (h->d_Sprof) (void)hipFree(h->d_Sprof);
     if (h->d_srec) (void)hipFree(h->d_srec);
+    if (h->d_srecs) (void)hipFree(h->d_srecs);
     if (h->d_toprec) (void)hipFree(h->d_toprec);
     if (h->d_Hprev) (void)hipFree(h->d_Hprev);
     if (h->d_topres) (void)hipFree(h->d_topres);
@@ -1282,6 +1280,59 @@ __global__ void __launch_bounds__(256) k_zero_f64(double* p, long n)
     if (q < n) p[q] = 0.0;
 }
 
+static WaveShape step_shape(const obme_handle* h, int nsteps)
+{
+    const bool general = h->scaling || h->sediment;
+    return h->prec == OBME_FP64 ? wave_shape<double>(h, TILE_STEP, nsteps, general)
+                                : wave_shape<float>(h, TILE_STEP, nsteps, general);
+}
+
+// Within a step call: the handle's records of several steps in the place of the
+// one step's, allocated where no call has had them (not under capture, where
+// the call goes by one step per launch, nor in obme_step_noalloc, which brings
+// its own; memory that is not there is done without).
+struct RecordsOfCall {
+    obme_handle* h;
+    void* srec;
+    int steps;
+    RecordsOfCall(obme_handle* handle, int nsteps, hipStream_t s) : h(handle), srec(handle->d_srec), steps(handle->srec_steps)
+    {
+        const obme_config& c = h->cfg;
+        if (h->noalloc || nsteps < 1 || !(c.model == OBME_LOBSTER && c.carbonate_system && c.co2.enabled)) return;
+        const size_t ncol = (size_t)c.grid.Nx * c.grid.Ny, es = h->prec == OBME_FP64 ? 8 : 4;
+        if (h->co2_inline) {
+            if (!h->d_toprec && step_shape(h, 1).levels) grow(&h->d_toprec, &h->toprec_steps, TOP_REC * ncol * es, s);
+            return;
+        }
+        if (nsteps < 2 || !step_shape(h, 2).levels) return;
+        if (!h->d_srecs && steps_within(RECORD_BYTES, SURF_REC * ncol * es) > 1)
+            grow(&h->d_srecs, &h->srecs_steps, SURF_REC * ncol * es, s);
+        if (h->d_srecs) {
+            h->d_srec = h->d_srecs;
+            h->srec_steps = h->srecs_steps;
+        }
+    }
+    ~RecordsOfCall()
+    {
+        h->d_srec = srec;
+        h->srec_steps = steps;
+    }
+    static void grow(void** p, int* steps, size_t per_step, hipStream_t s)
+    {
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(s, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) {
+            (void)hipGetLastError();
+            return;
+        }
+        const int n = steps_within(RECORD_BYTES, per_step);
+        if (hipMalloc(p, n * per_step) == hipSuccess) *steps = n;
+        else {
+            *p = nullptr;
+            (void)hipGetLastError();
+        }
+    }
+};
+
 extern "C" obme_status obme_step_with_sediment(obme_handle* h, void* const* tracers, const void* T, const void* S,
                                                double* storage, int32_t nsteps, double dt, double t0, void* stream)
 {
@@ -1329,14 +1380,12 @@ extern "C" obme_status obme_step_with_sediment(obme_handle* h, void* const* trac
     obme_status r = OBME_OK;
     h->o2c_ready = false;
     {
-        const bool general = h->scaling || h->sediment;
-        const bool f64 = h->prec == OBME_FP64;
+        RecordsOfCall records(h, nsteps, s);
         const int steps = launch_steps(h, nsteps);
-        const WaveShape ws = f64 ? wave_shape<double>(h, TILE_STEP, steps, general)
-                                 : wave_shape<float>(h, TILE_STEP, steps, general);
+        const WaveShape ws = step_shape(h, steps);
         if (ws.levels && steps > 0) {
-            r = f64 ? run_wave_steps<double>(h, ws, tracers, T, S, storage, nsteps, t0, dt, s)
-                    : run_wave_steps<float>(h, ws, tracers, T, S, storage, nsteps, t0, dt, s);
+            r = h->prec == OBME_FP64 ? run_wave_steps<double>(h, ws, tracers, T, S, storage, nsteps, t0, dt, s)
+                                     : run_wave_steps<float>(h, ws, tracers, T, S, storage, nsteps, t0, dt, s);
             h->surfc_ready = false;
             return r;
         }
@@ -1450,28 +1499,34 @@ extern "C" obme_status obme_step_noalloc(obme_handle* h, void* const* tracers, c
     // the library would have to create
     struct Swap {
         obme_handle* h;
-        void* srec;
-        int srec_steps;
+        void *srec, *toprec;
+        int srec_steps, toprec_steps;
         double *hprev, *surfc, *o2c;
         float* topres;
         bool timing;
         ~Swap()
         {
+            h->noalloc = false;
             h->d_srec = srec;
             h->srec_steps = srec_steps;
+            h->d_toprec = toprec;
+            h->toprec_steps = toprec_steps;
             h->d_Hprev = hprev;
             h->d_surfc = surfc;
             h->d_o2c = o2c;
             h->d_topres = topres;
             h->timing = timing;
         }
-    } keep{h, h->d_srec, h->srec_steps, h->d_Hprev, h->d_surfc, h->d_o2c, h->d_topres, h->timing};
+    } keep{h,           h->d_srec,   h->d_toprec, h->srec_steps, h->toprec_steps,
+           h->d_Hprev, h->d_surfc, h->d_o2c,    h->d_topres,   h->timing};
+    h->noalloc = true;
     h->timing = false;
-    // (the records of one step are part of the limit; more steps of them take
-    // what the static array has left, at its end)
-    if (co2)
-        h->srec_steps = 1 + (int)std::min<size_t>(WAVE_MAX_STEPS - 1,
-                                                  (NOALLOC_SCRATCH_BYTES - need) / (SURF_REC * ncol * es));
+    // (the records of one step are part of the limit; more steps of them, or the
+    // top cells', take what the static array has left, at its end)
+    const size_t left = NOALLOC_SCRATCH_BYTES - need;
+    if (co2 && !h->co2_inline)
+        h->srec_steps = 1 + (int)std::min<size_t>(WAVE_MAX_STEPS - 1, left / (SURF_REC * ncol * es));
+    if (h->co2_inline) h->toprec_steps = (int)std::min<size_t>(WAVE_MAX_STEPS, left / (TOP_REC * ncol * es));
     size_t off = 0;
     if (co2) {
         h->d_Hprev = (double*)(base + off);
@@ -1491,6 +1546,7 @@ extern "C" obme_status obme_step_noalloc(obme_handle* h, void* const* tracers, c
     h->d_topres = b_topres ? (float*)(base + off) : nullptr;
     off += b_topres;
     if (co2) h->d_srec = base + off;
+    if (h->co2_inline) h->d_toprec = base + off + b_srec;
     return obme_step_with_sediment(h, tracers, T, S, nullptr, nsteps, dt, t0, s);
 }
 
