@@ -257,7 +257,7 @@ struct FastParams {
     FT rem, small_frac;           // Detritus rate and fraction
     FT nGrowP, nUp, nPonw, nOx;   // NPZD: (1 - gamma) mu0, (1 - alpha_x gamma) mu0, (1 - alpha_x) gamma mu0, Rp mu0
     FT logQ10_10, logQ10_10l;   // Q10^(T/10): FP32 log2(Q10)/10; FP64 ln|Q10|/10 and its rounding error
-    FT Q10;                     // (FP64)
+                                // (use_Q10 = 2: a Q10 of 0 or less, and it in its place)
     FT oRp, oRpn, oRpm;           // Oxygen(): Rp, Rp - Rn, Rp mu0/2
     int light_form, use_Q10, mort_form, graz_form;
 };
@@ -328,12 +328,13 @@ inline FastParams<FT> make_fast_params(const obme_npd_params& p, double Rp = 0.0
         f.logQ10_10 = (FT)lnQ;
         f.logQ10_10l = (FT)(lnQ - (long double)(double)lnQ);
     }
-    f.Q10 = (FT)p.temperature_coefficient;
+    const bool special = q10 && !F32 && p.use_temperature_coefficient && !(p.temperature_coefficient > 0);
+    if (special) f.logQ10_10l = (FT)p.temperature_coefficient;
     f.oRp = (FT)Rp;
     f.oRpn = (FT)(Rp - Rn);
     f.oRpm = (FT)(Rp * h);
     f.light_form = p.light_limitation;
-    f.use_Q10 = p.use_temperature_coefficient;
+    f.use_Q10 = special ? 2 : p.use_temperature_coefficient;
     f.mort_form = p.phytoplankton_mortality_formulation;
     f.graz_form = p.grazing_concentration_formulation;
     return f;
@@ -369,10 +370,9 @@ __device__ __forceinline__ FT q10_factor(const FastParams<FT>& f, FT T)
     } else {
         const double p = T * f.logQ10_10;
         const double e = exp(p);
-        double r = fma(e, fma(T, f.logQ10_10, -p) + T * f.logQ10_10l, e);
-        r = r < HUGE_VAL ? r : e;       // (overflow: the correction is inf * 0)
-        if (!(f.Q10 > 0)) r = pow_special(f.Q10, T / 10, r);
-        return r;
+        if (f.use_Q10 == 2) return pow_special(f.logQ10_10l, T / 10, fma(e, fma(T, f.logQ10_10, -p), e));
+        const double r = fma(e, fma(T, f.logQ10_10, -p) + T * f.logQ10_10l, e);
+        return r < HUGE_VAL ? r : e;    // (overflow: the correction is inf * 0)
     }
 }
 

@@ -172,8 +172,6 @@ struct StepArgs {
     FT invdz_u;                    // uniform grid: 1/Δz
     float rk_a[3], rk_b[3];        // FP32 path: Δt γ and Δt ζ per stage
     float kr2, kb2, xr2, xb2;      // FP32 path: attenuations × log2(e)
-    const double* light;           // FP32 path: [LIGHT_COUNT][Nz], the levels' chlorophyll attenuations
-    float erl, ebl;                // FP32 path: what er and eb lost to rounding
     float cr, cb;                  // FP32 path: e log2(R_chl / r) per band
     float xr2h, xb2h;              // FP32 uniform grid: xr2 dz/2, xb2 dz/2
     float wi0, wi1;                // FP32 uniform grid: w / dz of the two sinking tracers
@@ -222,6 +220,9 @@ struct StepArgs {
     unsigned ncell;
     FT* Dsc;
     FT* Gsc;
+    // FP32, the light hooks
+    const double* light;           // [LIGHT_COUNT][Nz], the levels' chlorophyll attenuations
+    float erl, ebl;                // what er and eb lost to rounding
 };
 
 // Per-level geometry rows in `lev` (each Nz entries).
