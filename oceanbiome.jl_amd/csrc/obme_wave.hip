@@ -22,9 +22,13 @@ template <int MODEL, int CARB, typename FT, int L>
 static WaveKernel<FT> wave_kernel_levels(int mode, bool uniform, int lpc, bool general, bool win)
 {
     constexpr int FM = default_fm<MODEL>();
-    constexpr int SEG = 64 / L;         // 64 levels
-    if (mode == TILE_STEP && !general && !win && uniform && lpc == SEG)
-        return k_column_wave<MODEL, CARB, FT, TILE_STEP, true, L, false, false, FM, SEG>;
+    // 64 levels (FP32 with more than one level per lane: wave_shape has one for
+    // them on any number of columns)
+    if constexpr (sizeof(FT) == 8 || L == 1) {
+        constexpr int SEG = 64 / L;
+        if (mode == TILE_STEP && !general && !win && uniform && lpc == SEG)
+            return k_column_wave<MODEL, CARB, FT, TILE_STEP, true, L, false, false, FM, SEG>;
+    }
     if (mode == TILE_STEP && !general && !win)
         return uniform ? k_column_wave<MODEL, CARB, FT, TILE_STEP, true, L, false, false, FM>
                        : k_column_wave<MODEL, CARB, FT, TILE_STEP, false, L, false, false, FM>;
