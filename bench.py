@@ -26,6 +26,11 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, os.path.join(ROOT, "oceanbiome.jl_amd"))
 
 HBM_PEAK_GBS = 8000.0
+# vector instructions of a wave (64 lanes, two operations in a multiply-add) at
+# the nominal vector rates, 157.3 TFLOP/s in FP32 and 78.6 in FP64: 256 CUs of
+# four SIMDs at 2.4 GHz, two and four cycles each.  (Unpacked FP32 measures 2.4 to
+# 4.5 by its operands.)
+VALU_PEAK = {"fp32": 1024 * 2.4e9 / 2, "fp64": 1024 * 2.4e9 / 4}
 
 
 def parse():
@@ -145,20 +150,28 @@ def cpu_threads(req):
     return max(1, min(HOST_SHARE, host_cpus()))
 
 
-def read_traffic(profile_dir, workload, precision):
-    """HBM bytes per sweep launch from a committed counter summary: a line
-    'traffic_bytes_per_launch <workload> <precision> <bytes>'."""
-    if not os.path.isdir(profile_dir):
+def read_profile(what, workload, precision):
+    """A counter of a committed profile: the words after
+    '<what> <workload> <precision>' of a line, as numbers."""
+    folder = os.path.join(ROOT, "profiles")
+    if not os.path.isdir(folder):
         return None
-    for fn in sorted(os.listdir(profile_dir)):
+    for fn in sorted(os.listdir(folder)):
         if not fn.endswith((".md", ".txt")):
             continue
-        for line in open(os.path.join(profile_dir, fn)):
+        for line in open(os.path.join(folder, fn)):
             parts = line.strip().strip("`").split()
-            if len(parts) == 4 and parts[0] == "traffic_bytes_per_launch" and parts[1] == workload \
-                    and parts[2] == precision:
-                return float(parts[3])
+            if len(parts) >= 4 and parts[:3] == [what, workload, precision]:
+                return [float(x) for x in parts[3:]]
     return None
+
+
+def read_traffic(workload, precision):
+    """HBM bytes of a launch from a committed counter summary, and the steps of
+    that launch: 'traffic_bytes_per_launch <workload> <precision> <bytes>
+    [<steps>]'."""
+    found = read_profile("traffic_bytes_per_launch", workload, precision)
+    return (None, None) if found is None else (found[0], found[1] if len(found) > 1 else 1)
 
 
 def main():
@@ -196,8 +209,8 @@ def main():
         bytes_step = wl.algorithmic_bytes_per_step(sbytes)
         ms = secs / args.steps * 1e3
         upd = nw * ncell * args.steps / secs
-        gbs = bytes_step / (secs / args.steps) / 1e9
         # (the state crosses HBM once per launch, whatever its steps)
+        gbs = bytes_step / spl / (secs / args.steps) / 1e9
         sweep_gbs = bytes_step / (sweep_ms * 1e-3) / 1e9
         results[prec] = {"ms_per_step": ms, "updates_per_s": upd, "achieved_GBs": gbs,
                          "sweep_ms_per_launch": sweep_ms, "steps_per_launch": spl, "sweep_achieved_GBs": sweep_gbs,
@@ -266,15 +279,22 @@ def main():
 
     head_prec = "fp32" if "fp32" in results else "fp64"
     head = results[head_prec]
-    traffic = read_traffic(os.path.join(ROOT, "profiles"), wl.name, head_prec)
+    traffic, traffic_steps = read_traffic(wl.name, head_prec)
+    spl, launch_s = head["steps_per_launch"], head["sweep_ms_per_launch"] * 1e-3
     # several steps per launch: the state stays in registers between them, and
-    # the vector ALUs are the bound
-    many = head["steps_per_launch"] > 1
-    dom = {"bound": "valu" if many else "hbm", "achieved": head["sweep_achieved_GBs"], "peak": HBM_PEAK_GBS,
-           "unit": "GB/s", "frac": head["sweep_achieved_GBs"] / HBM_PEAK_GBS, "traffic": traffic,
-           "kernel": "k_column_wave" if many else "k_column_lane (column sweep)",
-           "algorithmic_bytes_per_launch": head["bytes_per_step"], "steps_per_launch": head["steps_per_launch"],
-           "launch_ms": head["sweep_ms_per_launch"]}
+    # the vector ALUs are the bound (wave instructions per level of 64 lanes and
+    # stage, from the counters)
+    insts = read_profile("valu_instructions_per_level_and_stage", wl.name, head_prec) if spl > 1 else None
+    if insts:
+        rate = insts[0] * ncell / 64 * 3 * spl / launch_s
+        peak = VALU_PEAK[head_prec]
+        dom = {"bound": "valu", "achieved": rate, "peak": peak, "unit": "wave instructions/s", "frac": rate / peak}
+    else:
+        dom = {"bound": "valu" if spl > 1 else "hbm", "achieved": head["sweep_achieved_GBs"], "peak": HBM_PEAK_GBS,
+               "unit": "GB/s", "frac": None if spl > 1 else head["sweep_achieved_GBs"] / HBM_PEAK_GBS}
+    dom.update({"kernel": "k_column_wave" if spl > 1 else "k_column_lane (column sweep)", "steps_per_launch": spl,
+                "launch_ms": head["sweep_ms_per_launch"], "algorithmic_bytes_per_launch": head["bytes_per_step"],
+                "hbm_GBs": head["sweep_achieved_GBs"], "traffic": traffic, "traffic_steps_per_launch": traffic_steps})
     line = {
         "metric": "tracer-cell updates/s + % HBM roofline; FP32-mixed vs FP64 at stated error",
         "value": head["updates_per_s"],
@@ -373,7 +393,7 @@ def bench_hooks(args):
     calibration_copy(args)
     head_prec = "fp32" if "fp32" in res else "fp64"
     head = res[head_prec]
-    traffic = read_traffic(os.path.join(ROOT, "profiles"), wl.name + "_hooks", head_prec)
+    traffic, _ = read_traffic(wl.name + "_hooks", head_prec)
     print(json.dumps({
         "metric": "tracer-cell tendency evaluations/s of the coupled-model hooks (update-state + tendencies)",
         "value": head["tendency_evaluations_per_s"], "unit": "tracer-cell tendency evaluations/s",
@@ -633,8 +653,12 @@ def bench_pisces(args):
         secs = s.elapsed_time(e) / 1e3
         sb = 4 if prec == "fp32" else 8
         bytes_step = wl.algorithmic_bytes_per_step(sb)
+        # (the FP32 step takes up to 16 steps per launch, and the state crosses
+        # HBM once in each)
+        spl = steps / -(-steps // 16) if prec == "fp32" else 1
         res[prec] = {"ms_per_step": secs / steps * 1e3, "updates_per_s": nw * ncell * steps / secs,
-                     "achieved_GBs": bytes_step / (secs / steps) / 1e9, "bytes_per_step": bytes_step}
+                     "steps_per_launch": spl, "achieved_GBs": bytes_step / spl / (secs / steps) / 1e9,
+                     "bytes_per_step": bytes_step}
         log(f"pisces {prec}: {res[prec]['ms_per_step']:.3f} ms/step  {res[prec]['updates_per_s']:.3e} upd/s  "
             f"{res[prec]['achieved_GBs']:.0f} GB/s")
         if not args.no_check:
@@ -703,10 +727,11 @@ def bench_pisces(args):
         "ms_per_step": head["ms_per_step"], "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
         "dtype": "f32" if head_prec == "fp32" else "f64", "data": "synthetic (seeded lognormal tracers)",
         "config": {"workload": wl.name, "grid": [g.Nx, g.Ny, g.Nz], "tracers_written": nw, "dt": wl.dt},
-        "roofline": {"bound": "hbm", "achieved": head["achieved_GBs"], "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": head["achieved_GBs"] / HBM_PEAK_GBS, "traffic": None,
-                     "kernel": "whole PISCES step", "algorithmic_bytes_per_launch": head["bytes_per_step"],
-                     "launch_ms": head["ms_per_step"]},
+        "roofline": {"bound": "valu", "achieved": head["achieved_GBs"], "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                     "frac": None, "traffic": None, "kernel": "k_pisces_fused" if head_prec == "fp32" else "k_pisces_cell",
+                     "algorithmic_bytes_per_launch": head["bytes_per_step"],
+                     "steps_per_launch": head["steps_per_launch"],
+                     "launch_ms": head["ms_per_step"] * head["steps_per_launch"]},
         "cpu_baseline": cpu, "results": res, "errors_vs_oracle": errors}))
 
 
