@@ -573,8 +573,14 @@ extern "C" obme_status obme_create(const obme_config* cfg, obme_handle** out)
     h->scaling = cfg->scaling.n_groups > 0;
     {
         const FastParams<float> f = make_fast_params<float>(cfg->npd);
+        // (FP64: a Q10 of 0 or less and chlorophyll exponents that can overflow are
+        // for the kernels with the formulations read at run time)
+        const bool special =
+            h->prec == OBME_FP64 &&
+            (!tame_exponents(cfg->par.chlorophyll_red_exponent, cfg->par.chlorophyll_blue_exponent) ||
+             (cfg->npd.use_temperature_coefficient && !(cfg->npd.temperature_coefficient > 0)));
         h->default_forms =
-            fm_code(f) == (cfg->model == OBME_NPZD ? default_fm<OBME_NPZD>() : default_fm<OBME_LOBSTER>());
+            !special && fm_code(f) == (cfg->model == OBME_NPZD ? default_fm<OBME_NPZD>() : default_fm<OBME_LOBSTER>());
     }
     h->scheme = cfg->sinking.scheme;
     h->staged = h->scheme != OBME_UPWIND1;
@@ -882,10 +888,9 @@ static WaveShape wave_shape(const obme_handle* h, int mode, int nsteps, bool gen
     // (FP32 takes the logarithm of the chlorophyll attenuation)
     const obme_two_band_par& par = h->cfg.par;
     if (sizeof(FT) == 4 && !(par.chlorophyll_red_attenuation >= 0 && par.chlorophyll_blue_attenuation >= 0)) return best;
-    // exponents of 0 to 1: the powers of finite tracers are finite, and a level's
-    // own can be taken off the sum that includes it
-    auto tame = [](double e) { return e >= 0 && e <= 1; };
-    if (!tame(par.chlorophyll_red_exponent) || !tame(par.chlorophyll_blue_exponent)) return best;
+    // (the powers of finite tracers are finite, and a level's own can be taken off
+    // the sum that includes it)
+    if (!tame_exponents(par.chlorophyll_red_exponent, par.chlorophyll_blue_exponent)) return best;
     if (mode == TILE_STEP && h->sediment) {
         if (h->cfg.sediment.model == OBME_SEDIMENT_SIMPLE_MULTI_G) return best;
         // NPZD's sinking P takes the light's rounding into the FP64 storage
@@ -2158,7 +2163,9 @@ extern "C" obme_status obme_batch_create(const obme_config* cfg, int32_t n_colum
         q.remineralisation_rate = get(OBME_BP_REMINERALISATION_RATE, q.remineralisation_rate);
         q.small_particle_fraction = get(OBME_BP_SMALL_PARTICLE_FRACTION, q.small_particle_fraction);
         // (the formulations are the configuration's, the same for every column)
-        if (c == 0) b->default_forms = (fm_code(make_fast_params<float>(q)) == default_fm<OBME_NPZD>());
+        if (c == 0)
+            b->default_forms = fm_code(make_fast_params<float>(q)) == default_fm<OBME_NPZD>() &&
+                               (!f64 || tame_exponents(cfg->par.chlorophyll_red_exponent, cfg->par.chlorophyll_blue_exponent));
         if (f64) dpar[c] = make_fast_params<double>(q, 0.0, 0.0, false);
         else if (fixed) spar[c] = make_sediment_params(q);
         else fpar[c] = make_fast_params<float>(q, 0.0, 0.0, false);

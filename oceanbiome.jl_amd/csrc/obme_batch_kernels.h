@@ -422,7 +422,7 @@ __device__ __forceinline__ void batch_ragged(const BatchArgs<FT>& a)
                     pr[m] = m_exp2(fmaf(a.er_f, lg, a.cr));
                     pb[m] = m_exp2(fmaf(a.eb_f, lg, a.cb));
                 } else {
-                    pow_pair(X[1][m] * a.Rr, a.er, a.eb, pr[m], pb[m]);
+                    pow_pair<FM < 0>(X[1][m] * a.Rr, a.er, a.eb, pr[m], pb[m]);
                 }
                 totr = m == 0 ? pr[m] : totr + pr[m];
                 totb = m == 0 ? pb[m] : totb + pb[m];

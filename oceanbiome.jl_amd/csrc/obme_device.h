@@ -139,14 +139,15 @@ __device__ __forceinline__ double exp_product(double e, double L)
     const double r = exp(p);
     return fma(r, fma(e, L, -p), r);
 }
-// pow's value at x <= 0, infinite and NaN x, at e = 0 and where it overflows,
-// r = |x|^e elsewhere.
+// pow's value at x <= 0, infinite and NaN x, at e = 0 and (ANY) where it
+// overflows, r = |x|^e elsewhere.
+template <bool ANY = true>
 __device__ __forceinline__ double pow_special(double x, double e, double r)
 {
     if (e == 0.0) return 1.0;
     if (x != x || e != e) return x + e;
     const double inf = HUGE_VAL;
-    if (!(r < inf)) r = fabs(x) == 1.0 ? 1.0 : ((e > 0.0) == (fabs(x) > 1.0) ? inf : 0.0);
+    if (ANY && !(r < inf)) r = fabs(x) == 1.0 ? 1.0 : ((e > 0.0) == (fabs(x) > 1.0) ? inf : 0.0);
     if (x == 0.0) r = e > 0.0 ? 0.0 : inf;
     if (fabs(x) == inf) r = e > 0.0 ? inf : 0.0;
     if (x < 0.0) {
@@ -155,19 +156,26 @@ __device__ __forceinline__ double pow_special(double x, double e, double r)
     }
     return r;
 }
+// Exponents with which the power of a finite base does not overflow.
+__host__ __device__ __forceinline__ bool tame_exponents(double e1, double e2)
+{
+    return e1 >= 0.0 && e1 <= 1.0 && e2 >= 0.0 && e2 <= 1.0;
+}
 // x^e1 and x^e2 of one base in FP64, within a few ulp of pow: the logarithm
-// shared, pow's special cases behind one branch.  TAME: exponents of 0 to 1,
-// with which a power of a finite base does not overflow (LOBSTER's FP64 step
-// on 256x256x64, four steps: 628 us, 640 with the comparisons).
-template <bool TAME = false>
+// shared, pow's special cases behind one branch.  ANY: the exponents (the same
+// in every lane) need not be tame; with others every lane takes the branch.
+// (Only kernels with the formulations read at run time have ANY: the branch's
+// code alone cost the fused step of 512x512x64 697 -> 762 us.)
+template <bool ANY>
 __device__ __forceinline__ void pow_pair(double x, double e1, double e2, double& r1, double& r2)
 {
+    const bool plain = ANY ? tame_exponents(e1, e2) && e1 != 0.0 && e2 != 0.0 : e1 != 0.0 && e2 != 0.0;
     const double L = log_positive(fabs(x));
     r1 = exp_product(e1, L);
     r2 = exp_product(e2, L);
-    if (!(x > 0.0 && x < HUGE_VAL && e1 != 0.0 && e2 != 0.0) || !(TAME || (r1 < HUGE_VAL && r2 < HUGE_VAL))) {
-        r1 = pow_special(x, e1, r1);
-        r2 = pow_special(x, e2, r2);
+    if (!(x > 0.0 && x < HUGE_VAL && plain)) {
+        r1 = pow_special<ANY>(x, e1, r1);
+        r2 = pow_special<ANY>(x, e2, r2);
     }
 }
 // x^y: within a few ulp of pow (270 cycles of a wave where pow takes 600).
@@ -362,7 +370,9 @@ inline int fm_code(const FastParams<float>& f)
 }
 
 // Q10^(T/10) (plankton.jl:210-214); FP64 with the product's low part put back.
-template <typename FT>
+// (A Q10 of 0 or less: with the formulations read at run time, which such a
+// handle takes.)
+template <int FM, typename FT>
 __device__ __forceinline__ FT q10_factor(const FastParams<FT>& f, FT T)
 {
     if constexpr (sizeof(FT) == 4) {
@@ -370,9 +380,10 @@ __device__ __forceinline__ FT q10_factor(const FastParams<FT>& f, FT T)
     } else {
         const double p = T * f.logQ10_10;
         const double e = exp(p);
-        if (f.use_Q10 == 2) return pow_special(f.logQ10_10l, T / 10, fma(e, fma(T, f.logQ10_10, -p), e));
-        const double r = fma(e, fma(T, f.logQ10_10, -p) + T * f.logQ10_10l, e);
-        return r < HUGE_VAL ? r : e;    // (overflow: the correction is inf * 0)
+        if constexpr (FM < 0) {
+            if (f.use_Q10 == 2) return pow_special(f.logQ10_10l, T / 10, fma(e, fma(T, f.logQ10_10, -p), e));
+        }
+        return fma(e, fma(T, f.logQ10_10, -p) + T * f.logQ10_10l, e);
     }
 }
 

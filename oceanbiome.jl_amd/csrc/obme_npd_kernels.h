@@ -610,7 +610,7 @@ __device__ __forceinline__ void column_lane(const StepArgs<FT>& a, const int cw)
                 pb = m_exp2(fmaf(a.eb, lg, a.cb));
             } else {
                 // both bands' powers from one logarithm
-                pow_pair(X[PI] * a.Rr, a.er, a.eb, pr, pb);
+                pow_pair<FM < 0>(X[PI] * a.Rr, a.er, a.eb, pr, pb);
             }
             FT ir, ib;
             if constexpr (F32 && UNIFORM) {
@@ -654,7 +654,7 @@ __device__ __forceinline__ void column_lane(const StepArgs<FT>& a, const int cw)
                 constexpr bool FIXED = F32 && (EXTRA & 4) != 0;
                 if constexpr (MODEL == OBME_NPZD) {
                     FT Lt = FT(1);
-                    if (fm_q10<FM>(a.f)) Lt = q10_factor(a.f, v[3]);
+                    if (fm_q10<FM>(a.f)) Lt = q10_factor<FM>(a.f, v[3]);
                     if constexpr (FIXED)
                         npzd_sediment<FM>(a.fs, v[0], v[1], v[2], v[4], PARv, Lt, Gv[0], Gv[1], Gv[2], Gv[4],
                                           (CARB & 2) ? &Gv[NT - 1] : nullptr);
@@ -1116,7 +1116,7 @@ __global__ void __launch_bounds__(LightShape<FT>::THREADS, 4) k_light(StepArgs<F
             if constexpr (F32) {
                 chlorophyll_powers(a, p, r, b);
             } else {
-                pow_pair(p * a.Rr, a.er, a.eb, r, b);
+                pow_pair<true>(p * a.Rr, a.er, a.eb, r, b);
             }
             power(0, u) = r;
             power(1, u) = b;

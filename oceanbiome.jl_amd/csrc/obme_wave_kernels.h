@@ -310,7 +310,7 @@ __device__ __forceinline__ void column_wave(const WaveArgs<FT>& w, FT* lds)
         Lt[m] = FT(1);
         if constexpr (MODEL == OBME_NPZD) {
             // Q10^(T/10): T is fixed
-            if (fm_q10<FM>(a.f)) Lt[m] = q10_factor(a.f, U[3][m]);
+            if (fm_q10<FM>(a.f)) Lt[m] = q10_factor<FM>(a.f, U[3][m]);
         }
     }
     const bool top = r == 0;            // the column's top level is level 0 of its first lane
@@ -442,7 +442,7 @@ __device__ __forceinline__ void column_wave(const WaveArgs<FT>& w, FT* lds)
                     pr[m] = m_exp2(fmaf(a.er, lg, w.cr));
                     pb[m] = m_exp2(fmaf(a.eb, lg, w.cb));
                 } else {
-                    pow_pair<true>(I[PI][m] * a.Rr, a.er, a.eb, pr[m], pb[m]);
+                    pow_pair<false>(I[PI][m] * a.Rr, a.er, a.eb, pr[m], pb[m]);
                 }
             }
             // the integral to level j: with c = the half cells either side of the
@@ -831,7 +831,7 @@ __device__ __forceinline__ void top_steps(const WaveArgs<FT>& w, FT* rec)
                 const float h = w.uniform ? 1.0f : (float)dn;   // (a uniform grid's half cell is in cr, cb)
                 PAR = PAR0 * fmaf(wr, m_exp2(-(h * pr)), wb * m_exp2(-(h * pb)));
             } else {
-                pow_pair<true>(X[PI] * a.Rr, a.er, a.eb, pr, pb);
+                pow_pair<false>(X[PI] * a.Rr, a.er, a.eb, pr, pb);
                 PAR = PAR0 * (wr * m_exp(-a.xr * (dn * pr)) + wb * m_exp(-a.xb * (dn * pb)));
             }
             FT Gv[NT], v[NT];
