@@ -877,6 +877,73 @@ static int launch_steps(const obme_handle* h, int nsteps)
     return n;
 }
 
+// Up to how many (thousand) columns a launch of nsteps steps, or a hook, takes
+// the levels-along-the-lanes kernel; they count by the lanes that a column
+// takes, in columns' worth of levels (a launch of several steps, which computes
+// more: by its square), and from 131 072 columns on all alike.  Up to 65 536
+// columns the sweep, a thread per column, takes about as long as for one: this
+// kernel's lanes then win by all that they fill.  Where the sweep fills the chip
+// it is the faster in one step, having the longer runs of a level's values; from
+// three FP32 steps of a launch on, with the state in registers between them,
+// this is.  us per call, sweep | this:
+//                                FP32                     FP64
+//   one step, LOBSTER, 64 levels
+//     32 768 columns             60 | 41                  189 | 108
+//     65 536                     61 | 70                  184 | 225
+//     262 144                   193 | 536                 620 | 794
+//   two, three steps of it, 131 072 columns
+//                               203 | 202, 298 | 266      643 | 600, 969 | 813
+//   two steps of NPZD, 33 levels, 65 536 columns
+//                                67 | 57                  154 | 193
+//   a step with scaling, 64 levels
+//     65 536                    182 | 110                 407 | 269
+//     131 072                   223 | 247                 584 | 534
+//   the same with a sediment, 65 536
+//                               181 | 129                 411 | 263
+//   a step, then five, with a sediment, 33 levels (FP32: 31 of 64 lanes idle)
+//     16 384                     50 | 40, 238 | 113       101 | 52, 490 | 165
+//     65 536                     56 | 128, 271 | 394      114 | 157, 549 | 529
+//     131 072                    78 | 275, 376 | 771      188 | 333, 904 | 1035
+//   the hook, 64 levels
+//     32 768                     48 | 53                   94 | 102
+//     131 072                   147 | 325                 297 | 463
+//   the hook of WENO sinking, 64 levels (a flux solve in each thread's walk)
+//     65 536                    146 | 129                 254 | 217
+//     131 072                   240 | 332                 365 | 477
+// (One step without scaling or sediment from 40 960 columns on, and the hook from
+// 32 768, are the sweep's however well the lanes are filled: within 5 % there.)
+// Centred and WENO steps, a launch per stage otherwise, are this kernel's at
+// every size but 65 levels of FP64 (half the lanes idle; one WENO step of
+// 131 072 columns 1217 | 1393).
+template <typename FT>
+static double wave_columns(const obme_handle* h, int mode, int nsteps)
+{
+    const bool f64 = sizeof(FT) == 8;
+    const double all = HUGE_VAL;
+    if (mode != TILE_STEP) {
+        if (!h->staged) return f64 ? 31 : 41;
+        return h->scheme == OBME_WENO5 ? (f64 ? 80 : 94) : (f64 ? 48 : 52);
+    }
+    const int n = std::max(1, std::min(nsteps, 3)) - 1;
+    const bool co2 = h->cfg.model == OBME_LOBSTER && h->cfg.carbonate_system && h->cfg.co2.enabled;
+    if (h->staged) return f64 && h->scheme == OBME_WENO5 && n == 0 ? 190 : all;
+    if (h->sediment && !h->scaling) {
+        const double f32_cols[] = {40, 92, 124}, f64_cols[] = {49, 100, 150};
+        return f64 ? f64_cols[n] : f32_cols[n];
+    }
+    if (h->sediment && !f64 && !h->co2_inline) {
+        const double both[] = {80, 124, 160};
+        return both[n];
+    }
+    if (h->scaling) {
+        const double f32_cols[] = {112, 340, all};
+        return !f64 ? f32_cols[n] : h->co2_inline || n > 0 ? all : 190;
+    }
+    const double f32_cols[] = {co2 ? 41.0 : 48.0, co2 ? 104.0 : 127.0, all};
+    const double lobster[] = {52, 160, 220}, npzd[] = {52, 98, 150};
+    return !f64 ? f32_cols[n] : h->cfg.model == OBME_NPZD ? npzd[n] : lobster[n];
+}
+
 // nsteps: of a launch
 template <typename FT>
 static WaveShape wave_shape(const obme_handle* h, int mode, int nsteps, bool general)
@@ -897,20 +964,6 @@ static WaveShape wave_shape(const obme_handle* h, int mode, int nsteps, bool gen
         // (obme_sediment_order.h): FP32 keeps the sweep's running sums there
         if (sizeof(FT) == 4 && h->cfg.model == OBME_NPZD) return best;
     }
-    // One step or a hook: the sweep moves a level's values in longer runs and
-    // is the faster where its columns fill the chip.  On 64 levels, us per
-    // step, sweep | this: FP32 16 384 columns 59 | 26, 65 536 64 | 81; FP64
-    // 180 | 65, 197 | 247; FP32 hooks 57 | 35, 110 | 158; FP64 hooks on 38 400
-    // 222 | 238.  The hooks of the centred and WENO schemes cross later (on
-    // 38 400 columns FP32 154 | 65, FP64 275 | 134).  From two steps of a launch
-    // on, with the state in registers between them, this is the faster everywhere
-    // (262 144 columns, two steps: 507 | 486).  The centred and WENO steps and
-    // the scaling and sediment variants are: a launch per stage and the flux
-    // solve in the walk are what they replace.
-    long most = LONG_MAX;
-    if (mode != TILE_STEP) most = !h->staged ? 32768 : (sizeof(FT) == 4 ? 131072 : 65536);
-    else if (nsteps < 2 && !general && !h->staged) most = 40960;
-    if (ncol > most) return best;
     double cost = 0.0;
     for (int i = 0; i < 4 && wave_levels<FT>(i); i++) {
         const int L = wave_levels<FT>(i);
@@ -932,6 +985,11 @@ static WaveShape wave_shape(const obme_handle* h, int mode, int nsteps, bool gen
         }
     }
     if (!best.levels) return best;
+    const double lanes = 64.0 * best.levels / (Nz * (double)best.cpw);
+    const bool several = mode == TILE_STEP && nsteps > 1;
+    if (!general && !h->staged && !several && ncol > (mode == TILE_STEP ? 40960 : 32768)) return WaveShape();
+    if (std::min(ncol, 131072l) * (several ? lanes * lanes : lanes) > 1024.0 * wave_columns<FT>(h, mode, nsteps))
+        return WaveShape();
     // workgroups of eight waves, fewer where that leaves CUs without one
     best.nw = 8;
     const int es = (int)sizeof(FT);
@@ -1305,13 +1363,15 @@ struct RecordsOfCall {
         const obme_config& c = h->cfg;
         if (h->noalloc || nsteps < 1 || !(c.model == OBME_LOBSTER && c.carbonate_system && c.co2.enabled)) return;
         const size_t ncol = (size_t)c.grid.Nx * c.grid.Ny, es = h->prec == OBME_FP64 ? 8 : 4;
+        const size_t per_step = (h->co2_inline ? TOP_REC : SURF_REC) * ncol * es;
+        const int launch = std::min(nsteps, steps_within(RECORD_BYTES, per_step));
+        const bool used = step_shape(h, launch).levels > 0;
         if (h->co2_inline) {
-            if (!h->d_toprec && step_shape(h, 1).levels) grow(&h->d_toprec, &h->toprec_steps, TOP_REC * ncol * es, s);
+            if (!h->d_toprec && used) grow(&h->d_toprec, &h->toprec_steps, per_step, s);
             return;
         }
-        if (nsteps < 2 || !step_shape(h, 2).levels) return;
-        if (!h->d_srecs && steps_within(RECORD_BYTES, SURF_REC * ncol * es) > 1)
-            grow(&h->d_srecs, &h->srecs_steps, SURF_REC * ncol * es, s);
+        if (launch < 2 || !used) return;
+        if (!h->d_srecs) grow(&h->d_srecs, &h->srecs_steps, per_step, s);
         if (h->d_srecs) {
             h->d_srec = h->d_srecs;
             h->srec_steps = h->srecs_steps;
