@@ -238,7 +238,7 @@ enum { LEV_ZC = 0, LEV_UP, LEV_DN, LEV_INVDZ, LEV_WR, LEV_WB, LEV_COUNT };
 enum { LIGHT_ABOVE_R = 0, LIGHT_ABOVE_B, LIGHT_WHOLE_R, LIGHT_WHOLE_B, LIGHT_COUNT };
 
 // What a launch does: the fused RK3 step, the tendencies (hook), the PAR (hook;
-// k_light, and the sweep for many columns in FP64), one RK3 stage with its
+// k_light, and the sweep for many columns), one RK3 stage with its
 // substep (the step of the sinking schemes whose face values need the levels
 // below).
 enum { TILE_STEP = 0, TILE_TENDENCY = 1, TILE_PAR = 2, TILE_STAGE = 3 };
@@ -1029,17 +1029,20 @@ __device__ __forceinline__ void chlorophyll_powers(const StepArgs<FT>& a, float 
 // to unroll (eight levels: 27 us of fetching it on 17x76x58, 8 with a loop);
 // its levels wait in LDS.  Above 65536 columns FP64 takes the sweep, which keeps
 // the powers' constants in registers down the column (500x300x40: 50 us | 60;
-// with the tendencies 256x256x64 221 | 215, 333x187x20 65.6 | 65.1).
+// with the tendencies 256x256x64 221 | 215, 333x187x20 65.6 | 65.1).  FP32
+// above 163 840, where the sweep fills the chip three times (160 000 and 262 144
+// columns of 17 levels 12.3 | 14.6 and 14.6 | 19.4, of 64 26.5 | 24.2 and
+// 30.6 | 36.2).
 // FP32: the integral is summed in FP64 (which takes as long as FP32 and a
 // conversion) and its exponent rounded once, as the sweep's compensated sums
 // are: largest error on 64 levels of P about 0.1 1.4e-6 (the sweep 1.9e-6; with
 // sums in FP32 3.8e-6), on 400 of P about 3 5.7e-6 (9.3e-6; 3.0e-5).  With them
-// 384x384x64 took 20.1 us, 512x512x30 17.5 (now 18.9).
+// 384x384x64 took 20.1 us.
 template <typename FT>
 struct LightShape {
     static constexpr int COLS = sizeof(FT) == 4 ? 64 : 32;
     static constexpr int ROWS = 8, LEVELS = 8, THREADS = COLS * ROWS;
-    static constexpr unsigned MOST_COLUMNS = sizeof(FT) == 4 ? ~0u : 65536u;
+    static constexpr unsigned MOST_COLUMNS = sizeof(FT) == 4 ? 163840u : 65536u;
 };
 // A level: the thickness from zf(k+1) to zc(k) and the whole level's (FP32:
 // times the band's attenuation, see `light`), the light left by the water

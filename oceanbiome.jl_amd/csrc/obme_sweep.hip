@@ -29,12 +29,9 @@ LaneKernel<FT> lane_kernel(int mode, bool uniform, bool whole, bool forms, int s
                                     : k_column_lane<MODEL, CARB, FT, TILE_STAGE, false, -1, 0, true, OBME_CENTERED2>;
     }
     if (mode == TILE_PAR) {
-        if constexpr (sizeof(FT) == 8) {
-            if (whole && uniform) return k_column_lane<MODEL, CARB, FT, TILE_PAR, true, -1, 0, false>;
-            return uniform ? k_column_lane<MODEL, CARB, FT, TILE_PAR, true>
-                           : k_column_lane<MODEL, CARB, FT, TILE_PAR, false>;
-        }
-        return nullptr;
+        if (whole && uniform) return k_column_lane<MODEL, CARB, FT, TILE_PAR, true, -1, 0, false>;
+        return uniform ? k_column_lane<MODEL, CARB, FT, TILE_PAR, true>
+                       : k_column_lane<MODEL, CARB, FT, TILE_PAR, false>;
     }
     if (mode == TILE_TENDENCY) {
         if (scheme == OBME_WENO5) return k_column_lane<MODEL, CARB, FT, TILE_TENDENCY, false, -1, 0, true, OBME_WENO5>;
