@@ -16,12 +16,13 @@
 //    WAVE_MAX_STEPS steps of a launch (T, S and the light at the surface are
 //    given, columns are independent): each tracer is read and written once per
 //    launch.  Between steps the state is rounded as a store and a load would.
-// What it measured (us per call, the sweep of the columns | this): NPZD 160 x 32
-// FP64, one step 161 | 10.5; LOBSTER + DIC/Alk with the CO2 flux, FP32
-// 512 x 512 x 64, ten steps 2733 | 1828 (150 us of a step, 3.0 cycles of a wave
-// per vector instruction: issue-bound), FP64 256 x 256 x 64, four steps 1158 |
-// 644; WENO5 256 x 256 x 64, four steps 3491 (three launches a step) | 420;
-// scaling, CO2 flux and sediment 240 x 180 x 50, four steps 1786 | 364.
+// What it measured (us per call, the sweep of the columns, one launch a step |
+// this): NPZD 160 x 32 FP64, one step 161 | 10.5; LOBSTER + DIC/Alk with the CO2
+// flux, FP32 512 x 512 x 64, ten steps 2733 | 1755 (3.9 cycles of a SIMD per
+// vector instruction: issue-bound), FP64 256 x 256 x 64, four steps 1158 | 624;
+// WENO5 256 x 256 x 64, four steps 3491 (three launches a step) | 410; scaling,
+// CO2 flux and sediment 240 x 180 x 50, four steps 1786 | 365.  (Where the
+// sweep is the faster: wave_columns in obme_api.hip.)
 //
 // Loads and stores go through LDS: a workgroup moves its C = NW cpw columns
 // (neighbours in the flattened (i, j) order) level by level, C values per run,
@@ -34,7 +35,7 @@ namespace obme {
 
 // The model's default formulations (fm_code): LOBSTER Mondo light,
 // quadratic mortality and grazing; NPZD analytical light, linear
-// mortality, quadratic grazing, Q10 on.  FP32 kernels are compiled for these
+// mortality, quadratic grazing, Q10 on.  The kernels are compiled for these
 // with the choices folded in.
 template <int MODEL>
 constexpr int default_fm()
