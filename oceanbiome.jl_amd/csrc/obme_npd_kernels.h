@@ -233,8 +233,9 @@ enum { LEV_ZC = 0, LEV_UP, LEV_DN, LEV_INVDZ, LEV_WR, LEV_WB, LEV_COUNT };
 // of the red and blue bands, formed in FP64.
 
 // FP32: the rows of `light`, in powers of 2 per unit of the band's chlorophyll
-// power (and times what the rounding of cr or cb took from the power): the attenuation from the face above a level to its centre, and the
-// whole of its cell's (from its centre up and down; the bottom level: above).
+// power (and times what the rounding of cr or cb took from the power): the
+// attenuation from the face above a level to its centre, and the whole of its
+// cell's (from its centre up and down; the bottom level: above).
 enum { LIGHT_ABOVE_R = 0, LIGHT_ABOVE_B, LIGHT_WHOLE_R, LIGHT_WHOLE_B, LIGHT_COUNT };
 
 // What a launch does: the fused RK3 step, the tendencies (hook), the PAR (hook;
